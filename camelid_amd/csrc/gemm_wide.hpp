@@ -1,0 +1,482 @@
+// The wide matrix-core kernel: matmul of a K-quant weight with batches of more than 32 tokens
+// (prefill), and of the expert groups of a routed layer.  One workgroup per (block of weight rows,
+// column of up to 128 tokens); gemm_q6k_wide.hip supplies the format.
+//
+// A wave owns ONE 16-row tile and all tokens of its workgroup's column: what a super-block of
+// weights costs to unpack into int8 operands is paid once for up to eight token groups of 16.
+//
+// Everything a step reads -- the super-block of weights of every wave's tile, the activation slab
+// (256 values of every token of the column), now and then the activation scales -- goes from memory
+// to LDS without passing through registers (global_load_lds).  A lane's register loads of a weight
+// tile would touch 16 rows per instruction and keep the address unit busy for 31 - 39 cycles each,
+// more than the bytes take; here every request reads whole lines.  LDS is written at consecutive addresses, 16
+// bytes per lane, so bank conflicts are avoided by what each lane FETCHES: 16-byte slot p of
+// token t holds piece p ^ (t % 16) of its 256 values (the weights likewise).  A reader applies the
+// same exclusive-or.
+//
+// Results are the matvec's bits: the exact integers of a super-block, then its f32 steps, in order;
+// where the matvec cuts K for a weight shape the same parts are summed left to right here, on KS = 2
+// groups of waves (each walking half of the parts) or inside the lane (SPLIT).
+#pragma once
+
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <string>
+
+#include "cml_device.hpp"
+#include "cml_host.hpp"
+
+#pragma clang fp contract(off)
+
+namespace cml {
+
+typedef int v4i_w __attribute__((ext_vector_type(4)));
+typedef float v4f_w __attribute__((ext_vector_type(4)));
+typedef _Float16 v4h_w __attribute__((ext_vector_type(4)));
+
+// One wave's 1 KB: lane l's 16 bytes at base + off (off per lane) to LDS byte lds_byte + 16 * l (lds_byte wave-uniform).
+// Written as assembly because the compiler, which cannot tell which LDS bytes such a load will
+// write, puts a wait for all of them in front of every later LDS read; here the caller waits
+// (wide_wait) where the data is first needed.  s_nop: one wait state between a scalar write of m0
+// and an instruction that addresses LDS through it.
+__device__ __forceinline__ void wide_dma16(uint32_t lds_byte, const void *base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte), "v"(off), "s"(base) : "memory", "m0");
+}
+// The same with 4 bytes per lane.
+__device__ __forceinline__ void wide_dma4(uint32_t lds_byte, const void *base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_byte), "v"(off), "s"(base) : "memory", "m0");
+}
+// Waits until at most OUT of the wave's vector-memory operations are outstanding (loads complete in order).
+template <int OUT>
+__device__ __forceinline__ void wide_wait() {
+    static_assert(OUT < 64, "six bits");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(OUT) : "memory");
+}
+// Workgroup barrier after this wave's LDS operations (__syncthreads would also wait for every load in flight).
+__device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// LDS byte address of a shared-memory pointer.
+__device__ __forceinline__ uint32_t lds_address(const void *p) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void *)p));
+}
+
+// Workgroup id -> (row block, token column).  Consecutive ids go to the eight XCDs in turn; the columns of one row
+// block are given to ONE XCD, one after the other, so that its rows of the weight come through that XCD's L2 once.
+// The grid is padded to whole rounds of eight row blocks: row blocks past the end return false.
+__device__ __forceinline__ bool wide_block(int id, int n_row_blocks, int n_cols, int &row_block, int &col) {
+    const int j = id >> 3, r = j / n_cols;
+    row_block = r * 8 + (id & 7);
+    col = j - r * n_cols;
+    return row_block < n_row_blocks;
+}
+inline unsigned wide_grid(int64_t n_row_blocks, int64_t n_cols) { return static_cast<unsigned>((n_row_blocks + 7) / 8 * 8 * n_cols); }
+
+template <class F>
+struct WideArgs {
+    typename F::Weight w;
+    int rows, n_sb;     // rows of one band; super-blocks per row
+    int row_skip;       // leading rows of the first tile that precede this weight view (0..15)
+    int n_tiles;        // 16-row tiles of one band
+    int n_row_blocks;   // of both weights of a pair launch
+    int n_cols;         // token columns
+    int ksplit;         // association to reproduce (the matvec kernel's K cut)
+    const int8_t *q;    // [n_tokens][n_sb*256]
+    const float *yd;    // [n_tokens][n_sb]
+    float *out;         // [n_tokens][rows]
+    int n_tokens;       // plain: activation rows; grouped: the most assignments one group can hold
+    // Grouped call (mixture of experts): blockIdx.y -> group e (through group_ids when set; -1 = unused slot), which owns
+    // the weight band of rows [e*rows, (e+1)*rows) and the assignments [group_offsets[e], group_offsets[e+1]); assignment
+    // j reads activation row group_rows[j] (j itself when null) and writes output row j.
+    const int32_t *group_offsets;
+    const int32_t *group_rows;
+    const int32_t *group_ids;
+    // Pair launch (grouped calls): a second stacked weight of the same shape against the same activations, written to out2;
+    // its row blocks follow the first's.
+    typename F::Weight w2;
+    float *out2;
+};
+
+// LDS layout of one workgroup.
+template <class F, int G, int WAVES, int KS>
+struct WideLds {
+    static constexpr int NTOK = 16 * G;
+    static constexpr int kSlab = NTOK * 256;                   // one activation slab, pieces exclusive-ored
+    static constexpr int kRuns = F::kRunSums ? NTOK * 32 : 0;  // the sums of its 16-value runs, f16
+    static constexpr int kYd = (NTOK + 63) / 64 * 256;         // activation scales of one step
+    // weights: one super-block of every wave's tile, two steps ahead where that fits
+    static constexpr int kW = WAVES * F::kTileBytes;
+    static constexpr int kBase = 2 * KS * (kSlab + kRuns + kYd);
+    // (two workgroups per compute unit before two steps ahead)
+    static constexpr int kHalf = 80 * 1024;
+    static constexpr int WS = kBase + 2 * kW <= kHalf ? 2 : kBase + kW <= kHalf ? 1 : kBase + 2 * kW <= 2 * kHalf ? 2 : 1;
+    static constexpr int kTotal = kBase + WS * kW;
+};
+
+// F: the weight format.  G: token groups of 16 per column.  WAVES: waves per workgroup, WAVES / KS row tiles.
+// KS: groups of waves the K parts are shared over (1 or 2).  SPLIT: K parts are closed inside the lane.
+// GROUPED: expert groups (token groups past a group's last assignment are skipped, rows are gathered).
+template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED>
+__global__ __launch_bounds__(64 * WAVES, 2) void gemm_wide_kernel(WideArgs<F> a) {
+    typedef WideLds<F, G, WAVES, KS> L;
+    constexpr int NTOK = L::NTOK, RT = WAVES / KS, WS = L::WS;
+    constexpr int kThreads = 64 * WAVES, kRowsPass = kThreads / 16;        // tokens fetched per pass of the workgroup
+    constexpr int kPer = (NTOK + kRowsPass - 1) / kRowsPass;               // passes per slab
+    static_assert(KS == 1 || KS == 2, "K parts");
+    extern __shared__ uint4 smem[];
+    uint8_t *slabs = reinterpret_cast<uint8_t *>(smem);                      // [2][KS][NTOK][256]
+    uint8_t *runs = slabs + 2 * KS * L::kSlab;                               // [2][KS][NTOK][16] f16
+    constexpr int kYdAt = 2 * KS * (L::kSlab + L::kRuns);
+    const float *yds = reinterpret_cast<const float *>(slabs + kYdAt);       // [2][KS][NTOK rounded up to 64]
+    constexpr int kWAt = kYdAt + 2 * KS * L::kYd;
+    const uint8_t *wbuf = slabs + kWAt;                                      // [WS][WAVES][kTileBytes]
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int n_sb = a.n_sb;
+    const int n = lane & 15, kq = lane >> 4;
+    int row_block, col;
+    if (!wide_block(blockIdx.x, a.n_row_blocks, a.n_cols, row_block, col)) return;
+    const int64_t band = GROUPED ? (a.group_ids ? a.group_ids[blockIdx.y] : static_cast<int>(blockIdx.y)) : 0;
+    if (band < 0) return;
+    const int a0 = GROUPED ? a.group_offsets[band] : 0;
+    const int n_assign = GROUPED ? a.group_offsets[band + 1] - a0 : a.n_tokens;
+    const int tok0 = col * NTOK;
+    if (tok0 >= n_assign) return;  // the whole workgroup leaves
+    const int n_here = min(NTOK, n_assign - tok0);
+    const int n_blk = (a.n_tiles + RT - 1) / RT;
+    const bool second = GROUPED && row_block >= n_blk;
+    const int ks = KS == 2 ? wave / RT : 0;
+    const int tile = (row_block - (second ? n_blk : 0)) * RT + (KS == 2 ? wave - ks * RT : wave);
+    // this wave group's part of K
+    const int k_mid = KS == 2 ? (a.ksplit / 2) * n_sb / a.ksplit : n_sb;
+    const int s_begin = ks ? k_mid : 0, n_loc = ks ? n_sb - k_mid : k_mid;
+    const int n_max = KS == 2 ? max(k_mid, n_sb - k_mid) : n_sb;
+
+    auto act_row = [&](int t) __attribute__((always_inline)) -> uint32_t {  // (tokens past the end repeat the last one)
+        const int j = min(t, n_here - 1);
+        return static_cast<uint32_t>(GROUPED ? (a.group_rows ? a.group_rows[a0 + tok0 + j] : a0 + tok0 + j) : j);
+    };
+    const uint32_t lds0 = lds_address(smem);
+    // Activation: thread tid fetches slot tid % 16 of tokens tid / 16 + kRowsPass * k; a wave whose tokens lie past the column does not fetch.
+    const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
+    const uint32_t row_bytes = n_sb * 256u;
+    const int8_t *q_base = a.q + (GROUPED ? 0 : static_cast<int64_t>(tok0) * row_bytes);
+    uint32_t src[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) src[k] = act_row(t16 + kRowsPass * k) * row_bytes + piece * 16;
+    auto fetch = [&](int loc, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kp = 0; kp < KS; kp++) {
+            const int sb = min((kp ? k_mid : 0) + loc, n_sb - 1);
+#pragma unroll
+            for (int k = 0; k < kPer; k++)
+                if ((kPer * kRowsPass == NTOK || 4 * wave + kRowsPass * k < NTOK) && (!GROUPED || 4 * wave + kRowsPass * k < n_here))
+                    wide_dma16(lds0 + (buf * KS + kp) * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + sb * 256, src[k]);
+        }
+    };
+    // Scales: wave w of the first KS * NTOK / 64 fetches those of tokens 64 (w / KS) + lane for part w % KS.
+    const bool yd_wave = wave < KS * (L::kYd / 256);
+    const int ykp = wave % KS, yt = wave / KS * 64;
+    const float *yd_base = a.yd + (GROUPED ? 0 : static_cast<int64_t>(tok0) * n_sb);
+    const uint32_t yd_src = act_row(yt + lane) * n_sb * 4u;
+    auto fetch_yd = [&](int loc, int buf) __attribute__((always_inline)) {
+        if (yd_wave) wide_dma4(lds0 + kYdAt + (buf * KS + ykp) * L::kYd + yt * 4, yd_base + min((ykp ? k_mid : 0) + loc, n_sb - 1), yd_src);
+    };
+    // What is derived from a slab: after its wait a lane may read what it has fetched itself.
+    auto finish = [&](int buf) __attribute__((always_inline)) {
+        if constexpr (F::kRunSums) {
+#pragma unroll
+            for (int kp = 0; kp < KS; kp++)
+#pragma unroll
+                for (int k = 0; k < kPer; k++)
+                    if ((kPer * kRowsPass == NTOK || 4 * wave + kRowsPass * k < NTOK) && (!GROUPED || 4 * wave + kRowsPass * k < n_here)) {
+                        const uint4 v = *reinterpret_cast<const uint4 *>(slabs + (buf * KS + kp) * L::kSlab + (tid + kThreads * k) * 16);
+                        *reinterpret_cast<_Float16 *>(runs + (buf * KS + kp) * L::kRuns + (t16 + kRowsPass * k) * 32 + piece * 2) =
+                            static_cast<_Float16>(static_cast<float>(bytesum16(v)));
+                    }
+        }
+    };
+
+    F fmt(second ? a.w2 : a.w, band, a.rows, min(tile, a.n_tiles - 1), lane);
+    const uint32_t w_lds = lds0 + kWAt + wave * F::kTileBytes;
+    const uint8_t *w_mine = wbuf + wave * F::kTileBytes;
+    auto fetch_w = [&](int loc, int slot) __attribute__((always_inline)) { fmt.fetch(w_lds + slot * L::kW, min(s_begin + loc, n_sb - 1)); };
+
+    // A operand of step c: piece (lane's) ^ (step's) of token n
+    uint32_t a_addr[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) a_addr[c] = n * 256 + ((F::lane_piece(kq) ^ n ^ F::step_piece(c)) << 4);
+
+    fetch_yd(0, 0);
+    fetch(0, 0);
+    fetch_w(0, 0);
+    if constexpr (WS == 2) fetch_w(1, 1);
+    typename F::Raw raw;
+    wide_wait<(WS - 1) * F::kFetches>();
+    fmt.read(raw, w_mine, s_begin);
+    finish(0);
+    wide_barrier();
+
+    float acc[G][4], total[SPLIT ? G : 1][4];
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[g][j] = 0.0f;
+    // K parts closed inside the lane: of the whole row, or of this wave group's half of the parts
+    const int part0 = ks ? a.ksplit / 2 : 0;
+    int part = 0;
+    int next_cut = SPLIT ? (part0 + 1) * n_sb / a.ksplit : 0;
+
+    auto step = [&](int loc, int buf) __attribute__((always_inline)) {
+        if constexpr (SPLIT) {
+            if (s_begin + loc == next_cut && loc < n_loc) {  // the matvec kernel's K-split point: close the partial chain
+#pragma unroll
+                for (int g = 0; g < G; g++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        total[g][j] = part == 0 ? acc[g][j] : total[g][j] + acc[g][j];
+                        acc[g][j] = 0.0f;
+                    }
+                part++;
+                next_cut = (part0 + part + 1) * n_sb / a.ksplit;
+            }
+        }
+        // Requests: the next slab (and scales), then weights WS steps ahead, which alone may be outstanding at the end of the step.
+        // (Past the end the last super-block is fetched again: the number of requests in flight stays the same.)
+        fetch_yd(loc + 1, buf ^ 1);
+        fetch(loc + 1, buf ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        fmt.unpack(raw);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_w(loc + WS, WS == 2 ? buf : 0);  // (its slot was read into registers a step ago)
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t *slab = slabs + (buf * KS + ks) * L::kSlab;
+        const uint8_t *run = runs + (buf * KS + ks) * L::kRuns + n * 32 + kq * 8;
+        const float *ydp = yds + (buf * KS + ks) * (L::kYd / 4) + 4 * kq;
+        if (KS == 1 || loc < n_loc) {
+            // Software pipeline over the token groups: while the matrix cores work on group g, the operands of group g + 1
+            // are read from LDS and the f32 steps of group g - 1 run.
+            v4i_w av[2][4];
+            v4h_w rs[2];
+            float4 yd4[3];
+            typename F::Sums sums[2];
+            auto read = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) av[g & 1][c] = *reinterpret_cast<const v4i_w *>(slab + a_addr[c] + g * 4096);
+                if constexpr (F::kRunSums) rs[g & 1] = *reinterpret_cast<const v4h_w *>(run + g * 512);
+                yd4[g % 3] = *reinterpret_cast<const float4 *>(ydp + g * 16);
+            };
+            auto chain = [&](int g) __attribute__((always_inline)) {
+                const float yv[4] = {yd4[g % 3].x, yd4[g % 3].y, yd4[g % 3].z, yd4[g % 3].w};
+                fmt.chain(sums[g & 1], yv, acc[g]);
+                // (left alone, the compiler sinks the chains of all steps to the store and keeps every operand alive)
+#pragma unroll
+                for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[g][j]));
+            };
+            read(0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                if (!GROUPED || 16 * g < n_here) {
+                    if (g + 1 < G) read(g + 1);
+                    fmt.contract(av[g & 1], rs[g & 1], sums[g & 1]);
+                    if (g > 0) chain(g - 1);
+                    __builtin_amdgcn_sched_group_barrier(0x100, F::kRunSums ? 6 : 5, 0);
+#pragma unroll
+                    for (int m = 0; m < F::kMfma; m++) {
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, F::kChainPerMfma, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (g == G - 1 || (GROUPED && 16 * (g + 1) >= n_here)) chain(g);
+                }
+            }
+        }
+        wide_wait<(WS - 1) * F::kFetches>();
+        fmt.read(raw, w_mine + (WS == 2 ? (buf ^ 1) * L::kW : 0), min(s_begin + loc + 1, n_sb - 1));
+        finish(buf ^ 1);
+        wide_barrier();
+    };
+    // (two steps per round: buffer addresses are known at compile time)
+    int loc = 0;
+    for (; loc + 2 <= n_max; loc += 2) {
+        step(loc, 0);
+        step(loc + 1, 1);
+    }
+    if (loc < n_max) step(loc, 0);
+    wide_wait<0>();  // (nothing may still be on its way into LDS that is reused or given back)
+
+    if constexpr (KS == 2) {
+        // The second wave group's partial chains go to the first, which adds them in order (all slabs are free here:
+        // every wave has passed the last step's barrier and its own wait).
+        static_assert(KS * L::kSlab >= RT * G * 4 * 64 * 4, "partial chains fit a slab");
+        wide_barrier();
+        float *red = reinterpret_cast<float *>(slabs) + (wave - ks * RT) * (G * 4 * 64) + lane;
+        float *red2 = reinterpret_cast<float *>(slabs + KS * L::kSlab) + (wave - ks * RT) * (G * 4 * 64) + lane;
+        if (ks == 1) {
+#pragma unroll
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if constexpr (SPLIT) {
+                        red2[(g * 4 + j) * 64] = acc[g][j];
+                        red[(g * 4 + j) * 64] = total[g][j];
+                    } else {
+                        red[(g * 4 + j) * 64] = acc[g][j];
+                    }
+                }
+        }
+        wide_barrier();
+        if (ks == 1) return;
+#pragma unroll
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float v = acc[g][j];
+                if constexpr (SPLIT) v = total[g][j] + v;
+                v = v + red[(g * 4 + j) * 64];
+                if constexpr (SPLIT) v = v + red2[(g * 4 + j) * 64];
+                acc[g][j] = v;
+            }
+    }
+    const int row = tile * 16 + n - a.row_skip;
+    if (tile >= a.n_tiles || row < 0 || row >= a.rows) return;
+    float *out = (second ? a.out2 : a.out) + static_cast<int64_t>(a0 + tok0) * a.rows + row;
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int t = 16 * g + 4 * kq + j;
+            float v = acc[g][j];
+            if constexpr (SPLIT && KS == 1) v = part == 0 ? v : total[g][j] + v;
+            if (t < n_here) out[static_cast<int64_t>(t) * a.rows] = v;
+        }
+}
+
+template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED>
+static int launch_wide(WideArgs<F> ka, int slots, hipStream_t st) {
+    typedef WideLds<F, G, WAVES, KS> L;
+    static_assert(L::kTotal <= 160 * 1024, "LDS of a compute unit");
+    constexpr int RT = WAVES / KS;
+    ka.n_tiles = (ka.rows + ka.row_skip + 15) / 16;
+    ka.n_row_blocks = (ka.n_tiles + RT - 1) / RT * (ka.out2 ? 2 : 1);
+    ka.n_cols = (ka.n_tokens + L::NTOK - 1) / L::NTOK;
+    static std::atomic<bool> raised{false};  // per instantiation: allow more than 64 KB of dynamic LDS once
+    if (!raised.load(std::memory_order_acquire)) {
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wide_kernel<F, G, WAVES, KS, SPLIT, GROUPED>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        raised.store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL((gemm_wide_kernel<F, G, WAVES, KS, SPLIT, GROUPED>), dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * WAVES), L::kTotal, st, ka);
+    // "<format>.mfma.wide.g<token groups>w<waves>[.ksplit2][.serial_split][.grouped]"
+    CML_COUNT_LAUNCH(std::string(F::kName) + ".mfma.wide.g" + std::to_string(G) + "w" + std::to_string(WAVES) + (KS == 2 ? ".ksplit2" : "") +
+                     (SPLIT ? ".serial_split" : "") + (GROUPED ? ".grouped" : ""));
+    CML_HIP_TRY(hipGetLastError());
+    return CML_OK;
+}
+
+// The shape of a launch: token groups per column, waves per workgroup, and how a K cut is walked.
+struct WideShape {
+    int g = 0, waves = 0, ks = 1;
+};
+
+// Estimated us of a launch (less a constant), fitted on MI355X to 1800 launches: Q4_K and Q6_K weights of six and five shapes with
+// the three K cuts, 24 to 512 tokens, every shape of the kernel.  A step costs a fixed latency -- more for workgroups of four
+// waves and for two wave groups in F's measure --, and for every wave on a SIMD the unpacking of a super-block and then 0.12 us per token
+// group.  `rounds`: workgroups over what is resident at once, between their average and the last round at full length.  The shape
+// with the lowest estimate was the fastest or within 1 % of it on average over those launches (28 % off at worst).
+template <class F>
+static float wide_cost(int64_t tiles, int groups, int n_sb, int ksplit, const WideShape &s, int lds) {
+    const int rt = s.waves / s.ks;
+    const int64_t wgs = (tiles + rt - 1) / rt * ((groups + s.g - 1) / s.g);
+    const int resident = std::min(160 * 1024 / lds, 8 / s.waves);  // (registers: two waves per SIMD)
+    const float per_cu = wgs / 256.0f, full = per_cu / resident;
+    const float rounds = full <= 1.0f ? 1.0f : 0.4f * full + 0.6f * std::ceil(full);
+    const float m = (per_cu > 1.0f ? std::min<float>(resident, std::ceil(per_cu)) : 1.0f) * s.waves / 4;  // waves per SIMD
+    const int mid = s.ks == 2 ? ksplit / 2 * n_sb / ksplit : 0, steps = std::max(mid, n_sb - mid);
+    const float step = F::kStepUs + (s.ks == 2 ? F::kTwoPartsUs : 0.0f) + (s.waves == 4 ? F::kFourWavesUs : 0.0f);
+    return rounds * steps * (step + m * (F::kUnpackUs + 0.12f * s.g));
+}
+
+template <class F, int G, int WAVES, int KS>
+static void wide_consider(int64_t tiles, int groups, int n_sb, int ksplit, WideShape &best, float &cost) {
+    typedef WideLds<F, G, WAVES, KS> L;
+    if constexpr (L::kTotal <= 160 * 1024) {
+        const WideShape s{G, WAVES, KS};
+        const float c = wide_cost<F>(tiles, groups, n_sb, ksplit, s, L::kTotal);
+        if (c < cost) {
+            cost = c;
+            best = s;
+        }
+    }
+}
+
+template <class F, int WAVES, int KS>
+static void wide_consider_g(int64_t tiles, int groups, int n_sb, int ksplit, WideShape &best, float &cost) {
+    wide_consider<F, 1, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+    wide_consider<F, 2, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+    wide_consider<F, 3, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+    wide_consider<F, 4, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+    wide_consider<F, 5, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+    wide_consider<F, 6, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+    wide_consider<F, 7, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+    wide_consider<F, 8, WAVES, KS>(tiles, groups, n_sb, ksplit, best, cost);
+}
+
+template <class F, int G, int WAVES, int KS>
+static int launch_wide_split(const WideArgs<F> &ka, hipStream_t st) {
+    if constexpr (WideLds<F, G, WAVES, KS>::kTotal <= 160 * 1024) {
+        const bool split = KS == 2 ? ka.ksplit > 2 : ka.ksplit > 1;
+        return split ? launch_wide<F, G, WAVES, KS, true, false>(ka, 1, st) : launch_wide<F, G, WAVES, KS, false, false>(ka, 1, st);
+    } else {
+        return fail(CML_ERR_UNSUPPORTED, "wide matrix-core kernel: no such shape");
+    }
+}
+
+template <class F, int WAVES, int KS>
+static int launch_wide_g(const WideArgs<F> &ka, int g, hipStream_t st) {
+    switch (g) {
+        case 1: return launch_wide_split<F, 1, WAVES, KS>(ka, st);
+        case 2: return launch_wide_split<F, 2, WAVES, KS>(ka, st);
+        case 3: return launch_wide_split<F, 3, WAVES, KS>(ka, st);
+        case 4: return launch_wide_split<F, 4, WAVES, KS>(ka, st);
+        case 5: return launch_wide_split<F, 5, WAVES, KS>(ka, st);
+        case 6: return launch_wide_split<F, 6, WAVES, KS>(ka, st);
+        case 7: return launch_wide_split<F, 7, WAVES, KS>(ka, st);
+        default: return launch_wide_split<F, 8, WAVES, KS>(ka, st);
+    }
+}
+
+template <class F>
+static int launch_wide_plain(const MatArgs &a, hipStream_t st) {
+    const cml_weight *w = a.w;
+    WideArgs<F> ka{};
+    ka.w = F::weight(w);
+    ka.rows = static_cast<int>(w->rows);
+    ka.row_skip = w->row_skip;
+    ka.n_sb = static_cast<int>(w->nb);
+    ka.ksplit = F::ksplit(w->rows, w->nb);
+    ka.q = a.q;
+    ka.yd = a.scales;
+    ka.out = a.out;
+    ka.n_tokens = static_cast<int>(a.n_tokens);
+    const int64_t tiles = (w->rows + w->row_skip + 15) / 16;
+    const int groups = (ka.n_tokens + 15) / 16;
+    WideShape s;
+    float cost = 1e30f;
+    const bool two = ka.ksplit == 2 || ka.ksplit == 4;  // (other cuts are closed inside the lane)
+    wide_consider_g<F, 4, 1>(tiles, groups, ka.n_sb, ka.ksplit, s, cost);
+    wide_consider_g<F, 8, 1>(tiles, groups, ka.n_sb, ka.ksplit, s, cost);
+    if (two) {
+        wide_consider_g<F, 4, 2>(tiles, groups, ka.n_sb, ka.ksplit, s, cost);
+        wide_consider_g<F, 8, 2>(tiles, groups, ka.n_sb, ka.ksplit, s, cost);
+    }
+    // (forced shapes: tests and measurements)
+    s.g = env_int("CAMELID_HIP_WIDE_GROUPS", s.g);
+    s.waves = env_int("CAMELID_HIP_WIDE_WAVES", s.waves);
+    s.ks = two ? env_int("CAMELID_HIP_WIDE_PARTS", s.ks) : 1;
+    if (s.ks == 2) return s.waves == 4 ? launch_wide_g<F, 4, 2>(ka, s.g, st) : launch_wide_g<F, 8, 2>(ka, s.g, st);
+    return s.waves == 4 ? launch_wide_g<F, 4, 1>(ka, s.g, st) : launch_wide_g<F, 8, 1>(ka, s.g, st);
+}
+
+}  // namespace cml

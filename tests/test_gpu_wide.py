@@ -1,0 +1,72 @@
+"""The wide matrix-core kernel (batches on Q6_K weights): every cell is the
+matvec's, bit for bit, in every launch shape, at the edges of its tiles, token columns and K parts."""
+import numpy as np
+import pytest
+
+import oracle
+from camelid_amd import binding as B
+from camelid_amd.binding import Weight
+from tests import gpu_util as G
+
+pytestmark = pytest.mark.gpu
+
+K_FORMATS = [("Q6_K", B.CML_Q6_K, "q6k")]
+SHAPES = [(g, waves) for g in (1, 2, 3, 4, 5, 6, 7, 8) for waves in (4, 8)]
+
+
+def activations(n: int, cols: int, seed: int):
+    x = np.random.default_rng(seed).standard_normal((n, cols)).astype(np.float32)
+    x[0] = 0.0
+    x[-1, :256] = -np.abs(x[-1, :256]).max() * 4  # a super-block at the negative extreme
+    return oracle.quantize_activation(B.CML_Q4_K, x)
+
+
+# rows below a tile, a tile, past one; one super-block per row; K cut two ways (even and uneven parts), four ways (even and uneven)
+@pytest.mark.parametrize("rows,cols", [(1, 256), (16, 768), (130, 1280), (300, 2048), (145, 13 * 256), (300, 4096), (100, 18 * 256)])
+@pytest.mark.parametrize("name,fmt,tag", K_FORMATS)
+def test_wide_cells_are_bitwise_the_gemv(name, fmt, tag, rows, cols):
+    wire = G.synth_weight(fmt, rows, cols, seed=rows + cols)
+    w = Weight.upload(fmt, rows, cols, wire)
+    for n in (3, 16, 17, 47, 130):
+        s, q = activations(n, cols, seed=n)
+        with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+            ref = G.gpu_gemm(w, s, q)
+        for g, waves in SHAPES:
+            if n < 16 * (g - 1) and n != 3:
+                continue
+            for parts in (1, 2):
+                if (name, g, waves, parts) == ("Q4_K", 8, 8, 2):
+                    continue  # does not fit a compute unit's LDS
+                G.say(f"wide {name} {rows}x{cols} n={n} groups={g} waves={waves} parts={parts}")
+                with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g, CAMELID_HIP_WIDE_WAVES=waves, CAMELID_HIP_WIDE_PARTS=parts,
+                           CAMELID_HIP_Q4K_MFMA_MIN_TOKENS=1, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), \
+                        G.engaged(rf"^{tag}\.mfma\.wide\.g{g}w{waves}(\.|$)", none=(r"\.dot\.",)):
+                    assert G.same_bits(G.gpu_gemm(w, s, q), ref)
+        with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_EXACT_ORDER=1, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), G.engaged(rf"^{tag}\.mfma\.wide\."):
+            got = G.gpu_gemm(w, s, q)
+        order = oracle.ORDER_PRIMARY if fmt == B.CML_Q4_K else oracle.ORDER_ALT  # the fused chains of the reference
+        assert G.same_bits(got, oracle.matmul_q(fmt, wire, cols, s, q, order=order, threads=8))
+
+
+@pytest.mark.parametrize("name,fmt,tag", K_FORMATS)
+def test_wide_on_a_row_band(name, fmt, tag):
+    """A view that starts and ends inside a tile, of rows with an odd number of super-blocks (Q6_K: block scales at odd halves of a word)."""
+    rows, cols, n = 200, 5 * 256, 70
+    w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=5))
+    s, q = activations(n, cols, seed=1)
+    G.say(f"wide {name} row band")
+    with G.env(CAMELID_HIP_MFMA_WIDE=2), G.engaged(rf"^{tag}\.mfma\.wide\."):
+        whole, band = G.gpu_gemm(w, s, q), G.gpu_gemm(w.slice(7, 150), s, q)
+    assert G.same_bits(band, whole[:, 7:157])
+
+
+@pytest.mark.parametrize("name,fmt,tag", K_FORMATS)
+def test_batches_of_more_than_32_tokens_take_the_wide_kernel(name, fmt, tag):
+    rows, cols, n = 2048, 1024, 65
+    w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=6))
+    x = np.random.default_rng(2).standard_normal((n, cols)).astype(np.float32)
+    G.say(f"wide {name} default dispatch")
+    with G.engaged(rf"^{tag}\.mfma\.wide\."):
+        got = G.gpu_matmul_f32(w, x)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        assert G.same_bits(got, G.gpu_matmul_f32(w, x))
