@@ -1127,6 +1127,19 @@ int launch_gemm_q4k_mfma(const MatArgs &a, hipStream_t st) {
     // workgroup columns (grid.y), each a pass over the weight.  The other shapes stay selectable
     // for tuning.
     const int shape = env_int("CAMELID_HIP_Q4K_MFMA_SHAPE", 0);
+    // The wide kernel.  Plain: more than 32 tokens (14336 x 4096 at 24 / 40 / 64 / 128 / 200 / 512 tokens, this kernel / wide: 13.1 / 15.7,
+    // 18.8 / 17.8, 19.3 / 17.8, 30 / 24, 54 / 36, 98 / 76 us; 4096 x 14336 at 24 / 64 / 200 / 512: 18.8 / 20.9, 28.4 / 27.5, 88 / 49, 185 / 82).
+    // Expert groups: more than 12 assignments each on average where the launch has the tiles to fill the chip with its larger workgroups, from 24 on where
+    // a second token column would read the weight again (layer of 8 experts, top-2, us: 4096 / 14336 at 32 / 48 / 64 / 128 tokens 162 / 176, 217 / 190,
+    // 205 / 197, 340 / 256; 2048 / 8192 at 64 tokens 92 / 75; 2048 / 2048 at 128 tokens 61 / 48; 1024 / 2048 at 100 tokens 35 / 34).
+    // (32-bit offsets reach the activation rows)
+    const int wide = env_int("CAMELID_HIP_MFMA_WIDE", 1);  // 0 = never, 1 = by shape, 2 = always
+    if (shape == 0 && wide) {
+        const int64_t slots = grouped ? ng / (a.w2 ? 2 : 1) : 1, tiles = static_cast<int64_t>(ka.rows / 16) * ng;
+        const bool pays = !grouped ? a.n_tokens > 32 : (tiles > 2048 && a.n_assign_total > 12 * slots) || (tiles > 1024 && a.n_assign_total >= 24 * slots);
+        const bool reach = !grouped || std::max(a.n_assign_total, a.n_tokens) * ka.n_sb * 256 < (int64_t{1} << 32);
+        if ((wide == 2 || pays) && reach) return launch_gemm_q4k_wide(a, st);
+    }
     // One column of up to 16 tokens against rows of up to 16 super-blocks that the shape policy
     // does not cut: two waves per row tile, one chain.
     if (!grouped && mfma_pair_serves(ka.rows, ka.n_sb, a.n_tokens)) return launch_mfma_pair<false>(ka, nullptr, st);

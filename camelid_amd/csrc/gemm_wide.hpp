@@ -1,6 +1,6 @@
 // The wide matrix-core kernel: matmul of a K-quant weight with batches of more than 32 tokens
 // (prefill), and of the expert groups of a routed layer.  One workgroup per (block of weight rows,
-// column of up to 128 tokens); gemm_q6k_wide.hip supplies the format.
+// column of up to 128 tokens); gemm_q6k_wide.hip and gemm_q4k_wide.hip supply the formats.
 //
 // A wave owns ONE 16-row tile and all tokens of its workgroup's column: what a super-block of
 // weights costs to unpack into int8 operands is paid once for up to eight token groups of 16.
@@ -79,7 +79,7 @@ struct WideArgs {
     int row_skip;       // leading rows of the first tile that precede this weight view (0..15)
     int n_tiles;        // 16-row tiles of one band
     int n_row_blocks;   // of both weights of a pair launch
-    int n_cols;         // token columns
+    int n_cols;         // token columns in the grid (expert groups: one, which walks them all)
     int ksplit;         // association to reproduce (the matvec kernel's K cut)
     const int8_t *q;    // [n_tokens][n_sb*256]
     const float *yd;    // [n_tokens][n_sb]
@@ -117,12 +117,12 @@ struct WideLds {
 // KS: groups of waves the K parts are shared over (1 or 2).  SPLIT: K parts are closed inside the lane.
 // GROUPED: expert groups (token groups past a group's last assignment are skipped, rows are gathered).
 template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED>
-__global__ __launch_bounds__(64 * WAVES, 2) void gemm_wide_kernel(WideArgs<F> a) {
+__global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2) void gemm_wide_kernel(WideArgs<F> a) {
     typedef WideLds<F, G, WAVES, KS> L;
     constexpr int NTOK = L::NTOK, RT = WAVES / KS, WS = L::WS;
     constexpr int kThreads = 64 * WAVES, kRowsPass = kThreads / 16;        // tokens fetched per pass of the workgroup
     constexpr int kPer = (NTOK + kRowsPass - 1) / kRowsPass;               // passes per slab
-    static_assert(KS == 1 || KS == 2, "K parts");
+    static_assert(KS == 1 || (KS == 2 && !GROUPED), "K parts");
     extern __shared__ uint4 smem[];
     uint8_t *slabs = reinterpret_cast<uint8_t *>(smem);                      // [2][KS][NTOK][256]
     uint8_t *runs = slabs + 2 * KS * L::kSlab;                               // [2][KS][NTOK][16] f16
@@ -141,217 +141,224 @@ __global__ __launch_bounds__(64 * WAVES, 2) void gemm_wide_kernel(WideArgs<F> a)
     if (band < 0) return;
     const int a0 = GROUPED ? a.group_offsets[band] : 0;
     const int n_assign = GROUPED ? a.group_offsets[band + 1] - a0 : a.n_tokens;
-    const int tok0 = col * NTOK;
-    if (tok0 >= n_assign) return;  // the whole workgroup leaves
-    const int n_here = min(NTOK, n_assign - tok0);
-    const int n_blk = (a.n_tiles + RT - 1) / RT;
-    const bool second = GROUPED && row_block >= n_blk;
-    const int ks = KS == 2 ? wave / RT : 0;
-    const int tile = (row_block - (second ? n_blk : 0)) * RT + (KS == 2 ? wave - ks * RT : wave);
-    // this wave group's part of K
-    const int k_mid = KS == 2 ? (a.ksplit / 2) * n_sb / a.ksplit : n_sb;
-    const int s_begin = ks ? k_mid : 0, n_loc = ks ? n_sb - k_mid : k_mid;
-    const int n_max = KS == 2 ? max(k_mid, n_sb - k_mid) : n_sb;
+    // Expert groups: one workgroup walks all columns of its group (workgroups of a column of their own would mostly find
+    // it empty, each after two dependent loads: with two columns 282 us per Mixtral-shaped layer of 64 tokens, 200 so).
+    for (;; col++) {
+        const int tok0 = col * NTOK;
+        if (tok0 >= n_assign) return;  // the whole workgroup leaves
+        const int n_here = min(NTOK, n_assign - tok0);
+        const int n_blk = (a.n_tiles + RT - 1) / RT;
+        const bool second = GROUPED && row_block >= n_blk;
+        const int ks = KS == 2 ? wave / RT : 0;
+        const int tile = (row_block - (second ? n_blk : 0)) * RT + (KS == 2 ? wave - ks * RT : wave);
+        // this wave group's part of K
+        const int k_mid = KS == 2 ? (a.ksplit / 2) * n_sb / a.ksplit : n_sb;
+        const int s_begin = ks ? k_mid : 0, n_loc = ks ? n_sb - k_mid : k_mid;
+        const int n_max = KS == 2 ? max(k_mid, n_sb - k_mid) : n_sb;
 
-    auto act_row = [&](int t) __attribute__((always_inline)) -> uint32_t {  // (tokens past the end repeat the last one)
-        const int j = min(t, n_here - 1);
-        return static_cast<uint32_t>(GROUPED ? (a.group_rows ? a.group_rows[a0 + tok0 + j] : a0 + tok0 + j) : j);
-    };
-    const uint32_t lds0 = lds_address(smem);
-    // Activation: thread tid fetches slot tid % 16 of tokens tid / 16 + kRowsPass * k; a wave whose tokens lie past the column does not fetch.
-    const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
-    const uint32_t row_bytes = n_sb * 256u;
-    const int8_t *q_base = a.q + (GROUPED ? 0 : static_cast<int64_t>(tok0) * row_bytes);
-    uint32_t src[kPer];
+        auto act_row = [&](int t) __attribute__((always_inline)) -> uint32_t {  // (tokens past the end repeat the last one)
+            const int j = min(t, n_here - 1);
+            return static_cast<uint32_t>(GROUPED ? (a.group_rows ? a.group_rows[a0 + tok0 + j] : a0 + tok0 + j) : j);
+        };
+        const uint32_t lds0 = lds_address(smem);
+        // Activation: thread tid fetches slot tid % 16 of tokens tid / 16 + kRowsPass * k; a wave whose tokens lie past the column does not fetch.
+        const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
+        const uint32_t row_bytes = n_sb * 256u;
+        const int8_t *q_base = a.q + (GROUPED ? 0 : static_cast<int64_t>(tok0) * row_bytes);
+        uint32_t src[kPer];
 #pragma unroll
-    for (int k = 0; k < kPer; k++) src[k] = act_row(t16 + kRowsPass * k) * row_bytes + piece * 16;
-    auto fetch = [&](int loc, int buf) __attribute__((always_inline)) {
+        for (int k = 0; k < kPer; k++) src[k] = act_row(t16 + kRowsPass * k) * row_bytes + piece * 16;
+        auto fetch = [&](int loc, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kp = 0; kp < KS; kp++) {
-            const int sb = min((kp ? k_mid : 0) + loc, n_sb - 1);
-#pragma unroll
-            for (int k = 0; k < kPer; k++)
-                if ((kPer * kRowsPass == NTOK || 4 * wave + kRowsPass * k < NTOK) && (!GROUPED || 4 * wave + kRowsPass * k < n_here))
-                    wide_dma16(lds0 + (buf * KS + kp) * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + sb * 256, src[k]);
-        }
-    };
-    // Scales: wave w of the first KS * NTOK / 64 fetches those of tokens 64 (w / KS) + lane for part w % KS.
-    const bool yd_wave = wave < KS * (L::kYd / 256);
-    const int ykp = wave % KS, yt = wave / KS * 64;
-    const float *yd_base = a.yd + (GROUPED ? 0 : static_cast<int64_t>(tok0) * n_sb);
-    const uint32_t yd_src = act_row(yt + lane) * n_sb * 4u;
-    auto fetch_yd = [&](int loc, int buf) __attribute__((always_inline)) {
-        if (yd_wave) wide_dma4(lds0 + kYdAt + (buf * KS + ykp) * L::kYd + yt * 4, yd_base + min((ykp ? k_mid : 0) + loc, n_sb - 1), yd_src);
-    };
-    // What is derived from a slab: after its wait a lane may read what it has fetched itself.
-    auto finish = [&](int buf) __attribute__((always_inline)) {
-        if constexpr (F::kRunSums) {
-#pragma unroll
-            for (int kp = 0; kp < KS; kp++)
+            for (int kp = 0; kp < KS; kp++) {
+                const int sb = min((kp ? k_mid : 0) + loc, n_sb - 1);
 #pragma unroll
                 for (int k = 0; k < kPer; k++)
-                    if ((kPer * kRowsPass == NTOK || 4 * wave + kRowsPass * k < NTOK) && (!GROUPED || 4 * wave + kRowsPass * k < n_here)) {
-                        const uint4 v = *reinterpret_cast<const uint4 *>(slabs + (buf * KS + kp) * L::kSlab + (tid + kThreads * k) * 16);
-                        *reinterpret_cast<_Float16 *>(runs + (buf * KS + kp) * L::kRuns + (t16 + kRowsPass * k) * 32 + piece * 2) =
-                            static_cast<_Float16>(static_cast<float>(bytesum16(v)));
+                    if ((kPer * kRowsPass == NTOK || 4 * wave + kRowsPass * k < NTOK) && (!GROUPED || 4 * wave + kRowsPass * k < n_here))
+                        wide_dma16(lds0 + (buf * KS + kp) * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + sb * 256, src[k]);
+            }
+        };
+        // Scales: wave w of the first KS * NTOK / 64 fetches those of tokens 64 (w / KS) + lane for part w % KS.
+        const bool yd_wave = wave < KS * (L::kYd / 256);
+        const int ykp = wave % KS, yt = wave / KS * 64;
+        const float *yd_base = a.yd + (GROUPED ? 0 : static_cast<int64_t>(tok0) * n_sb);
+        const uint32_t yd_src = act_row(yt + lane) * n_sb * 4u;
+        auto fetch_yd = [&](int loc, int buf) __attribute__((always_inline)) {
+            if (yd_wave) wide_dma4(lds0 + kYdAt + (buf * KS + ykp) * L::kYd + yt * 4, yd_base + min((ykp ? k_mid : 0) + loc, n_sb - 1), yd_src);
+        };
+        // What is derived from a slab: after its wait a lane may read what it has fetched itself.
+        auto finish = [&](int buf) __attribute__((always_inline)) {
+            if constexpr (F::kRunSums) {
+#pragma unroll
+                for (int kp = 0; kp < KS; kp++)
+#pragma unroll
+                    for (int k = 0; k < kPer; k++)
+                        if ((kPer * kRowsPass == NTOK || 4 * wave + kRowsPass * k < NTOK) && (!GROUPED || 4 * wave + kRowsPass * k < n_here)) {
+                            const uint4 v = *reinterpret_cast<const uint4 *>(slabs + (buf * KS + kp) * L::kSlab + (tid + kThreads * k) * 16);
+                            *reinterpret_cast<_Float16 *>(runs + (buf * KS + kp) * L::kRuns + (t16 + kRowsPass * k) * 32 + piece * 2) =
+                                static_cast<_Float16>(static_cast<float>(bytesum16(v)));
+                        }
+            }
+        };
+
+        F fmt(second ? a.w2 : a.w, band, a.rows, min(tile, a.n_tiles - 1), lane);
+        const uint32_t w_lds = lds0 + kWAt + wave * F::kTileBytes;
+        const uint8_t *w_mine = wbuf + wave * F::kTileBytes;
+        auto fetch_w = [&](int loc, int slot) __attribute__((always_inline)) { fmt.fetch(w_lds + slot * L::kW, min(s_begin + loc, n_sb - 1)); };
+
+        // A operand of step c: piece (lane's) ^ (step's) of token n
+        uint32_t a_addr[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) a_addr[c] = n * 256 + ((F::lane_piece(kq) ^ n ^ F::step_piece(c)) << 4);
+
+        fetch_yd(0, 0);
+        fetch(0, 0);
+        fetch_w(0, 0);
+        if constexpr (WS == 2) fetch_w(1, 1);
+        typename F::Raw raw;
+        wide_wait<(WS - 1) * F::kFetches>();
+        fmt.read(raw, w_mine, s_begin);
+        finish(0);
+        wide_barrier();
+
+        float acc[G][4], total[SPLIT ? G : 1][4];
+#pragma unroll
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[g][j] = 0.0f;
+        // K parts closed inside the lane: of the whole row, or of this wave group's half of the parts
+        const int part0 = ks ? a.ksplit / 2 : 0;
+        int part = 0;
+        int next_cut = SPLIT ? (part0 + 1) * n_sb / a.ksplit : 0;
+
+        auto step = [&](int loc, int buf) __attribute__((always_inline)) {
+            if constexpr (SPLIT) {
+                if (s_begin + loc == next_cut && loc < n_loc) {  // the matvec kernel's K-split point: close the partial chain
+#pragma unroll
+                    for (int g = 0; g < G; g++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            total[g][j] = part == 0 ? acc[g][j] : total[g][j] + acc[g][j];
+                            acc[g][j] = 0.0f;
+                        }
+                    part++;
+                    next_cut = (part0 + part + 1) * n_sb / a.ksplit;
+                }
+            }
+            // Requests: the next slab (and scales), then weights WS steps ahead, which alone may be outstanding at the end of the step.
+            // (Past the end the last super-block is fetched again: the number of requests in flight stays the same.)
+            fetch_yd(loc + 1, buf ^ 1);
+            fetch(loc + 1, buf ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+            fmt.unpack(raw);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_w(loc + WS, WS == 2 ? buf : 0);  // (its slot was read into registers a step ago)
+            __builtin_amdgcn_sched_barrier(0);
+            const uint8_t *slab = slabs + (buf * KS + ks) * L::kSlab;
+            const uint8_t *run = runs + (buf * KS + ks) * L::kRuns + n * 32 + kq * 8;
+            const float *ydp = yds + (buf * KS + ks) * (L::kYd / 4) + 4 * kq;
+            if (KS == 1 || loc < n_loc) {
+                // Software pipeline over the token groups: while the matrix cores work on group g, the operands of group g + 1
+                // are read from LDS and the f32 steps of group g - 1 run.
+                v4i_w av[2][4];
+                v4h_w rs[2];
+                float4 yd4[3];
+                typename F::Sums sums[2];
+                auto read = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int c = 0; c < 4; c++) av[g & 1][c] = *reinterpret_cast<const v4i_w *>(slab + a_addr[c] + g * 4096);
+                    if constexpr (F::kRunSums) rs[g & 1] = *reinterpret_cast<const v4h_w *>(run + g * 512);
+                    yd4[g % 3] = *reinterpret_cast<const float4 *>(ydp + g * 16);
+                };
+                auto chain = [&](int g) __attribute__((always_inline)) {
+                    const float yv[4] = {yd4[g % 3].x, yd4[g % 3].y, yd4[g % 3].z, yd4[g % 3].w};
+                    fmt.chain(sums[g & 1], yv, acc[g]);
+                    // (left alone, the compiler sinks the chains of all steps to the store and keeps every operand alive)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[g][j]));
+                };
+                read(0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    if (!GROUPED || 16 * g < n_here) {
+                        if (g + 1 < G) read(g + 1);
+                        fmt.contract(av[g & 1], rs[g & 1], sums[g & 1]);
+                        if (g > 0) chain(g - 1);
+                        __builtin_amdgcn_sched_group_barrier(0x100, F::kRunSums ? 6 : 5, 0);
+#pragma unroll
+                        for (int m = 0; m < F::kMfma; m++) {
+                            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x2, F::kChainPerMfma, 0);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (g == G - 1 || (GROUPED && 16 * (g + 1) >= n_here)) chain(g);
                     }
+                }
+            }
+            wide_wait<(WS - 1) * F::kFetches>();
+            fmt.read(raw, w_mine + (WS == 2 ? (buf ^ 1) * L::kW : 0), min(s_begin + loc + 1, n_sb - 1));
+            finish(buf ^ 1);
+            wide_barrier();
+        };
+        // (two steps per round: buffer addresses are known at compile time)
+        int loc = 0;
+        for (; loc + 2 <= n_max; loc += 2) {
+            step(loc, 0);
+            step(loc + 1, 1);
         }
-    };
+        if (loc < n_max) step(loc, 0);
+        wide_wait<0>();  // (nothing may still be on its way into LDS that is reused or given back)
 
-    F fmt(second ? a.w2 : a.w, band, a.rows, min(tile, a.n_tiles - 1), lane);
-    const uint32_t w_lds = lds0 + kWAt + wave * F::kTileBytes;
-    const uint8_t *w_mine = wbuf + wave * F::kTileBytes;
-    auto fetch_w = [&](int loc, int slot) __attribute__((always_inline)) { fmt.fetch(w_lds + slot * L::kW, min(s_begin + loc, n_sb - 1)); };
-
-    // A operand of step c: piece (lane's) ^ (step's) of token n
-    uint32_t a_addr[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) a_addr[c] = n * 256 + ((F::lane_piece(kq) ^ n ^ F::step_piece(c)) << 4);
-
-    fetch_yd(0, 0);
-    fetch(0, 0);
-    fetch_w(0, 0);
-    if constexpr (WS == 2) fetch_w(1, 1);
-    typename F::Raw raw;
-    wide_wait<(WS - 1) * F::kFetches>();
-    fmt.read(raw, w_mine, s_begin);
-    finish(0);
-    wide_barrier();
-
-    float acc[G][4], total[SPLIT ? G : 1][4];
-#pragma unroll
-    for (int g = 0; g < G; g++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[g][j] = 0.0f;
-    // K parts closed inside the lane: of the whole row, or of this wave group's half of the parts
-    const int part0 = ks ? a.ksplit / 2 : 0;
-    int part = 0;
-    int next_cut = SPLIT ? (part0 + 1) * n_sb / a.ksplit : 0;
-
-    auto step = [&](int loc, int buf) __attribute__((always_inline)) {
-        if constexpr (SPLIT) {
-            if (s_begin + loc == next_cut && loc < n_loc) {  // the matvec kernel's K-split point: close the partial chain
+        if constexpr (KS == 2) {
+            // The second wave group's partial chains go to the first, which adds them in order (all slabs are free here:
+            // every wave has passed the last step's barrier and its own wait).
+            static_assert(KS * L::kSlab >= RT * G * 4 * 64 * 4, "partial chains fit a slab");
+            wide_barrier();
+            float *red = reinterpret_cast<float *>(slabs) + (wave - ks * RT) * (G * 4 * 64) + lane;
+            float *red2 = reinterpret_cast<float *>(slabs + KS * L::kSlab) + (wave - ks * RT) * (G * 4 * 64) + lane;
+            if (ks == 1) {
 #pragma unroll
                 for (int g = 0; g < G; g++)
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
-                        total[g][j] = part == 0 ? acc[g][j] : total[g][j] + acc[g][j];
-                        acc[g][j] = 0.0f;
+                        if constexpr (SPLIT) {
+                            red2[(g * 4 + j) * 64] = acc[g][j];
+                            red[(g * 4 + j) * 64] = total[g][j];
+                        } else {
+                            red[(g * 4 + j) * 64] = acc[g][j];
+                        }
                     }
-                part++;
-                next_cut = (part0 + part + 1) * n_sb / a.ksplit;
             }
-        }
-        // Requests: the next slab (and scales), then weights WS steps ahead, which alone may be outstanding at the end of the step.
-        // (Past the end the last super-block is fetched again: the number of requests in flight stays the same.)
-        fetch_yd(loc + 1, buf ^ 1);
-        fetch(loc + 1, buf ^ 1);
-        __builtin_amdgcn_sched_barrier(0);
-        fmt.unpack(raw);
-        __builtin_amdgcn_sched_barrier(0);
-        fetch_w(loc + WS, WS == 2 ? buf : 0);  // (its slot was read into registers a step ago)
-        __builtin_amdgcn_sched_barrier(0);
-        const uint8_t *slab = slabs + (buf * KS + ks) * L::kSlab;
-        const uint8_t *run = runs + (buf * KS + ks) * L::kRuns + n * 32 + kq * 8;
-        const float *ydp = yds + (buf * KS + ks) * (L::kYd / 4) + 4 * kq;
-        if (KS == 1 || loc < n_loc) {
-            // Software pipeline over the token groups: while the matrix cores work on group g, the operands of group g + 1
-            // are read from LDS and the f32 steps of group g - 1 run.
-            v4i_w av[2][4];
-            v4h_w rs[2];
-            float4 yd4[3];
-            typename F::Sums sums[2];
-            auto read = [&](int g) __attribute__((always_inline)) {
-#pragma unroll
-                for (int c = 0; c < 4; c++) av[g & 1][c] = *reinterpret_cast<const v4i_w *>(slab + a_addr[c] + g * 4096);
-                if constexpr (F::kRunSums) rs[g & 1] = *reinterpret_cast<const v4h_w *>(run + g * 512);
-                yd4[g % 3] = *reinterpret_cast<const float4 *>(ydp + g * 16);
-            };
-            auto chain = [&](int g) __attribute__((always_inline)) {
-                const float yv[4] = {yd4[g % 3].x, yd4[g % 3].y, yd4[g % 3].z, yd4[g % 3].w};
-                fmt.chain(sums[g & 1], yv, acc[g]);
-                // (left alone, the compiler sinks the chains of all steps to the store and keeps every operand alive)
-#pragma unroll
-                for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[g][j]));
-            };
-            read(0);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-                if (!GROUPED || 16 * g < n_here) {
-                    if (g + 1 < G) read(g + 1);
-                    fmt.contract(av[g & 1], rs[g & 1], sums[g & 1]);
-                    if (g > 0) chain(g - 1);
-                    __builtin_amdgcn_sched_group_barrier(0x100, F::kRunSums ? 6 : 5, 0);
-#pragma unroll
-                    for (int m = 0; m < F::kMfma; m++) {
-                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                        __builtin_amdgcn_sched_group_barrier(0x2, F::kChainPerMfma, 0);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (g == G - 1 || (GROUPED && 16 * (g + 1) >= n_here)) chain(g);
-                }
-            }
-        }
-        wide_wait<(WS - 1) * F::kFetches>();
-        fmt.read(raw, w_mine + (WS == 2 ? (buf ^ 1) * L::kW : 0), min(s_begin + loc + 1, n_sb - 1));
-        finish(buf ^ 1);
-        wide_barrier();
-    };
-    // (two steps per round: buffer addresses are known at compile time)
-    int loc = 0;
-    for (; loc + 2 <= n_max; loc += 2) {
-        step(loc, 0);
-        step(loc + 1, 1);
-    }
-    if (loc < n_max) step(loc, 0);
-    wide_wait<0>();  // (nothing may still be on its way into LDS that is reused or given back)
-
-    if constexpr (KS == 2) {
-        // The second wave group's partial chains go to the first, which adds them in order (all slabs are free here:
-        // every wave has passed the last step's barrier and its own wait).
-        static_assert(KS * L::kSlab >= RT * G * 4 * 64 * 4, "partial chains fit a slab");
-        wide_barrier();
-        float *red = reinterpret_cast<float *>(slabs) + (wave - ks * RT) * (G * 4 * 64) + lane;
-        float *red2 = reinterpret_cast<float *>(slabs + KS * L::kSlab) + (wave - ks * RT) * (G * 4 * 64) + lane;
-        if (ks == 1) {
+            wide_barrier();
+            if (ks == 1) return;
 #pragma unroll
             for (int g = 0; g < G; g++)
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    if constexpr (SPLIT) {
-                        red2[(g * 4 + j) * 64] = acc[g][j];
-                        red[(g * 4 + j) * 64] = total[g][j];
-                    } else {
-                        red[(g * 4 + j) * 64] = acc[g][j];
-                    }
+                    float v = acc[g][j];
+                    if constexpr (SPLIT) v = total[g][j] + v;
+                    v = v + red[(g * 4 + j) * 64];
+                    if constexpr (SPLIT) v = v + red2[(g * 4 + j) * 64];
+                    acc[g][j] = v;
                 }
         }
-        wide_barrier();
-        if (ks == 1) return;
+        const int row = tile * 16 + n - a.row_skip;
+        if (tile < a.n_tiles && row >= 0 && row < a.rows) {
+            float *out = (second ? a.out2 : a.out) + static_cast<int64_t>(a0 + tok0) * a.rows + row;
 #pragma unroll
-        for (int g = 0; g < G; g++)
+            for (int g = 0; g < G; g++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float v = acc[g][j];
-                if constexpr (SPLIT) v = total[g][j] + v;
-                v = v + red[(g * 4 + j) * 64];
-                if constexpr (SPLIT) v = v + red2[(g * 4 + j) * 64];
-                acc[g][j] = v;
-            }
-    }
-    const int row = tile * 16 + n - a.row_skip;
-    if (tile >= a.n_tiles || row < 0 || row >= a.rows) return;
-    float *out = (second ? a.out2 : a.out) + static_cast<int64_t>(a0 + tok0) * a.rows + row;
-#pragma unroll
-    for (int g = 0; g < G; g++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int t = 16 * g + 4 * kq + j;
-            float v = acc[g][j];
-            if constexpr (SPLIT && KS == 1) v = part == 0 ? v : total[g][j] + v;
-            if (t < n_here) out[static_cast<int64_t>(t) * a.rows] = v;
+                for (int j = 0; j < 4; j++) {
+                    const int t = 16 * g + 4 * kq + j;
+                    float v = acc[g][j];
+                    if constexpr (SPLIT && KS == 1) v = part == 0 ? v : total[g][j] + v;
+                    if (t < n_here) out[static_cast<int64_t>(t) * a.rows] = v;
+                }
         }
+        if constexpr (!GROUPED) return;
+        wide_barrier();  // (every wave's requests have arrived: the next column may use the buffers)
+    }
 }
 
 template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED>
@@ -361,7 +368,7 @@ static int launch_wide(WideArgs<F> ka, int slots, hipStream_t st) {
     constexpr int RT = WAVES / KS;
     ka.n_tiles = (ka.rows + ka.row_skip + 15) / 16;
     ka.n_row_blocks = (ka.n_tiles + RT - 1) / RT * (ka.out2 ? 2 : 1);
-    ka.n_cols = (ka.n_tokens + L::NTOK - 1) / L::NTOK;
+    ka.n_cols = GROUPED ? 1 : (ka.n_tokens + L::NTOK - 1) / L::NTOK;
     static std::atomic<bool> raised{false};  // per instantiation: allow more than 64 KB of dynamic LDS once
     if (!raised.load(std::memory_order_acquire)) {
         CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wide_kernel<F, G, WAVES, KS, SPLIT, GROUPED>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
@@ -477,6 +484,42 @@ static int launch_wide_plain(const MatArgs &a, hipStream_t st) {
     s.ks = two ? env_int("CAMELID_HIP_WIDE_PARTS", s.ks) : 1;
     if (s.ks == 2) return s.waves == 4 ? launch_wide_g<F, 4, 2>(ka, s.g, st) : launch_wide_g<F, 8, 2>(ka, s.g, st);
     return s.waves == 4 ? launch_wide_g<F, 4, 1>(ka, s.g, st) : launch_wide_g<F, 8, 1>(ka, s.g, st);
+}
+
+// Expert groups: four waves up to 64 assignments (three workgroups per compute unit up to 48), eight beyond; token groups per column enough for nearly every group of a routing whose assignments fall evenly
+// (mean and one and a half deviations); a fuller group takes another column, groups of 16 past a group's last are skipped.
+template <class F, int G, int WAVES>
+static int launch_wide_grouped_split(const WideArgs<F> &ka, int slots, hipStream_t st) {
+    return ka.ksplit > 1 ? launch_wide<F, G, WAVES, 1, true, true>(ka, slots, st) : launch_wide<F, G, WAVES, 1, false, true>(ka, slots, st);
+}
+
+template <class F>
+static int launch_wide_grouped(const MatArgs &a, hipStream_t st) {
+    const cml_weight *w = a.w;
+    WideArgs<F> ka{};
+    ka.w = F::weight(w);
+    ka.rows = static_cast<int>(a.band_rows);
+    ka.n_sb = static_cast<int>(w->nb);
+    ka.ksplit = F::ksplit(ka.rows, w->nb);
+    ka.q = a.q;
+    ka.yd = a.scales;
+    ka.out = a.out;
+    ka.n_tokens = static_cast<int>(a.n_tokens);
+    ka.group_offsets = a.group_offsets;
+    ka.group_rows = a.group_rows;
+    ka.group_ids = a.group_ids;
+    if (a.w2) {
+        ka.w2 = F::weight(a.w2);
+        ka.out2 = a.out2;
+    }
+    const int slots = static_cast<int>(a.group_ids ? a.max_active : a.n_groups);
+    const float mean = static_cast<float>(a.n_assign_total) / std::max(1, slots);
+    int g = static_cast<int>(std::ceil(std::min<float>(mean + 1.5f * std::sqrt(mean), static_cast<float>(ka.n_tokens)) / 16.0f));
+    g = env_int("CAMELID_HIP_WIDE_GROUPS", g);
+    if (g <= 2) return launch_wide_grouped_split<F, 2, 4>(ka, slots, st);
+    if (g <= 3) return launch_wide_grouped_split<F, 3, 4>(ka, slots, st);
+    if (g <= 4) return launch_wide_grouped_split<F, 4, 4>(ka, slots, st);
+    return launch_wide_grouped_split<F, 8, 8>(ka, slots, st);
 }
 
 }  // namespace cml

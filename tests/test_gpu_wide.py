@@ -1,4 +1,4 @@
-"""The wide matrix-core kernel (batches on Q6_K weights): every cell is the
+"""The wide matrix-core kernels (batches and expert groups): every cell is the
 matvec's, bit for bit, in every launch shape, at the edges of its tiles, token columns and K parts."""
 import numpy as np
 import pytest
@@ -7,10 +7,11 @@ import oracle
 from camelid_amd import binding as B
 from camelid_amd.binding import Weight
 from tests import gpu_util as G
+from tests.test_gpu_moe import gpu_moe, gpu_route
 
 pytestmark = pytest.mark.gpu
 
-K_FORMATS = [("Q6_K", B.CML_Q6_K, "q6k")]
+K_FORMATS = [("Q4_K", B.CML_Q4_K, "q4k"), ("Q6_K", B.CML_Q6_K, "q6k")]
 SHAPES = [(g, waves) for g in (1, 2, 3, 4, 5, 6, 7, 8) for waves in (4, 8)]
 
 
@@ -70,3 +71,26 @@ def test_batches_of_more_than_32_tokens_take_the_wide_kernel(name, fmt, tag):
         got = G.gpu_matmul_f32(w, x)
     with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
         assert G.same_bits(got, G.gpu_matmul_f32(w, x))
+
+
+def experts(E, hidden, ff, seed):
+    return [Weight.upload(B.CML_Q4_K, E * r, c, G.synth_weight(B.CML_Q4_K, E * r, c, seed=seed + i)) for i, (r, c) in enumerate([(ff, hidden), (ff, hidden), (hidden, ff)])]
+
+
+# gate and up in one launch, gathered rows, a group without assignments, one past a column, K cut inside the lane (down)
+@pytest.mark.parametrize("E,k,hidden,ff,T", [(8, 2, 1024, 4096, 100), (4, 1, 256, 768, 5), (3, 3, 512, 512, 17), (6, 2, 4096, 1280, 130)])
+def test_wide_expert_groups_are_bitwise_the_narrow_ones(E, k, hidden, ff, T):
+    w = experts(E, hidden, ff, E + T)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    logits[:, 0] += 1.0  # a crowded expert, one without assignments
+    logits[:, E - 1] -= 50.0 * (E > k)
+    idx, weight, _, _ = gpu_route(logits, k)
+    run = lambda: gpu_moe(*w, E, k, idx, weight, x)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        ref = run()
+    for g in (1, 3, 4, 8):
+        G.say(f"wide experts E={E} k={k} {hidden}/{ff} T={T} groups={g}")
+        with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g), G.engaged(r"^q4k\.mfma\.wide\..*grouped"):
+            assert G.same_bits(run(), ref)
