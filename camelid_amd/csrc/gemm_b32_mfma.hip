@@ -609,7 +609,10 @@ static int launch_b32_mfma_p(const B32MfmaArgs &ka, int n_groups, hipStream_t st
 }
 
 template <int FMT>
-static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, int n_groups, bool grouped, hipStream_t st) {
+static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_groups, bool grouped, hipStream_t st) {
+    const int wide = env_int("CAMELID_HIP_MFMA_WIDE", 1);  // 0 = never, 1 = by shape, 2 = always
+    const bool can_wide = wide && !grouped && reinterpret_cast<uintptr_t>(ka.xs) % 16 == 0 && env_int("CAMELID_HIP_B32_MFMA_SHAPE", 0) == 0;
+    if (can_wide && wide == 2) return launch_gemm_b32_wide(a, st);
     // Workgroup shape: token groups per wave x token blocks across waves.  Default: one wave per
     // row tile with 16 / 32 / 64 tokens; a matrix with fewer row tiles than the chip has SIMDs
     // spreads the tokens of a tile over 2 or 4 waves instead.
@@ -642,6 +645,11 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, int n_groups, bool grouped
             return launch_b32_mfma_kpar<FMT, 2, 2, 1>(ka, st);
         }
     }
+    // Plain calls: the wide kernel wherever several waves per row tile do not serve.  us per launch, the kernel below / wide, Q8_0: 14336 x 4096
+    // at 6 / 16 / 24 / 64 / 200 / 512 tokens 20.4 / 19.7, 20.5 / 19.8, 34.5 / 21.2, 67 / 24, 217 / 61, 434 / 115; 4096 x 14336 at 12 / 64 / 512
+    // 49 / 39, 73 / 39, 541 / 116; 11008 x 2048 at 6 / 16 10.6 / 8.4, 11.0 / 8.5; 32000 x 4096 at 16 35 / 32; 2048 x 2048 at 24 / 200 10.4 / 7.6, 19.3 / 10.
+    // Q4_0: 128256 x 3072 at 4 / 16 / 32 / 64 52.4 / 50.9, 57.7 / 51.5, 82 / 64, 156 / 101; 14336 x 4096 at 16 / 200 18.0 / 18.5, 200 / 62.
+    if (can_wide && (kpar != 0 || ka.n_tokens > 16)) return launch_gemm_b32_wide(a, st);
     switch (env_int("CAMELID_HIP_B32_MFMA_SHAPE", 0)) {
         case 1: return launch_b32_mfma_p<FMT, 1, 1>(ka, n_groups, st);   // 16 tokens, 1 wave per row tile
         case 2: return launch_b32_mfma_p<FMT, 2, 1>(ka, n_groups, st);   // 32 tokens, 1 wave per row tile
@@ -663,13 +671,14 @@ bool b32_mfma_usable(const cml_weight *w) {
            (reinterpret_cast<uintptr_t>(w->planes.p[1]) % 16 == 0) && (w->planes.row_stride[1] % 16 == 0);
 }
 
-// Batch size from which the matrix-core kernel beats the packed-dot kernel (which serves up to 8
-// tokens per pass over the weight).  Measured on MI355X: 8192x2048 Q8_0, 4 / 8 tokens: 7.0 / 10.0 us
-// packed dot against 10.9 us; 128256x3072 Q4_0: 62 / 105 us against 59 / 61 us.
+// Batch size from which the matrix cores beat the packed-dot kernel (which serves up to 8 tokens per pass over the weight).
+// us per launch at 4 / 8 tokens, packed dot against matrix cores: Q8_0 4096 x 14336 28 / 56 against 39, 14336 x 4096 20 / 27 against 20,
+// 11008 x 2048 8.2 / 12.4 against 8.4, 2048 x 2048 5.3 / 8.2 against 5.3; Q4_0 14336 x 4096 14 / 24 against 16 / 18, 5120 x 5120
+// 11 / 19 against 17.  Tall weights from 4 tokens: 128256 x 3072 Q4_0 62 / 105 against 51.
 int b32_mfma_min_tokens(int64_t rows) {
     const int forced = env_int("CAMELID_HIP_B32_MFMA_MIN_TOKENS", 0);
     if (forced > 0) return forced;
-    return (rows + 15) / 16 >= 2048 ? 4 : 9;  // 128256 x 3072 Q4_0, 4 tokens: 54.6 us against 61.8 us for the packed dot
+    return (rows + 15) / 16 >= 2048 ? 4 : 5;
 }
 
 // Q8_0 / Q4_0 matmul on the matrix cores: plain calls, or grouped by expert (mixture of experts).
@@ -693,8 +702,8 @@ int launch_gemm_b32_mfma(const MatArgs &a, hipStream_t st) {
     ka.group_rows = a.group_rows;
     ka.group_ids = a.group_ids;
     const int ng = grouped ? (a.group_ids ? a.max_active : a.n_groups) : 1;
-    if (w->fmt == CML_Q8_0) return launch_b32_mfma_fmt<CML_Q8_0>(ka, ng, grouped, st);
-    return launch_b32_mfma_fmt<CML_Q4_0>(ka, ng, grouped, st);
+    if (w->fmt == CML_Q8_0) return launch_b32_mfma_fmt<CML_Q8_0>(ka, a, ng, grouped, st);
+    return launch_b32_mfma_fmt<CML_Q4_0>(ka, a, ng, grouped, st);
 }
 
 }  // namespace cml

@@ -1,0 +1,372 @@
+// Q8_0 / Q4_0 x Q8_0 matmul for prefill batches on the int8 matrix cores (gfx950).
+//
+// Arithmetic: cell by cell that of the matvec kernels and of gemm_b32_mfma.hip: per 32-value block, in block order,
+//     isum = sum_j w_j * x_j  (exact i32),   acc = acc + ((float)isum * d_w) * d_x
+// so one v_mfma_i32_16x16x32_i8 per block and 16 x 16 cells, and an f32 step per block and cell: the vector
+// instructions bound this kernel (three of four cycles each per 64 cells and block: 14336 x 4096 x 200 tokens 29 us of issue, 61 measured).  Three
+// are the least: multiply, multiply, add, each rounded.  The conversion is left out: the matrix instruction
+// adds onto 0x4b400000, so that its result READ AS f32 is 12582912 + isum (|isum| <= 2^19), and
+//     fma(that, d_w, -12582912 * d_w)
+// is isum * d_w rounded once, the product (d_w has 11 significant bits, 1.5 * 2^23 * d_w is exact).  A slab
+// that holds a scale which is no finite number takes the subtraction instead (inf - inf).
+//
+// A wave owns 32 weight rows (two 16-row tiles) and all tokens of its workgroup's column, so that an activation
+// operand and the activation scales read from LDS serve two tiles; with one, LDS would carry as many cycles as the vector unit.
+// K is walked in slabs of 256 values.  Everything a slab needs goes from memory to LDS without passing through
+// registers (gemm_wide.hpp): the activation of the workgroup's tokens and their scales (two buffers), the rows
+// of every wave (one buffer: a wave holds the slab it works on in registers).  LDS is written at consecutive
+// addresses, 16 bytes per lane; bank conflicts are avoided by what each lane fetches (exclusive-or of the piece with the row).
+// Lane L supplies A-row t = L % 16 and B-column n = L % 16 at the k-octet L / 16 of a block and
+// receives D[4 * (L / 16) + j][L % 16], j < 4.  Q4_0: octets 0, 1 are the low nibbles of the block's first and second
+// eight bytes, octets 2, 3 the high ones.
+// us per launch, gemm_b32_mfma.hip before -> here: Q8_0 14336 x 4096 at 24 / 64 / 200 / 512 tokens 34.5 -> 21.2, 67 -> 24, 217 -> 61,
+// 434 -> 115 (523 TOP/s); 4096 x 14336 at 64 / 512 73 -> 39, 541 -> 116; Q4_0 128256 x 3072 at 16 / 64 57.7 -> 51.5, 156 -> 101.
+#include "gemm_wide.hpp"
+
+#pragma clang fp contract(off)
+
+namespace cml {
+
+typedef int v2i_w __attribute__((ext_vector_type(2)));
+
+struct B32WideArgs {
+    const uint8_t *quants;  // plane 0, row-major
+    const uint8_t *scales;  // plane 1: f16 per block, row-major
+    int64_t q_stride, s_stride;
+    int rows, n_slabs;
+    int n_row_blocks, n_cols;
+    const int8_t *q;   // [n_tokens][n_slabs*256]
+    const float *xs;   // [n_tokens][n_slabs*8], 16-byte aligned
+    float *out;        // [n_tokens][rows]
+    int n_tokens;
+};
+
+constexpr int kB32Waves = 4;
+
+// LDS layout of one workgroup.
+template <int FMT, int G, int RT, int D>
+struct B32WideLds {
+    static constexpr int NTOK = 16 * G;
+    static constexpr int kRowBytes = FMT == CML_Q8_0 ? 256 : 128;
+    static constexpr int kSlab = NTOK * 256;
+    static constexpr int kXs = (NTOK + 31) / 32 * 1024;         // activation scales [token][8]
+    static constexpr int kQuants = RT * 16 * kRowBytes;         // of a wave's rows
+    static constexpr int kWave = kQuants + RT * 256;            // + block scales [row][8] f16
+    static constexpr int kTotal = (D + 1) * (kSlab + kXs) + D * kB32Waves * kWave;
+};
+
+// G: token groups of 16 per column.  RT: row tiles of a wave.  D: slabs requested ahead.
+template <int FMT, int G, int RT, int D>
+__global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32WideArgs a) {
+    typedef B32WideLds<FMT, G, RT, D> L;
+    constexpr int NTOK = L::NTOK, WAVES = kB32Waves;
+    constexpr int kThreads = 64 * WAVES;
+    static_assert(kThreads == 256, "a pass of the workgroup fetches a token group");
+    extern __shared__ uint4 smem[];
+    uint8_t *slabs = reinterpret_cast<uint8_t *>(smem);  // [D + 1][NTOK][256]
+    constexpr int kXsAt = (D + 1) * L::kSlab, kWAt = kXsAt + (D + 1) * L::kXs;
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int n = lane & 15, kq = lane >> 4;
+    int row_block, col;
+    if (!wide_block(blockIdx.x, a.n_row_blocks, a.n_cols, row_block, col)) return;
+    const int tok0 = col * NTOK, n_here = min(NTOK, a.n_tokens - tok0);
+    const int n_slabs = a.n_slabs;
+    const int row0 = (row_block * WAVES + wave) * (16 * RT);
+
+    const uint32_t lds0 = lds_address(smem);
+    // Activation: thread tid fetches slot tid % 16 of tokens tid / 16 + 16 * k (tokens past the end repeat the last one).
+    const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
+    const uint32_t row_bytes = n_slabs * 256u;
+    const int8_t *q_base = a.q + static_cast<int64_t>(tok0) * row_bytes;
+    uint32_t src[G];
+#pragma unroll
+    for (int k = 0; k < G; k++) src[k] = static_cast<uint32_t>(min(t16 + 16 * k, n_here - 1)) * row_bytes + piece * 16;
+    // Scales: lane pairs of the first waves, token 32 * wave + lane / 2.
+    const bool xs_wave = wave < L::kXs / 1024;
+    const float *xs_base = a.xs + static_cast<int64_t>(tok0) * (n_slabs * 8);
+    const uint32_t xs_src = static_cast<uint32_t>(min(32 * wave + (lane >> 1), n_here - 1)) * (n_slabs * 32u) + (lane & 1) * 16;
+    auto fetch = [&](int slab, int buf) __attribute__((always_inline)) {
+        slab = min(slab, n_slabs - 1);
+        if (xs_wave) wide_dma16(lds0 + kXsAt + buf * L::kXs + wave * 1024, xs_base + slab * 8, xs_src);
+#pragma unroll
+        for (int k = 0; k < G; k++)
+            wide_dma16(lds0 + buf * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + slab * 256, src[k]);
+    };
+    // Weights: rows past the end repeat the last one.
+    const int first = min(row0, a.rows - 1), last = a.rows - 1 - first;  // (of this wave's rows)
+    const uint8_t *wq = a.quants + first * a.q_stride;
+    const uint8_t *wd = a.scales + first * a.s_stride;
+    constexpr int kRowsReq = 1024 / L::kRowBytes, kReqs = L::kQuants / 1024;
+    const uint32_t w_lds = lds0 + kWAt + wave * L::kWave;  // + slot * WAVES * kWave
+    uint32_t w_src[kReqs];
+#pragma unroll
+    for (int i = 0; i < kReqs; i++) {
+        const int r = kRowsReq * i + lane / (64 / kRowsReq);
+        const int slot = lane % (64 / kRowsReq);
+        const int p = FMT == CML_Q8_0 ? slot ^ (r & 15) : slot ^ ((r >> 1) & 7);
+        w_src[i] = static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(a.q_stride) + p * 16;
+    }
+    uint32_t d_src[RT];
+#pragma unroll
+    for (int r = 0; r < RT; r++) d_src[r] = static_cast<uint32_t>(min(16 * r + (lane >> 2), last)) * static_cast<uint32_t>(a.s_stride) + (lane & 3) * 4;
+    auto fetch_w = [&](int slab, int slot) __attribute__((always_inline)) {
+        slab = min(slab, n_slabs - 1);
+        const uint32_t to = w_lds + slot * (WAVES * L::kWave);
+#pragma unroll
+        for (int i = 0; i < kReqs; i++) wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
+#pragma unroll
+        for (int r = 0; r < RT; r++) wide_dma4(to + L::kQuants + r * 256, wd + slab * 16, d_src[r]);
+    };
+    constexpr int kAhead = (D - 1) * (G + kReqs + RT);  // requests that may be outstanding at the end of a step (some waves have more)
+
+    // Operands of a slab: the lane's octet of the eight blocks of either tile's row, the blocks' scales.
+    long bw[RT][8];
+    float dw[RT][8], md[RT][8];  // d_w; -12582912 * d_w
+    bool finite;
+    auto read_w = [&](int slot) __attribute__((always_inline)) {
+        const uint8_t *w_mine = slabs + kWAt + wave * L::kWave + slot * (WAVES * L::kWave);
+        uint32_t high = 0;
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const int row = 16 * r + n;
+            const uint4 d = *reinterpret_cast<const uint4 *>(w_mine + L::kQuants + row * 16);
+            const uint32_t dword[4] = {d.x, d.y, d.z, d.w};
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                const uint32_t bits = (dword[b >> 1] >> (16 * (b & 1))) & 0xffffu;
+                dw[r][b] = f16_bits_to_f32(bits);
+                md[r][b] = -12582912.0f * dw[r][b];
+                high = max(high, bits & 0x7c00u);
+                if constexpr (FMT == CML_Q8_0) {
+                    const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8);
+                    bw[r][b] = __builtin_bit_cast(long, o);
+                } else {
+                    const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 128 + ((b ^ ((n >> 1) & 7)) << 4) + (kq & 1) * 8);
+                    v2i_w v;
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {  // nibble - 8 as a signed byte
+                        const uint32_t nib = (static_cast<uint32_t>(o[i]) >> (4 * (kq >> 1))) & 0x0f0f0f0fu;
+                        v[i] = static_cast<int>((nib + 0x78787878u) ^ 0x80808080u);
+                    }
+                    bw[r][b] = __builtin_bit_cast(long, v);
+                }
+            }
+        }
+        finite = __builtin_amdgcn_ballot_w64(high == 0x7c00u) == 0;
+    };
+
+    // A operand of block b: octet kq of token n; the blocks' scales of tokens 4 kq .. + 3
+    uint32_t a_addr[8];
+#pragma unroll
+    for (int b = 0; b < 8; b++) a_addr[b] = n * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8;
+
+#pragma unroll
+    for (int i = 0; i < D; i++) {
+        fetch(i, i);
+        fetch_w(i, i);
+    }
+    wide_wait<kAhead>();
+    read_w(0);
+    wide_barrier();
+
+    float acc[RT][G][4];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int g = 0; g < G; g++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[r][g][j] = 0.0f;
+
+    const v4i_w magic = {0x4b400000, 0x4b400000, 0x4b400000, 0x4b400000};
+
+    auto step = [&](const uint8_t *slab, const float *xs, auto fin) __attribute__((always_inline)) {
+        // Software pipeline over units of two blocks of a token group: while the matrix cores work on unit i + 1, the
+        // f32 steps of unit i run and the operands of unit i + 2 are read.
+        constexpr int kUnits = G * 4;
+        long av[3][2];
+        float4 xv[2][4];  // scales of four blocks, of the lane's four tokens
+        v4i_w d[2][RT][2];
+        auto read_a = [&](int i) __attribute__((always_inline)) {
+            const int g = i >> 2, u = i & 3;
+#pragma unroll
+            for (int e = 0; e < 2; e++) av[i % 3][e] = *reinterpret_cast<const long *>(slab + a_addr[2 * u + e] + g * 4096);
+        };
+        auto read_x = [&](int i) __attribute__((always_inline)) {  // of units i and i + 1
+            const int g = i >> 2, h = (i >> 1) & 1;
+#pragma unroll
+            for (int j = 0; j < 4; j++) xv[h][j] = *reinterpret_cast<const float4 *>(xs + (16 * g + 4 * kq + j) * 8 + 4 * h);
+        };
+        auto contract = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+#pragma unroll
+                for (int r = 0; r < RT; r++) d[i & 1][r][e] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i % 3][e], bw[r][2 * (i & 3) + e], magic, 0, 0, 0);
+        };
+        auto chain = [&](int i) __attribute__((always_inline)) {
+            const int g = i >> 2, u = i & 3, h = u >> 1;
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int b = 2 * u + e, k = 2 * (u & 1) + e;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float x = k == 0 ? xv[h][j].x : k == 1 ? xv[h][j].y : k == 2 ? xv[h][j].z : xv[h][j].w;
+#pragma unroll
+                    for (int r = 0; r < RT; r++) {
+                        const float f = __builtin_bit_cast(float, static_cast<int>(d[i & 1][r][e][j]));
+                        const float p = decltype(fin)::value ? __builtin_fmaf(f, dw[r][b], md[r][b]) : (f - 12582912.0f) * dw[r][b];
+                        acc[r][g][j] = acc[r][g][j] + p * x;
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[r][g][j]));  // (keeps the compiler from sinking the chains to the store)
+        };
+        read_a(0);
+        read_x(0);
+        read_a(1);
+        contract(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kUnits; i++) {
+            if (i + 2 < kUnits) {
+                read_a(i + 2);
+                if ((i & 1) == 0) read_x(i + 2);
+            }
+            if (i + 1 < kUnits) contract(i + 1);
+            chain(i);
+            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+            for (int m = 0; m < 2 * RT; m++) {
+                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x2, 12, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    int buf = 0, slot = 0;  // of slab s: s % (D + 1), s % D
+    for (int s = 0; s < n_slabs; s++) {
+        fetch(s + D, buf == 0 ? D : buf - 1);  // (past the end the last slab again; the buffer of slab s - 1)
+        fetch_w(s + D, slot);                  // (slab s was read into registers before the barrier)
+        __builtin_amdgcn_sched_barrier(0);
+        const uint8_t *slab = slabs + buf * L::kSlab;
+        const float *xs = reinterpret_cast<const float *>(slabs + kXsAt + buf * L::kXs);
+        if (finite) step(slab, xs, std::true_type{});
+        else step(slab, xs, std::false_type{});
+        wide_wait<kAhead>();
+        buf = buf == D ? 0 : buf + 1;
+        slot = slot == D - 1 ? 0 : slot + 1;
+        read_w(slot);
+        wide_barrier();
+    }
+    wide_wait<0>();  // (nothing may still be on its way into LDS that is given back)
+
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        const int row = row0 + 16 * r + n;
+        if (row < a.rows) {
+            float *out = a.out + static_cast<int64_t>(tok0) * a.rows + row;
+#pragma unroll
+            for (int g = 0; g < G; g++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int t = 16 * g + 4 * kq + j;
+                    if (t < n_here) out[static_cast<int64_t>(t) * a.rows] = acc[r][g][j];
+                }
+        }
+    }
+}
+
+template <int FMT, int G, int RT, int D>
+static int launch_b32_wide(B32WideArgs ka, hipStream_t st) {
+    typedef B32WideLds<FMT, G, RT, D> L;
+    constexpr int kRows = kB32Waves * 16 * RT;
+    ka.n_row_blocks = (ka.rows + kRows - 1) / kRows;
+    ka.n_cols = (ka.n_tokens + L::NTOK - 1) / L::NTOK;
+    static std::atomic<bool> raised{false};  // per instantiation: allow more than 64 KB of dynamic LDS once
+    if (!raised.load(std::memory_order_acquire)) {
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_b32_wide_kernel<FMT, G, RT, D>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        raised.store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL((gemm_b32_wide_kernel<FMT, G, RT, D>), dim3(wide_grid(ka.n_row_blocks, ka.n_cols)), dim3(64 * kB32Waves), L::kTotal, st, ka);
+    // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>"
+    CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D));
+    CML_HIP_TRY(hipGetLastError());
+    return CML_OK;
+}
+
+struct B32WideShape {
+    int g = 0, rt = 0, d = 0;
+};
+
+// Estimated us of a launch (less a constant), fitted on MI355X to 750 launches of five weight shapes in both formats, 12 to 512 tokens.  A slab costs a
+// fixed latency and, for every wave on a SIMD and row tile, 0.165 us and 0.15 us per token group (a wave alone on its
+// SIMD stalls where two overlap: 1.4, not 1, times that).  A second slab ahead shortens the latency of long rows walked with one token
+// group (4096 x 14336 at 64 tokens 52 -> 40 us) and costs LDS elsewhere.  The shape with the lowest estimate was within 1.5 % of the
+// fastest on average (12 % off at worst).
+static float b32_wide_cost(int rows, int groups, int n_slabs, const B32WideShape &s) {
+    const int64_t wgs = static_cast<int64_t>((rows + s.rt * 64 - 1) / (s.rt * 64)) * ((groups + s.g - 1) / s.g);
+    const float per_cu = wgs / 256.0f, full = per_cu / 2;  // (two workgroups are resident at once)
+    const float rounds = full <= 1.0f ? 1.0f : 0.77f * full + 0.23f * std::ceil(full);
+    const float base = s.d == 1 ? 0.37f : n_slabs >= 24 ? 0.3f : 0.5f;
+    return rounds * n_slabs * (base + (per_cu > 1.0f ? 2.0f : 1.4f) * s.rt * (0.165f + 0.15f * s.g));
+}
+
+template <int FMT, int G, int RT, int D>
+static int b32_wide_visit(const B32WideArgs &ka, B32WideShape &best, float &cost, const B32WideShape *launch, hipStream_t st) {
+    typedef B32WideLds<FMT, G, RT, D> L;
+    static_assert(2 * L::kTotal <= 160 * 1024, "two workgroups per compute unit");
+    if (launch) return launch->g == G && launch->rt == RT && launch->d == D ? launch_b32_wide<FMT, G, RT, D>(ka, st) : -1;
+    const B32WideShape s{G, RT, D};
+    const float c = b32_wide_cost(ka.rows, (ka.n_tokens + 15) / 16, ka.n_slabs, s);
+    if (c < cost) {
+        cost = c;
+        best = s;
+    }
+    return -1;
+}
+
+// Every shape in turn: considers it (launch null) or, if it is the wanted one, launches it.
+template <int FMT, int I = 0>
+static int b32_wide_each(const B32WideArgs &ka, B32WideShape &best, float &cost, const B32WideShape *launch, hipStream_t st) {
+    if constexpr (I < 9) {
+        const int rc = b32_wide_visit<FMT, I == 8 ? 1 : I % 4 + 1, I == 8 ? 1 : I / 4 + 1, I == 8 ? 2 : 1>(ka, best, cost, launch, st);
+        return rc != -1 ? rc : b32_wide_each<FMT, I + 1>(ka, best, cost, launch, st);
+    }
+    return launch ? fail(CML_ERR_UNSUPPORTED, "wide matrix-core kernel: no such shape") : CML_OK;
+}
+
+template <int FMT>
+static int launch_b32_wide_fmt(const B32WideArgs &ka, hipStream_t st) {
+    B32WideShape s;
+    float cost = 1e30f;
+    b32_wide_each<FMT>(ka, s, cost, nullptr, st);
+    // (forced shapes: tests and measurements)
+    s.g = env_int("CAMELID_HIP_WIDE_GROUPS", s.g);
+    s.rt = env_int("CAMELID_HIP_WIDE_TILES", s.rt);
+    s.d = env_int("CAMELID_HIP_WIDE_AHEAD", s.d);
+    return b32_wide_each<FMT>(ka, s, cost, &s, st);
+}
+
+// A plain call on a weight that b32_mfma_usable accepts, activation scales 16-byte aligned.
+int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
+    const cml_weight *w = a.w;
+    B32WideArgs ka{};
+    ka.quants = w->planes.p[0];
+    ka.q_stride = w->planes.row_stride[0];
+    ka.scales = w->planes.p[1];
+    ka.s_stride = w->planes.row_stride[1];
+    ka.rows = static_cast<int>(w->rows);
+    ka.n_slabs = static_cast<int>(w->nb / 8);
+    ka.q = a.q;
+    ka.xs = a.scales;
+    ka.out = a.out;
+    ka.n_tokens = static_cast<int>(a.n_tokens);
+    return w->fmt == CML_Q8_0 ? launch_b32_wide_fmt<CML_Q8_0>(ka, st) : launch_b32_wide_fmt<CML_Q4_0>(ka, st);
+}
+
+}  // namespace cml

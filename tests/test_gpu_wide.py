@@ -94,3 +94,45 @@ def test_wide_expert_groups_are_bitwise_the_narrow_ones(E, k, hidden, ff, T):
         G.say(f"wide experts E={E} k={k} {hidden}/{ff} T={T} groups={g}")
         with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g), G.engaged(r"^q4k\.mfma\.wide\..*grouped"):
             assert G.same_bits(run(), ref)
+
+
+B32_FORMATS = [("Q8_0", B.CML_Q8_0, "q8_0"), ("Q4_0", B.CML_Q4_0, "q4_0")]
+
+
+# rows below a tile, past one, past a workgroup's; one slab, two, an odd number of them, rows long enough for two slabs ahead
+@pytest.mark.parametrize("rows,cols", [(1, 256), (16, 512), (70, 1280), (300, 2048), (130, 25 * 256)])
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_cells_are_bitwise_the_gemv(name, fmt, tag, rows, cols):
+    wire = G.synth_weight(fmt, rows, cols, seed=rows + cols)
+    blocks = wire.reshape(-1, 34 if fmt == B.CML_Q8_0 else 18)
+    for special in (False, True):
+        if special:  # scales that are no finite numbers, a zero one, a negative one
+            blocks[:: 37, :2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+            blocks[5:: 41, :2] = np.frombuffer(np.float16(-0.0).tobytes(), np.uint8)
+            blocks[7:: 43, 1] ^= 0x80
+        w = Weight.upload(fmt, rows, cols, wire)
+        for n in (3, 16, 17, 70):
+            x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+            x[0] = 0.0
+            s, q = oracle.quantize_activation(fmt, x)
+            with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+                ref = G.gpu_gemm(w, s, q)
+            for g, tiles, ahead in [(g, t, 1) for g in (1, 2, 3, 4) for t in (1, 2)] + [(1, 1, 2)]:
+                G.say(f"wide {name} {rows}x{cols} n={n} groups={g} tiles={tiles} ahead={ahead} special={special}")
+                with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g, CAMELID_HIP_WIDE_TILES=tiles, CAMELID_HIP_WIDE_AHEAD=ahead,
+                           CAMELID_HIP_B32_MFMA_MIN_TOKENS=1), G.engaged(rf"^{tag}\.mfma\.wide\.g{g}r{tiles}d{ahead}$", none=(r"\.dot\.",)):
+                    got = G.gpu_gemm(w, s, q)
+                assert np.array_equal(got, ref, equal_nan=True) if special else G.same_bits(got, ref)
+
+
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_on_a_row_band(name, fmt, tag):
+    rows, cols, n = 200, 5 * 256, 40
+    w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=5))
+    s, q = oracle.quantize_activation(fmt, np.random.default_rng(1).standard_normal((n, cols)).astype(np.float32))
+    G.say(f"wide {name} row band")
+    with G.engaged(rf"^{tag}\.mfma\.wide\."):
+        whole, band = G.gpu_gemm(w, s, q), G.gpu_gemm(w.slice(7, 150), s, q)
+    assert G.same_bits(band, whole[:, 7:157])
+    with G.env(CAMELID_HIP_MFMA_WIDE=0):
+        assert G.same_bits(whole, G.gpu_gemm(w, s, q))
