@@ -26,24 +26,28 @@
 //      APPROXIMATE incoming sum (any association);
 //   2. a chunk whose approximate incoming and outgoing sums, widened by the worst-case
 //      difference between any two f32 summation orders, lie in the same binade computes its
-//      (D0, D1) in that binade's units; any other chunk (the few where the sum crosses a power of
-//      two, the leading ones, anything not finite) is marked for in-order addition;
+//      (D0, D1): it adds its terms, in order, to two values of that binade, one with an even and one
+//      with an odd last bit, and takes how far their bits moved (any two sums of one parity move
+//      alike); any other chunk (the few where the sum crosses a power of two, the leading ones,
+//      anything not finite) is marked for in-order addition;
 //   3. neighbouring chunks of the same binade are composed by a segmented scan;
 //   4. one wave walks the groups in order: a composed run is applied in O(1) after checking on
 //      the EXACT running sum that it enters in the assumed binade and does not leave it (if the
 //      check fails the run's terms are added one by one -- the approximation only decides speed,
 //      never the result); marked chunks are added term by term as the scalar loop would.
-// 4096 values: about 12 marked chunks of 16 terms and as many runs instead of 4096 dependent
+// 4096 values: about 9 marked chunks of 16 terms and as many runs instead of 4096 dependent
 // additions.
-// Rows are independent: one workgroup per token.
+// Rows are independent: one workgroup per token.  Bound: latency -- a row is one chain of memory, scan and walk, and nearly every
+// instruction runs once, so the code itself (4 KB) has to be fetched: short straight phases are worth more than
+// parallel ones.  4 or 8 waves where 16 had longer scans and more groups to walk.
+#include <atomic>
+
 #include "cml_device.hpp"
 #include "cml_host.hpp"
 
 #pragma clang fp contract(off)
 
 namespace cml {
-
-constexpr uint32_t kRunBig = 1u << 26;  // saturation of run increments: anything >= 2^24 leaves the binade
 
 __device__ __forceinline__ float readlane_f32(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
@@ -56,77 +60,63 @@ struct RunPair {
 // `left` runs first, then `right`
 __device__ __forceinline__ RunPair run_then(const RunPair &left, const RunPair &right) {
     RunPair r;
-    r.d0 = min(left.d0 + ((left.d0 & 1u) ? right.d1 : right.d0), kRunBig);
-    r.d1 = min(left.d1 + ((left.d1 & 1u) ? right.d0 : right.d1), kRunBig);
+    r.d0 = left.d0 + ((left.d0 & 1u) ? right.d1 : right.d0);  // (the runs of a group climb through one binade, about 2^23 in all)
+    r.d1 = left.d1 + ((left.d1 & 1u) ? right.d0 : right.d1);
     return r;
 }
 
 // Segmented inclusive scan over the 64 lanes of a wave: every lane ends up with the composition
-// of the runs from its group's first lane to itself, and with that first lane's `first`.
-// `seen` enters as 1 in the lanes that start a group.  Rows of 16 lanes by DPP, then row by row
+// of the runs from its group's first lane to itself, `back` lanes before it.  Rows of 16 lanes by DPP, then row by row
 // through lane reads.
-__device__ __forceinline__ void run_scan64(RunPair &me, int &first, int &seen, int lane) {
+__device__ __forceinline__ void run_scan64(RunPair &me, int back, int lane) {
     const int rl = lane & 15, row = lane >> 4;
-    auto absorb = [&](uint32_t o0, uint32_t o1, int ofirst, int oseen, bool reach) __attribute__((always_inline)) {
-        if (reach && !seen) {
-            me = run_then(RunPair{o0, o1}, me);
-            first = ofirst;
-            seen = oseen;
-        }
+    auto absorb = [&](uint32_t o0, uint32_t o1, bool take) __attribute__((always_inline)) {
+        const RunPair both = run_then(RunPair{o0, o1}, me);
+        me.d0 = take ? both.d0 : me.d0;
+        me.d1 = take ? both.d1 : me.d1;
     };
-    absorb(row_shr_i32<1>(me.d0), row_shr_i32<1>(me.d1), row_shr_i32<1>(first), row_shr_i32<1>(seen), rl >= 1);
-    absorb(row_shr_i32<2>(me.d0), row_shr_i32<2>(me.d1), row_shr_i32<2>(first), row_shr_i32<2>(seen), rl >= 2);
-    absorb(row_shr_i32<4>(me.d0), row_shr_i32<4>(me.d1), row_shr_i32<4>(first), row_shr_i32<4>(seen), rl >= 4);
-    absorb(row_shr_i32<8>(me.d0), row_shr_i32<8>(me.d1), row_shr_i32<8>(first), row_shr_i32<8>(seen), rl >= 8);
+    const int in_row = min(rl, back);
+    absorb(row_shr_i32<1>(me.d0), row_shr_i32<1>(me.d1), in_row >= 1);
+    absorb(row_shr_i32<2>(me.d0), row_shr_i32<2>(me.d1), in_row >= 2);
+    absorb(row_shr_i32<4>(me.d0), row_shr_i32<4>(me.d1), in_row >= 4);
+    absorb(row_shr_i32<8>(me.d0), row_shr_i32<8>(me.d1), in_row >= 8);
 #pragma unroll
-    for (int r = 1; r < 4; r++) {  // the (by now complete) last lane of row r-1 into row r
-        const int src = 16 * r - 1;
-        absorb(__builtin_amdgcn_readlane(me.d0, src), __builtin_amdgcn_readlane(me.d1, src), __builtin_amdgcn_readlane(first, src),
-               __builtin_amdgcn_readlane(seen, src), row == r);
-    }
+    for (int r = 1; r < 4; r++)  // the (by now complete) last lane of row r-1 into row r
+        absorb(__builtin_amdgcn_readlane(me.d0, 16 * r - 1), __builtin_amdgcn_readlane(me.d1, 16 * r - 1), row == r && back > rl);
 }
 
-constexpr int kSumThreads = 1024, kSumWaves = kSumThreads / 64;
-
-// Terms xs[0 .. 4*1024*c4) (non-negative f32, zero padded) in LDS, thread t owning the contiguous
-// chunk of c4 float4 starting at t*c4.  Returns, in every lane of wave 0, the f32 sum
-// (((0 + xs[0]) + xs[1]) + ...) exactly as a scalar loop produces it.  1024 threads (short
-// chunks: the terms of a chunk that straddles a power of two are added one by one); n = number
+// Terms xs[0 .. 4*THREADS*C4) (non-negative f32, zero padded) in LDS, thread t owning the contiguous
+// chunk of C4 float4 starting at t*C4.  Returns, in every lane of wave 0, the f32 sum
+// (((0 + xs[0]) + xs[1]) + ...) exactly as a scalar loop produces it.  n = number
 // of real terms (sets the width of the binade guard).
-__device__ __forceinline__ float ordered_sum_nonneg(const float4 *xs4, int c4, int n, int tid) {
-    __shared__ float s_wave_total[kSumWaves];
-    __shared__ int s_E[kSumThreads];         // binade of the group ending at thread t (0: add in order)
-    __shared__ uint32_t s_D0[kSumThreads], s_D1[kSumThreads];
-    __shared__ int s_head[kSumThreads];      // first thread of the group ending at thread t
-    __shared__ int s_count[kSumWaves];       // groups per wave
-    __shared__ uint16_t s_list[kSumWaves][64];  // the last threads of a wave's groups, in order
+template <int THREADS, int C4>
+__device__ __forceinline__ float ordered_sum_nonneg(const float4 *xs4, int n, int tid) {
+    constexpr int kWaves = THREADS / 64;
+    __shared__ float s_wave_total[kWaves];
+    __shared__ int s_count[kWaves];          // groups per wave
+    __shared__ uint4 s_group[kWaves][64];    // in order: binade (0: add in order), D0, D1, first thread | chunks << 16
     const int lane = tid & 63, wave = tid >> 6, row = lane >> 4;
-    const float4 *mine = xs4 + tid * c4;
+    float4 mine[C4];
+#pragma unroll
+    for (int j = 0; j < C4; j++) mine[j] = xs4[tid * C4 + j];
 
     // 1. chunk sums and their exclusive scan (the association of this approximation is free):
     //    rows of 16 lanes by DPP, the three row totals by lane reads
     float local = 0.0f;
-    for (int j = 0; j < c4; j++) {
-        const float4 v = mine[j];
-        local = local + v.x;
-        local = local + v.y;
-        local = local + v.z;
-        local = local + v.w;
-    }
+#pragma unroll
+    for (int j = 0; j < C4; j++) local = local + ((mine[j].x + mine[j].y) + (mine[j].z + mine[j].w));
     float incl = local;
     incl = incl + row_shr_f32<1>(incl);  // lanes at the start of a row receive 0
     incl = incl + row_shr_f32<2>(incl);
     incl = incl + row_shr_f32<4>(incl);
     incl = incl + row_shr_f32<8>(incl);
-    const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, incl), 15));
-    const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, incl), 31));
-    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, incl), 47));
+    const float r0 = readlane_f32(incl, 15), r1 = readlane_f32(incl, 31), r2 = readlane_f32(incl, 47);
     incl = incl + (row == 0 ? 0.0f : (row == 1 ? r0 : (row == 2 ? r0 + r1 : (r0 + r1) + r2)));
     if (lane == 63) s_wave_total[wave] = incl;
     __syncthreads();
     float before = 0.0f;
 #pragma unroll
-    for (int w = 0; w < kSumWaves - 1; w++) {  // all reads at once, then the additions
+    for (int w = 0; w < kWaves - 1; w++) {  // all reads at once, then the additions
         const float tw = s_wave_total[w];
         before = before + (w < wave ? tw : 0.0f);
     }
@@ -135,138 +125,117 @@ __device__ __forceinline__ float ordered_sum_nonneg(const float4 *xs4, int c4, i
     // 2. same binade on both sides, with room for the difference between summation orders?
     const float delta = static_cast<float>(n + 64) * 2.384185791015625e-07f;  // (n + 64) * 2^-22
     const uint32_t e_lo = __float_as_uint(base * (1.0f - delta)) >> 23, e_hi = __float_as_uint(after * (1.0f + delta)) >> 23;
-    const bool run = e_lo == e_hi && e_lo >= 1 && e_lo < 255;
-    const int E = run ? static_cast<int>(e_lo) : 0;
-    RunPair me{0u, 0u};
-    if (run) {
-        for (int j = 0; j < c4; j++) {
-            const float4 v = mine[j];
-            const float t4[4] = {v.x, v.y, v.z, v.w};
+    const uint32_t even = __float_as_uint(base) & ~1u, odd = even | 1u;
+    float u0 = __uint_as_float(even), u1 = __uint_as_float(odd);
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                // branch-free: a right shift by 1..31 covers every term below the sum's binade
-                // (25 and more leave nothing: no increment, no tie), a left shift the others
-                const uint32_t bits = __float_as_uint(t4[k]);
-                const int Ea = static_cast<int>(bits >> 23);
-                const uint32_t ma = (bits & 0x7fffffu) | (Ea ? 0x800000u : 0u);
-                const int sh = E - max(Ea, 1);
-                const int rs = min(max(sh, 1), 31);
-                const uint32_t floor_r = ma >> rs, rem = ma & ((1u << rs) - 1u), half = 1u << (rs - 1);
-                const uint32_t inc_r = floor_r + (rem > half ? 1u : 0u), tie_r = rem == half ? 1u : 0u;
-                const int ls = min(-sh, 8);
-                const uint32_t inc_l = ls == 8 ? (ma ? kRunBig : 0u) : min(ma << (ls & 7), kRunBig);
-                const bool right = sh >= 1;
-                const uint32_t inc = right ? inc_r : inc_l, floor_part = right ? floor_r : inc_l, tie = right ? tie_r : 0u;
-                // a tie goes to the even neighbour: up exactly when S + floor is odd
-                me.d0 = min(me.d0 + inc + (tie & (me.d0 ^ floor_part) & 1u), kRunBig);
-                me.d1 = min(me.d1 + inc + (tie & (me.d1 ^ floor_part ^ 1u) & 1u), kRunBig);
-            }
-        }
+    for (int j = 0; j < C4; j++) {
+        u0 = u0 + mine[j].x;
+        u1 = u1 + mine[j].x;
+        u0 = u0 + mine[j].y;
+        u1 = u1 + mine[j].y;
+        u0 = u0 + mine[j].z;
+        u1 = u1 + mine[j].z;
+        u0 = u0 + mine[j].w;
+        u1 = u1 + mine[j].w;
     }
+    const bool run = e_lo == e_hi && e_lo >= 1 && e_lo < 255 && (even >> 23) == e_lo && (__float_as_uint(u0) >> 23) == e_lo && (__float_as_uint(u1) >> 23) == e_lo;
+    const int E = run ? static_cast<int>(e_lo) : 0;
+    RunPair me{__float_as_uint(u0) - even, __float_as_uint(u1) - odd};
 
-    // 3. compose neighbouring runs of one binade: a segmented inclusive scan, rows of 16 lanes by
-    //    DPP, then row by row through lane reads (a wave boundary ends a group; the walk below
-    //    simply meets one more group there)
-    const int E_prev = __shfl_up(E, 1);
-    const bool head = lane == 0 || E_prev != E;  // neighbouring in-order chunks (E = 0) form one range
-    int first = tid;
-    int seen = head ? 1 : 0;  // a group head lies inside the span composed so far
-    run_scan64(me, first, seen, lane);
+    // 3. compose neighbouring runs of one binade (a wave boundary ends a group; neighbouring in-order chunks form one range)
+    const int E_prev = __builtin_amdgcn_update_dpp(0, E, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+    const unsigned long long heads = __ballot(lane == 0 || E_prev != E);
+    const int back = lane - (63 - __builtin_clzll(heads & (~0ull >> (63 - lane))));  // to the group's first lane
+    run_scan64(me, back, lane);
     // the zero padding behind the last real chunk is not walked at all
-    const int n_chunks = (n + 4 * c4 - 1) / (4 * c4);
-    const int next_head = __shfl_down(static_cast<int>(head), 1);
-    const bool tail = tid < n_chunks && (lane == 63 || next_head != 0 || tid == n_chunks - 1);
-    s_E[tid] = E;
-    s_D0[tid] = me.d0;
-    s_D1[tid] = me.d1;
-    s_head[tid] = first;
+    const int n_chunks = (n + 4 * C4 - 1) / (4 * C4);
+    const bool tail = tid < n_chunks && (lane == 63 || (heads >> (lane + 1 & 63) & 1) != 0 || tid == n_chunks - 1);
     const unsigned long long tails = __ballot(tail);
     if (lane == 0) s_count[wave] = __builtin_popcountll(tails);
-    if (tail) s_list[wave][__builtin_popcountll(tails & ((1ull << lane) - 1ull))] = static_cast<uint16_t>(tid);
+    if (tail) s_group[wave][__builtin_popcountll(tails & ((1ull << lane) - 1ull))] = make_uint4(E, me.d0, me.d1, (tid - back) | (back + 1) << 16);
     __syncthreads();
     if (wave != 0) return 0.0f;
 
     // 4. the walk, every lane of wave 0 alike.  Lane g first fetches the g-th group of a batch of
-    //    up to 64 (its last thread from the tail masks, then the group's record), so that the
+    //    up to 64 and, for the case that it is an in-order one, its first chunk, so that the
     //    chain through the running sum reads lanes, not memory.
     float s = 0.0f;
-    auto add_in_order = [&](const float4 *p, int cnt) __attribute__((always_inline)) {  // cnt float4, the next one read ahead
-        float4 v = p[0];
-        for (int j = 0; j < cnt; j++) {
-            const float4 nx = p[min(j + 1, cnt - 1)];
-            s = s + v.x;
-            s = s + v.y;
-            s = s + v.z;
-            s = s + v.w;
-            v = nx;
-        }
-    };
-    int cnt_w[kSumWaves];
+    int cnt_w[kWaves], n_groups = 0;
 #pragma unroll
-    for (int w = 0; w < kSumWaves; w++) cnt_w[w] = s_count[w];
-    int n_groups = 0;
+    for (int w = 0; w < kWaves; w++) cnt_w[w] = s_count[w];
 #pragma unroll
-    for (int w = 0; w < kSumWaves; w++) n_groups += cnt_w[w];
+    for (int w = 0; w < kWaves; w++) n_groups += cnt_w[w];
+    n_groups = __builtin_amdgcn_readfirstlane(n_groups);
     for (int g0 = 0; g0 < n_groups; g0 += 64) {
         // the (g0 + lane)-th group: which wave's list, which entry
         int k = g0 + lane, w_mine = 0;
-        bool found = false;
 #pragma unroll
-        for (int w = 0; w < kSumWaves; w++) {
-            if (!found) {
-                if (k < cnt_w[w]) {
-                    found = true;
-                    w_mine = w;
-                } else {
-                    k -= cnt_w[w];
+        for (int w = 0; w < kWaves - 1; w++) {
+            const bool past = w_mine == w && k >= cnt_w[w];
+            k -= past ? cnt_w[w] : 0;
+            w_mine += past ? 1 : 0;
+        }
+        const uint4 group = s_group[w_mine][min(k, 63)];  // (lanes past the last group read what nobody looks at)
+        const int g_first = min(static_cast<int>(group.w & 0xffffu), THREADS - 1);
+        float4 gV[C4];
+#pragma unroll
+        for (int j = 0; j < C4; j++) gV[j] = xs4[g_first * C4 + j];
+        const int here = min(64, n_groups - g0);
+        auto add_range = [&](const float4 *p, int chunks) __attribute__((always_inline)) {  // the next chunk read ahead
+            float4 next[C4];
+#pragma unroll
+            for (int j = 0; j < C4; j++) next[j] = p[j];
+#pragma unroll 1
+            for (int c = 1; c <= chunks; c++) {
+                float4 v[C4];
+                const float4 *pn = p + min(c, chunks - 1) * C4;
+#pragma unroll
+                for (int j = 0; j < C4; j++) {
+                    v[j] = next[j];
+                    next[j] = pn[j];
                 }
+#pragma unroll
+                for (int j = 0; j < C4; j++) {
+                    s = s + v[j].x;
+                    s = s + v[j].y;
+                    s = s + v[j].z;
+                    s = s + v[j].w;
+                }
+            }
+        };
+        auto add_marked = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < C4; j++) {
+                const float x = readlane_f32(gV[j].x, g), y = readlane_f32(gV[j].y, g), z = readlane_f32(gV[j].z, g), w = readlane_f32(gV[j].w, g);
+                s = s + x;
+                s = s + y;
+                s = s + z;
+                s = s + w;
+            }
+            const uint32_t where = __builtin_amdgcn_readlane(group.w, g);
+            if ((where >> 16) > 1) add_range(xs4 + ((where & 0xffffu) + 1) * C4, (where >> 16) - 1);
+        };
+        // A run enters with S even or odd; adding its increment to the BITS of s is adding it
+        // to S as long as no carry reaches the exponent field -- which is also the test that
+        // the sum stays in the binade.  The tests of a batch are looked at once, behind it.
+        const float s_in = s;
+        uint32_t off = 0;
+        for (int g = 0; g < here; g++) {
+            const uint32_t Eg = __builtin_amdgcn_readlane(group.x, g);
+            if (Eg == 0) {
+                add_marked(g);
+            } else {
+                const uint32_t D0 = __builtin_amdgcn_readlane(group.y, g), D1 = __builtin_amdgcn_readlane(group.z, g);
+                const uint32_t sb = __float_as_uint(s), to = sb + ((sb & 1u) ? D1 : D0);
+                off |= (sb ^ (Eg << 23)) | (to ^ (Eg << 23));
+                s = __uint_as_float(to);
             }
         }
-        const int t_mine = found ? s_list[w_mine][k] : kSumThreads - 1;
-        // Groups that a wave boundary cut apart are put together again here, in parallel: the same
-        // scan over the batch's records (lanes past the last group form groups of their own).
-        const int gE = g0 + lane < n_groups ? s_E[t_mine] : -1 - lane;
-        const int gE_prev = __shfl_up(gE, 1);
-        RunPair gD{s_D0[t_mine], s_D1[t_mine]};
-        int gH = s_head[t_mine];
-        int gSeen = (lane == 0 || gE_prev != gE) ? 1 : 0;
-        const int gE_next = __shfl_down(gE, 1);
-        const bool gTail = g0 + lane < n_groups && (lane == 63 || gE_next != gE);
-        run_scan64(gD, gH, gSeen, lane);
-        // an in-order range usually is one or two float4 long: fetch those with the record
-        const int gCnt = (t_mine - gH + 1) * c4;
-        const float4 gV0 = xs4[gH * c4], gV1 = xs4[gH * c4 + (gCnt > 1 ? 1 : 0)];
-        unsigned long long todo = __ballot(gTail);
-        while (todo) {
-            const int g = __builtin_ctzll(todo);
-            todo &= todo - 1;
-            const int Eg = __builtin_amdgcn_readlane(gE, g);
-            if (Eg == 0) {
-                const int cnt = __builtin_amdgcn_readlane(gCnt, g);
-                s = s + readlane_f32(gV0.x, g);
-                s = s + readlane_f32(gV0.y, g);
-                s = s + readlane_f32(gV0.z, g);
-                s = s + readlane_f32(gV0.w, g);
-                if (cnt > 1) {
-                    s = s + readlane_f32(gV1.x, g);
-                    s = s + readlane_f32(gV1.y, g);
-                    s = s + readlane_f32(gV1.z, g);
-                    s = s + readlane_f32(gV1.w, g);
-                    if (cnt > 2) add_in_order(xs4 + __builtin_amdgcn_readlane(gH, g) * c4 + 2, cnt - 2);
-                }
-                continue;
-            }
-            // The run enters with S even or odd; adding its increment to the BITS of s is adding it
-            // to S as long as no carry reaches the exponent field -- which is also the test that
-            // the sum stays in the binade.  D1 - D0 is a handful of ties: a 24-bit multiply.
-            const uint32_t D0 = __builtin_amdgcn_readlane(gD.d0, g), D1 = __builtin_amdgcn_readlane(gD.d1, g);
-            const uint32_t sb = __float_as_uint(s);
-            const uint32_t after = sb + D0 + static_cast<uint32_t>(__mul24(static_cast<int>(sb & 1u), static_cast<int>(D1 - D0)));
-            const uint32_t e_bits = static_cast<uint32_t>(Eg) << 23;
-            if (((sb ^ e_bits) | (after ^ e_bits)) < (1u << 23) && D0 < (1u << 24)) {
-                s = __uint_as_float(after);
-            } else {  // the guard was too narrow for this data: still exact
-                add_in_order(xs4 + __builtin_amdgcn_readlane(gH, g) * c4, __builtin_amdgcn_readlane(gCnt, g));
+        if (__builtin_amdgcn_readfirstlane(off) >> 23) {  // the guard was too narrow for this data: still exact
+            s = s_in;
+            for (int g = 0; g < here; g++) {
+                const uint32_t where = __builtin_amdgcn_readlane(group.w, g);
+                add_range(xs4 + (where & 0xffffu) * C4, where >> 16);
             }
         }
     }
@@ -278,10 +247,10 @@ __device__ __forceinline__ float ordered_sum_nonneg(const float4 *xs4, int c4, i
 // Every thread keeps its share of the row in registers (up to kRmsRegs float4) and puts the
 // squares into LDS, where ordered_sum_nonneg adds them up; the LDS row is reused for the
 // normalised values the quantizers read.
-constexpr int kRmsRegs = 4;  // float4 per thread: rows of up to 4 * 1024 * 4 = 16384 values
+constexpr int kRmsRegs = 4;  // most float4 per thread: rows of up to 4 * 1024 * 4 = 16384 values
 
-template <int ACT>
-__global__ __launch_bounds__(kSumThreads) void rms_norm_quantize_kernel(const float *__restrict__ x, const float *__restrict__ weight,
+template <int ACT, int THREADS, int C4>
+__global__ __launch_bounds__(THREADS) void rms_norm_quantize_kernel(const float *__restrict__ x, const float *__restrict__ weight,
                                                                 float eps, int cols, float *__restrict__ normed,
                                                                 int8_t *__restrict__ q, float *__restrict__ scales) {
     extern __shared__ float4 xs4[];  // the row, padded to whole batches: squares first, then the normalised values
@@ -290,22 +259,33 @@ __global__ __launch_bounds__(kSumThreads) void rms_norm_quantize_kernel(const fl
     const int64_t token = blockIdx.x;
     const int n4 = cols >> 2;
     const float4 *x4 = reinterpret_cast<const float4 *>(x + token * cols);
-    float4 xv[kRmsRegs];
+    const float4 *w4 = reinterpret_cast<const float4 *>(weight);
+    float4 xv[C4], wv[C4];  // (the weight is requested with the row: at the end it would be a second round trip)
 #pragma unroll
-    for (int k = 0; k < kRmsRegs; k++) {
-        const int i = tid + k * kSumThreads;
+    for (int k = 0; k < C4; k++) {
+        const int i = tid + k * THREADS;
+        if (i < n4) xv[k] = x4[i];
+    }
+    if constexpr (ACT != 3) {
+#pragma unroll
+        for (int k = 0; k < C4; k++) {
+            const int i = tid + k * THREADS;
+            if (i < n4) wv[k] = w4[i];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < C4; k++) {
+        const int i = tid + k * THREADS;
         if (i < n4) {
-            const float4 v = x4[i];
-            xv[k] = v;
+            const float4 v = xv[k];
             xs4[i] = make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
         }
     }
-    // zeros from the end of the row up to 1024 whole chunks: sum + 0 == sum exactly (the sum of
+    // zeros from the end of the row up to THREADS whole chunks: sum + 0 == sum exactly (the sum of
     // squares is never negative) and a zero term has increment 0
-    const int c4 = (n4 + kSumThreads - 1) / kSumThreads;  // float4 per thread chunk
-    for (int i = n4 + tid; i < kSumThreads * c4; i += kSumThreads) xs4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i = n4 + tid; i < THREADS * C4; i += THREADS) xs4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     __syncthreads();
-    const float sum = ordered_sum_nonneg(xs4, c4, cols, tid);  // valid in wave 0
+    const float sum = ordered_sum_nonneg<THREADS, C4>(xs4, cols, tid);  // valid in wave 0
     if constexpr (ACT == 3) {
         if (tid == 0) normed[token] = sum;
         return;
@@ -316,13 +296,12 @@ __global__ __launch_bounds__(kSumThreads) void rms_norm_quantize_kernel(const fl
     }
     __syncthreads();
     const float scale = s_scale;
-    const float4 *w4 = reinterpret_cast<const float4 *>(weight);
     float4 *n4out = normed ? reinterpret_cast<float4 *>(normed + token * cols) : nullptr;
 #pragma unroll
-    for (int k = 0; k < kRmsRegs; k++) {
-        const int i = tid + k * kSumThreads;
+    for (int k = 0; k < C4; k++) {
+        const int i = tid + k * THREADS;
         if (i < n4) {
-            const float4 v = xv[k], w = w4[i];
+            const float4 v = xv[k], w = wv[k];
             float4 y;
             y.x = (v.x * scale) * w.x;
             y.y = (v.y * scale) * w.y;
@@ -338,7 +317,7 @@ __global__ __launch_bounds__(kSumThreads) void rms_norm_quantize_kernel(const fl
     if constexpr (ACT == 1) {
         // eight lanes per 32-value block; cols/4 is a multiple of 8, so groups enter and leave together
         float *sc = scales + token * (cols / 32);
-        for (int i = tid; i < n4; i += kSumThreads) {
+        for (int i = tid; i < n4; i += THREADS) {
             float s;
             const uint32_t packed = q8_0_quantize_lane8(xs4[i], s);
             q32[i] = packed;
@@ -347,7 +326,7 @@ __global__ __launch_bounds__(kSumThreads) void rms_norm_quantize_kernel(const fl
     } else {
         // one wave per 256-value super-block
         float *d = scales + token * (cols / 256);
-        for (int sb = wave; sb < cols / 256; sb += kSumWaves) {
+        for (int sb = wave; sb < cols / 256; sb += THREADS / 64) {
             float dv;
             int bsum;
             const uint32_t packed = q8k_quantize_wave(xs4[sb * 64 + lane], dv, bsum);
@@ -357,32 +336,50 @@ __global__ __launch_bounds__(kSumThreads) void rms_norm_quantize_kernel(const fl
     }
 }
 
-int launch_rms_norm_quantize(int act, const float *x, const float *weight, float eps, int64_t n_tokens, int64_t cols,
-                             float *normed, int8_t *q, float *scales, hipStream_t st) {
-    if (n_tokens == 0 || cols == 0) return CML_OK;
-    if (cols > static_cast<int64_t>(kRmsRegs) * kSumThreads * 4)
-        return fail(CML_ERR_UNSUPPORTED, "rms_norm row of %lld values exceeds the staging limit of %d", (long long)cols, kRmsRegs * kSumThreads * 4);
-    // the row in 1024 whole chunks (zero padded)
-    const size_t lds = static_cast<size_t>((cols / 4 + kSumThreads - 1) / kSumThreads) * kSumThreads * sizeof(float4);
-    static bool raised = false;
-    if (!raised) {
-        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<0>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<1>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<2>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<3>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
-        raised = true;
+template <int THREADS, int C4>
+static int launch_rms_norm(int act, const float *x, const float *weight, float eps, int64_t n_tokens, int cols, float *normed, int8_t *q, float *scales, hipStream_t st) {
+    constexpr size_t lds = static_cast<size_t>(THREADS) * C4 * sizeof(float4);  // the row in whole chunks (zero padded)
+    static std::atomic<bool> raised{false};
+    if (lds > 48 * 1024 && !raised.load(std::memory_order_acquire)) {
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<0, THREADS, C4>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<1, THREADS, C4>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<2, THREADS, C4>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<3, THREADS, C4>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
+        raised.store(true, std::memory_order_release);
     }
-    const dim3 grid(static_cast<unsigned>(n_tokens)), block(kSumThreads);
-    const int c = static_cast<int>(cols);
+    const dim3 grid(static_cast<unsigned>(n_tokens)), block(THREADS);
     switch (act) {
-        case 0: hipLaunchKernelGGL(rms_norm_quantize_kernel<0>, grid, block, lds, st, x, weight, eps, c, normed, q, scales); break;
-        case 1: hipLaunchKernelGGL(rms_norm_quantize_kernel<1>, grid, block, lds, st, x, weight, eps, c, normed, q, scales); break;
-        case 3: hipLaunchKernelGGL(rms_norm_quantize_kernel<3>, grid, block, lds, st, x, weight, eps, c, normed, q, scales); break;
-        default: hipLaunchKernelGGL(rms_norm_quantize_kernel<2>, grid, block, lds, st, x, weight, eps, c, normed, q, scales); break;
+        case 0: hipLaunchKernelGGL((rms_norm_quantize_kernel<0, THREADS, C4>), grid, block, lds, st, x, weight, eps, cols, normed, q, scales); break;
+        case 1: hipLaunchKernelGGL((rms_norm_quantize_kernel<1, THREADS, C4>), grid, block, lds, st, x, weight, eps, cols, normed, q, scales); break;
+        case 3: hipLaunchKernelGGL((rms_norm_quantize_kernel<3, THREADS, C4>), grid, block, lds, st, x, weight, eps, cols, normed, q, scales); break;
+        default: hipLaunchKernelGGL((rms_norm_quantize_kernel<2, THREADS, C4>), grid, block, lds, st, x, weight, eps, cols, normed, q, scales); break;
     }
     CML_COUNT_LAUNCH("producer.rms_norm");
     CML_HIP_TRY(hipGetLastError());
     return CML_OK;
+}
+
+template <int THREADS>
+static int launch_rms_norm_chunks(int act, const float *x, const float *weight, float eps, int64_t n_tokens, int cols, float *normed, int8_t *q, float *scales, hipStream_t st) {
+    switch ((cols / 4 + THREADS - 1) / THREADS) {
+        case 1: return launch_rms_norm<THREADS, 1>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
+        case 2: return launch_rms_norm<THREADS, 2>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
+        case 3: return launch_rms_norm<THREADS, 3>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
+        default: return launch_rms_norm<THREADS, 4>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
+    }
+}
+
+int launch_rms_norm_quantize(int act, const float *x, const float *weight, float eps, int64_t n_tokens, int64_t cols,
+                             float *normed, int8_t *q, float *scales, hipStream_t st) {
+    if (n_tokens == 0 || cols == 0) return CML_OK;
+    if (cols > static_cast<int64_t>(kRmsRegs) * 1024 * 4)
+        return fail(CML_ERR_UNSUPPORTED, "rms_norm row of %lld values exceeds the staging limit of %d", (long long)cols, kRmsRegs * 1024 * 4);
+    // us per launch of one row, 256 / 512 / 1024 threads: 2048 values 4.7 / 4.9 / 5.9, 3072 5.4 / 5.4 / 6.6, 4096 6.0 / 5.6 / 7.3, 8192 - / 7.2 / 7.9
+    // (512 rows of 4096: 7.9 / 8.0 / 10.5); before, always 1024 threads: 4096 8.0, 512 rows 15.
+    const int c = static_cast<int>(cols), threads = env_int("CAMELID_HIP_RMS_THREADS", cols <= 3072 ? 256 : 512);
+    if (threads <= 256 && cols <= 4 * kRmsRegs * 256) return launch_rms_norm_chunks<256>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
+    if (threads <= 512 && cols <= 4 * kRmsRegs * 512) return launch_rms_norm_chunks<512>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
+    return launch_rms_norm_chunks<1024>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
 }
 
 // h = silu(g) * u = (g / (1 + exp(-g))) * u, quantized on the fly.  Q8_K: one wave per

@@ -112,6 +112,12 @@ def test_sum_of_squares_is_the_scalar_loop(cols):
         assert finite.sum() >= 12
 
 
+# one to four float4 per thread in workgroups of 256, 512 and 1024 threads: the last width of a shape and the first of the next
+@pytest.mark.parametrize("cols", [1024, 1028, 3072, 3076, 4100, 6144, 6148, 8196, 12288, 12292])
+def test_sum_of_squares_at_the_widths_where_the_launch_changes(cols):
+    test_sum_of_squares_is_the_scalar_loop(cols)
+
+
 @pytest.mark.parametrize("cols", [256, 2048, 2816, 4096, 14336])
 def test_rms_norm_rows_are_bit_exact(cols):
     x, w = _rows(5, cols, 900 + cols)
