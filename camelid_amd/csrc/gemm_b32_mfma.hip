@@ -619,8 +619,8 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_gr
     // Up to 16 tokens, rows of at most 16 slabs, few row tiles: several waves per row tile, one chain.
     // Workgroup shapes by measurement (16 tokens, kernel us cache-cold, against the kernel below):
     //   rows of <= 8 slabs:  <= 256 tiles: 8 waves per tile (4096 x 2048 Q8_0 10.0 -> 6.0);
-    //                        <= 768 tiles: 4 waves per tile, 2 tiles per workgroup (8192 x 2048 Q8_0 10.6 -> 8.0, Q4_0 11.8 -> 7.0);
-    //                        more tiles: no gain (16384 x 2048 12.3 -> 12.2), the kernel below stays;
+    //                        <= 512 tiles: 4 waves per tile, 2 tiles per workgroup (8192 x 2048 Q8_0 7.5 us, Q4_0 6.6; the wide kernel 8.2, 8.7);
+    //                        more tiles lose to the wide kernel (10240 x 2048 Q8_0 11.1, Q4_0 9.6; wide 8.4, 8.9; rows of 2 or 3 slabs alike: 12288 x 768 7.5, 5.7; 5.2);
     //   rows of 9..16 slabs: the staged activation fills half of a compute unit's LDS, one workgroup per unit:
     //                        <= 256 tiles: 8 waves per tile (4096 x 4096 Q8_0 15.6 -> 10.8, Q4_0 18.6 -> 8.8);
     //                        <= 512 tiles: the same, 2 tiles per workgroup (8192 x 4096 Q8_0 16.9 -> 14.3, Q4_0 19.1 -> 11.1);
@@ -634,14 +634,14 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_gr
             if (kpar == 3) return launch_b32_mfma_kpar<FMT, 8, 1, 1>(ka, st);
             if (kpar == 4) return launch_b32_mfma_kpar<FMT, 8, 1, 2>(ka, st);
             if (tiles <= 256) return launch_b32_mfma_kpar<FMT, 8, 1, 1>(ka, st);
-            if (tiles <= 768) return launch_b32_mfma_kpar<FMT, 4, 2, 2>(ka, st);
+            if (tiles <= 512) return launch_b32_mfma_kpar<FMT, 4, 2, 2>(ka, st);
         } else if (ka.n_slabs > 8 && ka.n_slabs <= 16) {
             if (kpar == 1) return launch_b32_mfma_kpar<FMT, 4, 4, 1>(ka, st);
             if (kpar == 2) return launch_b32_mfma_kpar<FMT, 8, 2, 1>(ka, st);
             if (kpar == 3) return launch_b32_mfma_kpar<FMT, 8, 2, 2>(ka, st);
             if (tiles <= 256) return launch_b32_mfma_kpar<FMT, 8, 2, 1>(ka, st);
             if (tiles <= 512) return launch_b32_mfma_kpar<FMT, 8, 2, 2>(ka, st);
-        } else if (ka.n_slabs >= 2 && ka.n_slabs < 4 && (kpar > 0 || tiles <= 768)) {
+        } else if (ka.n_slabs >= 2 && ka.n_slabs < 4 && (kpar > 0 || tiles <= 512)) {
             return launch_b32_mfma_kpar<FMT, 2, 2, 1>(ka, st);
         }
     }
