@@ -4,6 +4,7 @@ array, the second smaller than the first; sizes beyond the array are refused."""
 import numpy as np
 import pytest
 
+import oracle
 from camelid_amd import binding as B
 from camelid_amd.binding import DeviceBuffer, Weight, check, lib
 from tests import gpu_util as G
@@ -59,3 +60,21 @@ def test_static_workspace_refuses_what_does_not_fit():
     check(L.cml_stream_sync(None))
     assert np.all(od.to_numpy(np.float32, (n_fit, rows)) == 0)
     assert L.cml_matmul_f32_static(None, xd.ptr, 1, od.ptr, None) == 2  # CML_ERR_INVALID
+
+
+# outputs of a row that is no multiple of 16 bytes; the last size through pinned memory and the first past it; then small again
+@pytest.mark.parametrize("rows,n", [(1, 1), (7, 3), (1025, 5), (69625, 4), (69633, 4), (33, 2)])
+def test_host_slice_calls_through_pinned_and_pageable_memory_agree(rows, n):
+    B.init(0)
+    fmt, cols = B.CML_Q8_0, 64
+    wire = G.synth_weight(fmt, rows, cols, seed=rows)
+    s, q = oracle.quantize_activation(fmt, np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32))
+    got = []
+    for limit in (0, 1 << 30):  # (a larger limit than the library's is the library's)
+        G.say(f"host slices {rows}x{cols} n={n} limit={limit}")
+        out = np.full((n, rows), 7.0, np.float32)
+        with G.env(CAMELID_HIP_SEAM_PINNED_BYTES=limit):
+            check(lib().cml_try_linear_rows(fmt, s.ctypes.data, q.ctypes.data, wire.ctypes.data, wire.nbytes, n, rows, cols, out.ctypes.data))
+        got.append(out)
+    assert G.same_bits(got[0], got[1])
+    assert G.same_bits(got[0], oracle.matmul_q(fmt, wire, cols, s, q, order=oracle.ORDER_PRIMARY, threads=8))
