@@ -184,7 +184,8 @@ int launch_gemm_q4k(const MatArgs &a, hipStream_t st);
 int launch_gemm_q4k_mfma(const MatArgs &a, hipStream_t st);  // plain calls, n_tokens >= 16
 int launch_gemm_q4k_wide(const MatArgs &a, hipStream_t st);  // gemm_wide.hpp: plain, or grouped (band rows in whole tiles)
 int launch_gemm_q6k_wide(const MatArgs &a, hipStream_t st);
-int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st);  // plain calls
+int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st);  // plain, or grouped where the next says so
+bool gemm_b32_wide_serves_groups(const MatArgs &a);
 int launch_gemm_b32_mfma(const MatArgs &a, hipStream_t st);  // Q8_0 / Q4_0 on the matrix cores; plain or grouped
 bool b32_mfma_usable(const cml_weight *w);                   // rows of whole 256-value slabs
 int b32_mfma_min_tokens(int64_t rows);                       // batch size from which it pays

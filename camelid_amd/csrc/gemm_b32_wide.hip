@@ -1,4 +1,4 @@
-// Q8_0 / Q4_0 x Q8_0 matmul for prefill batches on the int8 matrix cores (gfx950).
+// Q8_0 / Q4_0 x Q8_0 matmul for prefill batches and expert groups on the int8 matrix cores (gfx950).
 //
 // Arithmetic: cell by cell that of the matvec kernels and of gemm_b32_mfma.hip: per 32-value block, in block order,
 //     isum = sum_j w_j * x_j  (exact i32),   acc = acc + ((float)isum * d_w) * d_x
@@ -39,6 +39,10 @@ struct B32WideArgs {
     const float *xs;   // [n_tokens][n_slabs*8], 16-byte aligned
     float *out;        // [n_tokens][rows]
     int n_tokens;
+    // Grouped call (mixture of experts), as in WideArgs: blockIdx.y -> group, its band of rows and its assignments.
+    const int32_t *group_offsets;
+    const int32_t *group_rows;
+    const int32_t *group_ids;
 };
 
 constexpr int kB32Waves = 4;
@@ -56,12 +60,14 @@ struct B32WideLds {
 };
 
 // G: token groups of 16 per column.  RT: row tiles of a wave.  D: slabs requested ahead.
-template <int FMT, int G, int RT, int D>
+// GROUPED: expert groups; a workgroup walks all token columns of its group.
+template <int FMT, int G, int RT, int D, bool GROUPED>
 __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32WideArgs a) {
     typedef B32WideLds<FMT, G, RT, D> L;
     constexpr int NTOK = L::NTOK, WAVES = kB32Waves;
     constexpr int kThreads = 64 * WAVES;
     static_assert(kThreads == 256, "a pass of the workgroup fetches a token group");
+    static_assert(!GROUPED || D == 1, "waves of a grouped call may have fewer requests in flight");
     extern __shared__ uint4 smem[];
     uint8_t *slabs = reinterpret_cast<uint8_t *>(smem);  // [D + 1][NTOK][256]
     constexpr int kXsAt = (D + 1) * L::kSlab, kWAt = kXsAt + (D + 1) * L::kXs;
@@ -71,230 +77,245 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
     const int n = lane & 15, kq = lane >> 4;
     int row_block, col;
     if (!wide_block(blockIdx.x, a.n_row_blocks, a.n_cols, row_block, col)) return;
-    const int tok0 = col * NTOK, n_here = min(NTOK, a.n_tokens - tok0);
-    const int n_slabs = a.n_slabs;
-    const int row0 = (row_block * WAVES + wave) * (16 * RT);
+    const int64_t band = GROUPED ? (a.group_ids ? a.group_ids[blockIdx.y] : static_cast<int>(blockIdx.y)) : 0;
+    if (band < 0) return;  // a slot past the groups in use
+    const int a0 = GROUPED ? a.group_offsets[band] : 0;
+    const int n_assign = GROUPED ? a.group_offsets[band + 1] - a0 : a.n_tokens;
+    for (;; col++) {
+        const int tok0 = col * NTOK;
+        if (tok0 >= n_assign) return;  // the whole workgroup leaves
+        const int n_here = min(NTOK, n_assign - tok0);
+        auto act_row = [&](int t) __attribute__((always_inline)) -> uint32_t {  // (tokens past the end repeat the last one)
+            const int j = min(t, n_here - 1);
+            return static_cast<uint32_t>(GROUPED ? (a.group_rows ? a.group_rows[a0 + tok0 + j] : a0 + tok0 + j) : j);
+        };
+        const int n_slabs = a.n_slabs;
+        const int row0 = (row_block * WAVES + wave) * (16 * RT);
 
-    const uint32_t lds0 = lds_address(smem);
-    // Activation: thread tid fetches slot tid % 16 of tokens tid / 16 + 16 * k (tokens past the end repeat the last one).
-    const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
-    const uint32_t row_bytes = n_slabs * 256u;
-    const int8_t *q_base = a.q + static_cast<int64_t>(tok0) * row_bytes;
-    uint32_t src[G];
+        const uint32_t lds0 = lds_address(smem);
+        // Activation: thread tid fetches slot tid % 16 of tokens tid / 16 + 16 * k.
+        const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
+        const uint32_t row_bytes = n_slabs * 256u;
+        const int8_t *q_base = a.q + (GROUPED ? 0 : static_cast<int64_t>(tok0) * row_bytes);
+        uint32_t src[G];
 #pragma unroll
-    for (int k = 0; k < G; k++) src[k] = static_cast<uint32_t>(min(t16 + 16 * k, n_here - 1)) * row_bytes + piece * 16;
-    // Scales: lane pairs of the first waves, token 32 * wave + lane / 2.
-    const bool xs_wave = wave < L::kXs / 1024;
-    const float *xs_base = a.xs + static_cast<int64_t>(tok0) * (n_slabs * 8);
-    const uint32_t xs_src = static_cast<uint32_t>(min(32 * wave + (lane >> 1), n_here - 1)) * (n_slabs * 32u) + (lane & 1) * 16;
-    auto fetch = [&](int slab, int buf) __attribute__((always_inline)) {
-        slab = min(slab, n_slabs - 1);
-        if (xs_wave) wide_dma16(lds0 + kXsAt + buf * L::kXs + wave * 1024, xs_base + slab * 8, xs_src);
+        for (int k = 0; k < G; k++) src[k] = act_row(t16 + 16 * k) * row_bytes + piece * 16;
+        // Scales: lane pairs of the first waves, token 32 * wave + lane / 2.
+        const bool xs_wave = wave < L::kXs / 1024;
+        const float *xs_base = a.xs + (GROUPED ? 0 : static_cast<int64_t>(tok0) * (n_slabs * 8));
+        const uint32_t xs_src = act_row(32 * wave + (lane >> 1)) * (n_slabs * 32u) + (lane & 1) * 16;
+        auto fetch = [&](int slab, int buf) __attribute__((always_inline)) {
+            slab = min(slab, n_slabs - 1);
+            if (xs_wave) wide_dma16(lds0 + kXsAt + buf * L::kXs + wave * 1024, xs_base + slab * 8, xs_src);
 #pragma unroll
-        for (int k = 0; k < G; k++)
-            wide_dma16(lds0 + buf * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + slab * 256, src[k]);
-    };
-    // Weights: rows past the end repeat the last one.
-    const int first = min(row0, a.rows - 1), last = a.rows - 1 - first;  // (of this wave's rows)
-    const uint8_t *wq = a.quants + first * a.q_stride;
-    const uint8_t *wd = a.scales + first * a.s_stride;
-    constexpr int kRowsReq = 1024 / L::kRowBytes, kReqs = L::kQuants / 1024;
-    const uint32_t w_lds = lds0 + kWAt + wave * L::kWave;  // + slot * WAVES * kWave
-    uint32_t w_src[kReqs];
+            for (int k = 0; k < G; k++)
+                if (!GROUPED || 4 * wave + 16 * k < n_here)  // (what no token owns stays what it was: cells of its own, never stored)
+                    wide_dma16(lds0 + buf * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + slab * 256, src[k]);
+        };
+        // Weights: rows past the end repeat the last one.
+        const int first = min(row0, a.rows - 1), last = a.rows - 1 - first;  // (of this wave's rows)
+        const uint8_t *wq = a.quants + (band * a.rows + first) * a.q_stride;
+        const uint8_t *wd = a.scales + (band * a.rows + first) * a.s_stride;
+        constexpr int kRowsReq = 1024 / L::kRowBytes, kReqs = L::kQuants / 1024;
+        const uint32_t w_lds = lds0 + kWAt + wave * L::kWave;  // + slot * WAVES * kWave
+        uint32_t w_src[kReqs];
 #pragma unroll
-    for (int i = 0; i < kReqs; i++) {
-        const int r = kRowsReq * i + lane / (64 / kRowsReq);
-        const int slot = lane % (64 / kRowsReq);
-        const int p = FMT == CML_Q8_0 ? slot ^ (r & 15) : slot ^ ((r >> 1) & 7);
-        w_src[i] = static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(a.q_stride) + p * 16;
-    }
-    uint32_t d_src[RT];
-#pragma unroll
-    for (int r = 0; r < RT; r++) d_src[r] = static_cast<uint32_t>(min(16 * r + (lane >> 2), last)) * static_cast<uint32_t>(a.s_stride) + (lane & 3) * 4;
-    auto fetch_w = [&](int slab, int slot) __attribute__((always_inline)) {
-        slab = min(slab, n_slabs - 1);
-        const uint32_t to = w_lds + slot * (WAVES * L::kWave);
-#pragma unroll
-        for (int i = 0; i < kReqs; i++) wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
-#pragma unroll
-        for (int r = 0; r < RT; r++) wide_dma4(to + L::kQuants + r * 256, wd + slab * 16, d_src[r]);
-    };
-    constexpr int kAhead = (D - 1) * (G + kReqs + RT);  // requests that may be outstanding at the end of a step (some waves have more)
-
-    // Operands of a slab: the lane's octet of the eight blocks of either tile's row, the blocks' scales.
-    long bw[RT][8];
-    float dw[RT][8], md[RT][8];  // d_w; -12582912 * d_w
-    bool finite;
-    auto read_w = [&](int slot) __attribute__((always_inline)) {
-        const uint8_t *w_mine = slabs + kWAt + wave * L::kWave + slot * (WAVES * L::kWave);
-        uint32_t high = 0;
-#pragma unroll
-        for (int r = 0; r < RT; r++) {
-            const int row = 16 * r + n;
-            const uint4 d = *reinterpret_cast<const uint4 *>(w_mine + L::kQuants + row * 16);
-            const uint32_t dword[4] = {d.x, d.y, d.z, d.w};
-#pragma unroll
-            for (int b = 0; b < 8; b++) {
-                const uint32_t bits = (dword[b >> 1] >> (16 * (b & 1))) & 0xffffu;
-                dw[r][b] = f16_bits_to_f32(bits);
-                md[r][b] = -12582912.0f * dw[r][b];
-                high = max(high, bits & 0x7c00u);
-                if constexpr (FMT == CML_Q8_0) {
-                    const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8);
-                    bw[r][b] = __builtin_bit_cast(long, o);
-                } else {
-                    const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 128 + ((b ^ ((n >> 1) & 7)) << 4) + (kq & 1) * 8);
-                    v2i_w v;
-#pragma unroll
-                    for (int i = 0; i < 2; i++) {  // nibble - 8 as a signed byte
-                        const uint32_t nib = (static_cast<uint32_t>(o[i]) >> (4 * (kq >> 1))) & 0x0f0f0f0fu;
-                        v[i] = static_cast<int>((nib + 0x78787878u) ^ 0x80808080u);
-                    }
-                    bw[r][b] = __builtin_bit_cast(long, v);
-                }
-            }
+        for (int i = 0; i < kReqs; i++) {
+            const int r = kRowsReq * i + lane / (64 / kRowsReq);
+            const int slot = lane % (64 / kRowsReq);
+            const int p = FMT == CML_Q8_0 ? slot ^ (r & 15) : slot ^ ((r >> 1) & 7);
+            w_src[i] = static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(a.q_stride) + p * 16;
         }
-        finite = __builtin_amdgcn_ballot_w64(high == 0x7c00u) == 0;
-    };
-
-    // A operand of block b: octet kq of token n; the blocks' scales of tokens 4 kq .. + 3
-    uint32_t a_addr[8];
+        uint32_t d_src[RT];
 #pragma unroll
-    for (int b = 0; b < 8; b++) a_addr[b] = n * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8;
-
+        for (int r = 0; r < RT; r++) d_src[r] = static_cast<uint32_t>(min(16 * r + (lane >> 2), last)) * static_cast<uint32_t>(a.s_stride) + (lane & 3) * 4;
+        auto fetch_w = [&](int slab, int slot) __attribute__((always_inline)) {
+            slab = min(slab, n_slabs - 1);
+            const uint32_t to = w_lds + slot * (WAVES * L::kWave);
 #pragma unroll
-    for (int i = 0; i < D; i++) {
-        fetch(i, i);
-        fetch_w(i, i);
-    }
-    wide_wait<kAhead>();
-    read_w(0);
-    wide_barrier();
-
-    float acc[RT][G][4];
+            for (int i = 0; i < kReqs; i++) wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
 #pragma unroll
-    for (int r = 0; r < RT; r++)
-#pragma unroll
-        for (int g = 0; g < G; g++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[r][g][j] = 0.0f;
-
-    const v4i_w magic = {0x4b400000, 0x4b400000, 0x4b400000, 0x4b400000};
-
-    auto step = [&](const uint8_t *slab, const float *xs, auto fin) __attribute__((always_inline)) {
-        // Software pipeline over units of two blocks of a token group: while the matrix cores work on unit i + 1, the
-        // f32 steps of unit i run and the operands of unit i + 2 are read.
-        constexpr int kUnits = G * 4;
-        long av[3][2];
-        float4 xv[2][4];  // scales of four blocks, of the lane's four tokens
-        v4i_w d[2][RT][2];
-        auto read_a = [&](int i) __attribute__((always_inline)) {
-            const int g = i >> 2, u = i & 3;
-#pragma unroll
-            for (int e = 0; e < 2; e++) av[i % 3][e] = *reinterpret_cast<const long *>(slab + a_addr[2 * u + e] + g * 4096);
+            for (int r = 0; r < RT; r++) wide_dma4(to + L::kQuants + r * 256, wd + slab * 16, d_src[r]);
         };
-        auto read_x = [&](int i) __attribute__((always_inline)) {  // of units i and i + 1
-            const int g = i >> 2, h = (i >> 1) & 1;
+        constexpr int kAhead = (D - 1) * (G + kReqs + RT);  // requests that may be outstanding at the end of a step (some waves have more)
+
+        // Operands of a slab: the lane's octet of the eight blocks of either tile's row, the blocks' scales.
+        long bw[RT][8];
+        float dw[RT][8], md[RT][8];  // d_w; -12582912 * d_w
+        bool finite;
+        auto read_w = [&](int slot) __attribute__((always_inline)) {
+            const uint8_t *w_mine = slabs + kWAt + wave * L::kWave + slot * (WAVES * L::kWave);
+            uint32_t high = 0;
 #pragma unroll
-            for (int j = 0; j < 4; j++) xv[h][j] = *reinterpret_cast<const float4 *>(xs + (16 * g + 4 * kq + j) * 8 + 4 * h);
-        };
-        auto contract = [&](int i) __attribute__((always_inline)) {
+            for (int r = 0; r < RT; r++) {
+                const int row = 16 * r + n;
+                const uint4 d = *reinterpret_cast<const uint4 *>(w_mine + L::kQuants + row * 16);
+                const uint32_t dword[4] = {d.x, d.y, d.z, d.w};
 #pragma unroll
-            for (int e = 0; e < 2; e++)
+                for (int b = 0; b < 8; b++) {
+                    const uint32_t bits = (dword[b >> 1] >> (16 * (b & 1))) & 0xffffu;
+                    dw[r][b] = f16_bits_to_f32(bits);
+                    md[r][b] = -12582912.0f * dw[r][b];
+                    high = max(high, bits & 0x7c00u);
+                    if constexpr (FMT == CML_Q8_0) {
+                        const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8);
+                        bw[r][b] = __builtin_bit_cast(long, o);
+                    } else {
+                        const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 128 + ((b ^ ((n >> 1) & 7)) << 4) + (kq & 1) * 8);
+                        v2i_w v;
 #pragma unroll
-                for (int r = 0; r < RT; r++) d[i & 1][r][e] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i % 3][e], bw[r][2 * (i & 3) + e], magic, 0, 0, 0);
-        };
-        auto chain = [&](int i) __attribute__((always_inline)) {
-            const int g = i >> 2, u = i & 3, h = u >> 1;
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int b = 2 * u + e, k = 2 * (u & 1) + e;
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float x = k == 0 ? xv[h][j].x : k == 1 ? xv[h][j].y : k == 2 ? xv[h][j].z : xv[h][j].w;
-#pragma unroll
-                    for (int r = 0; r < RT; r++) {
-                        const float f = __builtin_bit_cast(float, static_cast<int>(d[i & 1][r][e][j]));
-                        const float p = decltype(fin)::value ? __builtin_fmaf(f, dw[r][b], md[r][b]) : (f - 12582912.0f) * dw[r][b];
-                        acc[r][g][j] = acc[r][g][j] + p * x;
+                        for (int i = 0; i < 2; i++) {  // nibble - 8 as a signed byte
+                            const uint32_t nib = (static_cast<uint32_t>(o[i]) >> (4 * (kq >> 1))) & 0x0f0f0f0fu;
+                            v[i] = static_cast<int>((nib + 0x78787878u) ^ 0x80808080u);
+                        }
+                        bw[r][b] = __builtin_bit_cast(long, v);
                     }
                 }
             }
-#pragma unroll
-            for (int r = 0; r < RT; r++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[r][g][j]));  // (keeps the compiler from sinking the chains to the store)
+            finite = __builtin_amdgcn_ballot_w64(high == 0x7c00u) == 0;
         };
-        read_a(0);
-        read_x(0);
-        read_a(1);
-        contract(0);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < kUnits; i++) {
-            if (i + 2 < kUnits) {
-                read_a(i + 2);
-                if ((i & 1) == 0) read_x(i + 2);
-            }
-            if (i + 1 < kUnits) contract(i + 1);
-            chain(i);
-            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-#pragma unroll
-            for (int m = 0; m < 2 * RT; m++) {
-                __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x2, 12, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
 
-    int buf = 0, slot = 0;  // of slab s: s % (D + 1), s % D
-    for (int s = 0; s < n_slabs; s++) {
-        fetch(s + D, buf == 0 ? D : buf - 1);  // (past the end the last slab again; the buffer of slab s - 1)
-        fetch_w(s + D, slot);                  // (slab s was read into registers before the barrier)
-        __builtin_amdgcn_sched_barrier(0);
-        const uint8_t *slab = slabs + buf * L::kSlab;
-        const float *xs = reinterpret_cast<const float *>(slabs + kXsAt + buf * L::kXs);
-        if (finite) step(slab, xs, std::true_type{});
-        else step(slab, xs, std::false_type{});
+        // A operand of block b: octet kq of token n; the blocks' scales of tokens 4 kq .. + 3
+        uint32_t a_addr[8];
+#pragma unroll
+        for (int b = 0; b < 8; b++) a_addr[b] = n * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8;
+
+#pragma unroll
+        for (int i = 0; i < D; i++) {
+            fetch(i, i);
+            fetch_w(i, i);
+        }
         wide_wait<kAhead>();
-        buf = buf == D ? 0 : buf + 1;
-        slot = slot == D - 1 ? 0 : slot + 1;
-        read_w(slot);
+        read_w(0);
         wide_barrier();
-    }
-    wide_wait<0>();  // (nothing may still be on its way into LDS that is given back)
 
+        float acc[RT][G][4];
 #pragma unroll
-    for (int r = 0; r < RT; r++) {
-        const int row = row0 + 16 * r + n;
-        if (row < a.rows) {
-            float *out = a.out + static_cast<int64_t>(tok0) * a.rows + row;
+        for (int r = 0; r < RT; r++)
 #pragma unroll
             for (int g = 0; g < G; g++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int t = 16 * g + 4 * kq + j;
-                    if (t < n_here) out[static_cast<int64_t>(t) * a.rows] = acc[r][g][j];
+                for (int j = 0; j < 4; j++) acc[r][g][j] = 0.0f;
+
+        const v4i_w magic = {0x4b400000, 0x4b400000, 0x4b400000, 0x4b400000};
+
+        auto step = [&](const uint8_t *slab, const float *xs, auto fin) __attribute__((always_inline)) {
+            // Software pipeline over units of two blocks of a token group: while the matrix cores work on unit i + 1, the
+            // f32 steps of unit i run and the operands of unit i + 2 are read.
+            constexpr int kUnits = G * 4;
+            long av[3][2];
+            float4 xv[2][4];  // scales of four blocks, of the lane's four tokens
+            v4i_w d[2][RT][2];
+            auto read_a = [&](int i) __attribute__((always_inline)) {
+                const int g = i >> 2, u = i & 3;
+#pragma unroll
+                for (int e = 0; e < 2; e++) av[i % 3][e] = *reinterpret_cast<const long *>(slab + a_addr[2 * u + e] + g * 4096);
+            };
+            auto read_x = [&](int i) __attribute__((always_inline)) {  // of units i and i + 1
+                const int g = i >> 2, h = (i >> 1) & 1;
+#pragma unroll
+                for (int j = 0; j < 4; j++) xv[h][j] = *reinterpret_cast<const float4 *>(xs + (16 * g + 4 * kq + j) * 8 + 4 * h);
+            };
+            auto contract = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+#pragma unroll
+                    for (int r = 0; r < RT; r++) d[i & 1][r][e] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i % 3][e], bw[r][2 * (i & 3) + e], magic, 0, 0, 0);
+            };
+            auto chain = [&](int i) __attribute__((always_inline)) {
+                const int g = i >> 2, u = i & 3, h = u >> 1;
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int b = 2 * u + e, k = 2 * (u & 1) + e;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float x = k == 0 ? xv[h][j].x : k == 1 ? xv[h][j].y : k == 2 ? xv[h][j].z : xv[h][j].w;
+#pragma unroll
+                        for (int r = 0; r < RT; r++) {
+                            const float f = __builtin_bit_cast(float, static_cast<int>(d[i & 1][r][e][j]));
+                            const float p = decltype(fin)::value ? __builtin_fmaf(f, dw[r][b], md[r][b]) : (f - 12582912.0f) * dw[r][b];
+                            acc[r][g][j] = acc[r][g][j] + p * x;
+                        }
+                    }
                 }
+#pragma unroll
+                for (int r = 0; r < RT; r++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[r][g][j]));  // (keeps the compiler from sinking the chains to the store)
+            };
+            read_a(0);
+            read_x(0);
+            read_a(1);
+            contract(0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < kUnits; i++) {
+                if (i + 2 < kUnits) {
+                    read_a(i + 2);
+                    if ((i & 1) == 0) read_x(i + 2);
+                }
+                if (i + 1 < kUnits) contract(i + 1);
+                chain(i);
+                __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+                for (int m = 0; m < 2 * RT; m++) {
+                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, 12, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+
+        int buf = 0, slot = 0;  // of slab s: s % (D + 1), s % D
+        for (int s = 0; s < n_slabs; s++) {
+            fetch(s + D, buf == 0 ? D : buf - 1);  // (past the end the last slab again; the buffer of slab s - 1)
+            fetch_w(s + D, slot);                  // (slab s was read into registers before the barrier)
+            __builtin_amdgcn_sched_barrier(0);
+            const uint8_t *slab = slabs + buf * L::kSlab;
+            const float *xs = reinterpret_cast<const float *>(slabs + kXsAt + buf * L::kXs);
+            if (finite) step(slab, xs, std::true_type{});
+            else step(slab, xs, std::false_type{});
+            wide_wait<kAhead>();
+            buf = buf == D ? 0 : buf + 1;
+            slot = slot == D - 1 ? 0 : slot + 1;
+            read_w(slot);
+            wide_barrier();
         }
+        wide_wait<0>();  // (nothing may still be on its way into LDS that is given back)
+
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            const int row = row0 + 16 * r + n;
+            if (row < a.rows) {
+                float *out = a.out + static_cast<int64_t>(a0 + tok0) * a.rows + row;
+#pragma unroll
+                for (int g = 0; g < G; g++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const int t = 16 * g + 4 * kq + j;
+                        if (t < n_here) out[static_cast<int64_t>(t) * a.rows] = acc[r][g][j];
+                    }
+            }
+        }
+        if constexpr (!GROUPED) return;
+        wide_barrier();  // (every wave's requests have arrived: the next column may use the buffers)
     }
 }
 
-template <int FMT, int G, int RT, int D>
-static int launch_b32_wide(B32WideArgs ka, hipStream_t st) {
+template <int FMT, int G, int RT, int D, bool GROUPED = false>
+static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
     typedef B32WideLds<FMT, G, RT, D> L;
     constexpr int kRows = kB32Waves * 16 * RT;
     ka.n_row_blocks = (ka.rows + kRows - 1) / kRows;
-    ka.n_cols = (ka.n_tokens + L::NTOK - 1) / L::NTOK;
+    ka.n_cols = GROUPED ? 1 : (ka.n_tokens + L::NTOK - 1) / L::NTOK;
     static std::atomic<bool> raised{false};  // per instantiation: allow more than 64 KB of dynamic LDS once
     if (!raised.load(std::memory_order_acquire)) {
-        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_b32_wide_kernel<FMT, G, RT, D>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_b32_wide_kernel<FMT, G, RT, D, GROUPED>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((gemm_b32_wide_kernel<FMT, G, RT, D>), dim3(wide_grid(ka.n_row_blocks, ka.n_cols)), dim3(64 * kB32Waves), L::kTotal, st, ka);
-    // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>"
-    CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D));
+    hipLaunchKernelGGL((gemm_b32_wide_kernel<FMT, G, RT, D, GROUPED>), dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * kB32Waves), L::kTotal, st, ka);
+    // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>[.grouped]"
+    CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D) + (GROUPED ? ".grouped" : ""));
     CML_HIP_TRY(hipGetLastError());
     return CML_OK;
 }
@@ -320,7 +341,7 @@ template <int FMT, int G, int RT, int D>
 static int b32_wide_visit(const B32WideArgs &ka, B32WideShape &best, float &cost, const B32WideShape *launch, hipStream_t st) {
     typedef B32WideLds<FMT, G, RT, D> L;
     static_assert(2 * L::kTotal <= 160 * 1024, "two workgroups per compute unit");
-    if (launch) return launch->g == G && launch->rt == RT && launch->d == D ? launch_b32_wide<FMT, G, RT, D>(ka, st) : -1;
+    if (launch) return launch->g == G && launch->rt == RT && launch->d == D ? launch_b32_wide<FMT, G, RT, D>(ka, 1, st) : -1;
     const B32WideShape s{G, RT, D};
     const float c = b32_wide_cost(ka.rows, (ka.n_tokens + 15) / 16, ka.n_slabs, s);
     if (c < cost) {
@@ -352,7 +373,22 @@ static int launch_b32_wide_fmt(const B32WideArgs &ka, hipStream_t st) {
     return b32_wide_each<FMT>(ka, s, cost, &s, st);
 }
 
-// A plain call on a weight that b32_mfma_usable accepts, activation scales 16-byte aligned.
+// Expert groups: columns of 16 assignments, of 32 from 12 on average (a second column of 16 reads the weight again: 32 experts, top-8, 2816 / 1408 at
+// 64 tokens Q8_0 203 us with columns of 16, 185 so; at 24 tokens 117 / 122), one row tile per wave (two: 118 / 126).
+template <int FMT>
+static int launch_b32_wide_grouped(const B32WideArgs &ka, const MatArgs &a, hipStream_t st) {
+    const int slots = static_cast<int>(a.group_ids ? a.max_active : a.n_groups);
+    const int g = env_int("CAMELID_HIP_WIDE_GROUPS", a.n_assign_total >= 12 * static_cast<int64_t>(slots) ? 2 : 1);
+    return g == 1 ? launch_b32_wide<FMT, 1, 1, 1, true>(ka, slots, st) : launch_b32_wide<FMT, 2, 1, 1, true>(ka, slots, st);
+}
+
+// Whether the offsets of a grouped call's activation rows fit 32 bits and its weight and scales can be read 16 bytes at a time.
+bool gemm_b32_wide_serves_groups(const MatArgs &a) {
+    return b32_mfma_usable(a.w) && reinterpret_cast<uintptr_t>(a.scales) % 16 == 0 &&
+           std::max(a.n_assign_total, a.n_tokens) * a.w->nb * 32 < (int64_t{1} << 32);
+}
+
+// On a weight that b32_mfma_usable accepts, activation scales 16-byte aligned; grouped: gemm_b32_wide_serves_groups.
 int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
     const cml_weight *w = a.w;
     B32WideArgs ka{};
@@ -360,12 +396,16 @@ int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
     ka.q_stride = w->planes.row_stride[0];
     ka.scales = w->planes.p[1];
     ka.s_stride = w->planes.row_stride[1];
-    ka.rows = static_cast<int>(w->rows);
+    ka.rows = static_cast<int>(a.group_offsets ? a.band_rows : w->rows);
     ka.n_slabs = static_cast<int>(w->nb / 8);
     ka.q = a.q;
     ka.xs = a.scales;
     ka.out = a.out;
     ka.n_tokens = static_cast<int>(a.n_tokens);
+    ka.group_offsets = a.group_offsets;
+    ka.group_rows = a.group_rows;
+    ka.group_ids = a.group_ids;
+    if (a.group_offsets) return w->fmt == CML_Q8_0 ? launch_b32_wide_grouped<CML_Q8_0>(ka, a, st) : launch_b32_wide_grouped<CML_Q4_0>(ka, a, st);
     return w->fmt == CML_Q8_0 ? launch_b32_wide_fmt<CML_Q8_0>(ka, st) : launch_b32_wide_fmt<CML_Q4_0>(ka, st);
 }
 

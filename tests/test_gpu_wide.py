@@ -136,3 +136,24 @@ def test_wide_b32_on_a_row_band(name, fmt, tag):
     assert G.same_bits(band, whole[:, 7:157])
     with G.env(CAMELID_HIP_MFMA_WIDE=0):
         assert G.same_bits(whole, G.gpu_gemm(w, s, q))
+
+
+# gate | up fused (gathered rows), down on rows of whole slabs; groups of none, one, past a column; a band that ends inside a workgroup
+@pytest.mark.parametrize("E,k,hidden,ff,T", [(16, 4, 768, 512, 40), (8, 3, 256, 256, 1), (5, 2, 1280, 768, 33)])
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_expert_groups_are_bitwise_the_gemv(name, fmt, tag, E, k, hidden, ff, T):
+    gate_up = Weight.upload(fmt, E * 2 * ff, hidden, G.synth_weight(fmt, E * 2 * ff, hidden, seed=E))
+    down = Weight.upload(fmt, E * hidden, ff, G.synth_weight(fmt, E * hidden, ff, seed=E + 1))
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T + 1, hidden)).astype(np.float32)  # (a batch: a single token has a path of its own)
+    logits = rng.standard_normal((T + 1, E)).astype(np.float32)
+    logits[:, 0] += 1.0
+    logits[:, E - 1] -= 50.0
+    idx, weight, _, _ = gpu_route(logits, k)
+    run = lambda: gpu_moe(gate_up, None, down, E, k, idx, weight, x, glu=1)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        ref = run()
+    for g in (1, 2):
+        G.say(f"wide {name} experts E={E} k={k} {hidden}/{ff} T={T + 1} groups={g}")
+        with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g), G.engaged(rf"^{tag}\.mfma\.wide\.g{g}r1d1\.grouped$", none=(r"\.dot\.",)):
+            assert G.same_bits(run(), ref)
