@@ -648,8 +648,11 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_gr
     // Plain calls: the wide kernel wherever several waves per row tile do not serve.  us per launch, the kernel below / wide, Q8_0: 14336 x 4096
     // at 6 / 16 / 24 / 64 / 200 / 512 tokens 20.4 / 19.7, 20.5 / 19.8, 34.5 / 21.2, 67 / 24, 217 / 61, 434 / 115; 4096 x 14336 at 12 / 64 / 512
     // 49 / 39, 73 / 39, 541 / 116; 11008 x 2048 at 6 / 16 10.6 / 8.4, 11.0 / 8.5; 32000 x 4096 at 16 35 / 32; 2048 x 2048 at 24 / 200 10.4 / 7.6, 19.3 / 10.
-    // Q4_0: 128256 x 3072 at 4 / 16 / 32 / 64 52.4 / 50.9, 57.7 / 51.5, 82 / 64, 156 / 101; 14336 x 4096 at 16 / 200 18.0 / 18.5, 200 / 62.
-    if (can_wide && (kpar != 0 || ka.n_tokens > 16)) return launch_gemm_b32_wide(a, st);
+    // Q4_0: 128256 x 3072 at 16 / 32 / 64 57.7 / 51.5, 82 / 64, 156 / 101; 14336 x 4096 at 16 / 200 18.0 / 18.5, 200 / 62.
+    // (up to 16 tokens on weights of more than 49152 rows only 13 and more, on rows of 8 slabs and more: 90000 x 3072 at 6 / 16 Q4_0 41.1 / 44.3, 44.3 / 44.2,
+    // Q8_0 62.8 / 65.7, 67.8 / 66.4; 128256 x 1536 Q4_0 28.1 / 30.6, 30.2 / 30.9; 62848 x 2304 at 16 24.0 / 21.8; 40000 x 5120 at 6 34.7 / 30.9)
+    const bool tall_few = ka.n_tokens <= 16 && ka.rows > 49152 && (ka.n_tokens <= 12 || ka.n_slabs < 8);
+    if (can_wide && !tall_few && (kpar != 0 || ka.n_tokens > 16)) return launch_gemm_b32_wide(a, st);
     switch (env_int("CAMELID_HIP_B32_MFMA_SHAPE", 0)) {
         case 1: return launch_b32_mfma_p<FMT, 1, 1>(ka, n_groups, st);   // 16 tokens, 1 wave per row tile
         case 2: return launch_b32_mfma_p<FMT, 2, 1>(ka, n_groups, st);   // 32 tokens, 1 wave per row tile

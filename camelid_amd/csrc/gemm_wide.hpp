@@ -387,11 +387,11 @@ struct WideShape {
     int g = 0, waves = 0, ks = 1;
 };
 
-// Estimated us of a launch (less a constant), fitted on MI355X to 1800 launches: Q4_K and Q6_K weights of six and five shapes with
-// the three K cuts, 24 to 512 tokens, every shape of the kernel.  A step costs a fixed latency -- more for workgroups of four
-// waves and for two wave groups in F's measure --, and for every wave on a SIMD the unpacking of a super-block and then 0.12 us per token
-// group.  `rounds`: workgroups over what is resident at once, between their average and the last round at full length.  The shape
-// with the lowest estimate was the fastest or within 1 % of it on average over those launches (28 % off at worst).
+// Estimated us of a launch (less a constant), fitted on MI355X: Q6_K weights of five shapes with the three K cuts, 24 to 512 tokens, every shape of the
+// kernel; Q4_K four weights with the three cuts, 24 to 512 tokens, 2 to 8 groups (the lowest estimate was the fastest shape in all 16 pairs of weight and
+// tokens).  A step costs a fixed latency -- more for workgroups of four waves and for two wave groups in F's measure --, and for every wave on a
+// SIMD the unpacking of a super-block and then 0.12 us per token group.  `rounds`: workgroups over what is resident at once, between their average and
+// the last round at full length.
 template <class F>
 static float wide_cost(int64_t tiles, int groups, int n_sb, int ksplit, const WideShape &s, int lds) {
     const int rt = s.waves / s.ks;
