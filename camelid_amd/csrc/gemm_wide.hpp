@@ -38,14 +38,18 @@ typedef _Float16 v4h_w __attribute__((ext_vector_type(4)));
 // One wave's 1 KB: lane l's 16 bytes at base + off (off per lane) to LDS byte lds_byte + 16 * l (lds_byte wave-uniform).
 // Written as assembly because the compiler, which cannot tell which LDS bytes such a load will
 // write, puts a wait for all of them in front of every later LDS read; here the caller waits
-// (wide_wait) where the data is first needed.  s_nop: one wait state between a scalar write of m0
-// and an instruction that addresses LDS through it.
+// (wide_wait) where the data is first needed.  The compiler does not look inside for the wait states the hardware wants
+// either: five between a vector instruction that writes a scalar register (v_readlane: a base that was spilled) and a memory
+// instruction that addresses through it, one between a write of m0 and an instruction that addresses LDS through it.
+// The scalar move of the base is both: the hardware holds it back until the base is written, and it stands behind m0.
 __device__ __forceinline__ void wide_dma16(uint32_t lds_byte, const void *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_byte), "v"(off), "s"(base) : "memory", "m0");
+    const void *at;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(at) : "s"(lds_byte), "v"(off), "s"(base) : "memory", "m0");
 }
 // The same with 4 bytes per lane.
 __device__ __forceinline__ void wide_dma4(uint32_t lds_byte, const void *base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_byte), "v"(off), "s"(base) : "memory", "m0");
+    const void *at;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dword %2, %0" : "=&s"(at) : "s"(lds_byte), "v"(off), "s"(base) : "memory", "m0");
 }
 // Waits until at most OUT of the wave's vector-memory operations are outstanding (loads complete in order).
 template <int OUT>
