@@ -19,7 +19,7 @@ int q4k_ksplit_for(int64_t rows, int64_t n_sb);  // gemv_q4k.hip: the matvec ker
 struct Q4KWide {
     static constexpr const char *kName = "q4k";
     static constexpr int kTileBytes = 2304, kFetches = 3;  // LDS bytes of a wave's super-block (pieces a | pieces b | headers), requests for it
-    static constexpr float kStepUs = 0.40f, kTwoPartsUs = 0.10f, kFourWavesUs = 0.20f, kUnpackUs = 0.06f;  // (wide_cost)
+    static constexpr float kStepUs = 0.25f, kPartUs = 0.10f, kUnpackUs = 0.12f, kCellsUs = 0.06f, kSlabUs = 0.09f;  // (wide_cost)
     static constexpr bool kRunSums = true;
     struct Weight {
         const uint8_t *w;  // tiled layout [super-block][tile][2304 B]: 16 headers, then pieces a and b as [16 rows][4 chunks][16 B]

@@ -20,7 +20,7 @@ int q6k_ksplit_for(int64_t rows, int64_t n_sb);  // gemv_q6k.hip: the matvec ker
 struct Q6KWide {
     static constexpr const char *kName = "q6k";
     static constexpr int kTileBytes = 2048 + 1024 + 256 + 256, kFetches = 5;  // LDS bytes of a wave's super-block (ql | qh | scales | d), requests for it
-    static constexpr float kStepUs = 0.48f, kTwoPartsUs = 0.18f, kFourWavesUs = 0.00f, kUnpackUs = 0.12f;  // (wide_cost)
+    static constexpr float kStepUs = 0.30f, kPartUs = 0.18f, kUnpackUs = 0.12f, kCellsUs = 0.12f, kSlabUs = 0.00f;  // (wide_cost)
     static constexpr bool kRunSums = false;
     struct Weight {
         const uint8_t *ql, *qh, *sc, *d;

@@ -391,22 +391,23 @@ struct WideShape {
     int g = 0, waves = 0, ks = 1;
 };
 
-// Estimated us of a launch (less a constant), fitted on MI355X: Q6_K weights of five shapes with the three K cuts, 24 to 512 tokens, every shape of the
-// kernel; Q4_K four weights with the three cuts, 24 to 512 tokens, 2 to 8 groups (the lowest estimate was the fastest shape in all 16 pairs of weight and
-// tokens).  A step costs a fixed latency -- more for workgroups of four waves and for two wave groups in F's measure --, and for every wave on a
-// SIMD the unpacking of a super-block and then 0.12 us per token group.  `rounds`: workgroups over what is resident at once, between their average and
-// the last round at full length.
+// Estimated us of a launch (less a constant), fitted on MI355X to every shape of the kernel on cold weights (more than the last-level cache holds between
+// two launches on one) of 256 to 65536 rows and 512 to 14336 values with the three K cuts: Q6_K 1669 pairs of weight and tokens (5 to 512), Q4_K 1397 (33 to
+// 512).  The shape with the lowest estimate is on average 0.8 % / 0.7 % slower than the fastest (an earlier fit to few weights, some of them cached, took Q4_K
+// 4.3 % off).  A step costs a fixed latency, more for two wave groups; for every wave on a SIMD the unpacking of a super-block and the cells of its token groups;
+// and per token group the activation slabs that the compute unit's workgroups fetch (from three on they share what the cache holds).  Workgroups fill an XCD's 32
+// compute units row block by row block (wide_block).  `rounds`: workgroups over what is resident at once, between their average and the last round at full length.
 template <class F>
 static float wide_cost(int64_t tiles, int groups, int n_sb, int ksplit, const WideShape &s, int lds) {
     const int rt = s.waves / s.ks;
-    const int64_t wgs = (tiles + rt - 1) / rt * ((groups + s.g - 1) / s.g);
+    const int64_t blocks = (tiles + rt - 1) / rt, per_xcd = (blocks + 7) / 8 * ((groups + s.g - 1) / s.g);
     const int resident = std::min(160 * 1024 / lds, 8 / s.waves);  // (registers: two waves per SIMD)
-    const float per_cu = wgs / 256.0f, full = per_cu / resident;
+    const float per_cu = per_xcd / 32.0f, full = per_cu / resident;
     const float rounds = full <= 1.0f ? 1.0f : 0.4f * full + 0.6f * std::ceil(full);
-    const float m = (per_cu > 1.0f ? std::min<float>(resident, std::ceil(per_cu)) : 1.0f) * s.waves / 4;  // waves per SIMD
+    const int here = per_cu > 1.0f ? resident : 1;
+    const float waves = here * s.waves / 4;  // per SIMD
     const int mid = s.ks == 2 ? ksplit / 2 * n_sb / ksplit : 0, steps = std::max(mid, n_sb - mid);
-    const float step = F::kStepUs + (s.ks == 2 ? F::kTwoPartsUs : 0.0f) + (s.waves == 4 ? F::kFourWavesUs : 0.0f);
-    return rounds * steps * (step + m * (F::kUnpackUs + 0.12f * s.g));
+    return rounds * steps * (F::kStepUs + F::kPartUs * s.ks + F::kUnpackUs * waves + s.g * (F::kCellsUs * waves + F::kSlabUs * std::min(3, s.ks * here)));
 }
 
 template <class F, int G, int WAVES, int KS>

@@ -157,3 +157,23 @@ def test_wide_b32_expert_groups_are_bitwise_the_gemv(name, fmt, tag, E, k, hidde
         G.say(f"wide {name} experts E={E} k={k} {hidden}/{ff} T={T + 1} groups={g}")
         with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g), G.engaged(rf"^{tag}\.mfma\.wide\.g{g}r1d1\.grouped$", none=(r"\.dot\.",)):
             assert G.same_bits(run(), ref)
+
+
+# Which kernel a call without knobs takes, on either side of each line of the rules
+ROUTES = [
+    ("Q4_K", 2560, 4096, 33, r"^q4k\.mfma\.wide\.g1w4\.ksplit2$"),  # the smallest workgroups, where they alone have a compute unit each
+]
+
+
+@pytest.mark.parametrize("name,rows,cols,n,kernel", ROUTES)
+def test_calls_take_the_kernel_that_is_ahead(name, rows, cols, n, kernel):
+    fmt = {"Q4_K": B.CML_Q4_K, "Q6_K": B.CML_Q6_K, "Q8_0": B.CML_Q8_0, "Q4_0": B.CML_Q4_0}[name]
+    w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=rows + n))
+    x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    G.say(f"route {name} {rows}x{cols} n={n}")
+    with G.engaged(kernel, none=(r"\.mfma\.",) if ".dot" in kernel else (r"\.dot\.",)):
+        got = G.gpu_matmul_f32(w, x)
+    # the packed-dot kernel on the same inputs
+    with G.env(CAMELID_HIP_Q4K_MFMA_MIN_TOKENS=1 << 30, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1 << 30, CAMELID_HIP_B32_MFMA_MIN_TOKENS=1 << 30, CAMELID_HIP_FUSED_QUANT=0), \
+            G.engaged(r"\.dot\.", none=(r"\.mfma\.",)):
+        assert G.same_bits(got, G.gpu_matmul_f32(w, x))
