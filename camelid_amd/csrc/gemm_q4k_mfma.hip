@@ -1092,6 +1092,24 @@ static int launch_mfma(const Q4KMfmaArgs &ka, int n_groups, hipStream_t st) {
     return ka.ksplit > 1 ? launch_mfma_entry<GPW, TB, true, 1>(ka, n_groups, st) : launch_mfma_entry<GPW, TB, false, 1>(ka, n_groups, st);
 }
 
+// Plain calls of more than 32 tokens on a weight whose K is cut two or four ways: whether the launch with one wave per K part (32 tokens per workgroup)
+// beats the wide kernel, whose workgroups of two row tiles or more leave compute units idle where a weight has few tiles.  us per launch, this kernel /
+// the wide one's fastest shape, weights cold in every cache:
+//   cut four ways, up to one workgroup per compute unit: 1024 x 4096 at 48 / 100 tokens 7.1 / 8.8, 7.2 / 8.8; 1024 x 14336 at 48 17.8 / 21.6;
+//     up to two, where the wide kernel's smallest workgroups come to more than one as well: 2560 x 8192 at 64 15.9 / 17.3, 2048 x 8192 at 80 15.9 / 17.2, 512 x 11008 at 300
+//     19.4 / 21.3 -- unless more than a third of a part is added to fill this kernel's steps of four super-blocks (parts of five: 2048 x 5120 at 80 1.07 times the wide kernel's time);
+//   cut two ways: parts of four super-blocks up to two workgroups per unit: 2048 x 2048 at 48 / 128 6.1 / 6.2, 6.3 / 6.9; longer ones as above: 2048 x 3072 at 80 8.2 / 8.4.
+// A third workgroup per unit loses: 3072 x 8192 at 80 tokens 23.6 / 17.5, 3072 x 2048 8.4 / 7.0.
+static bool mfma_ksplit_beats_wide(int64_t tiles, int64_t n_tokens, int n_sb, int ksplit) {
+    if ((ksplit != 2 && ksplit != 4) || n_sb > 512) return false;  // (longer rows do not fit this kernel's LDS)
+    const int64_t workgroups = tiles * ((n_tokens + 31) / 32), wide_workgroups = (tiles + 1) / 2 * ((n_tokens + 15) / 16);
+    const int part = (n_sb + ksplit - 1) / ksplit, idle = -part & 3;
+    if (workgroups > 512) return false;
+    if (ksplit == 2 && part <= 4) return true;
+    if (workgroups <= 256) return ksplit == 4;
+    return wide_workgroups > 256 && (ksplit == 2 || 3 * idle <= part);
+}
+
 // Q4_K matmul on the matrix cores: plain calls, or grouped by expert (mixture of experts).
 int launch_gemm_q4k_mfma(const MatArgs &a, hipStream_t st) {
     const cml_weight *w = a.w;
@@ -1127,7 +1145,7 @@ int launch_gemm_q4k_mfma(const MatArgs &a, hipStream_t st) {
     // workgroup columns (grid.y), each a pass over the weight.  The other shapes stay selectable
     // for tuning.
     const int shape = env_int("CAMELID_HIP_Q4K_MFMA_SHAPE", 0);
-    // The wide kernel.  Plain: more than 32 tokens (14336 x 4096 at 24 / 40 / 64 / 128 / 200 / 512 tokens, this kernel / wide: 13.1 / 15.7,
+    // The wide kernel.  Plain: more than 32 tokens, but for small weights (above) (14336 x 4096 at 24 / 40 / 64 / 128 / 200 / 512 tokens, this kernel / wide: 13.1 / 15.7,
     // 18.8 / 17.8, 19.3 / 17.8, 30 / 24, 54 / 36, 98 / 76 us; 4096 x 14336 at 24 / 64 / 200 / 512: 18.8 / 20.9, 28.4 / 27.5, 88 / 49, 185 / 82).
     // Expert groups: more than 12 assignments each on average where the launch has the tiles to fill the chip with its larger workgroups, from 24 on where
     // a second token column would read the weight again (layer of 8 experts, top-2, us: 4096 / 14336 at 32 / 48 / 64 / 128 tokens 162 / 176, 217 / 190,
@@ -1136,7 +1154,8 @@ int launch_gemm_q4k_mfma(const MatArgs &a, hipStream_t st) {
     const int wide = env_int("CAMELID_HIP_MFMA_WIDE", 1);  // 0 = never, 1 = by shape, 2 = always
     if (shape == 0 && wide) {
         const int64_t slots = grouped ? ng / (a.w2 ? 2 : 1) : 1, tiles = static_cast<int64_t>(ka.rows / 16) * ng;
-        const bool pays = !grouped ? a.n_tokens > 32 : (tiles > 2048 && a.n_assign_total > 12 * slots) || (tiles > 1024 && a.n_assign_total >= 24 * slots);
+        const bool pays = !grouped ? a.n_tokens > 32 && !mfma_ksplit_beats_wide((ka.rows + ka.row_skip + 15) / 16, a.n_tokens, ka.n_sb, ka.ksplit)
+                                   : (tiles > 2048 && a.n_assign_total > 12 * slots) || (tiles > 1024 && a.n_assign_total >= 24 * slots);
         const bool reach = !grouped || std::max(a.n_assign_total, a.n_tokens) * ka.n_sb * 256 < (int64_t{1} << 32);
         if ((wide == 2 || pays) && reach) return launch_gemm_q4k_wide(a, st);
     }

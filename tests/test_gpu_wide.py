@@ -162,6 +162,12 @@ def test_wide_b32_expert_groups_are_bitwise_the_gemv(name, fmt, tag, E, k, hidde
 # Which kernel a call without knobs takes, on either side of each line of the rules
 ROUTES = [
     ("Q4_K", 2560, 4096, 33, r"^q4k\.mfma\.wide\.g1w4\.ksplit2$"),  # the smallest workgroups, where they alone have a compute unit each
+    ("Q4_K", 1024, 4096, 48, r"^q4k\.mfma\.ksplit4"),  # K cut four ways, a workgroup of the narrow kernel per compute unit at most
+    ("Q4_K", 4096, 4096, 33, r"^q4k\.mfma\.ksplit4"),  # up to two, the wide kernel's come to more than one as well
+    ("Q4_K", 2048, 5120, 80, r"^q4k\.mfma\.wide\."),  # K parts of five super-blocks
+    ("Q4_K", 2048, 2048, 100, r"^q4k\.mfma\.ksplit2"),  # cut two ways, parts of four
+    ("Q4_K", 2056, 2048, 129, r"^q4k\.mfma\.wide\."),  # a third workgroup per compute unit
+    ("Q4_K", 2048, 1024, 33, r"^q4k\.mfma\.wide\."),  # no cut
 ]
 
 
