@@ -1147,15 +1147,18 @@ int launch_gemm_q4k_mfma(const MatArgs &a, hipStream_t st) {
     const int shape = env_int("CAMELID_HIP_Q4K_MFMA_SHAPE", 0);
     // The wide kernel.  Plain: more than 32 tokens, but for small weights (above) (14336 x 4096 at 24 / 40 / 64 / 128 / 200 / 512 tokens, this kernel / wide: 13.1 / 15.7,
     // 18.8 / 17.8, 19.3 / 17.8, 30 / 24, 54 / 36, 98 / 76 us; 4096 x 14336 at 24 / 64 / 200 / 512: 18.8 / 20.9, 28.4 / 27.5, 88 / 49, 185 / 82).
-    // Expert groups: more than 12 assignments each on average where the launch has the tiles to fill the chip with its larger workgroups, from 24 on where
-    // a second token column would read the weight again (layer of 8 experts, top-2, us: 4096 / 14336 at 32 / 48 / 64 / 128 tokens 162 / 176, 217 / 190,
-    // 205 / 197, 340 / 256; 2048 / 8192 at 64 tokens 92 / 75; 2048 / 2048 at 128 tokens 61 / 48; 1024 / 2048 at 100 tokens 35 / 34).
+    // Expert groups: from 24 assignments each on average, where a second token column would read the weight again; from 12 on weights whose K is cut (which this kernel walks
+    // inside the lane there) from 1024 tiles on, and on the gate | up pair where rows of more than 16 super-blocks keep this kernel to one token group per wave.  Layer of 8
+    // experts, top-2, us, both launches here / gate and up wide / both wide: 4096 / 14336 at 32 / 64 / 90 / 128 tokens 168, 220, 244, 349 / -, 217, 248, - / 179, 202, 224, 271;
+    // 2048 / 8192 at 64 / 90 91, 98 / 93, 102 / 87, 93; 3072 / 8192 at 56 128 / 128 / 104; 4096 / 4096 at 72 84 / 87 / 84; 1024 / 14336 at 64 (down 512 tiles) 89 / 86 / 103;
+    // 6144 / 16384 at 56 408 / - / 301.
     // (32-bit offsets reach the activation rows)
     const int wide = env_int("CAMELID_HIP_MFMA_WIDE", 1);  // 0 = never, 1 = by shape, 2 = always
     if (shape == 0 && wide) {
         const int64_t slots = grouped ? ng / (a.w2 ? 2 : 1) : 1, tiles = static_cast<int64_t>(ka.rows / 16) * ng;
+        const bool from12 = a.w2 ? tiles > 2048 && ka.n_sb > 16 : tiles > 2048 || (ka.ksplit > 1 && tiles >= 1024);
         const bool pays = !grouped ? a.n_tokens > 32 && !mfma_ksplit_beats_wide((ka.rows + ka.row_skip + 15) / 16, a.n_tokens, ka.n_sb, ka.ksplit)
-                                   : (tiles > 2048 && a.n_assign_total > 12 * slots) || (tiles > 1024 && a.n_assign_total >= 24 * slots);
+                                   : (from12 && a.n_assign_total > 12 * slots) || (tiles > 1024 && a.n_assign_total >= 24 * slots);
         const bool reach = !grouped || std::max(a.n_assign_total, a.n_tokens) * ka.n_sb * 256 < (int64_t{1} << 32);
         if ((wide == 2 || pays) && reach) return launch_gemm_q4k_wide(a, st);
     }

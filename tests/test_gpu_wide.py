@@ -183,3 +183,20 @@ def test_calls_take_the_kernel_that_is_ahead(name, rows, cols, n, kernel):
     with G.env(CAMELID_HIP_Q4K_MFMA_MIN_TOKENS=1 << 30, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1 << 30, CAMELID_HIP_B32_MFMA_MIN_TOKENS=1 << 30, CAMELID_HIP_FUSED_QUANT=0), \
             G.engaged(r"\.dot\.", none=(r"\.mfma\.",)):
         assert G.same_bits(got, G.gpu_matmul_f32(w, x))
+
+
+# 10, 18 and 25 assignments per expert on average: both launches narrow; down (K cut, 1024 tiles) wide; both, two token groups per column
+@pytest.mark.parametrize("T,expect,none", [(40, (r"^q4k\.mfma\.(tile|serial_split)\..*grouped",), (r"\.wide\.",)),
+                                           (72, (r"^q4k\.mfma\.wide\.g2w4\.serial_split\.grouped$", r"^q4k\.mfma\.(tile|serial_split)\..*grouped"), ()),
+                                           (100, (r"^q4k\.mfma\.wide\.g2w4\.serial_split\.grouped$",), ())])
+def test_expert_groups_take_the_kernel_that_is_ahead(T, expect, none):
+    E, k, hidden, ff = 8, 2, 2048, 2048
+    w = experts(E, hidden, ff, 3)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    idx, weight, _, _ = gpu_route(rng.standard_normal((T, E)).astype(np.float32), k)
+    G.say(f"expert groups, default dispatch, T={T}")
+    with G.engaged(*expect, none=none):
+        got = gpu_moe(*w, E, k, idx, weight, x)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        assert G.same_bits(got, gpu_moe(*w, E, k, idx, weight, x))
