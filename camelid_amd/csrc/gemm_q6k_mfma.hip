@@ -441,15 +441,19 @@ int launch_gemm_q6k_mfma(const MatArgs &a, hipStream_t st) {
     const int ng = grouped ? (a.group_ids ? a.max_active : a.n_groups) : 1;
     const int shape = env_int("CAMELID_HIP_Q6K_MFMA_SHAPE", 0);
     // The wide kernel (one product of code and scale per weight instead of one integer multiply-add per cell and sub-block):
-    // any batch of more than 16 tokens, and smaller ones on weights without a K cut.  us per launch, this kernel / wide:
+    // any batch of more than 16 tokens, and most smaller ones on weights without a K cut.  us per launch, this kernel / wide:
     // 4096 x 14336 at 16 / 32 / 64 / 512 tokens 18.2 / 24.6, 27.0 / 24.7, 41 / 27, 281 / 81; 4096 x 4096 8.2 / 9.3, 10.6 / 9.5,
-    // 15.5 / 10.4, 90 / 27; uncut 18944 x 3584 at 8 / 16 / 37 / 512: 21.0 / 18.4, 21.2 / 18.5, 44 / 23, 204 / 91;
-    // 128256 x 3072 at 16 / 64: 78 / 77, 145 / 104.
+    // 15.5 / 10.4, 90 / 27; uncut 18944 x 3584 at 8 / 16 / 37 / 512: 21.0 / 18.4, 21.2 / 18.5, 44 / 23, 204 / 91; 128256 x 3072 at 16 / 64: 78 / 77, 145 / 104.
     const int wide = env_int("CAMELID_HIP_MFMA_WIDE", 1);  // 0 = never, 1 = by shape, 2 = always
-    // (up to 16 tokens on short rows of tall weights the stream is the same and this kernel's rounds are shorter: 81872 x 1536 at 6 / 16 25.4 / 27.4,
-    // 26.3 / 28.0; 128256 x 2048 50.4 / 51.1, 53.2 / 53.0; 50000 x 2560 31.3 / 30.8; 32000 x 1024 8.7 / 8.7; 20000 x 512 6.5 / 5.8)
-    const bool tall_short = a.n_tokens <= 16 && ka.rows > 49152 && ka.n_sb <= 8;
-    if (!grouped && shape == 0 && wide && (wide == 2 || a.n_tokens > 16 || (ka.ksplit == 1 && !tall_short))) return launch_gemm_q6k_wide(a, st);
+    // Up to 16 tokens this kernel keeps weights whose row tiles come to at most one wave per SIMD, its steps being shorter (8200 x 512 / 1024 at 8 tokens 4.8 / 4.9,
+    // 6.2 / 6.5; 16384 x 3072 / 4096 / 8192 at 5 14.0 / 14.6, 17.6 / 18.0, 31.6 / 32.3; 14336 x 14336 48.2 / 46.5), and short rows of tall weights, where either kernel does
+    // little but start (40000 x 512 / 1024 at 8 7.2 / 8.3, 11.8 / 12.3; 49000 x 1536 / 2048 17.8 / 18.7, 21.6 / 21.5; 81872 x 1536 25.4 / 27.4; 128256 x 2048 at 6 50.4 / 51.1).
+    // Up to 32: rows of four super-blocks, one phase of this kernel, while its tiles are few (6144 x 1024 at 17 / 32 6.2 / 6.4), and the shortest of tall weights
+    // (56000 x 512 at 17 / 32 10.7 / 11.6, 11.6 / 12.3).
+    const int tiles16 = (ka.rows + 15) / 16;
+    const bool stays = a.n_tokens <= 16 ? ka.ksplit > 1 || (tiles16 <= 1024 && ka.n_sb <= 32) || (ka.rows > 32768 && ka.n_sb <= 6) || (ka.rows > 49152 && ka.n_sb <= 8)
+                                        : a.n_tokens <= 32 && ((tiles16 <= 512 && ka.n_sb == 4) || (ka.rows > 49152 && ka.n_sb <= 2));
+    if (!grouped && shape == 0 && wide && (wide == 2 || !stays)) return launch_gemm_q6k_wide(a, st);
     // K split across waves where the matvec kernel splits K two or four ways and the launch has
     // fewer row tiles than the chip has SIMDs: 16 or 32 tokens per workgroup, more tokens = more
     // workgroup columns.

@@ -168,6 +168,12 @@ ROUTES = [
     ("Q4_K", 2048, 2048, 100, r"^q4k\.mfma\.ksplit2"),  # cut two ways, parts of four
     ("Q4_K", 2056, 2048, 129, r"^q4k\.mfma\.wide\."),  # a third workgroup per compute unit
     ("Q4_K", 2048, 1024, 33, r"^q4k\.mfma\.wide\."),  # no cut
+    ("Q6_K", 8200, 1024, 8, r"^q6k\.mfma\.tile\."),  # at most one wave per SIMD
+    ("Q6_K", 16400, 1024, 8, r"^q6k\.mfma\.wide\."),  # more
+    ("Q6_K", 33000, 512, 16, r"^q6k\.mfma\.tile\."),  # short rows of a tall weight
+    ("Q6_K", 8192, 1024, 32, r"^q6k\.mfma\.tile\."),  # rows of four super-blocks
+    ("Q6_K", 8192, 1024, 33, r"^q6k\.mfma\.wide\."),  # more tokens
+    ("Q6_K", 8192, 1280, 17, r"^q6k\.mfma\.wide\."),  # longer rows
 ]
 
 
