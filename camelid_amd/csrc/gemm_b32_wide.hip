@@ -324,17 +324,18 @@ struct B32WideShape {
     int g = 0, rt = 0, d = 0;
 };
 
-// Estimated us of a launch (less a constant), fitted on MI355X to 750 launches of five weight shapes in both formats, 12 to 512 tokens.  A slab costs a
-// fixed latency and, for every wave on a SIMD and row tile, 0.165 us and 0.15 us per token group (a wave alone on its
-// SIMD stalls where two overlap: 1.4, not 1, times that).  A second slab ahead shortens the latency of long rows walked with one token
-// group (4096 x 14336 at 64 tokens 52 -> 40 us) and costs LDS elsewhere.  The shape with the lowest estimate was within 1.5 % of the
-// fastest on average (12 % off at worst).
+// Estimated us of a launch (less a constant), fitted on MI355X to 2200 pairs of weight and tokens on cold weights (more than the last-level cache holds
+// between two launches on one): both formats, 512 to 152064 rows, 512 to 14336 values, 6 to 200 tokens.  A slab costs a fixed latency and, for every wave
+// on a SIMD and row tile, 0.3 us and 0.1 us per token group (a wave alone on its SIMD stalls where two overlap: 1.4, not 1, times that).  A second
+// slab ahead shortens the latency of workgroups that have a compute unit of their own (8 tokens, one slab ahead / two: 4096 x 4096 Q8_0 17.8 / 13.5 us, Q4_0
+// 18.9 / 15.7; 14336 x 5120 27.4 / 19.2, 24.5 / 20.2); where two share one it is on par.  Workgroups fill an XCD's 32 compute units row block by row block
+// (wide_block).  The shape with the lowest estimate is on average 0.7 % (Q8_0) and 1.3 % (Q4_0) slower than the fastest, 20 % at worst.
 static float b32_wide_cost(int rows, int groups, int n_slabs, const B32WideShape &s) {
-    const int64_t wgs = static_cast<int64_t>((rows + s.rt * 64 - 1) / (s.rt * 64)) * ((groups + s.g - 1) / s.g);
-    const float per_cu = wgs / 256.0f, full = per_cu / 2;  // (two workgroups are resident at once)
-    const float rounds = full <= 1.0f ? 1.0f : 0.77f * full + 0.23f * std::ceil(full);
-    const float base = s.d == 1 ? 0.37f : n_slabs >= 24 ? 0.3f : 0.5f;
-    return rounds * n_slabs * (base + (per_cu > 1.0f ? 2.0f : 1.4f) * s.rt * (0.165f + 0.15f * s.g));
+    const int64_t blocks = (rows + s.rt * 64 - 1) / (s.rt * 64), per_xcd = (blocks + 7) / 8 * ((groups + s.g - 1) / s.g);
+    const float per_cu = per_xcd / 32.0f, full = per_cu / 2;  // (two workgroups are resident at once)
+    const float rounds = full <= 1.0f ? 1.0f : 0.5f * full + 0.5f * std::ceil(full);
+    const float base = per_cu > 1.0f ? 0.25f : s.d == 1 ? 0.35f : 0.22f;
+    return rounds * n_slabs * (base + (per_cu > 1.0f ? 2.0f : 1.4f) * s.rt * (0.3f + 0.1f * s.g));
 }
 
 template <int FMT, int G, int RT, int D>

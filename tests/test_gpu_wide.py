@@ -174,6 +174,9 @@ ROUTES = [
     ("Q6_K", 8192, 1024, 32, r"^q6k\.mfma\.tile\."),  # rows of four super-blocks
     ("Q6_K", 8192, 1024, 33, r"^q6k\.mfma\.wide\."),  # more tokens
     ("Q6_K", 8192, 1280, 17, r"^q6k\.mfma\.wide\."),  # longer rows
+    ("Q8_0", 8320, 5120, 8, r"^q8_0\.mfma\.wide\.g1r1d2$"),  # two slabs ahead where a workgroup has a compute unit
+    ("Q4_0", 8320, 4096, 16, r"^q4_0\.mfma\.wide\.g1r1d2$"),  # the same
+    ("Q4_0", 33000, 1024, 16, r"^q4_0\.mfma\.wide\.g1r1d1$"),  # two share one
 ]
 
 
