@@ -619,14 +619,15 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_gr
     // Up to 16 tokens, rows of at most 16 slabs, few row tiles: several waves per row tile, one chain.
     // Workgroup shapes by measurement (16 tokens, kernel us cache-cold, against the kernel below):
     //   rows of <= 8 slabs:  <= 256 tiles: 8 waves per tile (4096 x 2048 Q8_0 10.0 -> 6.0);
-    //                        <= 512 tiles: 4 waves per tile, 2 tiles per workgroup (8192 x 2048 Q8_0 7.5 us, Q4_0 6.6; the wide kernel 8.2, 8.7);
-    //                        more tiles lose to the wide kernel (10240 x 2048 Q8_0 11.1, Q4_0 9.6; wide 8.4, 8.9; rows of 2 or 3 slabs alike: 12288 x 768 7.5, 5.7; 5.2);
+    //                        <= 512 tiles: 4 waves per tile, 2 tiles per workgroup (8192 x 2048 Q8_0 7.5 us, Q4_0 6.6; the wide kernel 8.2, 8.7), in Q4_0 on rows of up to
+    //                        seven slabs <= 768 (8320 x 512 / 1024 / 1536 / 1792 4.9, 6.0, 7.8, 8.6; wide 5.1, 6.6, 8.2, 8.9; x 2048 10.0; 9.8); Q8_0 there loses to the wide
+    //                        kernel (8320 x 1024 / 2048 7.0, 11.6; 6.2, 8.9);
     //   rows of 9..16 slabs: the staged activation fills half of a compute unit's LDS, one workgroup per unit:
     //                        <= 256 tiles: 8 waves per tile (4096 x 4096 Q8_0 15.6 -> 10.8, Q4_0 18.6 -> 8.8);
     //                        <= 512 tiles: the same, 2 tiles per workgroup (8192 x 4096 Q8_0 16.9 -> 14.3, Q4_0 19.1 -> 11.1);
     //                        896 tiles lose (14336 x 4096 20.6 -> 26.0).
     const int kpar = env_int("CAMELID_HIP_B32_MFMA_KPAR", -1);
-    const int tiles = (ka.rows + 15) / 16;
+    const int tiles = (ka.rows + 15) / 16, short_row_tiles = FMT == CML_Q4_0 && ka.n_slabs <= 7 ? 768 : 512;
     if (!grouped && ka.n_tokens <= 16 && env_int("CAMELID_HIP_B32_MFMA_SHAPE", 0) == 0 && kpar != 0) {
         if (ka.n_slabs >= 4 && ka.n_slabs <= 8) {
             if (kpar == 1) return launch_b32_mfma_kpar<FMT, 4, 2, 1>(ka, st);
@@ -634,14 +635,14 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_gr
             if (kpar == 3) return launch_b32_mfma_kpar<FMT, 8, 1, 1>(ka, st);
             if (kpar == 4) return launch_b32_mfma_kpar<FMT, 8, 1, 2>(ka, st);
             if (tiles <= 256) return launch_b32_mfma_kpar<FMT, 8, 1, 1>(ka, st);
-            if (tiles <= 512) return launch_b32_mfma_kpar<FMT, 4, 2, 2>(ka, st);
+            if (tiles <= short_row_tiles) return launch_b32_mfma_kpar<FMT, 4, 2, 2>(ka, st);
         } else if (ka.n_slabs > 8 && ka.n_slabs <= 16) {
             if (kpar == 1) return launch_b32_mfma_kpar<FMT, 4, 4, 1>(ka, st);
             if (kpar == 2) return launch_b32_mfma_kpar<FMT, 8, 2, 1>(ka, st);
             if (kpar == 3) return launch_b32_mfma_kpar<FMT, 8, 2, 2>(ka, st);
             if (tiles <= 256) return launch_b32_mfma_kpar<FMT, 8, 2, 1>(ka, st);
             if (tiles <= 512) return launch_b32_mfma_kpar<FMT, 8, 2, 2>(ka, st);
-        } else if (ka.n_slabs >= 2 && ka.n_slabs < 4 && (kpar > 0 || tiles <= 512)) {
+        } else if (ka.n_slabs >= 2 && ka.n_slabs < 4 && (kpar > 0 || tiles <= short_row_tiles)) {
             return launch_b32_mfma_kpar<FMT, 2, 2, 1>(ka, st);
         }
     }
@@ -650,8 +651,11 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_gr
     // 49 / 39, 73 / 39, 541 / 116; 11008 x 2048 at 6 / 16 10.6 / 8.4, 11.0 / 8.5; 32000 x 4096 at 16 35 / 32; 2048 x 2048 at 24 / 200 10.4 / 7.6, 19.3 / 10.
     // Q4_0: 128256 x 3072 at 16 / 32 / 64 57.7 / 51.5, 82 / 64, 156 / 101; 14336 x 4096 at 16 / 200 18.0 / 18.5, 200 / 62.
     // (up to 16 tokens on weights of more than 49152 rows only 13 and more, on rows of 8 slabs and more: 90000 x 3072 at 6 / 16 Q4_0 41.1 / 44.3, 44.3 / 44.2,
-    // Q8_0 62.8 / 65.7, 67.8 / 66.4; 128256 x 1536 Q4_0 28.1 / 30.6, 30.2 / 30.9; 62848 x 2304 at 16 24.0 / 21.8; 40000 x 5120 at 6 34.7 / 30.9)
-    const bool tall_few = ka.n_tokens <= 16 && ka.rows > 49152 && (ka.n_tokens <= 12 || ka.n_slabs < 8);
+    // Q8_0 62.8 / 65.7, 67.8 / 66.4; 128256 x 1536 Q4_0 28.1 / 30.6, 30.2 / 30.9; 62848 x 2304 at 16 24.0 / 21.8; 40000 x 5120 at 6 34.7 / 30.9; Q4_0 rows of 4 to 7 slabs
+    // from 40960 rows on: 45000 x 1536 at 6 / 16 13.7 / 14.2, 13.9 / 14.0, 45000 x 1024 at 12 10.5 / 10.6, 40000 x 1024 at 6 9.7 / 9.5; Q8_0 rows of two slabs on tall
+    // weights: 49152 / 100000 x 512 at 20 10.6 / 11.8, 18.1 / 21.4, 36000 x 512 10.1 / 9.7; 100000 x 512 at 64 / 128 26.5 / 28.2, 41.3 / 42.6)
+    const bool tall_few = ka.n_tokens <= 16 ? (ka.rows > 49152 ? ka.n_tokens <= 12 || ka.n_slabs < 8 : FMT == CML_Q4_0 && ka.rows > 40960 && ka.n_slabs >= 4 && ka.n_slabs < 8)
+                                            : FMT == CML_Q8_0 && ka.n_slabs <= 2 && ka.rows > 40960 && ka.n_tokens <= (ka.rows > 49152 ? 128 : 32);
     if (can_wide && !tall_few && (kpar != 0 || ka.n_tokens > 16)) return launch_gemm_b32_wide(a, st);
     switch (env_int("CAMELID_HIP_B32_MFMA_SHAPE", 0)) {
         case 1: return launch_b32_mfma_p<FMT, 1, 1>(ka, n_groups, st);   // 16 tokens, 1 wave per row tile

@@ -177,6 +177,13 @@ ROUTES = [
     ("Q8_0", 8320, 5120, 8, r"^q8_0\.mfma\.wide\.g1r1d2$"),  # two slabs ahead where a workgroup has a compute unit
     ("Q4_0", 8320, 4096, 16, r"^q4_0\.mfma\.wide\.g1r1d2$"),  # the same
     ("Q4_0", 33000, 1024, 16, r"^q4_0\.mfma\.wide\.g1r1d1$"),  # two share one
+    ("Q4_0", 8320, 1024, 16, r"^q4_0\.mfma\.kpar\."),  # up to 768 tiles of short rows
+    ("Q4_0", 8320, 2048, 16, r"^q4_0\.mfma\.wide\."),  # longer rows
+    ("Q8_0", 8320, 1024, 16, r"^q8_0\.mfma\.wide\."),  # Q8_0: up to 512
+    ("Q4_0", 41000, 1024, 12, r"^q4_0\.mfma\.tile\."),  # rows of four to seven slabs of tall weights
+    ("Q4_0", 40960, 1024, 12, r"^q4_0\.mfma\.wide\."),  # less tall
+    ("Q8_0", 41000, 512, 32, r"^q8_0\.mfma\.tile\."),  # rows of two slabs of tall weights
+    ("Q8_0", 41000, 512, 33, r"^q8_0\.mfma\.wide\."),  # more tokens
 ]
 
 
