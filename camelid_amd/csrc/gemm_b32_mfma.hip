@@ -681,11 +681,15 @@ bool b32_mfma_usable(const cml_weight *w) {
 // Batch size from which the matrix cores beat the packed-dot kernel (which serves up to 8 tokens per pass over the weight).
 // us per launch at 4 / 8 tokens, packed dot against matrix cores: Q8_0 4096 x 14336 28 / 56 against 39, 14336 x 4096 20 / 27 against 20,
 // 11008 x 2048 8.2 / 12.4 against 8.4, 2048 x 2048 5.3 / 8.2 against 5.3; Q4_0 14336 x 4096 14 / 24 against 16 / 18, 5120 x 5120
-// 11 / 19 against 17.  Tall weights from 4 tokens: 128256 x 3072 Q4_0 62 / 105 against 51.
-int b32_mfma_min_tokens(int64_t rows) {
+// 11 / 19 against 17.  Tall weights from 4 tokens: 128256 x 3072 Q4_0 62 / 105 against 51.  Small weights stay on the packed dot at 8 tokens: on rows of three slabs (Q8_0
+// 2048 / 7000 x 768 4.9, 6.0 against 6.0, 6.9, Q4_0 4.8, 5.8 against 5.0, 5.8) and, up to 256 row tiles in Q4_0, of 17 to 24, which several waves per row tile do not
+// serve (4096 x 4608 / 5120 / 6144 16.3, 16.5, 19.7 against 17.2, 18.7, 22.0; 5120 x 5120 19.1 against 19.0; 4096 x 7168 25.6 against 24.9).
+int b32_mfma_min_tokens(const cml_weight *w) {
     const int forced = env_int("CAMELID_HIP_B32_MFMA_MIN_TOKENS", 0);
     if (forced > 0) return forced;
-    return (rows + 15) / 16 >= 2048 ? 4 : 5;
+    const int64_t tiles = (w->rows + 15) / 16, slabs = w->nb / 8;
+    if ((slabs == 3 && tiles <= (w->fmt == CML_Q8_0 ? 512 : 256)) || (w->fmt == CML_Q4_0 && tiles <= 256 && slabs > 16 && slabs <= 24)) return 9;
+    return tiles >= 2048 ? 4 : 5;
 }
 
 // Q8_0 / Q4_0 matmul on the matrix cores: plain calls, or grouped by expert (mixture of experts).

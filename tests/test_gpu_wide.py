@@ -184,6 +184,10 @@ ROUTES = [
     ("Q4_0", 40960, 1024, 12, r"^q4_0\.mfma\.wide\."),  # less tall
     ("Q8_0", 41000, 512, 32, r"^q8_0\.mfma\.tile\."),  # rows of two slabs of tall weights
     ("Q8_0", 41000, 512, 33, r"^q8_0\.mfma\.wide\."),  # more tokens
+    ("Q4_0", 4096, 5120, 8, r"^q4_0\.dot\."),  # eight tokens on rows of 17 to 24 slabs, up to 256 tiles
+    ("Q4_0", 4100, 5120, 8, r"^q4_0\.mfma\.wide\."),  # more
+    ("Q8_0", 7000, 768, 8, r"^q8_0\.dot\."),  # rows of three slabs
+    ("Q4_0", 2048, 1024, 8, r"^q4_0\.mfma\.kpar\."),  # four
 ]
 
 
