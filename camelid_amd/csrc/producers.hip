@@ -339,8 +339,9 @@ __global__ __launch_bounds__(THREADS) void rms_norm_quantize_kernel(const float 
 template <int THREADS, int C4>
 static int launch_rms_norm(int act, const float *x, const float *weight, float eps, int64_t n_tokens, int cols, float *normed, int8_t *q, float *scales, hipStream_t st) {
     constexpr size_t lds = static_cast<size_t>(THREADS) * C4 * sizeof(float4);  // the row in whole chunks (zero padded)
+    constexpr size_t fixed = THREADS / 64 * (64 * sizeof(uint4) + 8) + 16;      // and what the kernel declares: ordered_sum_nonneg's lists, the scale
     static std::atomic<bool> raised{false};
-    if (lds > 48 * 1024 && !raised.load(std::memory_order_acquire)) {
+    if (lds + fixed > 64 * 1024 && !raised.load(std::memory_order_acquire)) {  // (a launch may use that much without asking)
         CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<0, THREADS, C4>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
         CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<1, THREADS, C4>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));
         CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&rms_norm_quantize_kernel<2, THREADS, C4>), hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024));

@@ -4,6 +4,8 @@ the reference's left-to-right sum of squares), quantized outputs bit-exact, fuse
 (the reference's own claim, src/cuda_resident/tests.rs:4114-4190).  silu uses expf: its f32
 values may differ from the host libm in the last bit, so that path is checked as fused ==
 device-composed bit for bit and against the oracle within 1 quantization step."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -116,6 +118,21 @@ def test_sum_of_squares_is_the_scalar_loop(cols):
 @pytest.mark.parametrize("cols", [1024, 1028, 3072, 3076, 4100, 6144, 6148, 8196, 12288, 12292])
 def test_sum_of_squares_at_the_widths_where_the_launch_changes(cols):
     test_sum_of_squares_is_the_scalar_loop(cols)
+
+
+# the kernel <threads, float4 per thread> of a width; a launch that uses more than 64 KB of LDS, its own lists included, has to have asked for it
+@pytest.mark.parametrize("cols,threads,chunks", [(8200, 1024, 3), (12288, 1024, 3), (12292, 1024, 4), (16384, 1024, 4)])
+def test_norm_launches_ask_for_the_lds_they_use(cols, threads, chunks):
+    G.say(f"sum of squares cols={cols}")
+    xd, od = DeviceBuffer.from_numpy(np.ones((1, cols), np.float32)), DeviceBuffer(16)
+    check(lib().cml_sum_squares_f32(xd.ptr, 1, cols, od.ptr, None), "cml_sum_squares_f32")
+    check(lib().cml_stream_sync(None))
+    assert od.to_numpy(np.float32, (1,))[0] == cols
+    attributes = (C.c_int * 14)()  # hipFuncAttributes: word 6 is maxDynamicSharedSizeBytes, words 12 and 13 sharedSizeBytes
+    kernel = C.c_void_p.in_dll(lib(), f"_ZN3cml24rms_norm_quantize_kernelILi3ELi{threads}ELi{chunks}EEEvPKfS2_fiPfPaS3_")
+    assert C.CDLL("libamdhip64.so").hipFuncGetAttributes(attributes, C.c_void_p(C.addressof(kernel))) == 0
+    used = threads * chunks * 16
+    assert used + attributes[12] > 64 * 1024 and used <= attributes[6] == 96 * 1024
 
 
 @pytest.mark.parametrize("cols", [256, 2048, 2816, 4096, 14336])
