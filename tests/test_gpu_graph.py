@@ -71,7 +71,7 @@ OUT_SCRUB = [None]   # the output buffer of the case at hand, scrubbed between t
 
 
 @pytest.mark.parametrize("name,fmt", [("Q8_0", oracle.Q8_0), ("Q4_0", oracle.Q4_0), ("Q4_K", oracle.Q4_K), ("Q6_K", oracle.Q6_K)])
-@pytest.mark.parametrize("n", [1, 3, 16])
+@pytest.mark.parametrize("n", [1, 3, 16, 40])  # (40: the wide kernels, but for Q4_K)
 def test_matmul_f32_replays_are_the_eager_bits(stream, name, fmt, n):
     rows, cols = 300, 2048
     w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=500 + fmt))

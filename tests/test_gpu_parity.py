@@ -1090,7 +1090,8 @@ def test_q4k_matrix_core_cells_are_bitwise_the_gemv(rows, cols):
             with G.env(CAMELID_HIP_Q4K_MFMA_SHAPE=shape), G.engaged(want_kernel, none=(r"^q4k\.dot\.",)):
                 got = G.gpu_gemm(w, s, q)                      # default K-split policy, reproduced across waves or in-lane
             if shape == 0:
-                with G.env(CAMELID_HIP_Q4K_MFMA_SERIAL_SPLIT=1), G.engaged(r"^q4k\.mfma\.", none=(r"^q4k\.mfma\.ksplit", r"^q4k\.dot\.")):
+                in_lane = r"^q4k\.mfma\.serial_split\." if rows in (4096, 2000, 1600, 6400, 300) else r"^q4k\.mfma\.(tile\.|pair$)"
+                with G.env(CAMELID_HIP_Q4K_MFMA_SERIAL_SPLIT=1, CAMELID_HIP_MFMA_WIDE=0), G.engaged(in_lane, none=(r"^q4k\.mfma\.ksplit", r"^q4k\.dot\.")):
                     assert G.same_bits(got, G.gpu_gemm(w, s, q))
             with G.env(CAMELID_HIP_Q4K_MFMA_MIN_TOKENS=1 << 30), G.engaged(r"^q4k\.dot\.", none=(r"^q4k\.mfma\.",)):
                 ref = G.gpu_gemm(w, s, q)                      # the packed-dot kernel on the same inputs
@@ -1297,8 +1298,9 @@ def test_q6k_matrix_core_cells_are_bitwise_the_gemv(rows, cols):
                         G.engaged(want_kernel, none=(r"^q6k\.dot\.",)):
                     got = G.gpu_gemm(w, s, q)
                 assert G.same_bits(got, ref)
-        with G.env(CAMELID_HIP_Q6K_MFMA_SERIAL_SPLIT=1, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), \
-                G.engaged(r"^q6k\.mfma\.", none=(r"^q6k\.mfma\.ksplit", r"^q6k\.dot\.")):   # the split inside the lane
+        in_lane = r"^q6k\.mfma\.serial_split\." if rows in (300, 4000, 1000) else r"^q6k\.mfma\.tile\."
+        with G.env(CAMELID_HIP_Q6K_MFMA_SERIAL_SPLIT=1, CAMELID_HIP_MFMA_WIDE=0, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), \
+                G.engaged(in_lane, none=(r"^q6k\.mfma\.ksplit", r"^q6k\.dot\.")):   # the split inside the lane
             assert G.same_bits(G.gpu_gemm(w, s, q), ref)
         check_outputs(fmt, wire, cols, s, q, got, expect_exact=False)
         with G.env(CAMELID_HIP_EXACT_ORDER="1", CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1):

@@ -5,7 +5,7 @@ import pytest
 
 import oracle
 from camelid_amd import binding as B
-from camelid_amd.binding import Weight
+from camelid_amd.binding import DeviceBuffer, Weight, check, lib
 from tests import gpu_util as G
 from tests.test_gpu_moe import gpu_moe, gpu_route
 
@@ -28,6 +28,7 @@ def activations(n: int, cols: int, seed: int):
 def test_wide_cells_are_bitwise_the_gemv(name, fmt, tag, rows, cols):
     wire = G.synth_weight(fmt, rows, cols, seed=rows + cols)
     w = Weight.upload(fmt, rows, cols, wire)
+    cut = {1: 1, 3: 1, 5: 1, 8: 2, 13: 2, 16: 4, 18: 4}[cols // 256]  # the matvec's K cut of these rows
     for n in (3, 16, 17, 47, 130):
         s, q = activations(n, cols, seed=n)
         with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
@@ -38,10 +39,12 @@ def test_wide_cells_are_bitwise_the_gemv(name, fmt, tag, rows, cols):
             for parts in (1, 2):
                 if (name, g, waves, parts) == ("Q4_K", 8, 8, 2):
                     continue  # does not fit a compute unit's LDS
+                two = parts == 2 and cut > 1
+                walk = (r"\.ksplit2" if two else "") + (r"\.serial_split" if cut > (2 if two else 1) else "")
                 G.say(f"wide {name} {rows}x{cols} n={n} groups={g} waves={waves} parts={parts}")
                 with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g, CAMELID_HIP_WIDE_WAVES=waves, CAMELID_HIP_WIDE_PARTS=parts,
                            CAMELID_HIP_Q4K_MFMA_MIN_TOKENS=1, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), \
-                        G.engaged(rf"^{tag}\.mfma\.wide\.g{g}w{waves}(\.|$)", none=(r"\.dot\.",)):
+                        G.engaged(rf"^{tag}\.mfma\.wide\.g{g}w{waves}{walk}$", none=(r"\.dot\.",)):
                     assert G.same_bits(G.gpu_gemm(w, s, q), ref)
         with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_EXACT_ORDER=1, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), G.engaged(rf"^{tag}\.mfma\.wide\."):
             got = G.gpu_gemm(w, s, q)
@@ -159,9 +162,24 @@ def test_wide_b32_expert_groups_are_bitwise_the_gemv(name, fmt, tag, E, k, hidde
             assert G.same_bits(run(), ref)
 
 
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_scales_that_cannot_be_read_16_bytes_at_a_time_stay_off_the_wide_kernel(name, fmt, tag):
+    rows, cols, n = 70, 768, 40
+    w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=8))
+    s, q = oracle.quantize_activation(fmt, np.random.default_rng(3).standard_normal((n, cols)).astype(np.float32))
+    want = G.gpu_gemm(w, s, q)
+    qd, od = DeviceBuffer.from_numpy(q), DeviceBuffer(n * rows * 4)
+    sd = DeviceBuffer.from_numpy(np.concatenate([[0.0], s.reshape(-1)]).astype(np.float32))
+    G.say(f"wide {name} scales at 4 bytes past a 16-byte boundary")
+    with G.engaged(rf"^{tag}\.mfma\.tile\.", none=(r"\.wide\.",)):
+        check(lib().cml_gemm(w.handle, qd.ptr, sd.ptr + 4, n, od.ptr, None), "cml_gemm")
+        check(lib().cml_stream_sync(None))
+    assert G.same_bits(od.to_numpy(np.float32, (n, rows)), want)
+
+
 # Which kernel a call without knobs takes, on either side of each line of the rules
 ROUTES = [
-    ("Q4_K", 2560, 4096, 33, r"^q4k\.mfma\.wide\.g1w4\.ksplit2$"),  # the smallest workgroups, where they alone have a compute unit each
+    ("Q4_K", 2560, 4096, 33, r"^q4k\.mfma\.wide\.g1w4\.ksplit2\.serial_split$"),  # the smallest workgroups, where they alone have a compute unit each
     ("Q4_K", 1024, 4096, 48, r"^q4k\.mfma\.ksplit4"),  # K cut four ways, a workgroup of the narrow kernel per compute unit at most
     ("Q4_K", 4096, 4096, 33, r"^q4k\.mfma\.ksplit4"),  # up to two, the wide kernel's come to more than one as well
     ("Q4_K", 2048, 5120, 80, r"^q4k\.mfma\.wide\."),  # K parts of five super-blocks
