@@ -360,14 +360,12 @@ static int launch_rms_norm(int act, const float *x, const float *weight, float e
     return CML_OK;
 }
 
-template <int THREADS>
+// `CHUNKS` float4 per thread, the fewest that hold the row; FIRST: the fewest that a row of this workgroup's widths needs.
+template <int THREADS, int FIRST, int CHUNKS = kRmsRegs>
 static int launch_rms_norm_chunks(int act, const float *x, const float *weight, float eps, int64_t n_tokens, int cols, float *normed, int8_t *q, float *scales, hipStream_t st) {
-    switch ((cols / 4 + THREADS - 1) / THREADS) {
-        case 1: return launch_rms_norm<THREADS, 1>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
-        case 2: return launch_rms_norm<THREADS, 2>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
-        case 3: return launch_rms_norm<THREADS, 3>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
-        default: return launch_rms_norm<THREADS, 4>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
-    }
+    if constexpr (CHUNKS > FIRST)
+        if (cols <= (CHUNKS - 1) * THREADS * 4) return launch_rms_norm_chunks<THREADS, FIRST, CHUNKS - 1>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
+    return launch_rms_norm<THREADS, CHUNKS>(act, x, weight, eps, n_tokens, cols, normed, q, scales, st);
 }
 
 int launch_rms_norm_quantize(int act, const float *x, const float *weight, float eps, int64_t n_tokens, int64_t cols,
@@ -377,10 +375,10 @@ int launch_rms_norm_quantize(int act, const float *x, const float *weight, float
         return fail(CML_ERR_UNSUPPORTED, "rms_norm row of %lld values exceeds the staging limit of %d", (long long)cols, kRmsRegs * 1024 * 4);
     // us per launch of one row, 256 / 512 / 1024 threads: 2048 values 4.7 / 4.9 / 5.9, 3072 5.4 / 5.4 / 6.6, 4096 6.0 / 5.6 / 7.3, 8192 - / 7.2 / 7.9
     // (512 rows of 4096: 7.9 / 8.0 / 10.5); before, always 1024 threads: 4096 8.0, 512 rows 15.
-    const int c = static_cast<int>(cols), threads = env_int("CAMELID_HIP_RMS_THREADS", cols <= 3072 ? 256 : 512);
-    if (threads <= 256 && cols <= 4 * kRmsRegs * 256) return launch_rms_norm_chunks<256>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
-    if (threads <= 512 && cols <= 4 * kRmsRegs * 512) return launch_rms_norm_chunks<512>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
-    return launch_rms_norm_chunks<1024>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
+    const int c = static_cast<int>(cols);
+    if (cols <= 3072) return launch_rms_norm_chunks<256, 1, 3>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
+    if (cols <= 4 * kRmsRegs * 512) return launch_rms_norm_chunks<512, 2>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
+    return launch_rms_norm_chunks<1024, 3>(act, x, weight, eps, n_tokens, c, normed, q, scales, st);
 }
 
 // h = silu(g) * u = (g / (1 + exp(-g))) * u, quantized on the fly.  Q8_K: one wave per

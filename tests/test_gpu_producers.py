@@ -114,8 +114,8 @@ def test_sum_of_squares_is_the_scalar_loop(cols):
         assert finite.sum() >= 12
 
 
-# one to four float4 per thread in workgroups of 256, 512 and 1024 threads: the last width of a shape and the first of the next
-@pytest.mark.parametrize("cols", [1024, 1028, 3072, 3076, 4100, 6144, 6148, 8196, 12288, 12292])
+# the last width of a launch and the first of the next: workgroups of 256 threads with one to three float4 each, of 512 with two to four, of 1024 with three or four
+@pytest.mark.parametrize("cols", [1024, 1028, 2052, 3072, 3076, 4100, 6144, 6148, 8196, 12288, 12292])
 def test_sum_of_squares_at_the_widths_where_the_launch_changes(cols):
     test_sum_of_squares_is_the_scalar_loop(cols)
 
