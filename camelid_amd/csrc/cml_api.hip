@@ -1049,7 +1049,8 @@ int cml_matmul_f32_static(const cml_weight *w, const float *x_dev, int64_t n_tok
 
 // Calls that move no more than this each way go through pinned memory and the copy kernel: three launches and one wait, where
 // copies from and to pageable memory wait for themselves (us per call, pageable / pinned: Q8_0 8192 x 2048, one row 29.6 / 20.1;
-// Q4_K 16384 x 4096 34.8 / 24.0; 448 KB of outputs 55 / 42).
+// Q4_K 16384 x 4096 34.8 / 24.0; outputs of 0.5 / 1.1 / 2 / 4 / 8 MB 56 / 46, 104 / 84, 143 / 131, 282 / 256, 520 / 540; activations of 0.6 / 2.3 / 4.6 MB 82 / 63,
+// 148 / 154, 219 / 253).  The limit keeps what the process pins for good at one megabyte; past it there is a tenth to be had up to 4 MB of outputs.
 constexpr size_t kSeamHostBytes = 1088 * 1024;
 
 static void launch_seam_copy(void *dst, const void *src, size_t nbytes) {

@@ -667,6 +667,7 @@ static int launch_b32_mfma_fmt(const B32MfmaArgs &ka, const MatArgs &a, int n_gr
         default: break;
     }
     if (grouped || ka.n_tokens <= 16) return launch_b32_mfma_p<FMT, 1, 1>(ka, n_groups, st);
+    // (more than 16 tokens: Q8_0 rows of two slabs on tall weights, scales off a 16-byte boundary, and CAMELID_HIP_MFMA_WIDE=0, the tests' second implementation)
     const bool few_tiles = (ka.rows + 15) / 16 < 1024;
     if (ka.n_tokens <= 32) return few_tiles ? launch_b32_mfma_p<FMT, 1, 2>(ka, n_groups, st) : launch_b32_mfma_p<FMT, 2, 1>(ka, n_groups, st);
     return few_tiles ? launch_b32_mfma_p<FMT, 1, 4>(ka, n_groups, st) : launch_b32_mfma_p<FMT, 4, 1>(ka, n_groups, st);

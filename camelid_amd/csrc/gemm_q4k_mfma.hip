@@ -1190,7 +1190,7 @@ int launch_gemm_q4k_mfma(const MatArgs &a, hipStream_t st) {
             return launch_mfma<2, 1>(ka, ng, st);
         return launch_mfma<1, 1>(ka, ng, st);
     }
-    if (a.n_tokens > 32) return launch_mfma<4, 1>(ka, ng, st);
+    if (a.n_tokens > 32) return launch_mfma<4, 1>(ka, ng, st);  // (only with tuning variables: the tests' second implementation)
     if (a.n_tokens > 16) return launch_mfma<2, 1>(ka, ng, st);
     return launch_mfma<1, 1>(ka, ng, st);
 }

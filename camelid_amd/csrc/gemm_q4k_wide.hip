@@ -1,5 +1,5 @@
-// Q4_K x Q8_K on the wide matrix-core kernel (gemm_wide.hpp): batches of more than 32 tokens, and expert
-// groups that hold more than a few assignments each.
+// Q4_K x Q8_K on the wide matrix-core kernel (gemm_wide.hpp): batches of more than 32 tokens, but for small weights whose
+// K is cut, and expert groups that hold more than a few assignments each (launch_gemm_q4k_mfma holds the lines).
 //
 // The integers are those of gemm_q4k_mfma.hip: the 6-bit scale of a sub-block as two 3-bit digits inside the int8 weight
 // operand (S = lo + 8 hi, two contractions over the whole super-block), the mins against the sums of the

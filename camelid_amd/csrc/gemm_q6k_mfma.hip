@@ -456,7 +456,7 @@ int launch_gemm_q6k_mfma(const MatArgs &a, hipStream_t st) {
     if (!grouped && shape == 0 && wide && (wide == 2 || !stays)) return launch_gemm_q6k_wide(a, st);
     // K split across waves where the matvec kernel splits K two or four ways and the launch has
     // fewer row tiles than the chip has SIMDs: 16 or 32 tokens per workgroup, more tokens = more
-    // workgroup columns.
+    // workgroup columns.  (More than 16 tokens come here, and more than 32 past the switch, only with CAMELID_HIP_MFMA_WIDE=0: the tests' second implementation.)
     const int64_t launch_tiles = static_cast<int64_t>((ka.rows + 15) / 16) * ng;
     if (shape == 0 && launch_tiles < 1024 && !env_int("CAMELID_HIP_Q6K_MFMA_SERIAL_SPLIT", 0)) {
         const bool small = grouped || a.n_tokens <= 16;

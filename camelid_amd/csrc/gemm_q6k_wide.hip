@@ -1,5 +1,5 @@
-// Q6_K x Q8_K on the wide matrix-core kernel (gemm_wide.hpp): batches of any size on weights without a K cut,
-// of more than 16 tokens on the others.
+// Q6_K x Q8_K on the wide matrix-core kernel (gemm_wide.hpp): batches of more than 16 tokens, and smaller ones on weights
+// of more than 1024 row tiles, but for short rows of tall weights (launch_gemm_q6k_mfma holds the lines).
 //
 // gemm_q6k_mfma.hip contracts one 16-value sub-block at a time (half of the matrix instruction's K is zero) and
 // scales its sums with an integer multiply-add per cell and sub-block: sixteen matrix and 64 vector instructions per

@@ -1,5 +1,6 @@
-// The wide matrix-core kernel: matmul of a K-quant weight with batches of more than 32 tokens
-// (prefill), and of the expert groups of a routed layer.  One workgroup per (block of weight rows,
+// The wide matrix-core kernel: matmul of a K-quant weight with batches (Q4_K of more than 32 tokens,
+// Q6_K of more than 16 and fewer on weights without a K cut; the launchers of the narrow kernels say which),
+// and of the expert groups of a routed layer.  One workgroup per (block of weight rows,
 // column of up to 128 tokens); gemm_q6k_wide.hip and gemm_q4k_wide.hip supply the formats.
 //
 // A wave owns ONE 16-row tile and all tokens of its workgroup's column: what a super-block of
@@ -10,7 +11,8 @@
 // to LDS without passing through registers (global_load_lds).  A lane's register loads of a weight
 // tile would touch 16 rows per instruction and keep the address unit busy for 31 - 39 cycles each,
 // more than the bytes take; here every request reads whole lines.  LDS is written at consecutive addresses, 16
-// bytes per lane, so bank conflicts are avoided by what each lane FETCHES: 16-byte slot p of
+// bytes per lane, so bank conflicts are kept down by what each lane FETCHES (a tenth of the LDS cycles are left on Q4_K,
+// 14336 x 4096 at 512 tokens): 16-byte slot p of
 // token t holds piece p ^ (t % 16) of its 256 values (the weights likewise).  A reader applies the
 // same exclusive-or.
 //

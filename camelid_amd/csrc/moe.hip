@@ -246,8 +246,8 @@ __global__ __launch_bounds__(kPlanThreads) void moe_plan_kernel(const int32_t *_
     }
 }
 
-// Expert-grouped matmul: the packed-dot kernel for a few tokens, the matrix cores from 4 tokens
-// up (the same crossover as for plain calls).  Both produce the same bits per cell.
+// Expert-grouped matmul: the packed-dot kernels for a few assignments per expert, the matrix cores for more (Q4_K: from 4
+// tokens; Q6_K: from six assignments per group on average; Q8_0 / Q4_0: below).  All produce the same bits per cell.
 static int launch_expert_matmul(const MatArgs &a, hipStream_t st) {
     if (a.w->fmt == CML_Q6_K) {
         const int64_t groups = a.group_ids ? a.max_active : a.n_groups;
@@ -255,13 +255,13 @@ static int launch_expert_matmul(const MatArgs &a, hipStream_t st) {
         return launch_gemv_q6k(a, st);
     }
     if (a.w->fmt != CML_Q4_K) {
-        // matrix cores once the groups in use hold enough assignments on average to fill a 16-token tile reasonably
         const int64_t groups = a.group_ids ? a.max_active : a.n_groups;
         // The wide kernel from three assignments per group on average.  us per layer, packed dot or narrow matrix-core kernel / wide, Q4_0: 128 experts, top-8,
         // 2816 / 704 at 32 / 64 tokens (2 and 4 each; down has no whole slabs) 121 / 123, 177 / 154; 64 experts, 2048 / 1024 at 16 / 40 (2 and 5) 64 / 64,
         // 108 / 72; 32 experts, 2816 / 1408 at 24 / 64 (6 and 16) 148 / 86, 243 / 157.
         const int wide = env_int("CAMELID_HIP_MFMA_WIDE", 1);  // 0 = never, 1 = by shape, 2 = always
         if (a.group_offsets && wide && (wide == 2 || a.n_assign_total >= 3 * groups) && gemm_b32_wide_serves_groups(a)) return launch_gemm_b32_wide(a, st);
+        // (scales off a 16-byte boundary, activation rows past 4 GB of offsets: the narrow matrix-core kernel once the groups fill a 16-token tile reasonably)
         if (a.group_offsets && b32_mfma_usable(a.w) && a.n_assign_total >= groups * env_int("CAMELID_HIP_B32_MFMA_MIN_GROUP", 6))
             return launch_gemm_b32_mfma(a, st);
         return launch_gemv_b32_grouped(a, GroupedPrologue{}, st);
