@@ -485,7 +485,8 @@ static int launch_wide_plain(const MatArgs &a, hipStream_t st) {
         wide_consider_g<F, 4, 2>(tiles, groups, ka.n_sb, ka.ksplit, s, cost);
         wide_consider_g<F, 8, 2>(tiles, groups, ka.n_sb, ka.ksplit, s, cost);
     }
-    // (forced shapes: tests and measurements)
+    // (forced shapes: tests and measurements.  Of the 31 / 32 compiled ones the estimate never takes, over 1 to 9500 tiles, 1 to 128 groups and the three cuts, Q4_K 8 groups and
+    // 4 to 8 on two parts with four waves, Q6_K eight waves alone and with 1 to 4 groups on two parts: the tests' other implementations of the same cells)
     s.g = env_int("CAMELID_HIP_WIDE_GROUPS", s.g);
     s.waves = env_int("CAMELID_HIP_WIDE_WAVES", s.waves);
     s.ks = two ? env_int("CAMELID_HIP_WIDE_PARTS", s.ks) : 1;
