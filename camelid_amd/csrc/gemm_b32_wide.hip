@@ -3,7 +3,8 @@
 // Arithmetic: cell by cell that of the matvec kernels and of gemm_b32_mfma.hip: per 32-value block, in block order,
 //     isum = sum_j w_j * x_j  (exact i32),   acc = acc + ((float)isum * d_w) * d_x
 // so one v_mfma_i32_16x16x32_i8 per block and 16 x 16 cells, and an f32 step per block and cell: the vector
-// instructions bound this kernel (three of four cycles each per 64 cells and block: 14336 x 4096 x 200 tokens 29 us of issue, 61 measured).  Three
+// instructions bound this kernel (three per 64 cells and block, the fused one four cycles and the others two with two waves to take turns: 14336 x 4096 x 200 tokens
+// 24 us of issue, 57 measured).  Three
 // are the least: multiply, multiply, add, each rounded.  The conversion is left out: the matrix instruction
 // adds onto 0x4b400000, so that its result READ AS f32 is 12582912 + isum (|isum| <= 2^19), and
 //     fma(that, d_w, -12582912 * d_w)
@@ -19,8 +20,10 @@
 // Lane L supplies A-row t = L % 16 and B-column n = L % 16 at the k-octet L / 16 of a block and
 // receives D[4 * (L / 16) + j][L % 16], j < 4.  Q4_0: octets 0, 1 are the low nibbles of the block's first and second
 // eight bytes, octets 2, 3 the high ones.
-// us per launch, gemm_b32_mfma.hip before -> here: Q8_0 14336 x 4096 at 24 / 64 / 200 / 512 tokens 34.5 -> 21.2, 67 -> 24, 217 -> 61,
-// 434 -> 115 (523 TOP/s); 4096 x 14336 at 64 / 512 73 -> 39, 541 -> 116; Q4_0 128256 x 3072 at 16 / 64 57.7 -> 51.5, 156 -> 101.
+// With one token group the weight costs Q4_0 more than the cells do: its words and scales are converted where they are used, in four instructions per word pair and two per
+// scale where they were eight and four, and in registers enough fewer that four waves fit a SIMD (32000 x 4096 at 16 tokens 22.8 -> 20.2 us, 4096 x 14336 46 -> 39).
+// us per launch, gemm_b32_mfma.hip -> here: Q8_0 14336 x 4096 at 24 / 64 / 200 / 512 tokens 34.5 -> 21.2, 67 -> 24, 217 -> 58,
+// 434 -> 115 (523 TOP/s); 4096 x 14336 at 64 / 512 73 -> 39, 541 -> 116; Q4_0 128256 x 3072 at 16 / 64 57.7 -> 51, 156 -> 100.
 #include "gemm_wide.hpp"
 
 #pragma clang fp contract(off)
@@ -35,6 +38,7 @@ struct B32WideArgs {
     int64_t q_stride, s_stride;
     int rows, n_slabs;
     int n_row_blocks, n_cols;
+    int base, more;    // token groups of a column; columns that have one more
     const int8_t *q;   // [n_tokens][n_slabs*256]
     const float *xs;   // [n_tokens][n_slabs*8], 16-byte aligned
     float *out;        // [n_tokens][rows]
@@ -46,6 +50,25 @@ struct B32WideArgs {
 };
 
 constexpr int kB32Waves = 4;
+
+typedef unsigned short us2_w __attribute__((ext_vector_type(2)));
+typedef _Float16 h2_w __attribute__((ext_vector_type(2)));
+
+// The eight bytes of a block that a lane holds, as the matrix instruction's operand.  Q4_0: the nibbles of its k-quarter (low ones in lanes of quarters
+// 0 and 1) in the upper half of the bytes with the top bit turned over, 16 (nibble - 8): two instructions per word, four to bring nibble - 8 down.
+template <int FMT>
+__device__ __forceinline__ v2i_w b32_operand(v2i_w o, int kq) {
+    if constexpr (FMT == CML_Q8_0) return o;
+    const int up = 4 - 4 * (kq >> 1);
+    return v2i_w{static_cast<int>(((static_cast<uint32_t>(o.x) << up) & 0xf0f0f0f0u) ^ 0x80808080u), static_cast<int>(((static_cast<uint32_t>(o.y) << up) & 0xf0f0f0f0u) ^ 0x80808080u)};
+}
+// d_w, over the 16 that a Q4_0 operand carries (both steps exact: 2^-28 is a normal f32)
+template <int FMT>
+__device__ __forceinline__ float b32_scale(uint32_t two, int odd) {
+    const h2_w h = __builtin_bit_cast(h2_w, two);
+    const float d = static_cast<float>(odd ? h.y : h.x);
+    return FMT == CML_Q8_0 ? d : d * 0.0625f;
+}
 
 // LDS layout of one workgroup.
 template <int FMT, int G, int RT, int D>
@@ -60,12 +83,13 @@ struct B32WideLds {
 };
 
 // G: token groups of 16 per column.  RT: row tiles of a wave.  D: slabs requested ahead.
-// GROUPED: expert groups; a workgroup walks all token columns of its group.
-template <int FMT, int G, int RT, int D, bool GROUPED>
-__global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32WideArgs a) {
+// GROUPED: expert groups; a workgroup walks all token columns of its group.  ONCE: the weight is read by one column.
+template <int FMT, int G, int RT, int D, bool GROUPED, bool ONCE>
+__global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 1 ? 4 : 3) : 2) void gemm_b32_wide_kernel(B32WideArgs a) {
     typedef B32WideLds<FMT, G, RT, D> L;
     constexpr int NTOK = L::NTOK, WAVES = kB32Waves;
     constexpr int kThreads = 64 * WAVES;
+    constexpr bool kLate = FMT == CML_Q4_0 && G == 1;  // a slab's weight is used once: it is unpacked where it is used
     static_assert(kThreads == 256, "a pass of the workgroup fetches a token group");
     static_assert(!GROUPED || D == 1, "waves of a grouped call may have fewer requests in flight");
     extern __shared__ uint4 smem[];
@@ -81,10 +105,9 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
     if (band < 0) return;  // a slot past the groups in use
     const int a0 = GROUPED ? a.group_offsets[band] : 0;
     const int n_assign = GROUPED ? a.group_offsets[band + 1] - a0 : a.n_tokens;
-    for (;; col++) {
-        const int tok0 = col * NTOK;
-        if (tok0 >= n_assign) return;  // the whole workgroup leaves
-        const int n_here = min(NTOK, n_assign - tok0);
+    // The walk over K of one column of NG token groups.
+    auto walk = [&](int tok0, int n_here, auto groups) __attribute__((always_inline)) {
+        constexpr int NG = decltype(groups)::value;
         auto act_row = [&](int t) __attribute__((always_inline)) -> uint32_t {  // (tokens past the end repeat the last one)
             const int j = min(t, n_here - 1);
             return static_cast<uint32_t>(GROUPED ? (a.group_rows ? a.group_rows[a0 + tok0 + j] : a0 + tok0 + j) : j);
@@ -97,9 +120,9 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
         const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
         const uint32_t row_bytes = n_slabs * 256u;
         const int8_t *q_base = a.q + (GROUPED ? 0 : static_cast<int64_t>(tok0) * row_bytes);
-        uint32_t src[G];
+        uint32_t src[NG];
 #pragma unroll
-        for (int k = 0; k < G; k++) src[k] = act_row(t16 + 16 * k) * row_bytes + piece * 16;
+        for (int k = 0; k < NG; k++) src[k] = act_row(t16 + 16 * k) * row_bytes + piece * 16;
         // Scales: lane pairs of the first waves, token 32 * wave + lane / 2.
         const bool xs_wave = wave < L::kXs / 1024;
         const float *xs_base = a.xs + (GROUPED ? 0 : static_cast<int64_t>(tok0) * (n_slabs * 8));
@@ -108,7 +131,7 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
             slab = min(slab, n_slabs - 1);
             if (xs_wave) wide_dma16(lds0 + kXsAt + buf * L::kXs + wave * 1024, xs_base + slab * 8, xs_src);
 #pragma unroll
-            for (int k = 0; k < G; k++)
+            for (int k = 0; k < NG; k++)
                 if (!GROUPED || 4 * wave + 16 * k < n_here)  // (what no token owns stays what it was: cells of its own, never stored)
                     wide_dma16(lds0 + buf * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + slab * 256, src[k]);
         };
@@ -133,46 +156,48 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
             slab = min(slab, n_slabs - 1);
             const uint32_t to = w_lds + slot * (WAVES * L::kWave);
 #pragma unroll
-            for (int i = 0; i < kReqs; i++) wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
+            for (int i = 0; i < kReqs; i++) {
+                if constexpr (ONCE) wide_dma16_once(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
+                else wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
+            }
 #pragma unroll
             for (int r = 0; r < RT; r++) wide_dma4(to + L::kQuants + r * 256, wd + slab * 16, d_src[r]);
         };
-        constexpr int kAhead = (D - 1) * (G + kReqs + RT);  // requests that may be outstanding at the end of a step (some waves have more)
+        constexpr int kAhead = (D - 1) * (NG + kReqs + RT);  // requests that may be outstanding at the end of a step (some waves have more)
 
-        // Operands of a slab: the lane's octet of the eight blocks of either tile's row, the blocks' scales.
-        long bw[RT][8];
-        float dw[RT][8], md[RT][8];  // d_w; -12582912 * d_w
-        bool finite;
+        // Operands of a slab: the lane's octet of the eight blocks of either tile's row, the blocks' scales.  With one token group they are
+        // used once and stay as they were read until then (28 registers fewer per tile: a third or fourth wave on a SIMD).
+        v2i_w bw[RT][8];
+        uint32_t dh[RT][4];                                             // scales of two blocks each, as read
+        float dw[kLate ? 1 : RT][kLate ? 1 : 8], md[kLate ? 1 : RT][kLate ? 1 : 8];  // d_w; -12582912 * d_w
+        bool finite = true;
         auto read_w = [&](int slot) __attribute__((always_inline)) {
             const uint8_t *w_mine = slabs + kWAt + wave * L::kWave + slot * (WAVES * L::kWave);
-            uint32_t high = 0;
+            us2_w high = {0, 0};
 #pragma unroll
             for (int r = 0; r < RT; r++) {
                 const int row = 16 * r + n;
                 const uint4 d = *reinterpret_cast<const uint4 *>(w_mine + L::kQuants + row * 16);
-                const uint32_t dword[4] = {d.x, d.y, d.z, d.w};
+                dh[r][0] = d.x;
+                dh[r][1] = d.y;
+                dh[r][2] = d.z;
+                dh[r][3] = d.w;
 #pragma unroll
                 for (int b = 0; b < 8; b++) {
-                    const uint32_t bits = (dword[b >> 1] >> (16 * (b & 1))) & 0xffffu;
-                    dw[r][b] = f16_bits_to_f32(bits);
-                    md[r][b] = -12582912.0f * dw[r][b];
-                    high = max(high, bits & 0x7c00u);
-                    if constexpr (FMT == CML_Q8_0) {
-                        const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8);
-                        bw[r][b] = __builtin_bit_cast(long, o);
-                    } else {
-                        const v2i_w o = *reinterpret_cast<const v2i_w *>(w_mine + row * 128 + ((b ^ ((n >> 1) & 7)) << 4) + (kq & 1) * 8);
-                        v2i_w v;
-#pragma unroll
-                        for (int i = 0; i < 2; i++) {  // nibble - 8 as a signed byte
-                            const uint32_t nib = (static_cast<uint32_t>(o[i]) >> (4 * (kq >> 1))) & 0x0f0f0f0fu;
-                            v[i] = static_cast<int>((nib + 0x78787878u) ^ 0x80808080u);
-                        }
-                        bw[r][b] = __builtin_bit_cast(long, v);
+                    if constexpr (FMT == CML_Q8_0) bw[r][b] = *reinterpret_cast<const v2i_w *>(w_mine + row * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8);
+                    else bw[r][b] = *reinterpret_cast<const v2i_w *>(w_mine + row * 128 + ((b ^ ((n >> 1) & 7)) << 4) + (kq & 1) * 8);
+                    if constexpr (!kLate) {
+                        bw[r][b] = b32_operand<FMT>(bw[r][b], kq);
+                        dw[r][b] = b32_scale<FMT>(dh[r][b >> 1], b & 1);
+                        md[r][b] = -12582912.0f * dw[r][b];
+                        if (b & 1) high = __builtin_elementwise_max(high, __builtin_bit_cast(us2_w, dh[r][b >> 1] & 0x7c007c00u));
                     }
                 }
             }
-            finite = __builtin_amdgcn_ballot_w64(high == 0x7c00u) == 0;
+            if constexpr (!kLate) {
+                finite = __builtin_amdgcn_ballot_w64(max(high.x, high.y) == 0x7c00) == 0;
+                __builtin_amdgcn_sched_barrier(0);  // (in front of the workgroup barrier: behind it the check is 0.04 us of every slab)
+            }
         };
 
         // A operand of block b: octet kq of token n; the blocks' scales of tokens 4 kq .. + 3
@@ -189,11 +214,11 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
         read_w(0);
         wide_barrier();
 
-        float acc[RT][G][4];
+        float acc[RT][NG][4];
 #pragma unroll
         for (int r = 0; r < RT; r++)
 #pragma unroll
-            for (int g = 0; g < G; g++)
+            for (int g = 0; g < NG; g++)
 #pragma unroll
                 for (int j = 0; j < 4; j++) acc[r][g][j] = 0.0f;
 
@@ -202,7 +227,7 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
         auto step = [&](const uint8_t *slab, const float *xs, auto fin) __attribute__((always_inline)) {
             // Software pipeline over units of two blocks of a token group: while the matrix cores work on unit i + 1, the
             // f32 steps of unit i run and the operands of unit i + 2 are read.
-            constexpr int kUnits = G * 4;
+            constexpr int kUnits = NG * 4;
             long av[3][2];
             float4 xv[2][4];  // scales of four blocks, of the lane's four tokens
             v4i_w d[2][RT][2];
@@ -220,20 +245,27 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
 #pragma unroll
                 for (int e = 0; e < 2; e++)
 #pragma unroll
-                    for (int r = 0; r < RT; r++) d[i & 1][r][e] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i % 3][e], bw[r][2 * (i & 3) + e], magic, 0, 0, 0);
+                    for (int r = 0; r < RT; r++) {
+                        const v2i_w w = kLate ? b32_operand<FMT>(bw[r][2 * (i & 3) + e], kq) : bw[r][2 * (i & 3) + e];
+                        d[i & 1][r][e] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[i % 3][e], __builtin_bit_cast(long, w), magic, 0, 0, 0);
+                    }
             };
             auto chain = [&](int i) __attribute__((always_inline)) {
                 const int g = i >> 2, u = i & 3, h = u >> 1;
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const int b = 2 * u + e, k = 2 * (u & 1) + e;
+                    float late[RT];
+#pragma unroll
+                    for (int r = 0; r < RT; r++) late[r] = kLate ? b32_scale<FMT>(dh[r][b >> 1], b & 1) : 0.0f;
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         const float x = k == 0 ? xv[h][j].x : k == 1 ? xv[h][j].y : k == 2 ? xv[h][j].z : xv[h][j].w;
 #pragma unroll
                         for (int r = 0; r < RT; r++) {
                             const float f = __builtin_bit_cast(float, static_cast<int>(d[i & 1][r][e][j]));
-                            const float p = decltype(fin)::value ? __builtin_fmaf(f, dw[r][b], md[r][b]) : (f - 12582912.0f) * dw[r][b];
+                            const float d_w = kLate ? late[r] : dw[kLate ? 0 : r][kLate ? 0 : b];
+                            const float p = !kLate && decltype(fin)::value ? __builtin_fmaf(f, d_w, md[kLate ? 0 : r][kLate ? 0 : b]) : (f - 12582912.0f) * d_w;
                             acc[r][g][j] = acc[r][g][j] + p * x;
                         }
                     }
@@ -260,7 +292,7 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
 #pragma unroll
                 for (int m = 0; m < 2 * RT; m++) {
                     __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x2, 12, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x2, kLate ? 22 : 12, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -273,8 +305,8 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
             __builtin_amdgcn_sched_barrier(0);
             const uint8_t *slab = slabs + buf * L::kSlab;
             const float *xs = reinterpret_cast<const float *>(slabs + kXsAt + buf * L::kXs);
-            if (finite) step(slab, xs, std::true_type{});
-            else step(slab, xs, std::false_type{});
+            if (kLate || !finite) step(slab, xs, std::false_type{});
+            else step(slab, xs, std::true_type{});
             wide_wait<kAhead>();
             buf = buf == D ? 0 : buf + 1;
             slot = slot == D - 1 ? 0 : slot + 1;
@@ -289,7 +321,7 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
             if (row < a.rows) {
                 float *out = a.out + static_cast<int64_t>(a0 + tok0) * a.rows + row;
 #pragma unroll
-                for (int g = 0; g < G; g++)
+                for (int g = 0; g < NG; g++)
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
                         const int t = 16 * g + 4 * kq + j;
@@ -297,45 +329,78 @@ __global__ __launch_bounds__(64 * kB32Waves, 2) void gemm_b32_wide_kernel(B32Wid
                     }
             }
         }
-        if constexpr (!GROUPED) return;
-        wide_barrier();  // (every wave's requests have arrived: the next column may use the buffers)
+    };
+    if constexpr (GROUPED) {
+        for (int tok0 = 0; tok0 < n_assign; tok0 += NTOK) {
+            walk(tok0, min(NTOK, n_assign - tok0), std::integral_constant<int, G>{});
+            wide_barrier();  // (every wave's requests have arrived: the next column may use the buffers)
+        }
+    } else if constexpr (G == 1) {
+        walk(col * NTOK, min(NTOK, n_assign - col * NTOK), std::integral_constant<int, 1>{});
+    } else {
+        // The columns' token groups differ by one at most: those of 13 groups in columns of up to four are 4, 3, 3, 3.  Where they do differ, every other
+        // 32 workgroups of an XCD take the columns one further on: the two workgroups of a compute unit (it gets the 32nd after its first) are not both the
+        // larger ones.  14336 x 4096 at 200 tokens 63.3 -> 60.6 us (Q8_0), 61.6 -> 58.4 (Q4_0) against a last column padded to four.
+        const int turn = col + (a.more == 0 ? 0 : (row_block >> 3) * a.n_cols >> 5 & 1), c = turn == a.n_cols ? 0 : turn;
+        const int first = 16 * (c * a.base + min(c, a.more)), here = a.base + (c < a.more ? 1 : 0);
+        const int n_here = min(16 * here, n_assign - first);
+        if (here == G) walk(first, n_here, std::integral_constant<int, G>{});
+        else walk(first, n_here, std::integral_constant<int, G - 1>{});
     }
 }
 
-template <int FMT, int G, int RT, int D, bool GROUPED = false>
-static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
+template <int FMT, int G, int RT, int D, bool GROUPED, bool ONCE>
+static int launch_b32_wide_as(const B32WideArgs &ka, int slots, hipStream_t st) {
     typedef B32WideLds<FMT, G, RT, D> L;
-    constexpr int kRows = kB32Waves * 16 * RT;
-    ka.n_row_blocks = (ka.rows + kRows - 1) / kRows;
-    ka.n_cols = GROUPED ? 1 : (ka.n_tokens + L::NTOK - 1) / L::NTOK;
+    auto *kernel = &gemm_b32_wide_kernel<FMT, G, RT, D, GROUPED, ONCE>;
     static std::atomic<bool> raised{false};  // per instantiation: allow more than 64 KB of dynamic LDS once
     if (!raised.load(std::memory_order_acquire)) {
-        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_b32_wide_kernel<FMT, G, RT, D, GROUPED>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((gemm_b32_wide_kernel<FMT, G, RT, D, GROUPED>), dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * kB32Waves), L::kTotal, st, ka);
+    hipLaunchKernelGGL(kernel, dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * kB32Waves), L::kTotal, st, ka);
     // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>[.grouped]"
     CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D) + (GROUPED ? ".grouped" : ""));
     CML_HIP_TRY(hipGetLastError());
     return CML_OK;
 }
 
+// Weights that one column reads go past the caches: always those of expert groups, those of a plain call of up to 16 tokens (128256 x 3072 at 16 tokens in Q8_0
+// 85.3 -> 79.0 us, 32000 x 4096 34.4 -> 30.9; a single wider column gains half of that and no kernel of its own).
+template <int FMT, int G, int RT, int D, bool GROUPED = false>
+static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
+    constexpr int kRows = kB32Waves * 16 * RT;
+    ka.n_row_blocks = (ka.rows + kRows - 1) / kRows;
+    ka.n_cols = GROUPED ? 1 : (ka.n_tokens + 16 * G - 1) / (16 * G);
+    const int groups = (ka.n_tokens + 15) / 16;
+    ka.base = groups / ka.n_cols;
+    ka.more = groups % ka.n_cols;
+    if constexpr (GROUPED) return launch_b32_wide_as<FMT, G, RT, D, true, true>(ka, slots, st);
+    else if constexpr (G == 1)
+        if (ka.n_cols == 1) return launch_b32_wide_as<FMT, G, RT, D, false, true>(ka, slots, st);
+    if constexpr (!GROUPED) return launch_b32_wide_as<FMT, G, RT, D, false, false>(ka, slots, st);
+}
+
 struct B32WideShape {
     int g = 0, rt = 0, d = 0;
 };
 
-// Estimated us of a launch (less a constant), fitted on MI355X to 2200 pairs of weight and tokens on cold weights (more than the last-level cache holds
-// between two launches on one): both formats, 512 to 152064 rows, 512 to 14336 values, 6 to 200 tokens.  A slab costs a fixed latency and, for every wave
-// on a SIMD and row tile, 0.3 us and 0.1 us per token group (a wave alone on its SIMD stalls where two overlap: 1.4, not 1, times that).  A second
-// slab ahead shortens the latency of workgroups that have a compute unit of their own (8 tokens, one slab ahead / two: 4096 x 4096 Q8_0 17.8 / 13.5 us, Q4_0
-// 18.9 / 15.7; 14336 x 5120 27.4 / 19.2, 24.5 / 20.2); where two share one it is on par.  Workgroups fill an XCD's 32 compute units row block by row block
-// (wide_block).  The shape with the lowest estimate is on average 0.7 % (Q8_0) and 1.3 % (Q4_0) slower than the fastest, 20 % at worst.
-static float b32_wide_cost(int rows, int groups, int n_slabs, const B32WideShape &s) {
+// Estimated us of a launch (less a constant), fitted on MI355X to 900 pairs of weight and tokens in every shape on cold weights (more than the last-level cache
+// holds between two launches on one): both formats, 512 to 128256 rows, 512 to 14336 values, 6 to 400 tokens.  A slab costs a fixed latency and, for every wave
+// on a SIMD and row tile, 0.23 us (0.16 where Q4_0 is unpacked at its one use) and 0.1 us per token group (a wave alone on its SIMD stalls where others overlap: 1.5, not 1,
+// times that).  A second slab ahead shortens the latency of workgroups that have a compute unit of their own (8 tokens, one slab ahead / two: 4096 x 4096 Q8_0
+// 17.8 / 13.5 us; 14336 x 5120 27.4 / 19.2) and, from about eight slabs, pays for its longer start on tall weights too (65536 x 4096 Q8_0 at 6 tokens 67.7 / 55.5).
+// Workgroups fill an XCD's 32 compute units row block by row block (wide_block); `resident` of them by registers.  The shape with the lowest estimate is on
+// average 0.8 % slower than the fastest, 22 % at worst (the estimate without residence and start: 0.9 % in Q8_0, 2.4 % in Q4_0).
+static float b32_wide_cost(bool late, int rows, int groups, int n_slabs, const B32WideShape &s) {
     const int64_t blocks = (rows + s.rt * 64 - 1) / (s.rt * 64), per_xcd = (blocks + 7) / 8 * ((groups + s.g - 1) / s.g);
-    const float per_cu = per_xcd / 32.0f, full = per_cu / 2;  // (two workgroups are resident at once)
-    const float rounds = full <= 1.0f ? 1.0f : 0.5f * full + 0.5f * std::ceil(full);
-    const float base = per_cu > 1.0f ? 0.25f : s.d == 1 ? 0.35f : 0.22f;
-    return rounds * n_slabs * (base + (per_cu > 1.0f ? 2.0f : 1.4f) * s.rt * (0.3f + 0.1f * s.g));
+    const int resident = s.rt == 1 ? (late ? 4 : s.g <= 3 ? 3 : 2) : late ? 3 : 2;
+    const float per_cu = per_xcd / 32.0f, full = per_cu / resident;
+    const bool shared = per_cu > 1.0f;
+    const float rounds = full <= 1.0f ? 1.0f : 0.28f * full + 0.72f * std::ceil(full);
+    const float base = shared ? (s.d == 1 ? 0.27f : 0.253f) : s.d == 1 ? 0.35f : 0.22f;
+    const float waves = shared ? std::max(1.9f, std::min<float>(resident, per_cu)) : 1.52f;
+    return rounds * (n_slabs * (base + waves * s.rt * ((late ? 0.164f : 0.229f) + 0.095f * s.g)) + (s.d == 2 ? 0.47f : 0.0f));
 }
 
 template <int FMT, int G, int RT, int D>
@@ -344,7 +409,9 @@ static int b32_wide_visit(const B32WideArgs &ka, B32WideShape &best, float &cost
     static_assert(2 * L::kTotal <= 160 * 1024, "two workgroups per compute unit");
     if (launch) return launch->g == G && launch->rt == RT && launch->d == D ? launch_b32_wide<FMT, G, RT, D>(ka, 1, st) : -1;
     const B32WideShape s{G, RT, D};
-    const float c = b32_wide_cost(ka.rows, (ka.n_tokens + 15) / 16, ka.n_slabs, s);
+    const int groups = (ka.n_tokens + 15) / 16;
+    if (G > 1 && (groups + G - 1) / G == (groups + G - 2) / std::max(1, G - 1)) return -1;  // (as few columns have room with a group less)
+    const float c = b32_wide_cost(FMT == CML_Q4_0 && G == 1, ka.rows, groups, ka.n_slabs, s);
     if (c < cost) {
         cost = c;
         best = s;

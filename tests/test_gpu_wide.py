@@ -128,6 +128,21 @@ def test_wide_b32_cells_are_bitwise_the_gemv(name, fmt, tag, rows, cols):
                 assert np.array_equal(got, ref, equal_nan=True) if special else G.same_bits(got, ref)
 
 
+# token columns that differ by a group, on enough row blocks that they change places between the workgroups of a compute unit
+@pytest.mark.parametrize("n,groups", [(200, 4), (135, 3), (70, 4), (33, 2)])
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_columns_of_unequal_width(name, fmt, tag, n, groups):
+    rows, cols = 9300, 512
+    w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=n))
+    s, q = oracle.quantize_activation(fmt, np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32))
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        ref = G.gpu_gemm(w, s, q)
+    for tiles in (1, 2):
+        G.say(f"wide {name} unequal columns n={n} groups={groups} tiles={tiles}")
+        with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=groups, CAMELID_HIP_WIDE_TILES=tiles, CAMELID_HIP_WIDE_AHEAD=1), G.engaged(rf"^{tag}\.mfma\.wide\.g{groups}r{tiles}d1$"):
+            assert G.same_bits(G.gpu_gemm(w, s, q), ref)
+
+
 @pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
 def test_wide_b32_on_a_row_band(name, fmt, tag):
     rows, cols, n = 200, 5 * 256, 40
