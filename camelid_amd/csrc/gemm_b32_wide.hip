@@ -22,6 +22,8 @@
 // eight bytes, octets 2, 3 the high ones.
 // With one token group the weight costs Q4_0 more than the cells do: its words and scales are converted where they are used, in four instructions per word pair and two per
 // scale where they were eight and four, and in registers enough fewer that four waves fit a SIMD (32000 x 4096 at 16 tokens 22.8 -> 20.2 us, 4096 x 14336 46 -> 39).
+// Rows of no whole slabs (cols no multiple of 256) had the packed dot alone, eight tokens per pass over the weight: 4096 x 4160 at 16 / 40 / 200 tokens 31.5 -> 16.1,
+// 78 -> 16.5, 394 -> 26.6 us, 14336 x 2912 at 64 161 -> 23.5.
 // us per launch, gemm_b32_mfma.hip -> here: Q8_0 14336 x 4096 at 24 / 64 / 200 / 512 tokens 34.5 -> 21.2, 67 -> 24, 217 -> 58,
 // 434 -> 115 (523 TOP/s); 4096 x 14336 at 64 / 512 73 -> 39, 541 -> 116; Q4_0 128256 x 3072 at 16 / 64 57.7 -> 51, 156 -> 100.
 #include "gemm_wide.hpp"
@@ -37,10 +39,11 @@ struct B32WideArgs {
     const uint8_t *scales;  // plane 1: f16 per block, row-major
     int64_t q_stride, s_stride;
     int rows, n_slabs;
+    int nb;            // blocks per row
     int n_row_blocks, n_cols;
     int base, more;    // token groups of a column; columns that have one more
-    const int8_t *q;   // [n_tokens][n_slabs*256]
-    const float *xs;   // [n_tokens][n_slabs*8], 16-byte aligned
+    const int8_t *q;   // [n_tokens][nb*32]
+    const float *xs;   // [n_tokens][nb], 16-byte aligned (rows of whole slabs)
     float *out;        // [n_tokens][rows]
     int n_tokens;
     // Grouped call (mixture of experts), as in WideArgs: blockIdx.y -> group, its band of rows and its assignments.
@@ -71,22 +74,25 @@ __device__ __forceinline__ float b32_scale(uint32_t two, int odd) {
 }
 
 // LDS layout of one workgroup.
-template <int FMT, int G, int RT, int D>
+template <int FMT, int G, int RT, int D, bool RAGGED>
 struct B32WideLds {
     static constexpr int NTOK = 16 * G;
     static constexpr int kRowBytes = FMT == CML_Q8_0 ? 256 : 128;
     static constexpr int kSlab = NTOK * 256;
     static constexpr int kXs = (NTOK + 31) / 32 * 1024;         // activation scales [token][8]
     static constexpr int kQuants = RT * 16 * kRowBytes;         // of a wave's rows
-    static constexpr int kWave = kQuants + RT * 256;            // + block scales [row][8] f16
+    static constexpr int kScales = RAGGED ? 512 : 256;          // block scales of 16 rows, [row][8] f16; RAGGED: the eight aligned words from the first on
+    static constexpr int kWave = kQuants + RT * kScales;
     static constexpr int kTotal = (D + 1) * (kSlab + kXs) + D * kB32Waves * kWave;
 };
 
 // G: token groups of 16 per column.  RT: row tiles of a wave.  D: slabs requested ahead.
 // GROUPED: expert groups; a workgroup walks all token columns of its group.  ONCE: the weight is read by one column.
-template <int FMT, int G, int RT, int D, bool GROUPED, bool ONCE>
-__global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 1 ? 4 : 3) : 2) void gemm_b32_wide_kernel(B32WideArgs a) {
-    typedef B32WideLds<FMT, G, RT, D> L;
+// RAGGED: rows of no whole slabs.  Their last slab is short: requests past the row repeat its last piece, the blocks it does not have take no f32 step;
+// scale rows may start at any even address, activation scales come a word per lane.
+template <int FMT, int G, int RT, int D, bool GROUPED, bool ONCE, bool RAGGED>
+__global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? 5 - RT - RAGGED : 2) void gemm_b32_wide_kernel(B32WideArgs a) {
+    typedef B32WideLds<FMT, G, RT, D, RAGGED> L;
     constexpr int NTOK = L::NTOK, WAVES = kB32Waves;
     constexpr int kThreads = 64 * WAVES;
     constexpr bool kLate = FMT == CML_Q4_0 && G == 1;  // a slab's weight is used once: it is unpacked where it is used
@@ -118,22 +124,37 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 
         const uint32_t lds0 = lds_address(smem);
         // Activation: thread tid fetches slot tid % 16 of tokens tid / 16 + 16 * k.
         const int t16 = tid >> 4, piece = (tid & 15) ^ (t16 & 15);
-        const uint32_t row_bytes = n_slabs * 256u;
+        const uint32_t row_bytes = RAGGED ? a.nb * 32u : n_slabs * 256u;
         const int8_t *q_base = a.q + (GROUPED ? 0 : static_cast<int64_t>(tok0) * row_bytes);
         uint32_t src[NG];
 #pragma unroll
         for (int k = 0; k < NG; k++) src[k] = act_row(t16 + 16 * k) * row_bytes + piece * 16;
-        // Scales: lane pairs of the first waves, token 32 * wave + lane / 2.
+        // Scales: lane pairs of the first waves, token 32 * wave + lane / 2; RAGGED: eight tokens per request, a block per lane.
         const bool xs_wave = wave < L::kXs / 1024;
-        const float *xs_base = a.xs + (GROUPED ? 0 : static_cast<int64_t>(tok0) * (n_slabs * 8));
-        const uint32_t xs_src = act_row(32 * wave + (lane >> 1)) * (n_slabs * 32u) + (lane & 1) * 16;
+        const float *xs_base = a.xs + (GROUPED ? 0 : static_cast<int64_t>(tok0) * (RAGGED ? a.nb : n_slabs * 8));
+        const uint32_t xs_src = RAGGED ? 0 : act_row(32 * wave + (lane >> 1)) * (n_slabs * 32u) + (lane & 1) * 16;
+        constexpr int kXsReqs = RAGGED ? (NG + 1) / 2 : 0;
+        uint32_t xs_row[RAGGED ? kXsReqs : 1];
+#pragma unroll
+        for (int i = 0; i < kXsReqs; i++) xs_row[i] = act_row(8 * wave + 32 * i + (lane >> 3)) * (a.nb * 4u);
         auto fetch = [&](int slab, int buf) __attribute__((always_inline)) {
             slab = min(slab, n_slabs - 1);
-            if (xs_wave) wide_dma16(lds0 + kXsAt + buf * L::kXs + wave * 1024, xs_base + slab * 8, xs_src);
+            uint32_t cut = 0;  // what a lane's piece lies past the row
+            if constexpr (RAGGED) {
+                const int left = a.nb - 8 * slab;
+                cut = max(piece - 2 * left + 1, 0) * 16;
+                const uint32_t block = min(lane & 7, left - 1) * 4;
+#pragma unroll
+                for (int i = 0; i < kXsReqs; i++)
+                    if (wave + 4 * i < 2 * NG)  // (the address in a scalar register, which the compiler does not see to by itself)
+                        wide_dma4(__builtin_amdgcn_readfirstlane(lds0 + kXsAt + buf * L::kXs + (wave + 4 * i) * 256), xs_base + slab * 8, xs_row[i] + block);
+            } else if (xs_wave) {
+                wide_dma16(lds0 + kXsAt + buf * L::kXs + wave * 1024, xs_base + slab * 8, xs_src);
+            }
 #pragma unroll
             for (int k = 0; k < NG; k++)
                 if (!GROUPED || 4 * wave + 16 * k < n_here)  // (what no token owns stays what it was: cells of its own, never stored)
-                    wide_dma16(lds0 + buf * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + slab * 256, src[k]);
+                    wide_dma16(lds0 + buf * L::kSlab + k * (16 * kThreads) + wave * 1024, q_base + slab * 256, src[k] - cut);
         };
         // Weights: rows past the end repeat the last one.
         const int first = min(row0, a.rows - 1), last = a.rows - 1 - first;  // (of this wave's rows)
@@ -141,29 +162,46 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 
         const uint8_t *wd = a.scales + (band * a.rows + first) * a.s_stride;
         constexpr int kRowsReq = 1024 / L::kRowBytes, kReqs = L::kQuants / 1024;
         const uint32_t w_lds = lds0 + kWAt + wave * L::kWave;  // + slot * WAVES * kWave
+        auto w_row = [&](int i) __attribute__((always_inline)) { return kRowsReq * i + lane / (64 / kRowsReq); };
+        auto w_piece = [&](int i) __attribute__((always_inline)) {
+            const int slot = lane % (64 / kRowsReq), r = w_row(i);
+            return FMT == CML_Q8_0 ? slot ^ (r & 15) : slot ^ ((r >> 1) & 7);
+        };
         uint32_t w_src[kReqs];
 #pragma unroll
-        for (int i = 0; i < kReqs; i++) {
-            const int r = kRowsReq * i + lane / (64 / kRowsReq);
-            const int slot = lane % (64 / kRowsReq);
-            const int p = FMT == CML_Q8_0 ? slot ^ (r & 15) : slot ^ ((r >> 1) & 7);
-            w_src[i] = static_cast<uint32_t>(min(r, last)) * static_cast<uint32_t>(a.q_stride) + p * 16;
-        }
-        uint32_t d_src[RT];
+        for (int i = 0; i < kReqs; i++) w_src[i] = static_cast<uint32_t>(min(w_row(i), last)) * static_cast<uint32_t>(a.q_stride) + w_piece(i) * 16;
+        // Scales: four lanes per row; RAGGED: eight, from the aligned word that holds the slab's first scale (wd need not be one) up to the row's last word.
+        const uint32_t wd_off = RAGGED ? static_cast<uint32_t>(reinterpret_cast<uintptr_t>(wd) & 3) : 0;
+        constexpr int kDReqs = L::kScales / 256 * RT;
+        uint32_t d_src[kDReqs], d_end[RAGGED ? kDReqs : 1];
 #pragma unroll
-        for (int r = 0; r < RT; r++) d_src[r] = static_cast<uint32_t>(min(16 * r + (lane >> 2), last)) * static_cast<uint32_t>(a.s_stride) + (lane & 3) * 4;
+        for (int r = 0; r < kDReqs; r++) {
+            if constexpr (RAGGED) {
+                const uint32_t row_at = wd_off + static_cast<uint32_t>(min(8 * r + (lane >> 3), last)) * static_cast<uint32_t>(a.s_stride);
+                d_src[r] = (row_at & ~3u) + (lane & 7) * 4;
+                d_end[r] = (row_at + 2 * a.nb - 1) & ~3u;
+            } else {
+                d_src[r] = static_cast<uint32_t>(min(16 * r + (lane >> 2), last)) * static_cast<uint32_t>(a.s_stride) + (lane & 3) * 4;
+            }
+        }
         auto fetch_w = [&](int slab, int slot) __attribute__((always_inline)) {
             slab = min(slab, n_slabs - 1);
             const uint32_t to = w_lds + slot * (WAVES * L::kWave);
+            const int pieces = RAGGED ? (FMT == CML_Q8_0 ? 2 : 1) * (a.nb - 8 * slab) : 0;  // of the row from this slab on
 #pragma unroll
             for (int i = 0; i < kReqs; i++) {
-                if constexpr (ONCE) wide_dma16_once(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
-                else wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, w_src[i]);
+                uint32_t from = w_src[i];
+                if constexpr (RAGGED) from -= max(w_piece(i) - pieces + 1, 0) * 16;
+                if constexpr (ONCE) wide_dma16_once(to + i * 1024, wq + slab * L::kRowBytes, from);
+                else wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, from);
             }
 #pragma unroll
-            for (int r = 0; r < RT; r++) wide_dma4(to + L::kQuants + r * 256, wd + slab * 16, d_src[r]);
+            for (int r = 0; r < kDReqs; r++) {
+                if constexpr (RAGGED) wide_dma4(to + L::kQuants + r * 256, wd - wd_off, min(d_src[r] + slab * 16, d_end[r]));
+                else wide_dma4(to + L::kQuants + r * 256, wd + slab * 16, d_src[r]);
+            }
         };
-        constexpr int kAhead = (D - 1) * (NG + kReqs + RT);  // requests that may be outstanding at the end of a step (some waves have more)
+        constexpr int kAhead = (D - 1) * (NG + kReqs + kDReqs);  // requests that may be outstanding at the end of a step (some waves have more)
 
         // Operands of a slab: the lane's octet of the eight blocks of either tile's row, the blocks' scales.  With one token group they are
         // used once and stay as they were read until then (28 registers fewer per tile: a third or fourth wave on a SIMD).
@@ -177,11 +215,19 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 
 #pragma unroll
             for (int r = 0; r < RT; r++) {
                 const int row = 16 * r + n;
-                const uint4 d = *reinterpret_cast<const uint4 *>(w_mine + L::kQuants + row * 16);
+                const uint8_t *scales = w_mine + L::kQuants + row * (L::kScales / 16);
+                const uint4 d = *reinterpret_cast<const uint4 *>(scales);
                 dh[r][0] = d.x;
                 dh[r][1] = d.y;
                 dh[r][2] = d.z;
                 dh[r][3] = d.w;
+                if constexpr (RAGGED) {
+                    // (a row past the end repeats the last one, whose parity counts)
+                    const uint32_t up = ((wd_off + static_cast<uint32_t>(min(row, last)) * static_cast<uint32_t>(a.s_stride)) & 2) * 8;  // 16: the first scale is the upper half of its word
+                    const uint32_t fifth = reinterpret_cast<const uint32_t *>(scales)[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) dh[r][i] = __builtin_amdgcn_alignbit(i < 3 ? dh[r][i + 1] : fifth, dh[r][i], up);
+                }
 #pragma unroll
                 for (int b = 0; b < 8; b++) {
                     if constexpr (FMT == CML_Q8_0) bw[r][b] = *reinterpret_cast<const v2i_w *>(w_mine + row * 256 + (((2 * b + (kq >> 1)) ^ n) << 4) + (kq & 1) * 8);
@@ -224,7 +270,7 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 
 
         const v4i_w magic = {0x4b400000, 0x4b400000, 0x4b400000, 0x4b400000};
 
-        auto step = [&](const uint8_t *slab, const float *xs, auto fin) __attribute__((always_inline)) {
+        auto step = [&](const uint8_t *slab, const float *xs, int blocks, auto fin, auto tail) __attribute__((always_inline)) {
             // Software pipeline over units of two blocks of a token group: while the matrix cores work on unit i + 1, the
             // f32 steps of unit i run and the operands of unit i + 2 are read.
             constexpr int kUnits = NG * 4;
@@ -255,6 +301,7 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const int b = 2 * u + e, k = 2 * (u & 1) + e;
+                    if (decltype(tail)::value && b >= blocks) continue;
                     float late[RT];
 #pragma unroll
                     for (int r = 0; r < RT; r++) late[r] = kLate ? b32_scale<FMT>(dh[r][b >> 1], b & 1) : 0.0f;
@@ -305,8 +352,9 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 
             __builtin_amdgcn_sched_barrier(0);
             const uint8_t *slab = slabs + buf * L::kSlab;
             const float *xs = reinterpret_cast<const float *>(slabs + kXsAt + buf * L::kXs);
-            if (kLate || !finite) step(slab, xs, std::false_type{});
-            else step(slab, xs, std::true_type{});
+            if (RAGGED && s == n_slabs - 1) step(slab, xs, a.nb - 8 * s, std::false_type{}, std::integral_constant<bool, RAGGED>{});
+            else if (kLate || !finite) step(slab, xs, 8, std::false_type{}, std::false_type{});
+            else step(slab, xs, 8, std::true_type{}, std::false_type{});
             wide_wait<kAhead>();
             buf = buf == D ? 0 : buf + 1;
             slot = slot == D - 1 ? 0 : slot + 1;
@@ -349,18 +397,18 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? (RT == 
     }
 }
 
-template <int FMT, int G, int RT, int D, bool GROUPED, bool ONCE>
+template <int FMT, int G, int RT, int D, bool GROUPED, bool ONCE, bool RAGGED>
 static int launch_b32_wide_as(const B32WideArgs &ka, int slots, hipStream_t st) {
-    typedef B32WideLds<FMT, G, RT, D> L;
-    auto *kernel = &gemm_b32_wide_kernel<FMT, G, RT, D, GROUPED, ONCE>;
+    typedef B32WideLds<FMT, G, RT, D, RAGGED> L;
+    auto *kernel = &gemm_b32_wide_kernel<FMT, G, RT, D, GROUPED, ONCE, RAGGED>;
     static std::atomic<bool> raised{false};  // per instantiation: allow more than 64 KB of dynamic LDS once
     if (!raised.load(std::memory_order_acquire)) {
         CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised.store(true, std::memory_order_release);
     }
     hipLaunchKernelGGL(kernel, dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * kB32Waves), L::kTotal, st, ka);
-    // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>[.grouped]"
-    CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D) + (GROUPED ? ".grouped" : ""));
+    // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>[.ragged][.grouped]"
+    CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D) + (RAGGED ? ".ragged" : "") + (GROUPED ? ".grouped" : ""));
     CML_HIP_TRY(hipGetLastError());
     return CML_OK;
 }
@@ -375,10 +423,16 @@ static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
     const int groups = (ka.n_tokens + 15) / 16;
     ka.base = groups / ka.n_cols;
     ka.more = groups % ka.n_cols;
-    if constexpr (GROUPED) return launch_b32_wide_as<FMT, G, RT, D, true, true>(ka, slots, st);
-    else if constexpr (G == 1)
-        if (ka.n_cols == 1) return launch_b32_wide_as<FMT, G, RT, D, false, true>(ka, slots, st);
-    if constexpr (!GROUPED) return launch_b32_wide_as<FMT, G, RT, D, false, false>(ka, slots, st);
+    const bool ragged = ka.nb % 8 != 0;
+    if constexpr (G == 4 && RT == 2) {  // (no registers left for the ragged form)
+        return ragged ? fail(CML_ERR_UNSUPPORTED, "wide matrix-core kernel: no such shape") : launch_b32_wide_as<FMT, G, RT, D, false, false, false>(ka, slots, st);
+    } else if constexpr (GROUPED) {
+        return ragged ? launch_b32_wide_as<FMT, G, RT, D, true, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, true, true, false>(ka, slots, st);
+    } else {
+        if constexpr (G == 1)
+            if (ka.n_cols == 1) return ragged ? launch_b32_wide_as<FMT, G, RT, D, false, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, false, true, false>(ka, slots, st);
+        return ragged ? launch_b32_wide_as<FMT, G, RT, D, false, false, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, false, false, false>(ka, slots, st);
+    }
 }
 
 struct B32WideShape {
@@ -405,11 +459,12 @@ static float b32_wide_cost(bool late, int rows, int groups, int n_slabs, const B
 
 template <int FMT, int G, int RT, int D>
 static int b32_wide_visit(const B32WideArgs &ka, B32WideShape &best, float &cost, const B32WideShape *launch, hipStream_t st) {
-    typedef B32WideLds<FMT, G, RT, D> L;
+    typedef B32WideLds<FMT, G, RT, D, true> L;
     static_assert(2 * L::kTotal <= 160 * 1024, "two workgroups per compute unit");
     if (launch) return launch->g == G && launch->rt == RT && launch->d == D ? launch_b32_wide<FMT, G, RT, D>(ka, 1, st) : -1;
     const B32WideShape s{G, RT, D};
     const int groups = (ka.n_tokens + 15) / 16;
+    if (G == 4 && RT == 2 && ka.nb % 8 != 0) return -1;
     if (G > 1 && (groups + G - 1) / G == (groups + G - 2) / std::max(1, G - 1)) return -1;  // (as few columns have room with a group less)
     const float c = b32_wide_cost(FMT == CML_Q4_0 && G == 1, ka.rows, groups, ka.n_slabs, s);
     if (c < cost) {
@@ -450,13 +505,16 @@ static int launch_b32_wide_grouped(const B32WideArgs &ka, const MatArgs &a, hipS
     return g == 1 ? launch_b32_wide<FMT, 1, 1, 1, true>(ka, slots, st) : launch_b32_wide<FMT, 2, 1, 1, true>(ka, slots, st);
 }
 
+// Rows of no whole slabs (up to a slab the packed dot serves them).
+bool b32_wide_ragged(const cml_weight *w) { return (w->fmt == CML_Q8_0 || w->fmt == CML_Q4_0) && w->nb > 8 && w->nb % 8 != 0; }
+
 // Whether the offsets of a grouped call's activation rows fit 32 bits and its weight and scales can be read 16 bytes at a time.
 bool gemm_b32_wide_serves_groups(const MatArgs &a) {
-    return b32_mfma_usable(a.w) && reinterpret_cast<uintptr_t>(a.scales) % 16 == 0 &&
+    return (b32_wide_ragged(a.w) || (b32_mfma_usable(a.w) && reinterpret_cast<uintptr_t>(a.scales) % 16 == 0)) &&
            std::max(a.n_assign_total, a.n_tokens) * a.w->nb * 32 < (int64_t{1} << 32);
 }
 
-// On a weight that b32_mfma_usable accepts, activation scales 16-byte aligned; grouped: gemm_b32_wide_serves_groups.
+// On a weight that b32_mfma_usable accepts, activation scales 16-byte aligned, or one of b32_wide_ragged; grouped: gemm_b32_wide_serves_groups.
 int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
     const cml_weight *w = a.w;
     B32WideArgs ka{};
@@ -465,7 +523,8 @@ int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
     ka.scales = w->planes.p[1];
     ka.s_stride = w->planes.row_stride[1];
     ka.rows = static_cast<int>(a.group_offsets ? a.band_rows : w->rows);
-    ka.n_slabs = static_cast<int>(w->nb / 8);
+    ka.n_slabs = static_cast<int>((w->nb + 7) / 8);
+    ka.nb = static_cast<int>(w->nb);
     ka.q = a.q;
     ka.xs = a.scales;
     ka.out = a.out;

@@ -256,11 +256,11 @@ static int launch_expert_matmul(const MatArgs &a, hipStream_t st) {
     }
     if (a.w->fmt != CML_Q4_K) {
         const int64_t groups = a.group_ids ? a.max_active : a.n_groups;
-        // The wide kernel from three assignments per group on average.  us per layer, packed dot or narrow matrix-core kernel / wide, Q4_0: 128 experts, top-8,
-        // 2816 / 704 at 32 / 64 tokens (2 and 4 each; down has no whole slabs) 121 / 123, 177 / 154; 64 experts, 2048 / 1024 at 16 / 40 (2 and 5) 64 / 64,
-        // 108 / 72; 32 experts, 2816 / 1408 at 24 / 64 (6 and 16) 148 / 86, 243 / 157.
+        // The wide kernel from two assignments per group on average.  us per layer, packed dot / wide, Q4_0: 128 experts, top-8, 2816 / 704 at 24 / 32 / 40 tokens
+        // (1.5, 2, 2.5 each) 103 / 108, 121 / 118, 135 / 127; 64 experts, 2816 / 1408 at 10 / 16 (1.25, 2) 94 / 95, 118 / 111; 32 experts, 1280 / 704 at 10 (2.5) 40 / 32;
+        // Q8_0: 128 experts, 2048 / 768 at 28 / 36 (1.75, 2.25) 123 / 119, 141 / 127; 64 experts, 1280 / 704 at 14 (1.75) 53 / 57.
         const int wide = env_int("CAMELID_HIP_MFMA_WIDE", 1);  // 0 = never, 1 = by shape, 2 = always
-        if (a.group_offsets && wide && (wide == 2 || a.n_assign_total >= 3 * groups) && gemm_b32_wide_serves_groups(a)) return launch_gemm_b32_wide(a, st);
+        if (a.group_offsets && wide && (wide == 2 || a.n_assign_total >= 2 * groups) && gemm_b32_wide_serves_groups(a)) return launch_gemm_b32_wide(a, st);
         // (scales off a 16-byte boundary, activation rows past 4 GB of offsets: the narrow matrix-core kernel once the groups fill a 16-token tile reasonably)
         if (a.group_offsets && b32_mfma_usable(a.w) && a.n_assign_total >= groups * env_int("CAMELID_HIP_B32_MFMA_MIN_GROUP", 6))
             return launch_gemm_b32_mfma(a, st);

@@ -143,6 +143,34 @@ def test_wide_b32_columns_of_unequal_width(name, fmt, tag, n, groups):
             assert G.same_bits(G.gpu_gemm(w, s, q), ref)
 
 
+# a last slab of one, two, seven blocks; scale rows that start at odd halves of a word (an odd number of blocks), also where a band starts
+@pytest.mark.parametrize("rows,cols", [(1, 288), (70, 320), (300, 736), (131, 4128)])
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_rows_of_no_whole_slabs(name, fmt, tag, rows, cols):
+    wire = G.synth_weight(fmt, rows, cols, seed=rows + cols)
+    blocks = wire.reshape(-1, 34 if fmt == B.CML_Q8_0 else 18)
+    for special in (False, True):
+        if special:
+            blocks[:: 37, :2] = np.frombuffer(np.float16(np.inf).tobytes(), np.uint8)
+            blocks[7:: 43, 1] ^= 0x80
+        w = Weight.upload(fmt, rows, cols, wire)
+        for n in (5, 17, 70):
+            s, q = oracle.quantize_activation(fmt, np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32))
+            s = s.reshape(n, -1).copy()
+            if special:
+                s[1, -1] = np.inf  # the scale that a short slab's requests repeat
+            views = [w] + ([w.slice(3, rows - 5)] if rows > 16 else [])
+            for v in views:
+                with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(r"\.dot\.", none=(r"\.mfma\.",)):
+                    ref = G.gpu_gemm(v, s, q)
+                for g, tiles, ahead in [(g, t, 1) for g in (1, 2, 3, 4) for t in (1, 2) if (g, t) != (4, 2)] + [(1, 1, 2)]:
+                    G.say(f"ragged {name} {rows}x{cols} n={n} groups={g} tiles={tiles} ahead={ahead} special={special}")
+                    with G.env(CAMELID_HIP_WIDE_GROUPS=g, CAMELID_HIP_WIDE_TILES=tiles, CAMELID_HIP_WIDE_AHEAD=ahead, CAMELID_HIP_B32_MFMA_MIN_TOKENS=1), \
+                            G.engaged(rf"^{tag}\.mfma\.wide\.g{g}r{tiles}d{ahead}\.ragged$", none=(r"\.dot\.",)):
+                        got = G.gpu_gemm(v, s, q)
+                    assert np.array_equal(got, ref, equal_nan=True) if special else G.same_bits(got, ref)
+
+
 @pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
 def test_wide_b32_on_a_row_band(name, fmt, tag):
     rows, cols, n = 200, 5 * 256, 40
@@ -157,6 +185,24 @@ def test_wide_b32_on_a_row_band(name, fmt, tag):
 
 
 # gate | up fused (gathered rows), down on rows of whole slabs; groups of none, one, past a column; a band that ends inside a workgroup
+# rows of no whole slabs (down, then both)
+@pytest.mark.parametrize("E,k,hidden,ff,T", [(6, 3, 512, 352, 20), (4, 2, 1088, 704, 35)])
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_expert_groups_on_rows_of_no_whole_slabs(name, fmt, tag, E, k, hidden, ff, T):
+    gate_up = Weight.upload(fmt, E * 2 * ff, hidden, G.synth_weight(fmt, E * 2 * ff, hidden, seed=E))
+    down = Weight.upload(fmt, E * hidden, ff, G.synth_weight(fmt, E * hidden, ff, seed=E + 1))
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    idx, weight, _, _ = gpu_route(rng.standard_normal((T, E)).astype(np.float32), k)
+    run = lambda: gpu_moe(gate_up, None, down, E, k, idx, weight, x, glu=1)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        ref = run()
+    for g in (1, 2):
+        G.say(f"ragged {name} experts E={E} k={k} {hidden}/{ff} T={T} groups={g}")
+        with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g), G.engaged(rf"^{tag}\.mfma\.wide\.g{g}r1d1\.ragged\.grouped$", none=(r"\.dot\.",)):
+            assert G.same_bits(run(), ref)
+
+
 @pytest.mark.parametrize("E,k,hidden,ff,T", [(16, 4, 768, 512, 40), (8, 3, 256, 256, 1), (5, 2, 1280, 768, 33)])
 @pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
 def test_wide_b32_expert_groups_are_bitwise_the_gemv(name, fmt, tag, E, k, hidden, ff, T):
@@ -221,6 +267,12 @@ ROUTES = [
     ("Q4_0", 4100, 5120, 8, r"^q4_0\.mfma\.wide\."),  # more
     ("Q8_0", 7000, 768, 8, r"^q8_0\.dot\."),  # rows of three slabs
     ("Q4_0", 2048, 1024, 8, r"^q4_0\.mfma\.kpar\."),  # four
+    ("Q8_0", 4096, 2912, 8, r"^q8_0\.dot\."),  # rows of no whole slabs: one pass of the packed dot on small weights
+    ("Q8_0", 4096, 2912, 9, r"^q8_0\.mfma\.wide\..*ragged$"),  # two
+    ("Q4_0", 2048, 1056, 5, r"^q4_0\.mfma\.wide\..*ragged$"),  # up to four slabs and a part
+    ("Q4_0", 8192, 2912, 5, r"^q4_0\.dot\."),
+    ("Q4_0", 8192, 2912, 6, r"^q4_0\.mfma\.wide\..*ragged$"),
+    ("Q8_0", 14336, 1056, 3, r"^q8_0\.mfma\.wide\..*ragged$"),  # more than 767 tiles
 ]
 
 
