@@ -8,6 +8,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from camelid_amd import binding as B
@@ -339,3 +340,34 @@ def test_argmax_first_maximum_wins():
     got = out.to_numpy(np.float32, (2, cols))
     for r in range(2):
         assert G.same_bits(got[r], ref[int(np.argmax(logits[r]))])
+
+
+@pytest.mark.parametrize("n", [16383, 16384, 16385, 20480, 40001])  # one workgroup; parts: whole, one value more, rows off a 16-byte boundary
+def test_argmax_of_long_rows_does_not_depend_on_what_the_index_held(n):
+    rng = np.random.default_rng(n)
+    logits = rng.standard_normal((7, n)).astype(np.float32)
+    logits[1, 4095] = logits[1, 4096] = logits[1, n - 1] = 9.0  # equal maxima on both sides of a part's edge, and in the last
+    logits[2, :] = -np.inf                                      # nothing beats the starting value: index 0
+    logits[3, 0], logits[3, n - 1] = np.nan, 50.0
+    logits[4, :] = -0.0
+    logits[4, 1:] = 0.0                                         # all equal
+    logits[5, :] = np.arange(n)                                 # every part beats the ones before
+    logits[6, :] = np.nan
+    want = [int(np.argmax(r)) if r.max() > -3.4e38 else 0 for r in np.where(np.isnan(logits), -np.inf, logits)]
+    ld = DeviceBuffer.from_numpy(logits)
+    for before in (0, 1, n - 1, n, 4096, 0xFFFFFFFF):
+        od = DeviceBuffer.from_numpy(np.full(7, before, np.uint32))
+        G.say(f"argmax n={n} index held {before}")
+        for r in range(7):  # (row by row: several rows at once take a workgroup each)
+            check(lib().cml_argmax_f32(ld.ptr + 4 * n * r, 1, n, od.ptr + 4 * r, None), "cml_argmax_f32")
+        check(lib().cml_stream_sync(None))
+        assert list(od.to_numpy(np.uint32, (7,))) == want, before
+    host = torch.full((7,), 3, dtype=torch.int32, pin_memory=True)  # host memory that the GPU writes
+    for r in range(7):
+        check(lib().cml_argmax_f32(ld.ptr + 4 * n * r, 1, n, host.data_ptr() + 4 * r, None), "cml_argmax_f32")
+    check(lib().cml_stream_sync(None))
+    assert host.tolist() == want
+    two = DeviceBuffer.from_numpy(np.full(2, 7, np.uint32))  # (two rows of 32768 and more share the parts' launch)
+    check(lib().cml_argmax_f32(ld.ptr + 4 * n * 4, 2, n, two.ptr, None), "cml_argmax_f32")
+    check(lib().cml_stream_sync(None))
+    assert list(two.to_numpy(np.uint32, (2,))) == want[4:6]
