@@ -40,6 +40,7 @@ struct B32WideArgs {
     int64_t q_stride, s_stride;
     int rows, n_slabs;
     int nb;            // blocks per row
+    bool once;         // (chooses the kernel)
     int n_row_blocks, n_cols;
     int base, more;    // token groups of a column; columns that have one more
     const int8_t *q;   // [n_tokens][nb*32]
@@ -413,10 +414,11 @@ static int launch_b32_wide_as(const B32WideArgs &ka, int slots, hipStream_t st) 
     return CML_OK;
 }
 
-// Weights that one column reads go past the caches: always those of expert groups, those of a plain call of up to 16 tokens (128256 x 3072 at 16 tokens in Q8_0
-// 85.3 -> 79.0 us, 32000 x 4096 34.4 -> 30.9; a single wider column gains half of that and no kernel of its own).
+// Large weights that one column reads go past the caches (wide_reads_once): those of expert groups, those of a plain call of up to 16 tokens (128256 x 3072 at 16
+// tokens in Q8_0 85.3 -> 79.0 us; a single wider column gains half of that and no kernel of its own).
 template <int FMT, int G, int RT, int D, bool GROUPED = false>
 static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
+    const bool once = ka.once;
     constexpr int kRows = kB32Waves * 16 * RT;
     ka.n_row_blocks = (ka.rows + kRows - 1) / kRows;
     ka.n_cols = GROUPED ? 1 : (ka.n_tokens + 16 * G - 1) / (16 * G);
@@ -427,10 +429,11 @@ static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
     if constexpr (G == 4 && RT == 2) {  // (no registers left for the ragged form)
         return ragged ? fail(CML_ERR_UNSUPPORTED, "wide matrix-core kernel: no such shape") : launch_b32_wide_as<FMT, G, RT, D, false, false, false>(ka, slots, st);
     } else if constexpr (GROUPED) {
-        return ragged ? launch_b32_wide_as<FMT, G, RT, D, true, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, true, true, false>(ka, slots, st);
+        if (once) return ragged ? launch_b32_wide_as<FMT, G, RT, D, true, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, true, true, false>(ka, slots, st);
+        return ragged ? launch_b32_wide_as<FMT, G, RT, D, true, false, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, true, false, false>(ka, slots, st);
     } else {
         if constexpr (G == 1)
-            if (ka.n_cols == 1) return ragged ? launch_b32_wide_as<FMT, G, RT, D, false, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, false, true, false>(ka, slots, st);
+            if (once && ka.n_cols == 1) return ragged ? launch_b32_wide_as<FMT, G, RT, D, false, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, false, true, false>(ka, slots, st);
         return ragged ? launch_b32_wide_as<FMT, G, RT, D, false, false, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, false, false, false>(ka, slots, st);
     }
 }
@@ -525,6 +528,7 @@ int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
     ka.rows = static_cast<int>(a.group_offsets ? a.band_rows : w->rows);
     ka.n_slabs = static_cast<int>((w->nb + 7) / 8);
     ka.nb = static_cast<int>(w->nb);
+    ka.once = wide_reads_once(w);
     ka.q = a.q;
     ka.xs = a.scales;
     ka.out = a.out;

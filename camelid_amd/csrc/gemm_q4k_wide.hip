@@ -5,7 +5,9 @@
 // operand (S = lo + 8 hi, two contractions over the whole super-block), the mins against the sums of the
 // activation's 16-value runs in one f16 instruction.  There the 16 operand words of a super-block are formed again for every 64
 // tokens and the activation passes through registers on its way to LDS; here once for up to 128.
-// Bound: instruction issue, of which a super-block and 16 x 16 cells take nine matrix and 24 vector instructions, and LDS reads (5.5 KB).
+// Bound: instruction issue and LDS reads, which add up: a super-block and 16 x 16 cells take nine and a half matrix instructions, 16 vector ones and 4.6 KB of LDS (a read costs
+// the matrix unit about ten cycles of its register ports).  The products of the scales, eight vector instructions before, come from the matrix unit (chain below); with the
+// scales unpacked in fewer steps 14336 x 4096 at 64 / 200 / 512 tokens 20.1 -> 19.4, 38.8 -> 37.8, 80.0 -> 77.3.
 // us per launch, before -> after: 14336 x 4096 at 64 / 200 / 512 tokens 19.3 -> 17.8, 54 -> 36, 98 -> 76 (790 TOP/s); 4096 x 14336 at 200 / 512
 // 88 -> 49, 185 -> 82; a layer of 8 experts of 4096 / 14336, top-2, at 48 / 128 tokens 217 -> 190, 340 -> 256.
 #include "gemm_wide.hpp"
@@ -34,9 +36,12 @@ struct Q4KWide {
     int64_t sb_stride;
     uint32_t piece_src, lane4;
     int kq, hdr_at, piece_at[2];
-    v4i_w blo[4], bhi[4];
-    v4h_w mins;
-    float dw, dminw;
+    struct Operands {
+        v4i_w lo[4], hi[4];  // the values times the two digits of their sub-block's scale
+        v4h_w mins;
+        float scale;         // d in the lanes of even k-quarters, -dmin in the others
+        float d, dmin;
+    };
 
     // LDS: pieces a and b of 16 rows x 4 chunks, chunk c of row r in slot c ^ (r / 2 % 4); 16 headers.
     __device__ __forceinline__ Q4KWide(const Weight &w, int64_t band, int rows, int tile, int lane) {
@@ -50,10 +55,11 @@ struct Q4KWide {
         for (int q = 0; q < 2; q++) piece_at[q] = (kq & 1) * 1024 + n * 64 + (((2 * q + (kq >> 1)) ^ ((n >> 1) & 3)) << 4);
         hdr_at = 2048 + n * 16;
     }
+    template <bool ONCE>
     __device__ __forceinline__ void fetch(uint32_t lds, int sb) const {
         const uint8_t *p = base + sb * sb_stride;
-        wide_dma16(lds, p, piece_src);
-        wide_dma16(lds + 1024, p, piece_src + 1024u);
+        wide_dma16_hint<ONCE>(lds, p, piece_src);
+        wide_dma16_hint<ONCE>(lds + 1024, p, piece_src + 1024u);
         wide_dma4(lds + 2048, p, lane4);
     }
     __device__ __forceinline__ void read(Raw &r, const uint8_t *lds, int) const {
@@ -65,54 +71,76 @@ struct Q4KWide {
     // values 128 q + 64 (kq / 2) + 32 plane + 16 (kq % 2) .. + 15, piece 8 q + 4 (kq / 2) + 2 plane + kq % 2 of a token
     static __device__ __forceinline__ int lane_piece(int kq) { return 4 * (kq >> 1) + (kq & 1); }
     static __device__ constexpr int step_piece(int c) { return 8 * (c >> 1) + 2 * (c & 1); }
-    __device__ __forceinline__ void unpack(const Raw &r) {
-        typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-        uint32_t sc03, sc47, m03, m47;
-        q4k_unpack_scales(r.hdr.y, r.hdr.z, r.hdr.w, sc03, sc47, m03, m47);
-        dw = f16_bits_to_f32(r.hdr.x & 0xffffu);
-        dminw = f16_bits_to_f32(r.hdr.x >> 16);
-        // runs 4 kq .. + 3 of the activation: the mins of sub-blocks 2 kq and 2 kq + 1, twice each (exact in f16)
-        const uint32_t mw = ((kq & 2) ? m47 : m03) >> (16 * (kq & 1));
-        const _Float16 ma = static_cast<_Float16>(static_cast<float>(mw & 0xffu)), mb = static_cast<_Float16>(static_cast<float>((mw >> 8) & 0xffu));
-        mins = v4h_w{ma, ma, mb, mb};
+    // A super-block is unpacked in five parts: scales, then the operand words of one step each.
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+    static constexpr int kParts = 5;
+    struct Part {
+        us2 lo[2], hi[2];  // digits of the scales of chunk 2 q + kq / 2: sub-block 2 * chunk, 2 * chunk + 1
+    };
+    __device__ __forceinline__ void unpack(const Raw &r, Operands &o, Part &d, int p) const {
+        if (p == 0) {
+            const uint32_t word = (kq & 1) ? (r.hdr.x ^ 0x80000000u) >> 16 : r.hdr.x;
+            o.scale = f16_bits_to_f32(word & 0xffffu);
+            o.d = f16_bits_to_f32(r.hdr.x & 0xffffu);
+            o.dmin = f16_bits_to_f32(r.hdr.x >> 16);
+            // runs 4 kq .. + 3 of the activation: the mins of sub-blocks 2 kq and 2 kq + 1, twice each (exact in f16)
+            const int odd = 16 * (kq & 1);
+            const uint32_t m03 = r.hdr.z >> odd, m47 = ((r.hdr.w >> (odd + 4)) & 0x0f0fu) | ((m03 >> 2) & 0x3030u);
+            const uint32_t mw = (kq & 2) ? m47 : m03 & 0x3f3fu;
+            const us2 m2 = __builtin_bit_cast(us2, __builtin_amdgcn_perm(mw, mw, 0x0c010c00u));
+            const _Float16 ma = static_cast<_Float16>(m2.x), mb = static_cast<_Float16>(m2.y);
+            o.mins = v4h_w{ma, ma, mb, mb};
+            const int up = 16 * (kq >> 1);
+            const uint32_t s03 = r.hdr.y >> up, s47 = ((r.hdr.w >> up) & 0x0f0fu) | ((s03 >> 2) & 0x3030u);
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const uint32_t sc = (q ? sc47 : sc03) >> (16 * (kq >> 1));
-            const uint32_t dlo = sc & 0x0707u, dhi = (sc >> 3) & 0x0707u;
-            const uint32_t pc[4] = {r.piece[q].x, r.piece[q].y, r.piece[q].z, r.piece[q].w};
-#pragma unroll
-            for (int plane = 0; plane < 2; plane++) {  // low nibbles = sub-block 2 * chunk, high = 2 * chunk + 1
-                const us2 l2 = __builtin_bit_cast(us2, __builtin_amdgcn_perm(dlo, dlo, plane ? 0x0c010c01u : 0x0c000c00u));
-                const us2 h2 = __builtin_bit_cast(us2, __builtin_amdgcn_perm(dhi, dhi, plane ? 0x0c010c01u : 0x0c000c00u));
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-                    const us2 v = __builtin_bit_cast(us2, (pc[m] >> (4 * plane)) & 0x0f0f0f0fu);
-                    // (a byte pair times a digit, at most 15 * 7, never carries into its neighbour)
-                    blo[2 * q + plane][m] = __builtin_bit_cast(int, static_cast<us2>(v * l2));
-                    bhi[2 * q + plane][m] = __builtin_bit_cast(int, static_cast<us2>(v * h2));
-                }
+            for (int q = 0; q < 2; q++) {
+                const uint32_t sc = __builtin_amdgcn_perm(q ? s47 : s03, q ? s47 : s03, 0x0c010c00u);
+                d.lo[q] = __builtin_bit_cast(us2, sc & 0x00070007u);
+                d.hi[q] = __builtin_bit_cast(us2, (sc >> 3) & 0x00070007u);
             }
+            return;
+        }
+        const int c = p - 1, q = c >> 1, plane = c & 1;  // low nibbles = sub-block 2 * chunk, high = 2 * chunk + 1
+        const us2 l2 = plane ? us2{d.lo[q].y, d.lo[q].y} : us2{d.lo[q].x, d.lo[q].x};
+        const us2 h2 = plane ? us2{d.hi[q].y, d.hi[q].y} : us2{d.hi[q].x, d.hi[q].x};
+        const uint32_t pc[4] = {r.piece[q].x, r.piece[q].y, r.piece[q].z, r.piece[q].w};
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const us2 v = __builtin_bit_cast(us2, (pc[m] >> (4 * plane)) & 0x0f0f0f0fu);
+            // (a byte pair times a digit, at most 15 * 7, never carries into its neighbour)
+            o.lo[c][m] = __builtin_bit_cast(int, static_cast<us2>(v * l2));
+            o.hi[c][m] = __builtin_bit_cast(int, static_cast<us2>(v * h2));
         }
     }
     struct Sums {
         v4i_w lo, hi;
         v4f_w p;
     };
-    static constexpr int kMfma = 9, kChainPerMfma = 3;
-    __device__ __forceinline__ void contract(const v4i_w (&av)[4], const v4h_w rs, Sums &s) const {
+    static constexpr int kMfma = 9;
+    __device__ __forceinline__ void contract(const Operands &o, const v4i_w (&av)[4], const v4h_w rs, Sums &s) const {
         s.lo = s.hi = v4i_w{0, 0, 0, 0};
-        s.p = __builtin_amdgcn_mfma_f32_16x16x16f16(rs, mins, v4f_w{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            s.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], blo[c], s.lo, 0, 0, 0);
-            s.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], bhi[c], s.hi, 0, 0, 0);
+            s.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], o.lo[c], s.lo, 0, 0, 0);
+            s.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], o.hi[c], s.hi, 0, 0, 0);
         }
+        s.p = __builtin_amdgcn_mfma_f32_16x16x16f16(rs, o.mins, v4f_w{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
     }
-    __device__ __forceinline__ void chain(const Sums &s, const float (&yv)[4], float (&acc)[4]) const {
+    // One matrix instruction forms yd * d and yd * -dmin of two token groups: its four 16 x 16 products of K = 1 are
+    // (group 0, d), (group 0, -dmin), (group 1, d), (group 1, -dmin), each the rounded product that a vector multiplication gives.
+    static constexpr int kScaleGroups = 2;
+    __device__ __forceinline__ void chain(const Sums &s, const v16f_w &y, int g, float (&acc)[4]) const {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            acc[j] = __builtin_fmaf(-(yv[j] * dminw), s.p[j], acc[j]);
-            acc[j] = __builtin_fmaf(yv[j] * dw, static_cast<float>(s.lo[j] + 8 * s.hi[j]), acc[j]);
+            acc[j] = __builtin_fmaf(y[8 * g + 4 + j], s.p[j], acc[j]);
+            acc[j] = __builtin_fmaf(y[8 * g + j], static_cast<float>(s.lo[j] + 8 * s.hi[j]), acc[j]);
+        }
+    }
+    __device__ __forceinline__ void chain(const Sums &s, const float (&yv)[4], const Operands &o, float (&acc)[4]) const {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            acc[j] = __builtin_fmaf(-(yv[j] * o.dmin), s.p[j], acc[j]);
+            acc[j] = __builtin_fmaf(yv[j] * o.d, static_cast<float>(s.lo[j] + 8 * s.hi[j]), acc[j]);
         }
     }
 };

@@ -40,8 +40,10 @@ struct Q6KWide {
     const uint8_t *ql, *qh, *sc, *d;      // of the tile's first row (wave-uniform)
     uint32_t ql_src[2], qh_src, sc_src, d_src;  // where this lane's bytes of the requests lie from there
     int kq, ql_at[2], qh_at[2], n16, d_at, d_odd;
-    v4i_w blo[4], bhi[4];
-    float dw;
+    struct Operands {
+        v4i_w lo[4], hi[4];  // the bytes of the values times their sub-block's scale
+        float scale;         // d
+    };
 
     // LDS: 16 rows of 128 ql bytes, 16-byte piece p of row r in slot p ^ (r % 8); 16 rows of 64 qh bytes, piece p in slot
     // p ^ (r / 2 % 4); 16 rows of 16 scales; 16 words that hold the rows' d (one of the two halves of an aligned word).
@@ -74,6 +76,7 @@ struct Q6KWide {
         n16 = 3072 + n * 16;
         d_at = 3328 + n * 4;
     }
+    template <bool>
     __device__ __forceinline__ void fetch(uint32_t lds, int sb) const {
         wide_dma16(lds, ql + sb * 128, ql_src[0]);
         wide_dma16(lds + 1024, ql + sb * 128, ql_src[1]);
@@ -95,55 +98,49 @@ struct Q6KWide {
     // The product of a 6-bit value (code - 32) and its int8 scale needs 13 bits; as p = 256 hi + lo with lo a signed byte
     // both are int8 operands:  r = code * sc + (128 - 32 sc) = p + 128,  hi = r >> 8,  lo = (r & 255) ^ 0x80 as a signed byte.
     // One packed 16-bit multiply-add gives r for two values.
-    __device__ __forceinline__ void unpack(const Raw &r) {
+    static constexpr int kParts = 4;
+    struct Part {};
+    __device__ __forceinline__ void unpack(const Raw &r, Operands &o, Part &, int c) const {
         typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-        dw = f16_bits_to_f32(r.d);
+        const int h = c >> 1, plane = c & 1;
+        if (c == 0) o.scale = f16_bits_to_f32(r.d);
         const int jj = 2 * (kq >> 1);
         const uint32_t scw[4] = {r.sc.x, r.sc.y, r.sc.z, r.sc.w};
+        const uint32_t l[4] = {r.ql[h].x, r.ql[h].y, r.ql[h].z, r.ql[h].w};
+        const uint32_t u[4] = {r.qh[h].x, r.qh[h].y, r.qh[h].z, r.qh[h].w};
+        const int s = static_cast<int>(scw[c] << (24 - 8 * kq)) >> 24;  // sub-block 8 h + 4 plane + kq
+        const uint32_t s2 = __builtin_amdgcn_perm(static_cast<uint32_t>(s), static_cast<uint32_t>(s), 0x01000100u);
+        const us2 s16 = __builtin_bit_cast(us2, s2);
+        const us2 o16 = s16 * us2{static_cast<unsigned short>(-32), static_cast<unsigned short>(-32)} + us2{128, 128};
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const uint32_t l[4] = {r.ql[h].x, r.ql[h].y, r.ql[h].z, r.ql[h].w};
-            const uint32_t u[4] = {r.qh[h].x, r.qh[h].y, r.qh[h].z, r.qh[h].w};
-#pragma unroll
-            for (int plane = 0; plane < 2; plane++) {
-                const int c = 2 * h + plane;
-                const int s = static_cast<int>(scw[c] << (24 - 8 * kq)) >> 24;  // sub-block 8 h + 4 plane + kq
-                const uint32_t s2 = __builtin_amdgcn_perm(static_cast<uint32_t>(s), static_cast<uint32_t>(s), 0x01000100u);
-                const us2 s16 = __builtin_bit_cast(us2, s2);
-                const us2 o16 = s16 * us2{static_cast<unsigned short>(-32), static_cast<unsigned short>(-32)} + us2{128, 128};
-                uint32_t lo[4], hi[4];
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-                    const uint32_t up = (plane ? u[m] >> jj : u[m] << (4 - jj)) & 0x30303030u;
-                    uint32_t code = ((plane ? l[m] >> 4 : l[m]) & 0x0f0f0f0fu) | up;
-                    asm("" : "+v"(code));  // (the compiler otherwise rebuilds the code for either half of the bytes)
-                    const us2 even = __builtin_bit_cast(us2, code & 0x00ff00ffu), odd = __builtin_bit_cast(us2, __builtin_amdgcn_perm(code, code, 0x0c030c01u));
-                    const uint32_t re = __builtin_bit_cast(uint32_t, static_cast<us2>(even * s16 + o16));
-                    const uint32_t ro = __builtin_bit_cast(uint32_t, static_cast<us2>(odd * s16 + o16));
-                    // bytes of values 0..3: even low halves hold values 0 and 2, odd ones 1 and 3
-                    lo[m] = __builtin_amdgcn_perm(ro, re, 0x06020400u) ^ 0x80808080u;
-                    hi[m] = __builtin_amdgcn_perm(ro, re, 0x07030501u);
-                }
-                blo[c] = v4i_w{static_cast<int>(lo[0]), static_cast<int>(lo[1]), static_cast<int>(lo[2]), static_cast<int>(lo[3])};
-                bhi[c] = v4i_w{static_cast<int>(hi[0]), static_cast<int>(hi[1]), static_cast<int>(hi[2]), static_cast<int>(hi[3])};
-            }
+        for (int m = 0; m < 4; m++) {
+            const uint32_t up = (plane ? u[m] >> jj : u[m] << (4 - jj)) & 0x30303030u;
+            uint32_t code = ((plane ? l[m] >> 4 : l[m]) & 0x0f0f0f0fu) | up;
+            asm("" : "+v"(code));  // (the compiler otherwise rebuilds the code for either half of the bytes)
+            const us2 even = __builtin_bit_cast(us2, code & 0x00ff00ffu), odd = __builtin_bit_cast(us2, __builtin_amdgcn_perm(code, code, 0x0c030c01u));
+            const uint32_t re = __builtin_bit_cast(uint32_t, static_cast<us2>(even * s16 + o16));
+            const uint32_t ro = __builtin_bit_cast(uint32_t, static_cast<us2>(odd * s16 + o16));
+            // bytes of values 0..3: even low halves hold values 0 and 2, odd ones 1 and 3
+            o.lo[c][m] = static_cast<int>(__builtin_amdgcn_perm(ro, re, 0x06020400u) ^ 0x80808080u);
+            o.hi[c][m] = static_cast<int>(__builtin_amdgcn_perm(ro, re, 0x07030501u));
         }
     }
     struct Sums {
         v4i_w lo, hi;
     };
-    static constexpr int kMfma = 8, kChainPerMfma = 2;
-    __device__ __forceinline__ void contract(const v4i_w (&av)[4], const v4h_w, Sums &s) const {
+    static constexpr int kMfma = 8;
+    __device__ __forceinline__ void contract(const Operands &o, const v4i_w (&av)[4], const v4h_w, Sums &s) const {
         s.lo = s.hi = v4i_w{0, 0, 0, 0};
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            s.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], blo[c], s.lo, 0, 0, 0);
-            s.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], bhi[c], s.hi, 0, 0, 0);
+            s.lo = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], o.lo[c], s.lo, 0, 0, 0);
+            s.hi = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[c], o.hi[c], s.hi, 0, 0, 0);
         }
     }
-    __device__ __forceinline__ void chain(const Sums &s, const float (&yv)[4], float (&acc)[4]) const {
+    static constexpr int kScaleGroups = 0;  // (one multiplication per cell and super-block: not ahead as a matrix instruction)
+    __device__ __forceinline__ void chain(const Sums &s, const float (&yv)[4], const Operands &o, float (&acc)[4]) const {
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(dw * yv[j], static_cast<float>(s.lo[j] + 256 * s.hi[j]), acc[j]);
+        for (int j = 0; j < 4; j++) acc[j] = __builtin_fmaf(o.scale * yv[j], static_cast<float>(s.lo[j] + 256 * s.hi[j]), acc[j]);
     }
 };
 

@@ -35,6 +35,7 @@ namespace cml {
 
 typedef int v4i_w __attribute__((ext_vector_type(4)));
 typedef float v4f_w __attribute__((ext_vector_type(4)));
+typedef float v16f_w __attribute__((ext_vector_type(16)));
 typedef _Float16 v4h_w __attribute__((ext_vector_type(4)));
 
 // One wave's 1 KB: lane l's 16 bytes at base + off (off per lane) to LDS byte lds_byte + 16 * l (lds_byte wave-uniform).
@@ -58,6 +59,11 @@ __device__ __forceinline__ void wide_dma4(uint32_t lds_byte, const void *base, u
     const void *at;
     asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dword %2, %0" : "=&s"(at) : "s"(lds_byte), "v"(off), "s"(base) : "memory", "m0");
 }
+template <bool ONCE>
+__device__ __forceinline__ void wide_dma16_hint(uint32_t lds_byte, const void *base, uint32_t off) {
+    if constexpr (ONCE) wide_dma16_once(lds_byte, base, off);
+    else wide_dma16(lds_byte, base, off);
+}
 // Waits until at most OUT of the wave's vector-memory operations are outstanding (loads complete in order).
 template <int OUT>
 __device__ __forceinline__ void wide_wait() {
@@ -66,6 +72,14 @@ __device__ __forceinline__ void wide_wait() {
 }
 // Workgroup barrier after this wave's LDS operations (__syncthreads would also wait for every load in flight).
 __device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A weight of which little would be found again in the 256 MB last-level cache is requested past it (where one column reads it).  Between uses of a smaller one
+// that cache may hold it, and then the hint costs: Q8_0 20000 x 2048 at 8 tokens back to back 11.6 us plain, 13.3 so; expert layers of 8 x 3 tensors, Q4_K, 128 tokens, plain / so:
+// 1536 / 6144 (42 MB each) 77 / 81, 3072 / 8192 (113 MB) 139 / 135, 4096 / 14336 (264 MB) 261 / 253; Q8_0 32000 x 4096 (139 MB), one column, 34.3 / 31.6.
+inline bool wide_reads_once(const cml_weight *w) {
+    const int64_t block = w->fmt == CML_Q8_0 ? 34 : w->fmt == CML_Q4_0 ? 18 : w->fmt == CML_Q4_K ? 144 : 210;
+    return w->rows * w->nb * block >= 96ll << 20;
+}
 
 // LDS byte address of a shared-memory pointer.
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
@@ -126,14 +140,17 @@ struct WideLds {
 
 // F: the weight format.  G: token groups of 16 per column.  WAVES: waves per workgroup, WAVES / KS row tiles.
 // KS: groups of waves the K parts are shared over (1 or 2).  SPLIT: K parts are closed inside the lane.
-// GROUPED: expert groups (token groups past a group's last assignment are skipped, rows are gathered).
-template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED>
+// GROUPED: expert groups (token groups past a group's last assignment are skipped, rows are gathered).  ONCE: wide_reads_once.
+template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED, bool ONCE>
 __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2) void gemm_wide_kernel(WideArgs<F> a) {
     typedef WideLds<F, G, WAVES, KS> L;
     constexpr int NTOK = L::NTOK, RT = WAVES / KS, WS = L::WS;
     constexpr int kThreads = 64 * WAVES, kRowsPass = kThreads / 16;        // tokens fetched per pass of the workgroup
     constexpr int kPer = (NTOK + kRowsPass - 1) / kRowsPass;               // passes per slab
     static_assert(KS == 1 || (KS == 2 && !GROUPED), "K parts");
+    // A matrix instruction forms the products of the activation's and the weight's scales; not where three waves share a SIMD's registers (expert groups).
+    constexpr bool kProducts = F::kScaleGroups > 0 && !GROUPED;
+    constexpr int kPair = kProducts ? F::kScaleGroups : 1;
     extern __shared__ uint4 smem[];
     uint8_t *slabs = reinterpret_cast<uint8_t *>(smem);                      // [2][KS][NTOK][256]
     uint8_t *runs = slabs + 2 * KS * L::kSlab;                               // [2][KS][NTOK][16] f16
@@ -207,15 +224,15 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
                         if ((kPer * kRowsPass == NTOK || 4 * wave + kRowsPass * k < NTOK) && (!GROUPED || 4 * wave + kRowsPass * k < n_here)) {
                             const uint4 v = *reinterpret_cast<const uint4 *>(slabs + (buf * KS + kp) * L::kSlab + (tid + kThreads * k) * 16);
                             *reinterpret_cast<_Float16 *>(runs + (buf * KS + kp) * L::kRuns + (t16 + kRowsPass * k) * 32 + piece * 2) =
-                                static_cast<_Float16>(static_cast<float>(bytesum16(v)));
+                                static_cast<_Float16>(static_cast<short>(bytesum16(v)));  // (|sum| <= 2048: exact)
                         }
             }
         };
 
-        F fmt(second ? a.w2 : a.w, band, a.rows, min(tile, a.n_tiles - 1), lane);
+        const F fmt(second ? a.w2 : a.w, band, a.rows, min(tile, a.n_tiles - 1), lane);
         const uint32_t w_lds = lds0 + kWAt + wave * F::kTileBytes;
         const uint8_t *w_mine = wbuf + wave * F::kTileBytes;
-        auto fetch_w = [&](int loc, int slot) __attribute__((always_inline)) { fmt.fetch(w_lds + slot * L::kW, min(s_begin + loc, n_sb - 1)); };
+        auto fetch_w = [&](int loc, int slot) __attribute__((always_inline)) { fmt.template fetch<ONCE>(w_lds + slot * L::kW, min(s_begin + loc, n_sb - 1)); };
 
         // A operand of step c: piece (lane's) ^ (step's) of token n
         uint32_t a_addr[4];
@@ -227,6 +244,7 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
         fetch_w(0, 0);
         if constexpr (WS == 2) fetch_w(1, 1);
         typename F::Raw raw;
+        typename F::Operands ops;
         wide_wait<(WS - 1) * F::kFetches>();
         fmt.read(raw, w_mine, s_begin);
         finish(0);
@@ -261,29 +279,40 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
             fetch_yd(loc + 1, buf ^ 1);
             fetch(loc + 1, buf ^ 1);
             __builtin_amdgcn_sched_barrier(0);
-            fmt.unpack(raw);
+            {
+                typename F::Part part_of;
+#pragma unroll
+                for (int p = 0; p < F::kParts; p++) fmt.unpack(raw, ops, part_of, p);
+            }
             __builtin_amdgcn_sched_barrier(0);
             fetch_w(loc + WS, WS == 2 ? buf : 0);  // (its slot was read into registers a step ago)
             __builtin_amdgcn_sched_barrier(0);
             const uint8_t *slab = slabs + (buf * KS + ks) * L::kSlab;
             const uint8_t *run = runs + (buf * KS + ks) * L::kRuns + n * 32 + kq * 8;
-            const float *ydp = yds + (buf * KS + ks) * (L::kYd / 4) + 4 * kq;
+            const float *ydp = yds + (buf * KS + ks) * (L::kYd / 4) + (kProducts ? 16 * (lane / (64 / kPair)) + n : 4 * kq);
             if (KS == 1 || loc < n_loc) {
                 // Software pipeline over the token groups: while the matrix cores work on group g, the operands of group g + 1
                 // are read from LDS and the f32 steps of group g - 1 run.
                 v4i_w av[2][4];
                 v4h_w rs[2];
-                float4 yd4[3];
+                float4 yd4[kProducts ? 1 : 3];
+                float ya[kProducts ? 2 : 1];
+                v16f_w scale[kProducts ? 2 : 1];  // products of the scales of two or four token groups and of the weight's, all cells of a tile
                 typename F::Sums sums[2];
                 auto read = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
                     for (int c = 0; c < 4; c++) av[g & 1][c] = *reinterpret_cast<const v4i_w *>(slab + a_addr[c] + g * 4096);
                     if constexpr (F::kRunSums) rs[g & 1] = *reinterpret_cast<const v4h_w *>(run + g * 512);
-                    yd4[g % 3] = *reinterpret_cast<const float4 *>(ydp + g * 16);
+                    if constexpr (!kProducts) yd4[g % 3] = *reinterpret_cast<const float4 *>(ydp + g * 16);
+                    else if (g % kPair == 0) ya[g / kPair & 1] = ydp[g * 16];
                 };
                 auto chain = [&](int g) __attribute__((always_inline)) {
-                    const float yv[4] = {yd4[g % 3].x, yd4[g % 3].y, yd4[g % 3].z, yd4[g % 3].w};
-                    fmt.chain(sums[g & 1], yv, acc[g]);
+                    if constexpr (kProducts) {
+                        fmt.chain(sums[g & 1], scale[g / kPair & 1], g % kPair, acc[g]);
+                    } else {
+                        const float yv[4] = {yd4[g % 3].x, yd4[g % 3].y, yd4[g % 3].z, yd4[g % 3].w};
+                        fmt.chain(sums[g & 1], yv, ops, acc[g]);
+                    }
                     // (left alone, the compiler sinks the chains of all steps to the store and keeps every operand alive)
 #pragma unroll
                     for (int j = 0; j < 4; j++) asm volatile("" : "+v"(acc[g][j]));
@@ -294,13 +323,15 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
                 for (int g = 0; g < G; g++) {
                     if (!GROUPED || 16 * g < n_here) {
                         if (g + 1 < G) read(g + 1);
-                        fmt.contract(av[g & 1], rs[g & 1], sums[g & 1]);
+                        fmt.contract(ops, av[g & 1], rs[g & 1], sums[g & 1]);
+                        if constexpr (kProducts)
+                            if (g % kPair == 0) scale[g / kPair & 1] = __builtin_amdgcn_mfma_f32_16x16x1f32(ya[g / kPair & 1], ops.scale, v16f_w{}, 0, 0, 0);
                         if (g > 0) chain(g - 1);
                         __builtin_amdgcn_sched_group_barrier(0x100, F::kRunSums ? 6 : 5, 0);
 #pragma unroll
                         for (int m = 0; m < F::kMfma; m++) {
                             __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x2, F::kChainPerMfma, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x2, F::kScaleGroups == 0 || kProducts ? 2 : 3, 0);
                         }
                         __builtin_amdgcn_sched_barrier(0);
                         if (g == G - 1 || (GROUPED && 16 * (g + 1) >= n_here)) chain(g);
@@ -372,7 +403,7 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
     }
 }
 
-template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED>
+template <class F, int G, int WAVES, int KS, bool SPLIT, bool GROUPED, bool ONCE = false>
 static int launch_wide(WideArgs<F> ka, int slots, hipStream_t st) {
     typedef WideLds<F, G, WAVES, KS> L;
     static_assert(L::kTotal <= 160 * 1024, "LDS of a compute unit");
@@ -382,10 +413,10 @@ static int launch_wide(WideArgs<F> ka, int slots, hipStream_t st) {
     ka.n_cols = GROUPED ? 1 : (ka.n_tokens + L::NTOK - 1) / L::NTOK;
     static std::atomic<bool> raised{false};  // per instantiation: allow more than 64 KB of dynamic LDS once
     if (!raised.load(std::memory_order_acquire)) {
-        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wide_kernel<F, G, WAVES, KS, SPLIT, GROUPED>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        CML_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_wide_kernel<F, G, WAVES, KS, SPLIT, GROUPED, ONCE>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised.store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((gemm_wide_kernel<F, G, WAVES, KS, SPLIT, GROUPED>), dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * WAVES), L::kTotal, st, ka);
+    hipLaunchKernelGGL((gemm_wide_kernel<F, G, WAVES, KS, SPLIT, GROUPED, ONCE>), dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * WAVES), L::kTotal, st, ka);
     // "<format>.mfma.wide.g<token groups>w<waves>[.ksplit2][.serial_split][.grouped]"
     CML_COUNT_LAUNCH(std::string(F::kName) + ".mfma.wide.g" + std::to_string(G) + "w" + std::to_string(WAVES) + (KS == 2 ? ".ksplit2" : "") +
                      (SPLIT ? ".serial_split" : "") + (GROUPED ? ".grouped" : ""));
@@ -503,7 +534,8 @@ static int launch_wide_plain(const MatArgs &a, hipStream_t st) {
 // routing whose assignments fall evenly (mean and one deviation; with one and a half, three token groups where two are enough: layer of 8 experts, top-2, at 100 tokens
 // 2048 / 8192 101 -> 109 us, 4096 / 14336 241 -> 247); a fuller group takes another column, groups of 16 past a group's last are skipped.
 template <class F, int G, int WAVES>
-static int launch_wide_grouped_split(const WideArgs<F> &ka, int slots, hipStream_t st) {
+static int launch_wide_grouped_split(const WideArgs<F> &ka, int slots, bool once, hipStream_t st) {
+    if (once) return ka.ksplit > 1 ? launch_wide<F, G, WAVES, 1, true, true, true>(ka, slots, st) : launch_wide<F, G, WAVES, 1, false, true, true>(ka, slots, st);
     return ka.ksplit > 1 ? launch_wide<F, G, WAVES, 1, true, true>(ka, slots, st) : launch_wide<F, G, WAVES, 1, false, true>(ka, slots, st);
 }
 
@@ -530,10 +562,11 @@ static int launch_wide_grouped(const MatArgs &a, hipStream_t st) {
     const float mean = static_cast<float>(a.n_assign_total) / std::max(1, slots);
     int g = static_cast<int>(std::ceil(std::min<float>(mean + std::sqrt(mean), static_cast<float>(ka.n_tokens)) / 16.0f));
     g = env_int("CAMELID_HIP_WIDE_GROUPS", g);
-    if (g <= 2) return launch_wide_grouped_split<F, 2, 4>(ka, slots, st);
-    if (g <= 3) return launch_wide_grouped_split<F, 3, 4>(ka, slots, st);
-    if (g <= 4) return launch_wide_grouped_split<F, 4, 4>(ka, slots, st);
-    return launch_wide_grouped_split<F, 8, 8>(ka, slots, st);
+    const bool once = wide_reads_once(w);
+    if (g <= 2) return launch_wide_grouped_split<F, 2, 4>(ka, slots, once, st);
+    if (g <= 3) return launch_wide_grouped_split<F, 3, 4>(ka, slots, once, st);
+    if (g <= 4) return launch_wide_grouped_split<F, 4, 4>(ka, slots, once, st);
+    return launch_wide_grouped_split<F, 8, 8>(ka, slots, once, st);
 }
 
 }  // namespace cml
