@@ -32,7 +32,7 @@
 // A workgroup is 4 waves: 4/TB consecutive 16-row tiles x TB token blocks of
 // 16*GPW tokens, sharing the staged activations of NTOK = 16*GPW*TB tokens.  K is
 // walked in slabs of 256 values (8 blocks; rows must be whole slabs -- other
-// lengths take the packed-dot kernel), phases of KC slabs double-buffered in LDS
+// lengths go to gemm_b32_wide.hip or the packed dot), phases of KC slabs double-buffered in LDS
 // as in the Q4_K matrix-core kernel; weights stream through a register ring of
 // RING slabs per wave.
 #include <type_traits>
