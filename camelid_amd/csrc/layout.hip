@@ -421,10 +421,13 @@ __global__ __launch_bounds__(256) void argmax_f32_parts_kernel(const float *__re
 
 int launch_argmax_f32(const float *logits, int64_t n_rows, int64_t n, uint32_t *out_idx, hipStream_t st) {
     if (n_rows == 0) return CML_OK;
-    // Up to four rows of at least 16384 values each (more rows fill the chip by themselves), where out_idx is memory of this GPU (the exchanges; host
-    // memory, which a caller may pass too, takes the plain store).  us, one workgroup per row / parts: a row of 8192 values 3.66 / 3.67, 16384 3.83 / 3.66,
+    // Up to four rows, of at least 16384 values per row there is (more rows fill the chip by themselves), where out_idx is memory of this GPU (the exchanges; host
+    // memory, which a caller may pass too, takes the plain store), on a boundary that an exchange needs, and no part of the logits: a row whose first answers stand
+    // in it is no longer the row that the other workgroups read.  us, one workgroup per row / parts: a row of 8192 values 3.66 / 3.67, 16384 3.83 / 3.66,
     // 32768 4.62 / 4.04, 128256 8.29 / 4.96; four rows of 32768 4.80 / 4.99, 16 rows of 128256 13.6 / 15.5.
-    if (n_rows <= 4 && n >= 4 * kArgmaxPart * n_rows) {
+    const uintptr_t in = reinterpret_cast<uintptr_t>(logits), out = reinterpret_cast<uintptr_t>(out_idx);
+    const bool apart = out + 4 * static_cast<uintptr_t>(n_rows) <= in || in + 4 * static_cast<uintptr_t>(n_rows * n) <= out;
+    if (n_rows <= 4 && n >= 4 * kArgmaxPart * n_rows && apart && out % 4 == 0) {
         hipPointerAttribute_t where{};
         int device = -1;
         if (hipPointerGetAttributes(&where, out_idx) != hipSuccess) (void)hipGetLastError();  // (memory the runtime does not know)

@@ -371,3 +371,18 @@ def test_argmax_of_long_rows_does_not_depend_on_what_the_index_held(n):
     check(lib().cml_argmax_f32(ld.ptr + 4 * n * 4, 2, n, two.ptr, None), "cml_argmax_f32")
     check(lib().cml_stream_sync(None))
     assert list(two.to_numpy(np.uint32, (2,))) == want[4:6]
+
+
+@pytest.mark.parametrize("at", [0, 5000, 39999])
+def test_argmax_of_a_long_row_may_be_written_into_the_row(at):
+    n = 40000
+    logits = np.random.default_rng(at).standard_normal(n).astype(np.float32)
+    logits[0], logits[35000], logits[at] = 30.0, 30.0, 50.0  # the answer's bits are a value below all of these
+    ld = DeviceBuffer.from_numpy(logits)
+    G.say(f"argmax into value {at} of its row")
+    check(lib().cml_argmax_f32(ld.ptr, 1, n, ld.ptr + 4 * at, None), "cml_argmax_f32")
+    check(lib().cml_stream_sync(None))
+    got = ld.to_numpy(np.float32, (n,))
+    assert got.view(np.uint32)[at] == at
+    logits.view(np.uint32)[at] = at
+    assert np.array_equal(got, logits)
