@@ -508,8 +508,11 @@ static int launch_b32_wide_grouped(const B32WideArgs &ka, const MatArgs &a, hipS
     return g == 1 ? launch_b32_wide<FMT, 1, 1, 1, true>(ka, slots, st) : launch_b32_wide<FMT, 2, 1, 1, true>(ka, slots, st);
 }
 
-// Rows of no whole slabs (up to a slab the packed dot serves them).
-bool b32_wide_ragged(const cml_weight *w) { return (w->fmt == CML_Q8_0 || w->fmt == CML_Q4_0) && w->nb > 8 && w->nb % 8 != 0; }
+// Rows of no whole slabs (up to a slab the packed dot serves them).  The packed dot stages a row, 40 bytes per block, in 64 KB of LDS and refuses
+// longer ones: they stay refused in batches too, there is no single-token result that a batch of them could equal.
+bool b32_wide_ragged(const cml_weight *w) {
+    return (w->fmt == CML_Q8_0 || w->fmt == CML_Q4_0) && w->nb > 8 && w->nb % 8 != 0 && w->nb <= 64 * 1024 / 40;
+}
 
 // Whether the offsets of a grouped call's activation rows fit 32 bits and its weight and scales can be read 16 bytes at a time.
 bool gemm_b32_wide_serves_groups(const MatArgs &a) {

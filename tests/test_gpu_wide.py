@@ -171,6 +171,25 @@ def test_wide_b32_rows_of_no_whole_slabs(name, fmt, tag, rows, cols):
                     assert np.array_equal(got, ref, equal_nan=True) if special else G.same_bits(got, ref)
 
 
+# 1637 blocks, and 1641: three more than a row of the packed dot holds
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_rows_of_no_whole_slabs_are_refused_where_the_matvec_refuses_them(name, fmt, tag):
+    rows, n = 20, 9
+    for blocks, served in ((1637, True), (1641, False)):
+        cols = 32 * blocks
+        wire = G.synth_weight(fmt, rows, cols, seed=blocks)
+        w = Weight.upload(fmt, rows, cols, wire)
+        s, q = oracle.quantize_activation(fmt, np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32))
+        qd, sd, od = DeviceBuffer.from_numpy(q), DeviceBuffer.from_numpy(s), DeviceBuffer(n * rows * 4)
+        G.say(f"ragged {name} rows of {blocks} blocks")
+        for tokens in (1, 2, n):
+            rc = lib().cml_gemm(w.handle, qd.ptr, sd.ptr, tokens, od.ptr, None)
+            assert rc == (0 if served else 6), (blocks, tokens, rc)
+        check(lib().cml_stream_sync(None))
+        if served:
+            assert G.same_bits(od.to_numpy(np.float32, (n, rows)), oracle.matmul_q(fmt, wire, cols, s, q, order=oracle.ORDER_PRIMARY, threads=8))
+
+
 @pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
 def test_wide_b32_on_a_row_band(name, fmt, tag):
     rows, cols, n = 200, 5 * 256, 40
