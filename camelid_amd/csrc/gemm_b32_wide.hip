@@ -88,7 +88,8 @@ struct B32WideLds {
 };
 
 // G: token groups of 16 per column.  RT: row tiles of a wave.  D: slabs requested ahead.
-// GROUPED: expert groups; a workgroup walks all token columns of its group.  ONCE: the weight is read by one column.
+// GROUPED: expert groups; a workgroup walks all token columns of its group.  ONCE: the weight is requested past the caches (wide_reads_once) where one column
+// reads it: of expert groups, whose sizes only the device knows, by the workgroups of those that fill one column at most.
 // RAGGED: rows of no whole slabs.  Their last slab is short: requests past the row repeat its last piece, the blocks it does not have take no f32 step;
 // scale rows may start at any even address, activation scales come a word per lane.
 template <int FMT, int G, int RT, int D, bool GROUPED, bool ONCE, bool RAGGED>
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? 5 - RT 
     const int a0 = GROUPED ? a.group_offsets[band] : 0;
     const int n_assign = GROUPED ? a.group_offsets[band + 1] - a0 : a.n_tokens;
     // The walk over K of one column of NG token groups.
-    auto walk = [&](int tok0, int n_here, auto groups) __attribute__((always_inline)) {
+    auto walk = [&](int tok0, int n_here, auto groups, auto once) __attribute__((always_inline)) {
         constexpr int NG = decltype(groups)::value;
         auto act_row = [&](int t) __attribute__((always_inline)) -> uint32_t {  // (tokens past the end repeat the last one)
             const int j = min(t, n_here - 1);
@@ -193,8 +194,7 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? 5 - RT 
             for (int i = 0; i < kReqs; i++) {
                 uint32_t from = w_src[i];
                 if constexpr (RAGGED) from -= max(w_piece(i) - pieces + 1, 0) * 16;
-                if constexpr (ONCE) wide_dma16_once(to + i * 1024, wq + slab * L::kRowBytes, from);
-                else wide_dma16(to + i * 1024, wq + slab * L::kRowBytes, from);
+                wide_dma16_hint<decltype(once)::value>(to + i * 1024, wq + slab * L::kRowBytes, from);
             }
 #pragma unroll
             for (int r = 0; r < kDReqs; r++) {
@@ -380,12 +380,18 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? 5 - RT 
         }
     };
     if constexpr (GROUPED) {
+        if constexpr (ONCE) {
+            if (n_assign <= NTOK) {
+                if (n_assign > 0) walk(0, n_assign, std::integral_constant<int, G>{}, std::true_type{});
+                return;
+            }
+        }
         for (int tok0 = 0; tok0 < n_assign; tok0 += NTOK) {
-            walk(tok0, min(NTOK, n_assign - tok0), std::integral_constant<int, G>{});
+            walk(tok0, min(NTOK, n_assign - tok0), std::integral_constant<int, G>{}, std::false_type{});
             wide_barrier();  // (every wave's requests have arrived: the next column may use the buffers)
         }
     } else if constexpr (G == 1) {
-        walk(col * NTOK, min(NTOK, n_assign - col * NTOK), std::integral_constant<int, 1>{});
+        walk(col * NTOK, min(NTOK, n_assign - col * NTOK), std::integral_constant<int, 1>{}, std::integral_constant<bool, ONCE>{});
     } else {
         // The columns' token groups differ by one at most: those of 13 groups in columns of up to four are 4, 3, 3, 3.  Where they do differ, every other
         // 32 workgroups of an XCD take the columns one further on: the two workgroups of a compute unit (it gets the 32nd after its first) are not both the
@@ -393,8 +399,8 @@ __global__ __launch_bounds__(64 * kB32Waves, FMT == CML_Q4_0 && G == 1 ? 5 - RT 
         const int turn = col + (a.more == 0 ? 0 : (row_block >> 3) * a.n_cols >> 5 & 1), c = turn == a.n_cols ? 0 : turn;
         const int first = 16 * (c * a.base + min(c, a.more)), here = a.base + (c < a.more ? 1 : 0);
         const int n_here = min(16 * here, n_assign - first);
-        if (here == G) walk(first, n_here, std::integral_constant<int, G>{});
-        else walk(first, n_here, std::integral_constant<int, G - 1>{});
+        if (here == G) walk(first, n_here, std::integral_constant<int, G>{}, std::false_type{});
+        else walk(first, n_here, std::integral_constant<int, G - 1>{}, std::false_type{});
     }
 }
 
@@ -408,34 +414,31 @@ static int launch_b32_wide_as(const B32WideArgs &ka, int slots, hipStream_t st) 
         raised.store(true, std::memory_order_release);
     }
     hipLaunchKernelGGL(kernel, dim3(wide_grid(ka.n_row_blocks, ka.n_cols), slots), dim3(64 * kB32Waves), L::kTotal, st, ka);
-    // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>[.ragged][.grouped]"
-    CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D) + (RAGGED ? ".ragged" : "") + (GROUPED ? ".grouped" : ""));
+    // "<format>.mfma.wide.g<token groups>r<row tiles of a wave>d<slabs ahead>[.ragged][.grouped][.once]"
+    CML_COUNT_LAUNCH(std::string(FMT == CML_Q8_0 ? "q8_0" : "q4_0") + ".mfma.wide.g" + std::to_string(G) + "r" + std::to_string(RT) + "d" + std::to_string(D) + (RAGGED ? ".ragged" : "") + (GROUPED ? ".grouped" : "") + (ONCE ? ".once" : ""));
     CML_HIP_TRY(hipGetLastError());
     return CML_OK;
 }
 
-// Large weights that one column reads go past the caches (wide_reads_once): those of expert groups, those of a plain call of up to 16 tokens (128256 x 3072 at 16
-// tokens in Q8_0 85.3 -> 79.0 us; a single wider column gains half of that and no kernel of its own).
+// Past the caches (wide_reads_once): weights of expert groups, weights of a plain call of up to 16 tokens (128256 x 3072 at 16 tokens in Q8_0 85.3 -> 79.0 us; a
+// single wider column gains half of that and no kernel of its own).  Not rows of no whole slabs: two of them share a line of the caches, which the hint has fetched
+// twice (plain / so, weights that no cache holds, 8 tokens: Q8_0 32000 x 4128 42.3 / 45.2, 100000 x 2912 82.5 / 86.4; Q4_0 128256 x 3104 68.5 / 77.9, 65536 x 4128 59.6 / 66.6;
+// 128 experts 2816 / 704 at 64 tokens, gate and up by the hint, down both ways: 131.0 / 136.4).
 template <int FMT, int G, int RT, int D, bool GROUPED = false>
 static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
-    const bool once = ka.once;
     constexpr int kRows = kB32Waves * 16 * RT;
     ka.n_row_blocks = (ka.rows + kRows - 1) / kRows;
     ka.n_cols = GROUPED ? 1 : (ka.n_tokens + 16 * G - 1) / (16 * G);
     const int groups = (ka.n_tokens + 15) / 16;
     ka.base = groups / ka.n_cols;
     ka.more = groups % ka.n_cols;
-    const bool ragged = ka.nb % 8 != 0;
-    if constexpr (G == 4 && RT == 2) {  // (no registers left for the ragged form)
-        return ragged ? fail(CML_ERR_UNSUPPORTED, "wide matrix-core kernel: no such shape") : launch_b32_wide_as<FMT, G, RT, D, false, false, false>(ka, slots, st);
-    } else if constexpr (GROUPED) {
-        if (once) return ragged ? launch_b32_wide_as<FMT, G, RT, D, true, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, true, true, false>(ka, slots, st);
-        return ragged ? launch_b32_wide_as<FMT, G, RT, D, true, false, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, true, false, false>(ka, slots, st);
-    } else {
-        if constexpr (G == 1)
-            if (once && ka.n_cols == 1) return ragged ? launch_b32_wide_as<FMT, G, RT, D, false, true, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, false, true, false>(ka, slots, st);
-        return ragged ? launch_b32_wide_as<FMT, G, RT, D, false, false, true>(ka, slots, st) : launch_b32_wide_as<FMT, G, RT, D, false, false, false>(ka, slots, st);
+    if (ka.nb % 8 != 0) {
+        if constexpr (G == 4 && RT == 2) return fail(CML_ERR_UNSUPPORTED, "wide matrix-core kernel: no such shape");  // (no registers left for the ragged form)
+        else return launch_b32_wide_as<FMT, G, RT, D, GROUPED, false, true>(ka, slots, st);
     }
+    if constexpr (GROUPED || G == 1)
+        if (ka.once && ka.n_cols == 1) return launch_b32_wide_as<FMT, G, RT, D, GROUPED, true, false>(ka, slots, st);
+    return launch_b32_wide_as<FMT, G, RT, D, GROUPED, false, false>(ka, slots, st);
 }
 
 struct B32WideShape {
@@ -531,7 +534,7 @@ int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
     ka.rows = static_cast<int>(a.group_offsets ? a.band_rows : w->rows);
     ka.n_slabs = static_cast<int>((w->nb + 7) / 8);
     ka.nb = static_cast<int>(w->nb);
-    ka.once = wide_reads_once(w);
+    ka.once = wide_reads_once(w, a.group_offsets != nullptr);
     ka.q = a.q;
     ka.xs = a.scales;
     ka.out = a.out;

@@ -242,6 +242,97 @@ def test_wide_b32_expert_groups_are_bitwise_the_gemv(name, fmt, tag, E, k, hidde
             assert G.same_bits(run(), ref)
 
 
+# Kernels that request the weight past the caches, on weights that small calls can afford: plain calls of one column, never of two, never on rows of no whole slabs
+@pytest.mark.parametrize("rows,cols", [(70, 1280), (300, 512), (70, 1312)])
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_weights_requested_past_the_caches(name, fmt, tag, rows, cols):
+    w = Weight.upload(fmt, rows, cols, G.synth_weight(fmt, rows, cols, seed=rows))
+    for n in (3, 16, 17):
+        s, q = oracle.quantize_activation(fmt, np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32))
+        with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+            ref = G.gpu_gemm(w, s, q)
+        for g, tiles, ahead in ((1, 1, 1), (1, 2, 1), (1, 1, 2), (2, 1, 1)):
+            form = ".ragged" if cols % 256 else ".once" if g == 1 and n <= 16 else ""
+            G.say(f"past the caches {name} {rows}x{cols} n={n} groups={g} tiles={tiles} ahead={ahead}")
+            with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_ONCE=1, CAMELID_HIP_WIDE_GROUPS=g, CAMELID_HIP_WIDE_TILES=tiles, CAMELID_HIP_WIDE_AHEAD=ahead,
+                       CAMELID_HIP_B32_MFMA_MIN_TOKENS=1), G.engaged(rf"^{tag}\.mfma\.wide\.g{g}r{tiles}d{ahead}{form}$", none=(r"\.dot\.",)):
+                assert G.same_bits(G.gpu_gemm(w, s, q), ref)
+
+
+# groups of none, of one column and of several in one launch
+@pytest.mark.parametrize("hidden,ff,ragged", [(768, 512, False), (512, 352, True)])
+@pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
+def test_wide_b32_expert_groups_requested_past_the_caches(name, fmt, tag, hidden, ff, ragged):
+    E, k, T = 6, 2, 70
+    gate_up = Weight.upload(fmt, E * 2 * ff, hidden, G.synth_weight(fmt, E * 2 * ff, hidden, seed=E))
+    down = Weight.upload(fmt, E * hidden, ff, G.synth_weight(fmt, E * hidden, ff, seed=E + 1))
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    logits[:, 0] += 2.0
+    logits[:, E - 2] -= 1.5
+    logits[:, E - 1] -= 50.0
+    idx, weight, chosen, _ = gpu_route(logits, k)
+    held = np.bincount(chosen.reshape(-1), minlength=E)
+    assert held.min() == 0 and (held[held > 0].min() <= 16) and held.max() > 32
+    run = lambda: gpu_moe(gate_up, None, down, E, k, idx, weight, x, glu=1)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        ref = run()
+    for g in (1, 2):
+        G.say(f"past the caches {name} experts {hidden}/{ff} groups={g}")
+        down_form = r"\.ragged\.grouped$" if ragged else r"\.grouped\.once$"
+        with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_ONCE=1, CAMELID_HIP_WIDE_GROUPS=g), \
+                G.engaged(rf"^{tag}\.mfma\.wide\.g{g}r1d1\.grouped\.once$", rf"^{tag}\.mfma\.wide\.g{g}r1d1{down_form}", none=(r"\.dot\.", r"ragged.*once")):
+            assert G.same_bits(run(), ref)
+
+
+@pytest.mark.parametrize("hidden,ff", [(1024, 4096), (512, 768)])  # down with a K cut, without
+def test_wide_k_quant_expert_groups_requested_past_the_caches(hidden, ff):
+    E, k, T = 4, 2, 100
+    w = experts(E, hidden, ff, 9)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    logits = rng.standard_normal((T, E)).astype(np.float32)
+    logits[:, 0] += 1.0
+    logits[:, E - 1] -= 50.0
+    idx, weight, _, _ = gpu_route(logits, k)
+    run = lambda: gpu_moe(*w, E, k, idx, weight, x)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        ref = run()
+    for g, shape in ((2, "g2w4"), (3, "g3w4"), (4, "g4w4"), (8, "g8w8")):
+        G.say(f"past the caches Q4_K experts {hidden}/{ff} groups={g}")
+        down = r"\.serial_split" if ff == 4096 else ""
+        with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_ONCE=1, CAMELID_HIP_WIDE_GROUPS=g), \
+                G.engaged(rf"^q4k\.mfma\.wide\.{shape}.*\.grouped\.once$", rf"^q4k\.mfma\.wide\.{shape}{down}\.grouped\.once$", none=(r"grouped$",)):
+            assert G.same_bits(run(), ref)
+
+
+# 255.9 and 256.1 MB; the two tensors of a layer, 102 and 51 MB
+def test_which_weights_are_requested_past_the_caches():
+    cols, n = 4096, 16
+    some = G.synth_weight(B.CML_Q4_0, 128, cols, seed=1).reshape(128, -1)
+    s, q = oracle.quantize_activation(B.CML_Q4_0, np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32))
+    want = G.gpu_gemm(Weight.upload(B.CML_Q4_0, 128, cols, some), s, q)
+    for rows, past in ((116480, False), (116544, True)):
+        w = Weight.upload(B.CML_Q4_0, rows, cols, np.tile(some, ((rows + 127) // 128, 1))[:rows])
+        G.say(f"past the caches, {rows} rows")
+        with G.engaged(r"^q4_0\.mfma\.wide\.g1r\dd\d" + (r"\.once$" if past else "$")):
+            got = G.gpu_gemm(w, s, q)
+        assert G.same_bits(got, np.tile(want, (1, rows // 128 + 1))[:, :rows])  # (the weight repeats its first 128 rows)
+    E, k, T, hidden, ff = 4, 2, 8, 2048, 5888
+    row = G.synth_weight(B.CML_Q8_0, 256, hidden, seed=2).reshape(256, -1)
+    gate_up = Weight.upload(B.CML_Q8_0, E * 2 * ff, hidden, np.tile(row, (E * 2 * ff // 256, 1)))
+    down = Weight.upload(B.CML_Q8_0, E * hidden, ff, np.tile(G.synth_weight(B.CML_Q8_0, 256, ff, seed=3).reshape(256, -1), (E * hidden // 256, 1)))
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, hidden)).astype(np.float32)
+    idx, weight, _, _ = gpu_route(rng.standard_normal((T, E)).astype(np.float32), k)
+    G.say("past the caches, the tensors of a layer")
+    with G.engaged(r"^q8_0\.mfma\.wide\.g1r1d1\.grouped\.once$", r"^q8_0\.mfma\.wide\.g1r1d1\.grouped$"):
+        got = gpu_moe(gate_up, None, down, E, k, idx, weight, x, glu=1)
+    with G.env(CAMELID_HIP_MFMA_WIDE=0), G.engaged(none=(r"\.wide\.",)):
+        assert G.same_bits(got, gpu_moe(gate_up, None, down, E, k, idx, weight, x, glu=1))
+
+
 @pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
 def test_scales_that_cannot_be_read_16_bytes_at_a_time_stay_off_the_wide_kernel(name, fmt, tag):
     rows, cols, n = 70, 768, 40
