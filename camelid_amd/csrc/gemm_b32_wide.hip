@@ -445,22 +445,30 @@ struct B32WideShape {
     int g = 0, rt = 0, d = 0;
 };
 
-// Estimated us of a launch (less a constant), fitted on MI355X to 900 pairs of weight and tokens in every shape on cold weights (more than the last-level cache
-// holds between two launches on one): both formats, 512 to 128256 rows, 512 to 14336 values, 6 to 400 tokens.  A slab costs a fixed latency and, for every wave
-// on a SIMD and row tile, 0.23 us (0.16 where Q4_0 is unpacked at its one use) and 0.1 us per token group (a wave alone on its SIMD stalls where others overlap: 1.5, not 1,
-// times that).  A second slab ahead shortens the latency of workgroups that have a compute unit of their own (8 tokens, one slab ahead / two: 4096 x 4096 Q8_0
-// 17.8 / 13.5 us; 14336 x 5120 27.4 / 19.2) and, from about eight slabs, pays for its longer start on tall weights too (65536 x 4096 Q8_0 at 6 tokens 67.7 / 55.5).
-// Workgroups fill an XCD's 32 compute units row block by row block (wide_block); `resident` of them by registers.  The shape with the lowest estimate is on
-// average 0.8 % slower than the fastest, 22 % at worst (the estimate without residence and start: 0.9 % in Q8_0, 2.4 % in Q4_0).
-static float b32_wide_cost(bool late, int rows, int groups, int n_slabs, const B32WideShape &s) {
+// Workgroups that a compute unit holds by registers.
+static int b32_wide_resident(int fmt, bool ragged, const B32WideShape &s) {
+    if (s.rt == 2) return fmt == CML_Q4_0 && s.g == 1 && !ragged ? 3 : 2;
+    if (s.g == 1) return fmt == CML_Q4_0 && !ragged ? 4 : 3;
+    return s.g == 2 || (s.g == 3 && !ragged) ? 3 : 2;
+}
+
+// Estimated us of a launch (less a constant), fitted on MI355X to 1800 pairs of weight and tokens in every shape on cold weights (more than the last-level cache
+// holds between two launches on one): both formats, rows of whole slabs (102 weights) and of no whole ones (40), 512 to 152064 rows, 512 to 14336 values, 5 to 400 tokens.
+// A slab costs a fixed latency and, for every wave on a SIMD and row tile, 0.19 us (Q4_0 0.16, 0.14 where it is unpacked at its one use) and 0.18 (0.16) per token group; a wave
+// alone on its SIMD stalls where others overlap (1.9, not 1, times that).  A second slab ahead shortens the latency of workgroups that have a compute unit of their own (8 tokens,
+// one slab ahead / two: 4096 x 4096 Q8_0 17.8 / 13.5 us; 14336 x 5120 27.4 / 19.2) for a longer start.  Workgroups fill an XCD's 32 compute units row block by row block
+// (wide_block), and the compute unit that holds the most of them is the last.  The shape with the lowest estimate is on average 0.7 % (no whole slabs Q8_0 0.9, Q4_0 0.5 %) slower than
+// the fastest, 17 % at worst (30 % on one weight of no whole slabs, 1.5 of 5 us).
+static float b32_wide_cost(int fmt, bool ragged, int rows, int groups, int n_slabs, const B32WideShape &s) {
     const int64_t blocks = (rows + s.rt * 64 - 1) / (s.rt * 64), per_xcd = (blocks + 7) / 8 * ((groups + s.g - 1) / s.g);
-    const int resident = s.rt == 1 ? (late ? 4 : s.g <= 3 ? 3 : 2) : late ? 3 : 2;
+    const int resident = b32_wide_resident(fmt, ragged, s);
     const float per_cu = per_xcd / 32.0f, full = per_cu / resident;
     const bool shared = per_cu > 1.0f;
-    const float rounds = full <= 1.0f ? 1.0f : 0.28f * full + 0.72f * std::ceil(full);
-    const float base = shared ? (s.d == 1 ? 0.27f : 0.253f) : s.d == 1 ? 0.35f : 0.22f;
-    const float waves = shared ? std::max(1.9f, std::min<float>(resident, per_cu)) : 1.52f;
-    return rounds * (n_slabs * (base + waves * s.rt * ((late ? 0.164f : 0.229f) + 0.095f * s.g)) + (s.d == 2 ? 0.47f : 0.0f));
+    const float rounds = full <= 1.0f ? 1.0f : 0.35f * full + 0.65f * std::ceil(full);
+    const float base = shared ? 0.32f : s.d == 1 ? 0.56f : 0.26f;
+    const float waves = shared ? std::min<float>(resident, std::ceil(per_cu)) : 1.9f;
+    const float weight = fmt == CML_Q8_0 ? 0.19f : s.g == 1 ? 0.14f : 0.16f, cells = fmt == CML_Q8_0 ? 0.18f : 0.16f;
+    return rounds * (n_slabs * (base + waves * s.rt * (weight + cells * s.g)) + (s.d == 2 ? 0.5f : 0.0f));
 }
 
 template <int FMT, int G, int RT, int D>
@@ -472,7 +480,7 @@ static int b32_wide_visit(const B32WideArgs &ka, B32WideShape &best, float &cost
     const int groups = (ka.n_tokens + 15) / 16;
     if (G == 4 && RT == 2 && ka.nb % 8 != 0) return -1;
     if (G > 1 && (groups + G - 1) / G == (groups + G - 2) / std::max(1, G - 1)) return -1;  // (as few columns have room with a group less)
-    const float c = b32_wide_cost(FMT == CML_Q4_0 && G == 1, ka.rows, groups, ka.n_slabs, s);
+    const float c = b32_wide_cost(FMT, ka.nb % 8 != 0, ka.rows, groups, ka.n_slabs, s);
     if (c < cost) {
         cost = c;
         best = s;

@@ -366,6 +366,10 @@ ROUTES = [
     ("Q8_0", 8320, 5120, 8, r"^q8_0\.mfma\.wide\.g1r1d2$"),  # two slabs ahead where a workgroup has a compute unit
     ("Q4_0", 8320, 4096, 16, r"^q4_0\.mfma\.wide\.g1r1d2$"),  # the same
     ("Q4_0", 33000, 1024, 16, r"^q4_0\.mfma\.wide\.g1r1d1$"),  # two share one
+    ("Q8_0", 10000, 768, 8, r"^q8_0\.mfma\.wide\.g1r1d2$"),  # two slabs ahead on rows of three, too
+    ("Q8_0", 8832, 1280, 128, r"^q8_0\.mfma\.wide\.g3r1d1$"),  # three workgroups of three token groups on some compute units (14 of 12.3 us for four of two)
+    ("Q8_0", 39536, 768, 64, r"^q8_0\.mfma\.wide\.g2r1d1$"),  # two row tiles per wave double the slowest compute unit's work
+    ("Q4_0", 21888, 1280, 128, r"^q4_0\.mfma\.wide\.g2r1d1$"),  # the same
     ("Q4_0", 8320, 1024, 16, r"^q4_0\.mfma\.kpar\."),  # up to 768 tiles of short rows
     ("Q4_0", 8320, 2048, 16, r"^q4_0\.mfma\.wide\."),  # longer rows
     ("Q8_0", 8320, 1024, 16, r"^q8_0\.mfma\.wide\."),  # Q8_0: up to 512
