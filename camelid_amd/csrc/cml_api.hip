@@ -750,10 +750,9 @@ static int dispatch(const MatArgs &a, hipStream_t st) {
             break;
         case CML_Q8_0:
         case CML_Q4_0:
-            // the same split for the 32-value-block formats (rows of whole 256-value slabs, and longer ones of no whole slabs, whose line holds as it is)
+            // the same split for the 32-value-block formats (rows of whole 256-value slabs, and longer ones of no whole slabs)
             if (!a.group_offsets && !a.ints && !a.residual &&
-                (b32_wide_ragged(a.w) ? a.n_tokens >= b32_mfma_min_tokens(a.w)
-                                      : mfma_pays(a.n_tokens, b32_mfma_min_tokens(a.w), "CAMELID_HIP_B32_MFMA_MIN_TOKENS") && b32_mfma_usable(a.w)))
+                (b32_wide_ragged_pays(a.w, a.n_tokens) || (mfma_pays(a.n_tokens, b32_mfma_min_tokens(a.w), "CAMELID_HIP_B32_MFMA_MIN_TOKENS") && b32_mfma_usable(a.w))))
                 rc = launch_gemm_b32_mfma(a, st);
             else
                 rc = a.w->fmt == CML_Q8_0 ? launch_gemv_q8_0(a, st) : launch_gemv_q4_0(a, st);

@@ -189,6 +189,7 @@ bool gemm_b32_wide_serves_groups(const MatArgs &a);
 int launch_gemm_b32_mfma(const MatArgs &a, hipStream_t st);  // Q8_0 / Q4_0 on the matrix cores; plain or grouped
 bool b32_mfma_usable(const cml_weight *w);                   // rows of whole 256-value slabs
 bool b32_wide_ragged(const cml_weight *w);                   // longer rows of no whole slabs, which the wide kernel alone takes
+bool b32_wide_ragged_pays(const cml_weight *w, int64_t n);   // batches on them that it takes
 int b32_mfma_min_tokens(const cml_weight *w);                // batch size from which it pays
 int launch_gemm_q8_0(const MatArgs &a, hipStream_t st);
 int launch_gemm_q4_0(const MatArgs &a, hipStream_t st);

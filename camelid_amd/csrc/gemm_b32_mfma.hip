@@ -689,14 +689,6 @@ int b32_mfma_min_tokens(const cml_weight *w) {
     const int forced = env_int("CAMELID_HIP_B32_MFMA_MIN_TOKENS", 0);
     if (forced > 0) return forced;
     const int64_t tiles = (w->rows + 15) / 16, slabs = w->nb / 8;
-    // Rows of no whole slabs (packed dot / wide): 4096 x 2912 at 6 / 8 tokens Q8_0 12.0, 10.7 / 12.2, 12.1, at 16 31.5 / 16.1 (x 4160); x 1056 at 5 8.7 / 6.6; 8192 x 5216 at
-    // 4 / 5 Q8_0 14.7, 24.5 / 19.3, 19.2, Q4_0 at 5 / 6 21.0, 22.4 / 19.8, 20.1 (x 11040 34.3, 37.7 / 37.4, 37.4); 14336 x 2912 at 3 / 4 Q8_0 20.3, 13.8 / 13.3, 13.4, Q4_0 at 4 / 5
-    // 11.9, 18.3 / 13.1, 13.1; 32000 x 2912 at 3 / 4 Q4_0 25.5, 20.1 / 18.2, 18.2.
-    if (b32_wide_ragged(w)) {
-        if (tiles <= 256) return slabs <= 4 ? 5 : 9;
-        if (tiles < 768) return w->fmt == CML_Q8_0 ? 5 : 6;
-        return w->fmt == CML_Q8_0 || tiles >= 2000 ? 3 : 5;
-    }
     if ((slabs == 3 && tiles <= (w->fmt == CML_Q8_0 ? 512 : 256)) || (w->fmt == CML_Q4_0 && tiles <= 256 && slabs > 16 && slabs <= 24)) return 9;
     return tiles >= 2048 ? 4 : 5;
 }
@@ -706,7 +698,7 @@ int launch_gemm_b32_mfma(const MatArgs &a, hipStream_t st) {
     const cml_weight *w = a.w;
     const bool grouped = a.group_offsets != nullptr;
     if (w->rows == 0 || a.n_tokens == 0) return CML_OK;
-    if (!grouped && b32_wide_ragged(w) && env_int("CAMELID_HIP_MFMA_WIDE", 1)) return launch_gemm_b32_wide(a, st);
+    if (!grouped && b32_wide_ragged(w)) return launch_gemm_b32_wide(a, st);
     if (!b32_mfma_usable(w)) return fail(CML_ERR_UNSUPPORTED, "matrix-core path needs rows of whole 256-value slabs");
     B32MfmaArgs ka{};
     ka.quants = w->planes.p[0];

@@ -387,6 +387,15 @@ ROUTES = [
     ("Q4_0", 8192, 2912, 5, r"^q4_0\.dot\."),
     ("Q4_0", 8192, 2912, 6, r"^q4_0\.mfma\.wide\..*ragged$"),
     ("Q8_0", 14336, 1056, 3, r"^q8_0\.mfma\.wide\..*ragged$"),  # more than 767 tiles
+    ("Q4_0", 12288, 1312, 3, r"^q4_0\.mfma\.wide\..*ragged$"),
+    ("Q8_0", 14336, 1056, 4, r"^q8_0\.dot\."),  # four tokens are one pass of the packed dot
+    ("Q4_0", 31900, 800, 4, r"^q4_0\.dot\."),
+    ("Q4_0", 32000, 800, 4, r"^q4_0\.mfma\.wide\..*ragged$"),  # more than 1999 tiles
+    ("Q8_0", 1024, 928, 5, r"^q8_0\.dot\."),  # rows of 24 to 31 blocks
+    ("Q8_0", 1024, 928, 6, r"^q8_0\.mfma\.wide\..*ragged$"),
+    ("Q4_0", 2048, 1056, 8, r"^q4_0\.dot\."),  # eight on small weights, too
+    ("Q4_0", 8192, 832, 8, r"^q4_0\.dot\."),
+    ("Q4_0", 8208, 832, 8, r"^q4_0\.mfma\.wide\..*ragged$"),  # more than 512 tiles
 ]
 
 
