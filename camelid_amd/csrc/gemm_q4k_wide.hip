@@ -71,45 +71,38 @@ struct Q4KWide {
     // values 128 q + 64 (kq / 2) + 32 plane + 16 (kq % 2) .. + 15, piece 8 q + 4 (kq / 2) + 2 plane + kq % 2 of a token
     static __device__ __forceinline__ int lane_piece(int kq) { return 4 * (kq >> 1) + (kq & 1); }
     static __device__ constexpr int step_piece(int c) { return 8 * (c >> 1) + 2 * (c & 1); }
-    // A super-block is unpacked in five parts: scales, then the operand words of one step each.
-    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-    static constexpr int kParts = 5;
-    struct Part {
-        us2 lo[2], hi[2];  // digits of the scales of chunk 2 q + kq / 2: sub-block 2 * chunk, 2 * chunk + 1
-    };
-    __device__ __forceinline__ void unpack(const Raw &r, Operands &o, Part &d, int p) const {
-        if (p == 0) {
-            const uint32_t word = (kq & 1) ? (r.hdr.x ^ 0x80000000u) >> 16 : r.hdr.x;
-            o.scale = f16_bits_to_f32(word & 0xffffu);
-            o.d = f16_bits_to_f32(r.hdr.x & 0xffffu);
-            o.dmin = f16_bits_to_f32(r.hdr.x >> 16);
-            // runs 4 kq .. + 3 of the activation: the mins of sub-blocks 2 kq and 2 kq + 1, twice each (exact in f16)
-            const int odd = 16 * (kq & 1);
-            const uint32_t m03 = r.hdr.z >> odd, m47 = ((r.hdr.w >> (odd + 4)) & 0x0f0fu) | ((m03 >> 2) & 0x3030u);
-            const uint32_t mw = (kq & 2) ? m47 : m03 & 0x3f3fu;
-            const us2 m2 = __builtin_bit_cast(us2, __builtin_amdgcn_perm(mw, mw, 0x0c010c00u));
-            const _Float16 ma = static_cast<_Float16>(m2.x), mb = static_cast<_Float16>(m2.y);
-            o.mins = v4h_w{ma, ma, mb, mb};
-            const int up = 16 * (kq >> 1);
-            const uint32_t s03 = r.hdr.y >> up, s47 = ((r.hdr.w >> up) & 0x0f0fu) | ((s03 >> 2) & 0x3030u);
+    __device__ __forceinline__ void unpack(const Raw &r, Operands &o) const {
+        typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+        const uint32_t word = (kq & 1) ? (r.hdr.x ^ 0x80000000u) >> 16 : r.hdr.x;
+        o.scale = f16_bits_to_f32(word & 0xffffu);
+        o.d = f16_bits_to_f32(r.hdr.x & 0xffffu);
+        o.dmin = f16_bits_to_f32(r.hdr.x >> 16);
+        // runs 4 kq .. + 3 of the activation: the mins of sub-blocks 2 kq and 2 kq + 1, twice each (exact in f16)
+        const int odd = 16 * (kq & 1);
+        const uint32_t m03 = r.hdr.z >> odd, m47 = ((r.hdr.w >> (odd + 4)) & 0x0f0fu) | ((m03 >> 2) & 0x3030u);
+        const uint32_t mw = (kq & 2) ? m47 : m03 & 0x3f3fu;
+        const us2 m2 = __builtin_bit_cast(us2, __builtin_amdgcn_perm(mw, mw, 0x0c010c00u));
+        const _Float16 ma = static_cast<_Float16>(m2.x), mb = static_cast<_Float16>(m2.y);
+        o.mins = v4h_w{ma, ma, mb, mb};
+        // scales of chunk 2 q + kq / 2: sub-block 2 * chunk, 2 * chunk + 1
+        const int up = 16 * (kq >> 1);
+        const uint32_t s03 = r.hdr.y >> up, s47 = ((r.hdr.w >> up) & 0x0f0fu) | ((s03 >> 2) & 0x3030u);
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
-                const uint32_t sc = __builtin_amdgcn_perm(q ? s47 : s03, q ? s47 : s03, 0x0c010c00u);
-                d.lo[q] = __builtin_bit_cast(us2, sc & 0x00070007u);
-                d.hi[q] = __builtin_bit_cast(us2, (sc >> 3) & 0x00070007u);
+        for (int q = 0; q < 2; q++) {
+            const uint32_t sc = __builtin_amdgcn_perm(q ? s47 : s03, q ? s47 : s03, 0x0c010c00u);
+            const us2 lo = __builtin_bit_cast(us2, sc & 0x00070007u), hi = __builtin_bit_cast(us2, (sc >> 3) & 0x00070007u);
+            const uint32_t pc[4] = {r.piece[q].x, r.piece[q].y, r.piece[q].z, r.piece[q].w};
+#pragma unroll
+            for (int plane = 0; plane < 2; plane++) {  // low nibbles = sub-block 2 * chunk, high = 2 * chunk + 1
+                const us2 l2 = plane ? us2{lo.y, lo.y} : us2{lo.x, lo.x}, h2 = plane ? us2{hi.y, hi.y} : us2{hi.x, hi.x};
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    const us2 v = __builtin_bit_cast(us2, (pc[m] >> (4 * plane)) & 0x0f0f0f0fu);
+                    // (a byte pair times a digit, at most 15 * 7, never carries into its neighbour)
+                    o.lo[2 * q + plane][m] = __builtin_bit_cast(int, static_cast<us2>(v * l2));
+                    o.hi[2 * q + plane][m] = __builtin_bit_cast(int, static_cast<us2>(v * h2));
+                }
             }
-            return;
-        }
-        const int c = p - 1, q = c >> 1, plane = c & 1;  // low nibbles = sub-block 2 * chunk, high = 2 * chunk + 1
-        const us2 l2 = plane ? us2{d.lo[q].y, d.lo[q].y} : us2{d.lo[q].x, d.lo[q].x};
-        const us2 h2 = plane ? us2{d.hi[q].y, d.hi[q].y} : us2{d.hi[q].x, d.hi[q].x};
-        const uint32_t pc[4] = {r.piece[q].x, r.piece[q].y, r.piece[q].z, r.piece[q].w};
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const us2 v = __builtin_bit_cast(us2, (pc[m] >> (4 * plane)) & 0x0f0f0f0fu);
-            // (a byte pair times a digit, at most 15 * 7, never carries into its neighbour)
-            o.lo[c][m] = __builtin_bit_cast(int, static_cast<us2>(v * l2));
-            o.hi[c][m] = __builtin_bit_cast(int, static_cast<us2>(v * h2));
         }
     }
     struct Sums {

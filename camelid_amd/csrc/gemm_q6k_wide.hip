@@ -98,31 +98,35 @@ struct Q6KWide {
     // The product of a 6-bit value (code - 32) and its int8 scale needs 13 bits; as p = 256 hi + lo with lo a signed byte
     // both are int8 operands:  r = code * sc + (128 - 32 sc) = p + 128,  hi = r >> 8,  lo = (r & 255) ^ 0x80 as a signed byte.
     // One packed 16-bit multiply-add gives r for two values.
-    static constexpr int kParts = 4;
-    struct Part {};
-    __device__ __forceinline__ void unpack(const Raw &r, Operands &o, Part &, int c) const {
+    __device__ __forceinline__ void unpack(const Raw &r, Operands &o) const {
         typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-        const int h = c >> 1, plane = c & 1;
-        if (c == 0) o.scale = f16_bits_to_f32(r.d);
+        o.scale = f16_bits_to_f32(r.d);
         const int jj = 2 * (kq >> 1);
         const uint32_t scw[4] = {r.sc.x, r.sc.y, r.sc.z, r.sc.w};
-        const uint32_t l[4] = {r.ql[h].x, r.ql[h].y, r.ql[h].z, r.ql[h].w};
-        const uint32_t u[4] = {r.qh[h].x, r.qh[h].y, r.qh[h].z, r.qh[h].w};
-        const int s = static_cast<int>(scw[c] << (24 - 8 * kq)) >> 24;  // sub-block 8 h + 4 plane + kq
-        const uint32_t s2 = __builtin_amdgcn_perm(static_cast<uint32_t>(s), static_cast<uint32_t>(s), 0x01000100u);
-        const us2 s16 = __builtin_bit_cast(us2, s2);
-        const us2 o16 = s16 * us2{static_cast<unsigned short>(-32), static_cast<unsigned short>(-32)} + us2{128, 128};
 #pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const uint32_t up = (plane ? u[m] >> jj : u[m] << (4 - jj)) & 0x30303030u;
-            uint32_t code = ((plane ? l[m] >> 4 : l[m]) & 0x0f0f0f0fu) | up;
-            asm("" : "+v"(code));  // (the compiler otherwise rebuilds the code for either half of the bytes)
-            const us2 even = __builtin_bit_cast(us2, code & 0x00ff00ffu), odd = __builtin_bit_cast(us2, __builtin_amdgcn_perm(code, code, 0x0c030c01u));
-            const uint32_t re = __builtin_bit_cast(uint32_t, static_cast<us2>(even * s16 + o16));
-            const uint32_t ro = __builtin_bit_cast(uint32_t, static_cast<us2>(odd * s16 + o16));
-            // bytes of values 0..3: even low halves hold values 0 and 2, odd ones 1 and 3
-            o.lo[c][m] = static_cast<int>(__builtin_amdgcn_perm(ro, re, 0x06020400u) ^ 0x80808080u);
-            o.hi[c][m] = static_cast<int>(__builtin_amdgcn_perm(ro, re, 0x07030501u));
+        for (int h = 0; h < 2; h++) {
+            const uint32_t l[4] = {r.ql[h].x, r.ql[h].y, r.ql[h].z, r.ql[h].w};
+            const uint32_t u[4] = {r.qh[h].x, r.qh[h].y, r.qh[h].z, r.qh[h].w};
+#pragma unroll
+            for (int plane = 0; plane < 2; plane++) {
+                const int c = 2 * h + plane;
+                const int s = static_cast<int>(scw[c] << (24 - 8 * kq)) >> 24;  // sub-block 8 h + 4 plane + kq
+                const uint32_t s2 = __builtin_amdgcn_perm(static_cast<uint32_t>(s), static_cast<uint32_t>(s), 0x01000100u);
+                const us2 s16 = __builtin_bit_cast(us2, s2);
+                const us2 o16 = s16 * us2{static_cast<unsigned short>(-32), static_cast<unsigned short>(-32)} + us2{128, 128};
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    const uint32_t up = (plane ? u[m] >> jj : u[m] << (4 - jj)) & 0x30303030u;
+                    uint32_t code = ((plane ? l[m] >> 4 : l[m]) & 0x0f0f0f0fu) | up;
+                    asm("" : "+v"(code));  // (the compiler otherwise rebuilds the code for either half of the bytes)
+                    const us2 even = __builtin_bit_cast(us2, code & 0x00ff00ffu), odd = __builtin_bit_cast(us2, __builtin_amdgcn_perm(code, code, 0x0c030c01u));
+                    const uint32_t re = __builtin_bit_cast(uint32_t, static_cast<us2>(even * s16 + o16));
+                    const uint32_t ro = __builtin_bit_cast(uint32_t, static_cast<us2>(odd * s16 + o16));
+                    // bytes of values 0..3: even low halves hold values 0 and 2, odd ones 1 and 3
+                    o.lo[c][m] = static_cast<int>(__builtin_amdgcn_perm(ro, re, 0x06020400u) ^ 0x80808080u);
+                    o.hi[c][m] = static_cast<int>(__builtin_amdgcn_perm(ro, re, 0x07030501u));
+                }
+            }
         }
     }
     struct Sums {

@@ -249,7 +249,6 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
         fetch_w(0, 0);
         if constexpr (WS == 2) fetch_w(1, 1);
         typename F::Raw raw;
-        typename F::Operands ops;
         wide_wait<(WS - 1) * F::kFetches>();
         fmt.read(raw, w_mine, s_begin);
         finish(0);
@@ -284,11 +283,8 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
             fetch_yd(loc + 1, buf ^ 1);
             fetch(loc + 1, buf ^ 1);
             __builtin_amdgcn_sched_barrier(0);
-            {
-                typename F::Part part_of;
-#pragma unroll
-                for (int p = 0; p < F::kParts; p++) fmt.unpack(raw, ops, part_of, p);
-            }
+            typename F::Operands ops;
+            fmt.unpack(raw, ops);
             __builtin_amdgcn_sched_barrier(0);
             fetch_w(loc + WS, WS == 2 ? buf : 0);  // (its slot was read into registers a step ago)
             __builtin_amdgcn_sched_barrier(0);
@@ -302,7 +298,7 @@ __global__ __launch_bounds__(64 * WAVES, GROUPED && WAVES == 4 && G <= 3 ? 3 : 2
                 v4h_w rs[2];
                 float4 yd4[kProducts ? 1 : 3];
                 float ya[kProducts ? 2 : 1];
-                v16f_w scale[kProducts ? 2 : 1];  // products of the scales of two or four token groups and of the weight's, all cells of a tile
+                v16f_w scale[kProducts ? 2 : 1];  // products of the scales of two token groups and of the weight's, all cells of a tile
                 typename F::Sums sums[2];
                 auto read = [&](int g) __attribute__((always_inline)) {
 #pragma unroll
@@ -436,8 +432,9 @@ struct WideShape {
 
 // Estimated us of a launch (less a constant), fitted on MI355X to every shape of the kernel on cold weights (more than the last-level cache holds between
 // two launches on one) of 256 to 65536 rows and 512 to 14336 values with the three K cuts: Q6_K 1669 pairs of weight and tokens (5 to 512), Q4_K 1397 (33 to
-// 512).  The shape with the lowest estimate is on average 0.8 % / 0.7 % slower than the fastest (an earlier fit to few weights, some of them cached, took Q4_K
-// 4.3 % off).  A step costs a fixed latency, more for two wave groups; for every wave on a SIMD the unpacking of a super-block and the cells of its token groups;
+// 512).  The shape with the lowest estimate was on average 0.8 % / 0.7 % slower than the fastest (an earlier fit to few weights, some of them cached, took Q4_K
+// 4.3 % off).  Q4_K has since become 1 to 4 % faster in the cells and the unpacking; with the constants as they are 121 pairs of other Q4_K weights are 1.2 % off (36 % at worst: 33970 x 4864
+// at 33 tokens 50 us, four waves on three token groups 37), 107 of Q6_K, which the change left alone, 3.7 % (28904 x 5632 at 33 49.5, 39.7).  A step costs a fixed latency, more for two wave groups; for every wave on a SIMD the unpacking of a super-block and the cells of its token groups;
 // and per token group the activation slabs that the compute unit's workgroups fetch (from three on they share what the cache holds).  Workgroups fill an XCD's 32
 // compute units row block by row block (wide_block).  `rounds`: workgroups over what is resident at once, between their average and the last round at full length.
 template <class F>
