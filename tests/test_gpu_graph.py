@@ -159,3 +159,27 @@ def test_producers_and_lm_head_neighbours_replay(stream):
     want = oracle.rms_norm(xs[2], gamma.to_numpy(np.float32, (cols,)), 1e-5)
     assert G.same_bits(normed.to_numpy(np.float32, (n, cols)), want)
     assert list(am.to_numpy(np.uint32, (n,))) == [int(np.argmax(want[i])) for i in range(n)]
+
+
+@pytest.mark.parametrize("rows,n", [(1, 40001), (4, 65539)])
+def test_argmax_of_long_rows_replays(stream, rows, n):
+    """Long rows keep their running answer in the index: a replay starts from what the one before left, a valid index of a value that wins no longer."""
+    rng = np.random.default_rng(n)
+    cases = [rng.standard_normal((rows, n)).astype(np.float32) for _ in range(3)]
+    for i, c in enumerate(cases):
+        c[:, 1000 + 9000 * i] = 20.0
+    ld, od = DeviceBuffer(rows * n * 4), DeviceBuffer(rows * 4)
+    OUT_SCRUB[0] = DeviceBuffer(16)  # (the index itself is not scrubbed)
+    G.say(f"graph argmax {rows} rows of {n}")
+    replay_and_compare(stream, lambda st: check(lib().cml_argmax_f32(ld.ptr, rows, n, od.ptr, st), "cml_argmax_f32"), cases,
+                       lambda c: (h2d(ld, c), check(lib().cml_stream_sync(None))), lambda: od.to_numpy(np.uint32, (rows,)).astype(np.float32))
+    graph = capture(stream, lambda st: check(lib().cml_argmax_f32(ld.ptr, rows, n, od.ptr, st), "cml_argmax_f32"))
+    try:
+        for i in (1, 0, 2, 1, 0):  # replays alone, each on other logits
+            h2d(ld, cases[i])
+            check(lib().cml_stream_sync(None))
+            check(lib().cml_graph_launch(graph, stream), "cml_graph_launch")
+            check(lib().cml_stream_sync(stream))
+            assert list(od.to_numpy(np.uint32, (rows,))) == [1000 + 9000 * i] * rows
+    finally:
+        check(lib().cml_graph_destroy(graph))

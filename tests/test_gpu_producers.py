@@ -373,6 +373,22 @@ def test_argmax_of_long_rows_does_not_depend_on_what_the_index_held(n):
     assert list(two.to_numpy(np.uint32, (2,))) == want[4:6]
 
 
+# two to four rows in one launch, whole parts and not, rows that start off a 16-byte boundary; a vocabulary's row and a very long one
+@pytest.mark.parametrize("rows,n", [(2, 32768), (3, 49157), (4, 65536), (4, 65539), (1, 128256), (1, 1000003)])
+def test_argmax_of_several_long_rows(rows, n):
+    logits = np.random.default_rng(n).standard_normal((rows, n)).astype(np.float32)
+    for r in range(rows):
+        logits[r, [n - 1 - r, 7 * r + 1, 4096 * (r + 1)]] = 20.0 + r  # equal maxima in three parts
+    want = [int(np.argmax(r)) for r in logits]
+    ld = DeviceBuffer.from_numpy(logits)
+    for before in (0, n - 1, 0xFFFFFFFF):
+        od = DeviceBuffer.from_numpy(np.full(rows, before, np.uint32))
+        G.say(f"argmax {rows} rows of {n}, index held {before}")
+        check(lib().cml_argmax_f32(ld.ptr, rows, n, od.ptr, None), "cml_argmax_f32")
+        check(lib().cml_stream_sync(None))
+        assert list(od.to_numpy(np.uint32, (rows,))) == want, before
+
+
 @pytest.mark.parametrize("at", [0, 5000, 39999])
 def test_argmax_of_a_long_row_may_be_written_into_the_row(at):
     n = 40000

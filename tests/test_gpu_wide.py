@@ -52,6 +52,43 @@ def test_wide_cells_are_bitwise_the_gemv(name, fmt, tag, rows, cols):
         assert G.same_bits(got, oracle.matmul_q(fmt, wire, cols, s, q, order=order, threads=8))
 
 
+# d (and dmin) subnormal, zero of either sign, negative, infinite, no number; activation scales the same.  Cells are the narrow kernel's, and without a K cut the
+# oracle's, the ones that are no number among them (an infinite scale times a zero one, a difference of infinities).
+@pytest.mark.parametrize("rows,cols", [(70, 768), (145, 13 * 256)])  # without and with a K cut
+@pytest.mark.parametrize("name,fmt,tag", K_FORMATS)
+def test_wide_cells_of_extreme_scales(name, fmt, tag, rows, cols):
+    blocks = G.synth_weight(fmt, rows, cols, seed=rows).reshape(-1, 144 if fmt == B.CML_Q4_K else 210)
+    at = [0, 2] if fmt == B.CML_Q4_K else [208]
+    odd = np.array([0x0001, 0x83FF, 0x0000, 0x8000, 0x7C00, 0xFC00, 0x7E01, 0x7BFF, 0xFBFF], np.uint16).view(np.uint8).reshape(-1, 2)
+    rng = np.random.default_rng(rows)
+    for i, v in enumerate(odd):
+        for a in at:
+            hit = rng.choice(len(blocks), rows // 20 if 4 <= i <= 6 else len(blocks) // 12, replace=False)  # (most cells stay finite)
+            blocks[hit, a:a + 2] = v
+    w = Weight.upload(fmt, rows, cols, blocks.reshape(-1))
+    for n in (3, 17, 130):
+        s, q = activations(n, cols, seed=n)
+        s = s.reshape(n, -1).copy()
+        s[0], s[1] = 1e-39, -3e-42  # subnormal: products with d round among the subnormal numbers
+        s[2] = 2e-36                # products that become subnormal
+        if n > 16:
+            s[5, 0], s[6, -1], s[7, 0], s[8] = np.inf, -np.inf, np.nan, 3e38
+            s[9], s[16] = -0.0, 1e-38
+        with G.env(CAMELID_HIP_MFMA_WIDE=0, CAMELID_HIP_Q4K_MFMA_MIN_TOKENS=1, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), G.engaged(r"\.mfma\.", none=(r"\.wide\.",)):
+            ref = G.gpu_gemm(w, s, q)
+        assert np.isfinite(ref).mean() > 0.3 and not np.isfinite(ref).all() and (np.abs(ref[:3]) < 1e-37).any() and ref[:3].any()
+        if cols == 768:
+            order = oracle.ORDER_PRIMARY if fmt == B.CML_Q4_K else oracle.ORDER_ALT
+            assert np.array_equal(oracle.matmul_q(fmt, blocks.reshape(-1), cols, s, q, order=order, threads=8), ref, equal_nan=True)
+        for g, waves, parts in [(g, v, p) for g in (1, 2, 3, 8) for v in (4, 8) for p in (1, 2)]:
+            if n < 16 * (g - 1) and n != 3 or (name, g, waves, parts) == ("Q4_K", 8, 8, 2):
+                continue
+            G.say(f"wide {name} extreme scales {rows}x{cols} n={n} groups={g} waves={waves} parts={parts}")
+            with G.env(CAMELID_HIP_MFMA_WIDE=2, CAMELID_HIP_WIDE_GROUPS=g, CAMELID_HIP_WIDE_WAVES=waves, CAMELID_HIP_WIDE_PARTS=parts,
+                       CAMELID_HIP_Q4K_MFMA_MIN_TOKENS=1, CAMELID_HIP_Q6K_MFMA_MIN_TOKENS=1), G.engaged(rf"^{tag}\.mfma\.wide\.g{g}w{waves}", none=(r"\.dot\.",)):
+                assert np.array_equal(G.gpu_gemm(w, s, q), ref, equal_nan=True)
+
+
 @pytest.mark.parametrize("name,fmt,tag", K_FORMATS)
 def test_wide_on_a_row_band(name, fmt, tag):
     """A view that starts and ends inside a tile, of rows with an odd number of super-blocks (Q6_K: block scales at odd halves of a word)."""
@@ -203,7 +240,6 @@ def test_wide_b32_on_a_row_band(name, fmt, tag):
         assert G.same_bits(whole, G.gpu_gemm(w, s, q))
 
 
-# gate | up fused (gathered rows), down on rows of whole slabs; groups of none, one, past a column; a band that ends inside a workgroup
 # rows of no whole slabs (down, then both)
 @pytest.mark.parametrize("E,k,hidden,ff,T", [(6, 3, 512, 352, 20), (4, 2, 1088, 704, 35)])
 @pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
@@ -222,6 +258,7 @@ def test_wide_b32_expert_groups_on_rows_of_no_whole_slabs(name, fmt, tag, E, k, 
             assert G.same_bits(run(), ref)
 
 
+# gate | up fused (gathered rows), down on rows of whole slabs; groups of none, one, past a column; a band that ends inside a workgroup
 @pytest.mark.parametrize("E,k,hidden,ff,T", [(16, 4, 768, 512, 40), (8, 3, 256, 256, 1), (5, 2, 1280, 768, 33)])
 @pytest.mark.parametrize("name,fmt,tag", B32_FORMATS)
 def test_wide_b32_expert_groups_are_bitwise_the_gemv(name, fmt, tag, E, k, hidden, ff, T):
