@@ -560,7 +560,7 @@ int launch_gemm_b32_wide(const MatArgs &a, hipStream_t st) {
     ka.rows = static_cast<int>(a.group_offsets ? a.band_rows : w->rows);
     ka.n_slabs = static_cast<int>((w->nb + 7) / 8);
     ka.nb = static_cast<int>(w->nb);
-    ka.once = wide_reads_once(w, a.group_offsets != nullptr);
+    ka.once = wide_reads_once(w);
     ka.q = a.q;
     ka.xs = a.scales;
     ka.out = a.out;

@@ -73,17 +73,17 @@ __device__ __forceinline__ void wide_wait() {
 // Workgroup barrier after this wave's LDS operations (__syncthreads would also wait for every load in flight).
 __device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// Which weights are requested past the 256 MB last-level cache: those that it could not hold until they are used again.  A plain call's weight where it alone is larger: one
-// that fits is found there when the next call uses it again, and gains less when it is not (plain / so, back to back: Q8_0 32000 x 4096, 139 MB, at 8 tokens 26.4 / 32.0 us, Q4_0
-// 128256 x 3072, 222 MB, at 16 43.9 / 58.5; with 600 MB of other weights between 32.5 / 29.4, 57.3 / 56.5; Q8_0 128256 x 2048, 279 MB, at 16 57.4 / 54.7).  The tensors of an
-// expert layer from 96 MB each: a layer reads three of them (with 1 GB of other layers between, plain / so: Q4_K 8 x 4096 / 14336, 264 MB each, at 64 / 128 / 512 tokens
-// 229 / 216, 282 / 270, 679 / 668, 3072 / 8192, 113 MB, at 128 145 / 143; Q8_0 8 x 4096 / 4096, 143 MB, at 16 / 64 124 / 111, 115 / 107; one layer over and over, Q4_K
-// 1536 / 6144, 42 MB each, at 128 77 / 81).  That a K-quant group of more than a column reads its rows again costs nothing there (a column holds up to 128 assignments), with
-// columns of 16 and 32 it did: Q8_0 8 x 4096 / 4096 at 256 239 / 274, all assignments on few experts 267 / 315.
-inline bool wide_reads_once(const cml_weight *w, bool grouped) {
+// Which weights are requested past the 256 MB last-level cache: those of 96 MB and more.  A weight of that size is used once in a pass over a model, whose other weights have taken its
+// place when it is used again (plain / so, 600 MB of other weights between, us: Q8_0 32000 x 4096, 139 MB, at 8 tokens 32.5 / 29.4, 128256 x 2048, 279 MB, at 16 57.4 / 54.7; Q4_0
+// 128256 x 3072, 222 MB, at 16 57.3 / 55.8; expert layers, three tensors of the size each, 1 GB of other layers between: Q4_K 8 x 4096 / 14336, 264 MB, at 64 / 128 / 512 tokens
+// 229 / 216, 282 / 270, 679 / 668, 3072 / 8192, 113 MB, at 128 145 / 143; Q8_0 8 x 4096 / 4096, 143 MB, at 16 / 64 124 / 111, 115 / 107).  Where nothing is used in between, the cache holds
+// weights of up to 256 MB and the hint costs: the two plain ones above back to back 26.4 / 32.0 and 43.9 / 58.5.  Smaller weights stay: Q4_K 1536 / 6144, 42 MB, one layer over and over, at 128
+// 77 / 81.  That a K-quant group of more than a column reads its rows again costs nothing (a column holds up to 128 assignments); with columns of 16 and 32 it does: Q8_0
+// 8 x 4096 / 4096 at 256 239 / 274, all assignments on few experts 267 / 315.
+inline bool wide_reads_once(const cml_weight *w) {
     const int64_t block = w->fmt == CML_Q8_0 ? 34 : w->fmt == CML_Q4_0 ? 18 : w->fmt == CML_Q4_K ? 144 : 210;
     const int forced = env_int("CAMELID_HIP_WIDE_ONCE", -1);  // 0 = never, 1 = always
-    return forced >= 0 ? forced != 0 : w->rows * w->nb * block >= static_cast<int64_t>(grouped ? 96 : 256) << 20;
+    return forced >= 0 ? forced != 0 : w->rows * w->nb * block >= 96ll << 20;
 }
 
 // LDS byte address of a shared-memory pointer.
@@ -564,7 +564,7 @@ static int launch_wide_grouped(const MatArgs &a, hipStream_t st) {
     const float mean = static_cast<float>(a.n_assign_total) / std::max(1, slots);
     int g = static_cast<int>(std::ceil(std::min<float>(mean + std::sqrt(mean), static_cast<float>(ka.n_tokens)) / 16.0f));
     g = env_int("CAMELID_HIP_WIDE_GROUPS", g);
-    const bool once = wide_reads_once(w, true);
+    const bool once = wide_reads_once(w);
     if (g <= 2) return launch_wide_grouped_split<F, 2, 4>(ka, slots, once, st);
     if (g <= 3) return launch_wide_grouped_split<F, 3, 4>(ka, slots, once, st);
     if (g <= 4) return launch_wide_grouped_split<F, 4, 4>(ka, slots, once, st);

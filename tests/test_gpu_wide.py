@@ -344,13 +344,13 @@ def test_wide_k_quant_expert_groups_requested_past_the_caches(hidden, ff):
             assert G.same_bits(run(), ref)
 
 
-# 255.9 and 256.1 MB; the two tensors of a layer, 102 and 51 MB
+# a row tile below 96 MB and one above; the two tensors of a layer, 102 and 51 MB
 def test_which_weights_are_requested_past_the_caches():
     cols, n = 4096, 16
     some = G.synth_weight(B.CML_Q4_0, 128, cols, seed=1).reshape(128, -1)
     s, q = oracle.quantize_activation(B.CML_Q4_0, np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32))
     want = G.gpu_gemm(Weight.upload(B.CML_Q4_0, 128, cols, some), s, q)
-    for rows, past in ((116480, False), (116544, True)):
+    for rows, past in ((43680, False), (43696, True)):
         w = Weight.upload(B.CML_Q4_0, rows, cols, np.tile(some, ((rows + 127) // 128, 1))[:rows])
         G.say(f"past the caches, {rows} rows")
         with G.engaged(r"^q4_0\.mfma\.wide\.g1r\dd\d" + (r"\.once$" if past else "$")):
