@@ -4,18 +4,18 @@
 //     isum = sum_j w_j * x_j  (exact i32),   acc = acc + ((float)isum * d_w) * d_x
 // so one v_mfma_i32_16x16x32_i8 per block and 16 x 16 cells, and an f32 step per block and cell: the vector
 // instructions bound this kernel (three per 64 cells and block, the fused one four cycles and the others two with two waves to take turns: 14336 x 4096 x 200 tokens
-// 24 us of issue, 57 measured).  Three
+// 24 us of issue, 57 measured: in row blocks of 128 and columns of 4, 3, 3, 3 token groups a compute unit has up to 7 groups where 5.7 is the mean).  Three
 // are the least: multiply, multiply, add, each rounded.  The conversion is left out: the matrix instruction
 // adds onto 0x4b400000, so that its result READ AS f32 is 12582912 + isum (|isum| <= 2^19), and
 //     fma(that, d_w, -12582912 * d_w)
 // is isum * d_w rounded once, the product (d_w has 11 significant bits, 1.5 * 2^23 * d_w is exact).  A slab
 // that holds a scale which is no finite number takes the subtraction instead (inf - inf).
 //
-// A wave owns 32 weight rows (two 16-row tiles) and all tokens of its workgroup's column, so that an activation
-// operand and the activation scales read from LDS serve two tiles; with one, LDS would carry as many cycles as the vector unit.
+// A wave owns one or two 16-row tiles (RT) and all tokens of its workgroup's column.  With two, an activation operand and the activation scales read from
+// LDS serve both, with one a launch has more workgroups and a compute unit room for more of them: b32_wide_cost chooses.
 // K is walked in slabs of 256 values.  Everything a slab needs goes from memory to LDS without passing through
-// registers (gemm_wide.hpp): the activation of the workgroup's tokens and their scales (two buffers), the rows
-// of every wave (one buffer: a wave holds the slab it works on in registers).  LDS is written at consecutive
+// registers (gemm_wide.hpp): the activation of the workgroup's tokens and their scales (D + 1 buffers), the rows
+// of every wave (D buffers: a wave holds the slab it works on in registers).  LDS is written at consecutive
 // addresses, 16 bytes per lane; bank conflicts are avoided by what each lane fetches (exclusive-or of the piece with the row).
 // Lane L supplies A-row t = L % 16 and B-column n = L % 16 at the k-octet L / 16 of a block and
 // receives D[4 * (L / 16) + j][L % 16], j < 4.  Q4_0: octets 0, 1 are the low nibbles of the block's first and second
@@ -452,13 +452,13 @@ static int b32_wide_resident(int fmt, bool ragged, const B32WideShape &s) {
     return s.g == 2 || (s.g == 3 && !ragged) ? 3 : 2;
 }
 
-// Estimated us of a launch (less a constant), fitted on MI355X to 1800 pairs of weight and tokens in every shape on cold weights (more than the last-level cache
-// holds between two launches on one): both formats, rows of whole slabs (102 weights) and of no whole ones (40), 512 to 152064 rows, 512 to 14336 values, 5 to 400 tokens.
+// Estimated us of a launch (less a constant), fitted on MI355X to 2640 pairs of weight and tokens in every shape on cold weights (more than the last-level cache
+// holds between two launches on one): both formats, rows of whole slabs (152 weights) and of no whole ones (84), 512 to 152064 rows, 512 to 14336 values, 5 to 400 tokens.
 // A slab costs a fixed latency and, for every wave on a SIMD and row tile, 0.19 us (Q4_0 0.16, 0.14 where it is unpacked at its one use) and 0.18 (0.16) per token group; a wave
 // alone on its SIMD stalls where others overlap (1.9, not 1, times that).  A second slab ahead shortens the latency of workgroups that have a compute unit of their own (8 tokens,
-// one slab ahead / two: 4096 x 4096 Q8_0 17.8 / 13.5 us; 14336 x 5120 27.4 / 19.2) for a longer start.  Workgroups fill an XCD's 32 compute units row block by row block
-// (wide_block), and the compute unit that holds the most of them is the last.  The shape with the lowest estimate is on average 0.7 % (no whole slabs Q8_0 0.9, Q4_0 0.5 %) slower than
-// the fastest, 17 % at worst (30 % on one weight of no whole slabs, 1.5 of 5 us).
+// one slab ahead / two: 4096 x 4096 Q8_0 17.8 / 13.5 us; 14336 x 5120 27.4 / 19.2) for a longer start, on rows of no whole slabs nearly twice as long (736 x 704 at 200 tokens
+// 5.0 / 6.5).  Workgroups fill an XCD's 32 compute units row block by row block (wide_block), and the compute unit that holds the most of them is the last.  The shape with the
+// lowest estimate is on average 0.7 % slower than the fastest, 17 % at worst.
 static float b32_wide_cost(int fmt, bool ragged, int rows, int groups, int n_slabs, const B32WideShape &s) {
     const int64_t blocks = (rows + s.rt * 64 - 1) / (s.rt * 64), per_xcd = (blocks + 7) / 8 * ((groups + s.g - 1) / s.g);
     const int resident = b32_wide_resident(fmt, ragged, s);
@@ -468,7 +468,7 @@ static float b32_wide_cost(int fmt, bool ragged, int rows, int groups, int n_sla
     const float base = shared ? 0.32f : s.d == 1 ? 0.56f : 0.26f;
     const float waves = shared ? std::min<float>(resident, std::ceil(per_cu)) : 1.9f;
     const float weight = fmt == CML_Q8_0 ? 0.19f : s.g == 1 ? 0.14f : 0.16f, cells = fmt == CML_Q8_0 ? 0.18f : 0.16f;
-    return rounds * (n_slabs * (base + waves * s.rt * (weight + cells * s.g)) + (s.d == 2 ? 0.5f : 0.0f));
+    return rounds * (n_slabs * (base + waves * s.rt * (weight + cells * s.g)) + (s.d == 1 ? 0.0f : ragged ? 0.9f : 0.5f));
 }
 
 template <int FMT, int G, int RT, int D>

@@ -425,6 +425,8 @@ ROUTES = [
     ("Q4_0", 8192, 2912, 6, r"^q4_0\.mfma\.wide\..*ragged$"),
     ("Q8_0", 14336, 1056, 3, r"^q8_0\.mfma\.wide\..*ragged$"),  # more than 767 tiles
     ("Q4_0", 12288, 1312, 3, r"^q4_0\.mfma\.wide\..*ragged$"),
+    ("Q8_0", 736, 704, 200, r"^q8_0\.mfma\.wide\.g1r1d1\.ragged$"),  # rows of two slabs and a part are over before a second slab ahead pays
+    ("Q8_0", 736, 1056, 200, r"^q8_0\.mfma\.wide\.g1r1d2\.ragged$"),
     ("Q8_0", 14336, 1056, 4, r"^q8_0\.dot\."),  # four tokens are one pass of the packed dot
     ("Q4_0", 31900, 800, 4, r"^q4_0\.dot\."),
     ("Q4_0", 32000, 800, 4, r"^q4_0\.mfma\.wide\..*ragged$"),  # more than 1999 tiles
