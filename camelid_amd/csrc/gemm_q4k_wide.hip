@@ -5,10 +5,10 @@
 // operand (S = lo + 8 hi, two contractions over the whole super-block), the mins against the sums of the
 // activation's 16-value runs in one f16 instruction.  There the 16 operand words of a super-block are formed again for every 64
 // tokens and the activation passes through registers on its way to LDS; here once for up to 128.
-// Bound: instruction issue and LDS reads, which add up: a super-block and 16 x 16 cells take nine and a half matrix instructions, 16 vector ones and 4.6 KB of LDS (a read costs
-// the matrix unit about ten cycles of its register ports).  The products of the scales, eight vector instructions before, come from the matrix unit (chain below); with the
-// scales unpacked in fewer steps 14336 x 4096 at 64 / 200 / 512 tokens 20.1 -> 19.4, 38.8 -> 37.8, 80.0 -> 77.3.
-// us per launch, before -> after: 14336 x 4096 at 64 / 200 / 512 tokens 19.3 -> 17.8, 54 -> 36, 98 -> 76 (790 TOP/s); 4096 x 14336 at 200 / 512
+// Bound: instruction issue and LDS reads, which add up: a super-block and 16 x 16 cells take nine and a half matrix instructions, 16 vector ones and 4.6 KB of LDS.  The products of
+// the scales, eight vector instructions before, come from the matrix unit (chain below).
+// us per launch: 14336 x 4096 at 64 / 200 / 512 tokens, narrow kernel -> this one -> with the products of the scales from the matrix unit and fewer steps to unpack them (the last two with
+// other weights between two launches on one) 19.3 -> 20.1 -> 19.4, 54 -> 38.8 -> 37.8, 98 -> 80.0 -> 77.3 (778 TOP/s); 4096 x 14336 at 200 / 512, narrow -> this one on a weight that the caches hold
 // 88 -> 49, 185 -> 82; a layer of 8 experts of 4096 / 14336, top-2, at 48 / 128 tokens 217 -> 190, 340 -> 256.
 #include "gemm_wide.hpp"
 
