@@ -526,21 +526,21 @@ bool b32_wide_ragged(const cml_weight *w) {
 }
 
 // Whether a batch on such rows is ahead here of the packed dot, which makes one pass over the weight for 4 or 8 tokens, two or three for 3 and 5 to 7.  Time here over there at
-// 3 / 4 / 5 / 8 tokens, 50 weights of cold memory in either format: from 768 row tiles 0.57 - 0.89 / 0.81 - 1.28 (Q4_0 from 2000 tiles 0.61 - 1.02) / 0.44 - 0.80 / 0.31 - 0.81; from 257 tiles
-// at 5 / 6 Q8_0 0.61 - 0.92 / 0.60 - 0.88, Q4_0 0.63 - 1.08 / 0.59 - 1.01; up to 256 tiles at 5 / 7 / 8 / 9 on rows of up to four slabs 0.74 - 0.85 / 0.51 - 0.60 / 0.85 - 1.00 / 0.52 - 0.65, of longer
-// ones 1.01 - 1.41 / 0.71 - 1.00 / 0.96 - 1.16 / 0.75 - 0.85.  Rows of 24 to 31 blocks are two nearly full steps of the packed dot's 16 lanes: at 5 / 8 tokens 0.98 - 1.05 / 1.24 - 1.30 up to
-// 256 tiles, at 8 1.06 and 1.11 at 512.
+// 3 / 4 / 5 / 8 tokens on 640 weights of cold memory (980 pairs): from 768 row tiles 0.53 - 0.90 / 0.60 - 1.27 (from 2000 tiles 0.66 - 1.02) / 0.42 - 0.73 / 0.31 - 0.92; from 257
+// at 5 / 8 Q8_0 0.63 - 0.95 / 0.54 - 0.97, Q4_0 up to 512 tiles on rows of five slabs and more 0.93 - 1.15 / 0.79 - 0.97, else 0.66 - 0.90 / 0.58 - 0.97; up to 256 tiles at
+// 5 / 7 / 8 / 9 on rows of up to four slabs 0.77 - 0.86 / 0.56 - 0.57 / 0.81 - 1.06 / 0.69, of longer ones 0.89 - 1.43 / 0.66 - 0.95 / 0.86 - 1.15 / 0.73 - 0.87.  Rows of 24 to 31
+// blocks are two nearly full steps of the packed dot's 16 lanes: at 5 / 8 tokens 0.94 - 1.01 / 1.17 - 1.25 up to 256 tiles, at 8 1.06 - 1.10 up to 512.
 bool b32_wide_ragged_pays(const cml_weight *w, int64_t n) {
     const int forced = env_int("CAMELID_HIP_B32_MFMA_MIN_TOKENS", 0);
     if (!b32_wide_ragged(w) || env_int("CAMELID_HIP_MFMA_WIDE", 1) == 0) return false;
     if (forced > 0) return n >= forced;
     const int64_t tiles = (w->rows + 15) / 16, slabs = w->nb / 8;
     if (n == 3) return tiles >= 768;
-    if (n == 4) return w->fmt == CML_Q4_0 && tiles >= 2000;
+    if (n == 4) return tiles >= 2000;
     if (n >= 9 || n < 3) return n >= 9;
-    if (tiles <= 256) return slabs <= 4 && n < 8 && (n > 5 || slabs != 3);
-    if (n == 8 && tiles <= 512 && slabs <= 3) return false;
-    return n > 5 || w->fmt == CML_Q8_0 || tiles >= 768;
+    if (slabs == 3 && tiles <= 512 && (n == 8 || (n == 5 && tiles <= 256))) return false;
+    if (tiles <= 256) return slabs <= 4;
+    return n > 5 || w->fmt == CML_Q8_0 || tiles > 512 || slabs <= 4;
 }
 
 // Whether the offsets of a grouped call's activation rows fit 32 bits and its weight and scales can be read 16 bytes at a time.
