@@ -421,9 +421,10 @@ static int launch_b32_wide_as(const B32WideArgs &ka, int slots, hipStream_t st) 
 }
 
 // Past the caches (wide_reads_once): weights of expert groups, weights of a plain call of up to 16 tokens (128256 x 3072 at 16 tokens in Q8_0 85.3 -> 79.0 us; a
-// single wider column gains half of that and no kernel of its own).  Not rows of no whole slabs: two of them share a line of the caches, which the hint has fetched
-// twice (plain / so, weights that no cache holds, 8 tokens: Q8_0 32000 x 4128 42.3 / 45.2, 100000 x 2912 82.5 / 86.4; Q4_0 128256 x 3104 68.5 / 77.9, 65536 x 4128 59.6 / 66.6;
-// 128 experts 2816 / 704 at 64 tokens, gate and up by the hint, down both ways: 131.0 / 136.4).
+// single wider column gains half of that and no kernel of its own).  Not rows of no whole slabs whose 128-byte lines hold a piece of the next row too, which the hint has
+// fetched twice: any in Q4_0, in Q8_0 those of other than a multiple of four blocks (plain / so, weights that no cache holds, 8 tokens: Q8_0 32000 x 4128 42.3 / 45.2, 100000 x 2912
+// 82.5 / 86.4; Q4_0 128256 x 3104 68.5 / 77.9, 65536 x 4128 59.6 / 66.6; 128 experts 2816 / 704 at 64 tokens, gate and up by the hint, down both ways: 131.0 / 136.4; but Q8_0
+// 46552 x 8576 85.4 / 80.9, 84064 x 3712 71.4 / 68.0; 128 experts 1920 / 1152, Q8_0, at 64 tokens 181 / 171).
 template <int FMT, int G, int RT, int D, bool GROUPED = false>
 static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
     constexpr int kRows = kB32Waves * 16 * RT;
@@ -434,7 +435,9 @@ static int launch_b32_wide(B32WideArgs ka, int slots, hipStream_t st) {
     ka.more = groups % ka.n_cols;
     if (ka.nb % 8 != 0) {
         if constexpr (G == 4 && RT == 2) return fail(CML_ERR_UNSUPPORTED, "wide matrix-core kernel: no such shape");  // (no registers left for the ragged form)
-        else return launch_b32_wide_as<FMT, G, RT, D, GROUPED, false, true>(ka, slots, st);
+        if constexpr (FMT == CML_Q8_0 && (GROUPED || G == 1))
+            if (ka.once && ka.n_cols == 1 && ka.nb % 4 == 0) return launch_b32_wide_as<FMT, G, RT, D, GROUPED, true, true>(ka, slots, st);
+        if constexpr (G < 4 || RT < 2) return launch_b32_wide_as<FMT, G, RT, D, GROUPED, false, true>(ka, slots, st);
     }
     if constexpr (GROUPED || G == 1)
         if (ka.once && ka.n_cols == 1) return launch_b32_wide_as<FMT, G, RT, D, GROUPED, true, false>(ka, slots, st);
