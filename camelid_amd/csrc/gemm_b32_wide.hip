@@ -461,7 +461,8 @@ static int b32_wide_resident(int fmt, bool ragged, const B32WideShape &s) {
 // alone on its SIMD stalls where others overlap (1.9, not 1, times that).  A second slab ahead shortens the latency of workgroups that have a compute unit of their own (8 tokens,
 // one slab ahead / two: 4096 x 4096 Q8_0 17.8 / 13.5 us; 14336 x 5120 27.4 / 19.2) for a longer start, on rows of no whole slabs nearly twice as long (736 x 704 at 200 tokens
 // 5.0 / 6.5).  Workgroups fill an XCD's 32 compute units row block by row block (wide_block), and the compute unit that holds the most of them is the last.  The shape with the
-// lowest estimate is on average 0.7 % slower than the fastest, 17 % at worst.
+// lowest estimate is on average 0.7 % slower than the fastest, 17 % at worst; on 1000 other weights (5200 pairs) 0.6 % and 16 % (the estimate before, which took the residence of
+// whole slabs for rows of none, 1.4 % and 49 %; calls moved either way: Q4_0 105120 x 608 at 8 tokens 16.3 -> 18.3, 139360 x 1728 at 8 50.1 -> 39.8).
 static float b32_wide_cost(int fmt, bool ragged, int rows, int groups, int n_slabs, const B32WideShape &s) {
     const int64_t blocks = (rows + s.rt * 64 - 1) / (s.rt * 64), per_xcd = (blocks + 7) / 8 * ((groups + s.g - 1) / s.g);
     const int resident = b32_wide_resident(fmt, ragged, s);
@@ -529,19 +530,21 @@ bool b32_wide_ragged(const cml_weight *w) {
 }
 
 // Whether a batch on such rows is ahead here of the packed dot, which makes one pass over the weight for 4 or 8 tokens, two or three for 3 and 5 to 7.  Time here over there at
-// 3 / 4 / 5 / 8 tokens on 640 weights of cold memory (980 pairs): from 768 row tiles 0.53 - 0.90 / 0.60 - 1.27 (from 2000 tiles 0.66 - 1.02) / 0.42 - 0.73 / 0.31 - 0.92; from 257
-// at 5 / 8 Q8_0 0.63 - 0.95 / 0.54 - 0.97, Q4_0 up to 512 tiles on rows of five slabs and more 0.93 - 1.15 / 0.79 - 0.97, else 0.66 - 0.90 / 0.58 - 0.97; up to 256 tiles at
-// 5 / 7 / 8 / 9 on rows of up to four slabs 0.77 - 0.86 / 0.56 - 0.57 / 0.81 - 1.06 / 0.69, of longer ones 0.89 - 1.43 / 0.66 - 0.95 / 0.86 - 1.15 / 0.73 - 0.87.  Rows of 24 to 31
-// blocks are two nearly full steps of the packed dot's 16 lanes: at 5 / 8 tokens 0.94 - 1.01 / 1.17 - 1.25 up to 256 tiles, at 8 1.06 - 1.10 up to 512.
+// 3 / 4 / 5 / 8 tokens on 560 weights, more than 600 MB of others between two launches on one (1500 pairs): from 768 row tiles 0.53 - 0.91 / 0.64 - 1.27 (from 1500 tiles
+// 0.64 - 1.17, 0.86 on average) / 0.42 - 0.76 / 0.32 - 0.91; from 257 tiles at 5 / 8 on rows of more than 31 blocks Q8_0 0.59 - 1.02 / 0.51 - 0.97, Q4_0 0.67 - 0.87 / 0.56 - 0.81, but up to
+// 512 tiles on rows of five slabs and more 0.81 - 1.15 / 0.62 - 1.00; up to 256 tiles at 5 / 7 / 8 / 9 on rows of four slabs and a part 0.82 - 0.87 / 0.6 / 0.89 - 0.93 / 0.7, of
+// longer ones 0.87 - 1.43 / 0.63 - 0.96 / 0.86 - 1.21 / 0.73 - 0.88.  Rows of up to 31 blocks at 8 up to 256 tiles 1.08 - 1.32, up to 512 0.99 - 1.14; of 24 to 31, two nearly full
+// steps of the packed dot's 16 lanes, at 5 up to 256 tiles 0.97 - 1.03, of fewer 0.86 - 0.97.
 bool b32_wide_ragged_pays(const cml_weight *w, int64_t n) {
     const int forced = env_int("CAMELID_HIP_B32_MFMA_MIN_TOKENS", 0);
     if (!b32_wide_ragged(w) || env_int("CAMELID_HIP_MFMA_WIDE", 1) == 0) return false;
     if (forced > 0) return n >= forced;
     const int64_t tiles = (w->rows + 15) / 16, slabs = w->nb / 8;
     if (n == 3) return tiles >= 768;
-    if (n == 4) return tiles >= 2000;
+    if (n == 4) return tiles >= 1500;
     if (n >= 9 || n < 3) return n >= 9;
-    if (slabs == 3 && tiles <= 512 && (n == 8 || (n == 5 && tiles <= 256))) return false;
+    if (n == 8 && slabs <= 3 && tiles <= 512) return false;
+    if (n == 5 && slabs == 3 && tiles <= 256) return false;
     if (tiles <= 256) return slabs <= 4;
     return n > 5 || w->fmt == CML_Q8_0 || tiles > 512 || slabs <= 4;
 }

@@ -431,17 +431,17 @@ ROUTES = [
     ("Q8_0", 736, 704, 200, r"^q8_0\.mfma\.wide\.g1r1d1\.ragged$"),  # rows of two slabs and a part are over before a second slab ahead pays
     ("Q8_0", 736, 1056, 200, r"^q8_0\.mfma\.wide\.g1r1d2\.ragged$"),
     ("Q8_0", 14336, 1056, 4, r"^q8_0\.dot\."),  # four tokens are one pass of the packed dot
-    ("Q4_0", 31900, 800, 4, r"^q4_0\.dot\."),
-    ("Q4_0", 32000, 800, 4, r"^q4_0\.mfma\.wide\..*ragged$"),  # more than 1999 tiles
+    ("Q4_0", 23984, 800, 4, r"^q4_0\.dot\."),
+    ("Q4_0", 24000, 800, 4, r"^q4_0\.mfma\.wide\..*ragged$"),  # more than 1499 tiles
     ("Q8_0", 1024, 928, 5, r"^q8_0\.dot\."),  # rows of 24 to 31 blocks
     ("Q8_0", 1024, 928, 6, r"^q8_0\.mfma\.wide\..*ragged$"),
-    ("Q8_0", 768, 1152, 8, r"^q8_0\.mfma\.wide\..*ragged$"),  # eight on rows of up to four slabs and a part
+    ("Q8_0", 768, 1152, 8, r"^q8_0\.mfma\.wide\..*ragged$"),  # eight on rows of four slabs and a part
     ("Q4_0", 992, 1248, 8, r"^q4_0\.mfma\.wide\..*ragged$"),
-    ("Q8_0", 4624, 544, 8, r"^q8_0\.mfma\.wide\..*ragged$"),
-    ("Q4_0", 4096, 832, 8, r"^q4_0\.dot\."),  # but of 24 to 31 blocks
+    ("Q8_0", 4096, 544, 8, r"^q8_0\.dot\."),  # but of up to 31 blocks
+    ("Q4_0", 4096, 832, 8, r"^q4_0\.dot\."),
     ("Q4_0", 8192, 832, 8, r"^q4_0\.dot\."),
     ("Q4_0", 8208, 832, 8, r"^q4_0\.mfma\.wide\..*ragged$"),  # more than 512 tiles
-    ("Q8_0", 32000, 800, 4, r"^q8_0\.mfma\.wide\..*ragged$"),  # four tokens on more than 1999 tiles, as in Q4_0
+    ("Q8_0", 24000, 800, 4, r"^q8_0\.mfma\.wide\..*ragged$"),
     ("Q4_0", 8208, 2912, 5, r"^q4_0\.mfma\.wide\..*ragged$"),  # five on more than 512
     ("Q4_0", 8192, 1056, 5, r"^q4_0\.mfma\.wide\..*ragged$"),  # on less with short rows
 ]
