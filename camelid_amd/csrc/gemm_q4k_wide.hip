@@ -5,7 +5,7 @@
 // operand (S = lo + 8 hi, two contractions over the whole super-block), the mins against the sums of the
 // activation's 16-value runs in one f16 instruction.  There the 16 operand words of a super-block are formed again for every 64
 // tokens and the activation passes through registers on its way to LDS; here once for up to 128.
-// Bound: instruction issue and LDS reads, which add up: a super-block and 16 x 16 cells take nine and a half matrix instructions, 16 vector ones and 4.6 KB of LDS.  The products of
+// Bound: matrix and vector instructions, which add up to nine tenths of the busy cycles, and LDS reads, a few cycles of the matrix unit each: a super-block and 16 x 16 cells take nine and a half matrix instructions, 16 vector ones and 4.6 KB of LDS.  The products of
 // the scales, eight vector instructions before, come from the matrix unit (chain below).
 // us per launch: 14336 x 4096 at 64 / 200 / 512 tokens, narrow kernel -> this one -> with the products of the scales from the matrix unit and fewer steps to unpack them (the last two with
 // other weights between two launches on one) 19.3 -> 20.1 -> 19.4, 54 -> 38.8 -> 37.8, 98 -> 80.0 -> 77.3 (778 TOP/s); 4096 x 14336 at 200 / 512, narrow -> this one on a weight that the caches hold

@@ -274,7 +274,7 @@ int cml_gemv(const cml_weight *w, const int8_t *q_dev, const float *scales_dev, 
  * packed-dot kernel (up to 8 per pass over the weight), larger batches on the
  * int8 matrix cores (all four formats; Q8_0 / Q4_0 rows of fewer than 256 values
  * stay on the packed-dot kernel, and longer ones that are no whole multiple of
- * 256 leave it at larger batches than the others).  Every cell equals the
+ * 256 leave it at batch sizes of their own).  Every cell equals the
  * cml_gemv result for that token bit for bit. */
 int cml_gemm(const cml_weight *w, const int8_t *q_dev, const float *scales_dev, int64_t n_tokens,
              float *out_dev, cml_stream_t stream);
