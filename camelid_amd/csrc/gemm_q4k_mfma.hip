@@ -1100,6 +1100,8 @@ static int launch_mfma(const Q4KMfmaArgs &ka, int n_groups, hipStream_t st) {
 //     19.4 / 21.3 -- unless more than a third of a part is added to fill this kernel's steps of four super-blocks (parts of five: 2048 x 5120 at 80 1.07 times the wide kernel's time);
 //   cut two ways: parts of four super-blocks up to two workgroups per unit: 2048 x 2048 at 48 / 128 6.1 / 6.2, 6.3 / 6.9; longer ones as above: 2048 x 3072 at 80 8.2 / 8.4.
 // A third workgroup per unit loses: 3072 x 8192 at 80 tokens 23.6 / 17.5, 3072 x 2048 8.4 / 7.0.
+// (With the wide kernel 1 to 4 % faster than when these were taken the line still holds for all of 276 pairs of 70 weights but five, where the other kernel is 6 to 10 % ahead:
+// 3136 x 5632 at 38 to 63 tokens the wide one, 1656 x 14080 at 123 this one.)
 static bool mfma_ksplit_beats_wide(int64_t tiles, int64_t n_tokens, int n_sb, int ksplit) {
     if ((ksplit != 2 && ksplit != 4) || n_sb > 512) return false;  // (longer rows do not fit this kernel's LDS)
     const int64_t workgroups = tiles * ((n_tokens + 31) / 32), wide_workgroups = (tiles + 1) / 2 * ((n_tokens + 15) / 16);

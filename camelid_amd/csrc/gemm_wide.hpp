@@ -433,8 +433,9 @@ struct WideShape {
 // Estimated us of a launch (less a constant), fitted on MI355X to every shape of the kernel on cold weights (more than the last-level cache holds between
 // two launches on one) of 256 to 65536 rows and 512 to 14336 values with the three K cuts: Q6_K 1669 pairs of weight and tokens (5 to 512), Q4_K 1397 (33 to
 // 512).  The shape with the lowest estimate was on average 0.8 % / 0.7 % slower than the fastest (an earlier fit to few weights, some of them cached, took Q4_K
-// 4.3 % off).  Q4_K has since become 1 to 4 % faster in the cells and the unpacking; with the constants as they are 121 pairs of other Q4_K weights are 1.2 % off (36 % at worst: 33970 x 4864
-// at 33 tokens 50 us, four waves on three token groups 37), 107 of Q6_K, which the change left alone, 3.7 % (28904 x 5632 at 33 49.5, 39.7).  A step costs a fixed latency, more for two wave groups; for every wave on a SIMD the unpacking of a super-block and the cells of its token groups;
+// 4.3 % off).  Q4_K has since become 1 to 4 % faster in the cells and the unpacking; with the constants as they are 276 pairs of 70 other weights, equally cold, are 1.1 % off in Q4_K (29 %
+// at worst: 37336 x 1024 at 36 tokens 16.2 us, four waves on three token groups 12.6) and 279 of 70 in Q6_K, which the change left alone, 1.7 % (19 %: 42952 x 2816 at 40 38.4, 32.4).
+// A step costs a fixed latency, more for two wave groups; for every wave on a SIMD the unpacking of a super-block and the cells of its token groups;
 // and per token group the activation slabs that the compute unit's workgroups fetch (from three on they share what the cache holds).  Workgroups fill an XCD's 32
 // compute units row block by row block (wide_block).  `rounds`: workgroups over what is resident at once, between their average and the last round at full length.
 template <class F>
